@@ -214,15 +214,16 @@ int nmr_hip_mfma_rate(int64_t iters, int32_t reps, double* tflops);
 int nmr_hip_last_run_ms(nmr_ctx* ctx, double* ms, int64_t* sweeps);
 
 /* Device layout of the sweeps (no reference counterpart): 1 (the default)
- * keeps the state, the velocity (as the per-voxel face-velocity sums the
- * sweeps read) and the per-voxel coefficients, field and phase weights in
- * bricks of 128 bytes (8 x-voxels by 4 rows of one plane)
- * -- for the one-step sweep with any one-step tile variant and for the
- * general sweep -- so that all-solid bricks are never fetched.  The uploads
- * convert their arrays once; the state stays in bricks from run to run
- * (pulses rotate it there) and is converted back only for a download or a
- * learned solve.  0 always sweeps the row layout.  The fields are the same
- * bits either way. */
+ * keeps the state, the velocity (as per-voxel face-velocity sums) and the
+ * per-voxel coefficients, field and phase weights where the sweeps read them
+ * best.  With the automatic tile that is a list of the pores, in the grid's
+ * order (unless most of a large grid is pores, or a mask does not fit the
+ * list's offsets); with a tile variant set, or where the list does not pay,
+ * bricks of 128 bytes (8 x-voxels by 4 rows of one plane), so that all-solid
+ * bricks are never fetched.  The uploads convert their arrays once; the state
+ * stays converted from run to run (pulses rotate it there) and is converted
+ * back only for a download or a learned solve.  0 always sweeps the row
+ * layout.  The fields are the same bits either way. */
 int nmr_hip_set_layout(nmr_ctx* ctx, int32_t brick);
 /* Tile shape of the sweep kernel: variant index (-1 = automatic, -2 = a
  * one-thread-per-voxel kernel with the arithmetic of the sweeps, a

@@ -19,7 +19,7 @@
 #include "nmr_kernels.h"
 
 namespace nmri {
-constexpr int kHomeRows = 1, kHomeBricks = 2;
+constexpr int kHomeRows = 1, kHomeBricks = 2, kHomePores = 4;
 // Record a status detail for nmr_hip_last_error() and return code.
 int fail(int code, const char* fmt, ...);
 inline int round_up4(int n) { return (n + 3) & ~3; }
@@ -41,6 +41,49 @@ inline size_t biggest_array_bytes(int nx, int ny, int nz)
             return nmri::fail(e_ == hipErrorOutOfMemory ? NMR_ERR_NOMEM : NMR_ERR_DEVICE, "%s: %s (%s:%d)", \
                               #expr, hipGetErrorString(e_), __FILE__, __LINE__);               \
     } while (0)
+
+namespace nmri {
+
+// A list of the pores of one domain or of all instances of a batch
+// (nmr_pores.hip), its state and its per-slot data, in device memory.
+struct PoreList {
+    uint32_t nslots = 0;  // slots in use, the empty group 0 among them
+    size_t cap = 0;       // slots allocated
+    int nc = 0;
+    nmr::PoreGroup* groups = nullptr;
+    nmr::PoreGhost* ghost = nullptr;
+    uint2* off = nullptr;
+    uint32_t* xoff = nullptr;
+    uint32_t *vox = nullptr, *xy = nullptr;
+    float* state[2] = {nullptr, nullptr};
+    float* pred = nullptr;
+    float* vel = nullptr;
+    float* pv[6] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr}; // dn, r1v, r2v, bn, w[0], w[1]
+    int ngroups() const { return (int)(nslots / 64); }
+};
+// What of the list a problem needs beside the state.
+struct PoreNeeds {
+    int nc;
+    bool vel, ghosts, xoff, pred;
+};
+// Buffers for `nslots` slots, grown where they are too small or missing;
+// everything in them is cleared (the voxel numbers set to "empty").  The
+// per-voxel arrays pv are made by who gathers them; they go when the list grows.
+int pores_alloc(PoreList* L, uint32_t nslots, const PoreNeeds& n, hipStream_t s, int64_t* bytes);
+void pores_free(PoreList* L);
+// Slots of one domain (b.first is set, b's temporary arrays are made here):
+// counts them and gives the slot past the last one in *end (waits for the
+// stream).  pores_link then assigns and links them in the list's arrays
+// (waits too) and releases the temporary arrays; *ok: every offset fits.
+int pores_count(nmr::PoreBuild* b, hipStream_t s, uint64_t* end);
+int pores_link(const PoreList& L, nmr::PoreBuild* b, uint64_t end, hipStream_t s, bool* ok);
+void pores_drop_temp(nmr::PoreBuild* b);
+// Workgroups of a sweep over `groups` groups and the groups of each.
+void pores_tiles(int groups, int* gpt, int* ntiles);
+// Whether a list of this many slots stays inside the kernels' 32-bit byte offsets.
+bool pores_fit(uint64_t nslots);
+
+} // namespace nmri
 
 struct nmr_ctx {
     nmr_problem prob{};
@@ -89,6 +132,18 @@ struct nmr_ctx {
     // only home of the state.
     int home = 1;
     int bpar = 0;
+    // The list of the pores, the automatic choice of the sweeps while the
+    // layout switch is on: state[ppar] is the current state when home says
+    // so.  Built by the uploads; pl_tried says that the list was built, or
+    // found not to fit, for the current mask and velocity.
+    nmri::PoreList pl;
+    bool pl_tried = false, pl_ok = false;
+    bool pl_vel_ok = false, pl_pv_ok = false; // velocity sums and per-voxel arrays gathered
+    bool pl_zeroed = false;   // a MacCormack step ran on the list: solids hold 0
+    int ppar = 0;
+    // every solid's magnetization is finite (else the tile sweeps, which
+    // multiply it by a zero weight, decide what comes out)
+    bool solids_tried = false, solids_ok = false;
     // signal of the current state: host copy of the last row of the last run
     // (or of the last nmr_hip_signal); cleared when the state changes otherwise
     bool sig_valid = false;

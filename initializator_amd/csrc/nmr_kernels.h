@@ -174,6 +174,88 @@ struct FieldSumArgs {
     int nby, nb8;           // brick layout of f (0: rows)
 };
 
+// ---- list of pores (nmr_pores.hip) ----
+// 64 slots of the list, in the grid's order and of one plane: the lowest slot
+// of its neighbours per side (x-, x+, y-, y+, z-, z+), which the 16-bit z
+// offsets count from, and 64-bit lane masks.
+struct PoreGroup {
+    int32_t base[6];
+    float zc;               // plane + 1/2
+    int32_t inst;           // instance of a batch
+    uint64_t pore[6];       // the neighbour on this side counts as a pore
+    uint64_t active;        // the slot holds a pore (else a solid that pores read, or nothing)
+    uint64_t window;        // a pore inside the signal window
+    uint64_t xm, xp;        // the x neighbour is the slot before / after (else the own value is read)
+    uint64_t zm, zp;        // a z neighbour is read (else the own value)
+};
+static_assert(sizeof(PoreGroup) == 128, "group descriptor");
+
+// Lanes whose neighbour on a side is a ghost (only with ghosts other than
+// zero-derivative ones).
+struct PoreGhost {
+    uint64_t side[6];
+};
+
+struct PoreArgs {
+    const float* f;         // field the stage differentiates, nc floats per slot
+    const float* mavg;      // corrector stage: the state at the start of the step
+    float* out;
+    const PoreGroup* groups;
+    const PoreGhost* ghost; // or null
+    const uint2* off;       // 16-bit y-, y+ (distances) and z-, z+ (from the group's bases)
+    const uint32_t* xoff;   // of x-, x+ where they are not the slots next to it; or null
+    const uint32_t* xy;     // x | y << 16 (three components)
+    const float* vel;       // 3 velocity sums per slot (upwind or centred)
+    const float* dn;        // per-voxel diffusivity / reference, dt/T1, dt/T2, field: or null
+    const float* r1v;
+    const float* r2v;
+    const float* bn;
+    const float* w[2];      // phase weights, or null
+    double* partials;       // [ntiles][sums] of this step
+    int ngroups;            // one past the last group (group 0 is empty)
+    int gpt, ntiles;        // groups per workgroup, workgroups
+    int bnax, amask;
+    Coef c;
+};
+
+// Building the list of one domain; slots [first, ...), whole groups.
+struct PoreBuild {
+    const uint8_t* mask;
+    int nx, ny, nz, pitch;
+    int bc[3];
+    int read_solids;        // upwind velocity on pore-solid faces: solids next to pores get slots
+    int w[6];               // signal window
+    uint64_t first;         // first slot (a multiple of 64)
+    int64_t count;          // groups of this domain (linking)
+    uint32_t* rows;         // [nz*ny] slots before the row in its plane
+    uint64_t* planes;       // [nz + 1] first slot of each plane
+    uint32_t* slotmap;      // [nz][ny][pitch] slot of a voxel, 0: none
+    uint32_t* vox;          // voxel (row layout) of a slot, ~0: empty
+    PoreGroup* groups;
+    PoreGhost* ghost;       // or null
+    uint2* off;
+    uint32_t* xoff;         // or null
+    uint32_t* xy;           // or null
+    int* overflow;          // set when an offset does not fit
+};
+
+hipError_t launch_pore_count(const PoreBuild& b, hipStream_t s);
+hipError_t launch_pore_link(const PoreBuild& b, hipStream_t s);
+// out[stride*slot + at] = row[vox[slot]] for slots [s0, s1), 0 at empty ones
+hipError_t launch_pore_gather(const float* row, const uint32_t* vox, uint32_t s0, uint32_t s1, int stride, int at,
+                              float* out, hipStream_t s);
+// row[vox[slot]] (and row2, unless null) = f[stride*slot + at]
+hipError_t launch_pore_scatter(const float* f, const uint32_t* vox, uint32_t s0, uint32_t s1, int stride, int at,
+                               float* row, float* row2, hipStream_t s);
+// *flag = 1 when row is not finite at a solid
+hipError_t launch_solids_finite(const float* row, const uint8_t* mask, size_t n, int* flag, hipStream_t s);
+hipError_t launch_pore_sum(int nc, const PoreArgs& a, hipStream_t s);
+// a step (stage st) of the whole list; gen: anything but the plain problem
+// (per-voxel data, ghosts other than zero-derivative ones, masked advection)
+hipError_t launch_pores(int nc, bool vel, int st, bool exact, bool gen, bool coef, const PoreArgs& a, hipStream_t s);
+hipError_t launch_pore_pulse(const PulseArgs& a, float* f, int nc, const uint32_t* vox, uint32_t s0, uint32_t s1,
+                             hipStream_t s);
+
 // ---- learned corrector (nmr_learn_kernels.hip) ----
 // Tensors: BF16 channels-last on the grid padded by one zero voxel per side.
 constexpr int kWgradPart = 27 * 256 + 16; // floats per wavefront partial of wgrad

@@ -38,6 +38,7 @@
 
 #include <algorithm>
 
+#include "nmr_device.h"
 #include "nmr_kernels.h"
 
 
@@ -84,18 +85,6 @@ __device__ __forceinline__ void st4_state(float* base, uint32_t boff, f4 v)
     else st4_nt(base, boff, v);
 }
 
-// Harmonic mean 2ab/(a + b) of two (scaled) diffusivities for the face
-// between them, with the hardware reciprocal (v_rcp_f32, about 1 ulp) in
-// place of an IEEE division.  Sums below 1e-30 -- solids, which the
-// reference gives D = 1e-50 -- give 0: their reciprocal would overflow, and
-// the exact mean is below 1e-30 there anyway.  Both general kernels use it,
-// so they stay bit-identical.
-__device__ __forceinline__ float hmean(float a, float b)
-{
-    const float s = a + b;
-    return s > 1e-30f ? (2.f * a * b) * __builtin_amdgcn_rcpf(s) : 0.f;
-}
-
 // Float offset of voxel (x, y, z) of a field in bricks of 8 x-voxels by 4
 // rows (brick (z, y/4, x/8); nby brick rows per plane, nb8 bricks per brick
 // row), the layout brick_kernel converts to.
@@ -107,15 +96,6 @@ __device__ __forceinline__ size_t brick_off(int x, int y, int z, int nby, int nb
 
 // byte e (0/1) of a packed mask word as a float
 __device__ __forceinline__ float ub(uint32_t w, int e) { return (float)((w >> (8 * e)) & 0xffu); }
-
-// Block index -> tile index such that XCD x (blocks x, x+8, x+16, ...) gets
-// the contiguous tile range [x*q + min(x,r), ...), q = nb/8, r = nb%8.
-__device__ __forceinline__ int xcd_tile(int b, int nb)
-{
-    const int xcd = b & 7, ib = b >> 3;
-    const int q = nb >> 3, r = nb & 7;
-    return xcd * q + (xcd < r ? xcd : r) + ib;
-}
 
 // Replace the elements of a chunk that lie beyond the domain end (index >
 // last) by element `last`: the zero-derivative ghost value.
@@ -1574,12 +1554,7 @@ hipError_t launch_adv(const AdvArgs& a, hipStream_t s)
     return hipGetLastError();
 }
 
-// Instantaneous RF / gradient pulse: every pore voxel's M is rotated by an
-// angle about an axis, as AddImpulse + OrtTransform do it
-// (src/NmrRelaxationSolve.cpp:2536-2608).  Angles and the rotation are
-// evaluated in FP64 in the reference's order of operations; the state stays
-// FP32.  Reference index i maps to x + 1 here (no ghost layer: ghost cells
-// are refilled from the interior after every pulse in the reference anyway).
+// A pulse on the row or brick layout, one voxel per thread.
 __global__ void __launch_bounds__(256) pulse_kernel(PulseArgs a)
 {
     const int x = blockIdx.x * 256 + threadIdx.x;
@@ -1588,37 +1563,7 @@ __global__ void __launch_bounds__(256) pulse_kernel(PulseArgs a)
     const size_t o = ((size_t)z * a.ny + y) * a.pitch + x;
     if (a.mask[o] == 0) return;
     const size_t fo = a.nb8 > 0 ? brick_off(x, y, z, a.nby, a.nb8) : o; // state offset
-    double len = sqrt(a.ax * a.ax + a.ay * a.ay + a.az * a.az);
-    if (len == 0.0) len = 1.0;
-    const double n0x = a.ax / len, n0y = a.ay / len, n0z = a.az / len;
-    const double i = (double)(x + 1), j = (double)(y + 1), k = (double)(z + 1);
-    double angle, rx, ry, rz;
-    if (a.flag == 1) { // narrow gradient pulse, axis = unit gradient direction
-        angle = a.param * a.gamma * ((i - 1) * a.dx * a.ax + (j - 1) * a.dy * a.ay + (k - 1) * a.dz * a.az);
-        rx = n0x; ry = n0y; rz = n0z;
-    } else if (a.flag == 2) { // RF pulse of angle param about the (unnormalised) axis
-        angle = a.param;
-        rx = a.ax; ry = a.ay; rz = a.az;
-    } else if (a.flag == 3) { // multi-gradient pulse about a far-away origin
-        const double distance = 10e+12;
-        const double eff = sqrt(a.ax * a.ax + a.ay * a.ay + a.az * a.az);
-        const double t = (i - 1.0 - distance) * a.dx * n0x + (j - 1.0 - distance) * a.dy * n0y +
-                         (k - 1.0 - distance) * a.dz * n0z;
-        angle = a.gamma * eff * sqrt(t * t);
-        rx = n0x; ry = n0y; rz = n0z;
-    } else { // flag 4: radial phase about the domain centre
-        const double tx = (i - 0.5) * a.dx * a.ax - 0.5 * a.nx * a.dx * a.ax;
-        const double ty = (j - 0.5) * a.dy * a.ay - 0.5 * a.ny * a.dy * a.ay;
-        const double tz = (k - 0.5) * a.dz * a.az - 0.5 * a.nz * a.dz * a.az;
-        angle = 0.0 - a.gamma * sqrt(tx * tx + ty * ty + tz * tz);
-        rx = a.ax; ry = a.ay; rz = a.az;
-    }
-    const double c = cos(angle), s = sin(angle);
-    const double vx = a.m[0][fo], vy = a.m[1][fo], vz = a.nc == 3 ? (double)a.m[2][fo] : 0.0;
-    const double scal = rx * vx + ry * vy + rz * vz;
-    a.m[0][fo] = (float)(vx * c + rx * (1.0 - c) * scal + s * (ry * vz - rz * vy));
-    a.m[1][fo] = (float)(vy * c + ry * (1.0 - c) * scal + s * (rz * vx - rx * vz));
-    if (a.nc == 3) a.m[2][fo] = (float)(vz * c + rz * (1.0 - c) * scal + s * (rx * vy - ry * vx));
+    pulse_voxel(a, x, y, z, a.m[0] + fo, a.m[1] + fo, a.nc == 3 ? a.m[2] + fo : nullptr);
 }
 
 hipError_t launch_pulse(const PulseArgs& a, hipStream_t s)

@@ -1,0 +1,157 @@
+// nmr_pore_list.hip -- host side of the pore list (nmr_pores.hip): its
+// buffers, and building it from a mask on the device.
+#include "nmr_internal.h"
+
+using nmri::fail;
+
+namespace nmri {
+
+namespace {
+
+template <typename T>
+int grow(T** p, size_t count, int fill, hipStream_t s, int64_t* bytes, size_t old_count)
+{
+    const size_t n = std::max<size_t>(count * sizeof(T), 256);
+    if (*p) {
+        HIP_TRY(hipStreamSynchronize(s));
+        HIP_TRY(hipFree(*p));
+        *p = nullptr;
+        *bytes -= (int64_t)std::max<size_t>(old_count * sizeof(T), 256);
+    }
+    HIP_TRY(hipMalloc((void**)p, n));
+    *bytes += (int64_t)n;
+    HIP_TRY(hipMemsetAsync(*p, fill, n, s));
+    return NMR_OK;
+}
+
+} // namespace
+
+bool pores_fit(uint64_t nslots)
+{
+    return nslots > 64 && (nslots + 64) * 12 < ((uint64_t)1 << 32) - 256;
+}
+
+int pores_alloc(PoreList* L, uint32_t nslots, const PoreNeeds& n, hipStream_t s, int64_t* bytes)
+{
+    const bool more = nslots > L->cap || n.nc != L->nc;
+    const size_t old = L->cap, cap = more ? (size_t)nslots : L->cap;
+    const size_t all = cap + 64, was = old + 64; // a spare group past the end: the last slot reads the one after it
+    int rc = NMR_OK;
+    auto need = [&](auto** p, size_t per, int fill) {
+        if (rc) return;
+        if (more || !*p) rc = grow(p, all * per, fill, s, bytes, was * per);
+        else if (hipMemsetAsync(*p, fill, all * per * sizeof(**p), s) != hipSuccess)
+            rc = fail(NMR_ERR_DEVICE, "pore list: clearing a buffer failed");
+    };
+    auto groups = [&](auto** p) {
+        if (rc) return;
+        if (more || !*p) rc = grow(p, all / 64, 0, s, bytes, was / 64);
+        else if (hipMemsetAsync(*p, 0, all / 64 * sizeof(**p), s) != hipSuccess)
+            rc = fail(NMR_ERR_DEVICE, "pore list: clearing a buffer failed");
+    };
+    if (L->nc != n.nc) { // sizes below are in slots of nc words
+        for (float** p : {&L->state[0], &L->state[1], &L->pred})
+            if (*p) {
+                HIP_TRY(hipStreamSynchronize(s));
+                HIP_TRY(hipFree(*p));
+                *p = nullptr;
+                *bytes -= (int64_t)(was * 4 * (size_t)L->nc);
+            }
+        L->nc = n.nc;
+    }
+    groups(&L->groups);
+    if (n.ghosts || L->ghost) groups(&L->ghost);
+    need(&L->off, 1, 0xff);
+    if (n.xoff || L->xoff) need(&L->xoff, 1, 0xff);
+    need(&L->vox, 1, 0xff);
+    if (n.nc == 3 || L->xy) need(&L->xy, 1, 0);
+    need(&L->state[0], (size_t)n.nc, 0);
+    need(&L->state[1], (size_t)n.nc, 0);
+    if (n.pred || L->pred) need(&L->pred, (size_t)n.nc, 0);
+    if (n.vel || L->vel) need(&L->vel, 3, 0);
+    if (more)
+        for (float*& p : L->pv)
+            if (p && !rc) {
+                if (hipStreamSynchronize(s) != hipSuccess || hipFree(p) != hipSuccess)
+                    rc = fail(NMR_ERR_DEVICE, "pore list: freeing a buffer failed");
+                p = nullptr;
+                *bytes -= (int64_t)(was * 4);
+            }
+    if (rc) return rc;
+    L->cap = cap;
+    L->nslots = nslots;
+    return NMR_OK;
+}
+
+void pores_free(PoreList* L)
+{
+    for (void* p : {(void*)L->groups, (void*)L->ghost, (void*)L->off, (void*)L->xoff, (void*)L->vox, (void*)L->xy,
+                    (void*)L->state[0], (void*)L->state[1], (void*)L->pred, (void*)L->vel, (void*)L->pv[0],
+                    (void*)L->pv[1], (void*)L->pv[2], (void*)L->pv[3], (void*)L->pv[4], (void*)L->pv[5]})
+        if (p) (void)hipFree(p);
+    *L = PoreList{};
+}
+
+void pores_drop_temp(nmr::PoreBuild* b)
+{
+    for (void* p : {(void*)b->rows, (void*)b->planes, (void*)b->slotmap, (void*)b->overflow})
+        if (p) (void)hipFree(p);
+    b->rows = nullptr;
+    b->planes = nullptr;
+    b->slotmap = nullptr;
+    b->overflow = nullptr;
+}
+
+int pores_count(nmr::PoreBuild* b, hipStream_t s, uint64_t* end)
+{
+    const size_t rows = (size_t)b->ny * (size_t)b->nz;
+    b->rows = nullptr;
+    b->planes = nullptr;
+    b->slotmap = nullptr;
+    b->overflow = nullptr;
+    int rc = NMR_OK;
+    auto check = [&](hipError_t e) {
+        if (!rc && e != hipSuccess)
+            rc = fail(e == hipErrorOutOfMemory ? NMR_ERR_NOMEM : NMR_ERR_DEVICE, "pore list: %s", hipGetErrorString(e));
+        return !rc;
+    };
+    if (check(hipMalloc((void**)&b->rows, rows * sizeof(uint32_t))) &&
+        check(hipMalloc((void**)&b->planes, ((size_t)b->nz + 1) * sizeof(uint64_t))) &&
+        check(hipMalloc((void**)&b->slotmap, rows * (size_t)b->pitch * sizeof(uint32_t))) &&
+        check(hipMalloc((void**)&b->overflow, 256)) && check(hipMemsetAsync(b->overflow, 0, 256, s)) &&
+        check(nmr::launch_pore_count(*b, s)) &&
+        check(hipMemcpyAsync(end, b->planes + b->nz, sizeof(uint64_t), hipMemcpyDeviceToHost, s)))
+        check(hipStreamSynchronize(s));
+    if (rc) pores_drop_temp(b);
+    return rc;
+}
+
+int pores_link(const PoreList& L, nmr::PoreBuild* b, uint64_t end, hipStream_t s, bool* ok)
+{
+    b->vox = L.vox;
+    b->groups = L.groups;
+    b->ghost = L.ghost;
+    b->off = L.off;
+    b->xoff = L.xoff;
+    b->xy = L.xy;
+    b->count = (int64_t)((end - b->first) / 64);
+    int over = 0, rc = NMR_OK;
+    hipError_t e = nmr::launch_pore_link(*b, s);
+    if (e == hipSuccess) e = hipMemcpyAsync(&over, b->overflow, sizeof(int), hipMemcpyDeviceToHost, s);
+    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    if (e != hipSuccess) rc = fail(NMR_ERR_DEVICE, "pore list: %s", hipGetErrorString(e));
+    pores_drop_temp(b);
+    *ok = rc == NMR_OK && over == 0;
+    return rc;
+}
+
+void pores_tiles(int groups, int* gpt, int* ntiles)
+{
+    // two groups a wavefront: 256^3 (52 K groups) 21.0 / 20.6 / 21.5 / 24.7 / 25.4 us
+    // a step at 4 / 8 / 16 / 32 / 64 groups a workgroup; fewer than a few
+    // workgroups per CU: one (64^3, 1.2 K groups: 3.0 / 3.4 / 4.5 us at 4 / 8 / 16)
+    *gpt = groups <= 8192 ? 4 : 8;
+    *ntiles = std::max(1, (groups + *gpt - 1) / *gpt);
+}
+
+} // namespace nmri
