@@ -769,20 +769,21 @@ bool pore_plain(const nmr_ctx* c)
            !c->weighted && !((p.flags & NMR_F_ADVECT_MASK) && c->vel);
 }
 
-// Whether the list beats the tiles: where at most half of the voxels are
-// pores, or the list's data (the state's two buffers, the predictor, the
-// velocity sums, offsets and descriptors) stay well inside the memory-side
-// cache.  Measured per step, list against tiles on bricks: 256^3 flow, two
-// components, porosity 0.2 / 0.4 / 0.5 / 0.7 / 1: 20.6 / 37.6 / 70 / 99 / 142
-// against 58 / 69 / 75 / 82 / 84 us; 512x512x256, porosity 1: 555 against 391;
-// 64^3, one component, porosity 1: 4.8 against 9.4; 160^3 MacCormack, porosity
-// 1 (188 MB): 56.5 against 54.6.
+// Whether the list beats the tiles: where at most 0.6 of the voxels are pores,
+// or the list's data (the state's two buffers, the predictor, the velocity
+// sums, offsets and descriptors) stay well inside the memory-side cache.
+// Measured per step, list against tiles on bricks: 256^3 flow, two components,
+// porosity 0.2 / 0.35 / 0.5 / 0.65 / 0.8 / 1: 19.9 / 31.2 / 61.2 / 81.9 / 101 /
+// 124 against 57.9 / 66.2 / 74.1 / 80.1 / 84.0 / 84.2 us; 256^3, one component
+// without flow, 0.5 / 0.8 (188 MB) / 1: 29.3 / 41.0 / 47.8 against 36.4 / 39.0 /
+// 39.2; 160^3 MacCormack, 1 (172 MB): 47.9 against 54.1; 512x512x256, 1: 511
+// against 388; 64^3, one component, 1: 2.9 against 9.4.
 bool pores_pay(const nmr_ctx* c, uint64_t slots)
 {
     const nmr_problem& p = c->prob;
     const double vox = (double)p.nx * p.ny * p.nz;
-    const double words = (p.scheme == NMR_SCHEME_MACCORMACK ? 3 : 2) * c->nc + (c->vel ? 3 : 0) + 2.5;
-    return (double)slots <= 0.5 * vox || 4.0 * words * (double)slots <= 160e6;
+    const double words = (p.scheme == NMR_SCHEME_MACCORMACK ? 3 : 2) * c->nc + (c->vel ? 3 : 0) + 1.5;
+    return (double)slots <= 0.6 * vox || 4.0 * words * (double)slots <= 180e6;
 }
 
 // Builds the list for the current mask and velocity.
@@ -791,6 +792,7 @@ int build_pores(nmr_ctx* c)
     const nmr_problem& p = c->prob;
     c->pl_tried = true;
     c->pl_ok = c->pl_vel_ok = c->pl_pv_ok = false;
+    c->pl_reads_solids = false;
     if (c->nc == 3 && (p.nx > 65536 || p.ny > 65536)) return NMR_OK; // positions are 16 + 16 bits
     int rc = refresh_inert(c);
     if (rc) return rc;
@@ -814,12 +816,14 @@ int build_pores(nmr_ctx* c)
         nmri::pores_drop_temp(&b);
         return NMR_OK;
     }
-    const nmri::PoreNeeds n{c->nc, c->vel, ghosts, p.bc[0] != NMR_BC_NEUMANN, p.scheme == NMR_SCHEME_MACCORMACK};
+    const nmri::PoreNeeds n{c->nc, c->vel, ghosts || b.read_solids, p.bc[0] != NMR_BC_NEUMANN,
+                            p.scheme == NMR_SCHEME_MACCORMACK};
     if ((rc = nmri::pores_alloc(&c->pl, (uint32_t)end, n, c->stream, &c->device_bytes))) {
         nmri::pores_drop_temp(&b);
         return rc;
     }
-    return nmri::pores_link(c->pl, &b, end, c->stream, &c->pl_ok);
+    c->pl_reads_solids = b.read_solids != 0;
+    return nmri::pores_link(&c->pl, &b, end, c->stream, &c->pl_ok);
 }
 
 // Whether the solids' magnetization is finite: their value reaches no pore
@@ -897,8 +901,9 @@ int pore_data(nmr_ctx* c)
         const bool centred = c->prob.scheme == NMR_SCHEME_MACCORMACK;
         if ((rc = velocity_sums(c, false, centred))) return rc;
         for (int q = 0; q < 3; q++)
-            HIP_TRY(nmr::launch_pore_gather(centred ? c->csum[q] : c->adv[q], c->pl.vox, 64, c->pl.nslots, 3, q,
-                                            c->pl.vel, c->stream));
+            HIP_TRY(nmr::launch_pore_gather(centred ? c->csum[q] : c->adv[q], c->pl.vox, 64, c->pl.nslots, 4, 1 + q,
+                                            reinterpret_cast<float*>(c->pl.rec), c->stream));
+        HIP_TRY(nmr::launch_pore_record(c->pl.off8, c->pl.nslots, c->pl.rec, c->stream));
         c->pl_vel_ok = true;
     }
     if (!c->pl_pv_ok) {
@@ -918,11 +923,19 @@ int pore_args(nmr_ctx* c, nmr::PoreArgs* a)
 {
     const nmri::PoreList& L = c->pl;
     a->groups = L.groups;
-    a->ghost = L.ghost;
-    a->off = L.off;
+    bool zeros = false, ghosts = false;
+    for (int q = 0; q < 3; q++) {
+        zeros = zeros || c->prob.bc[q] == NMR_BC_DIRICHLET;
+        ghosts = ghosts || c->prob.bc[q] != NMR_BC_NEUMANN;
+    }
+    a->aux = zeros || c->pl_reads_solids ? L.aux : nullptr;
+    a->ghost = ghosts ? L.aux : nullptr;
+    a->wide = L.wide ? 1 : 0;
+    a->rec = L.rec;
+    a->off8 = L.off8;
+    a->off16 = L.off16;
     a->xoff = L.xoff;
     a->xy = L.xy;
-    a->vel = L.vel;
     a->dn = c->dn ? L.pv[0] : nullptr;
     a->r1v = c->r1v ? L.pv[1] : nullptr;
     a->r2v = c->r2v ? L.pv[2] : nullptr;
@@ -933,9 +946,18 @@ int pore_args(nmr_ctx* c, nmr::PoreArgs* a)
         a->w[1] = L.pv[5];
     }
     a->ngroups = L.ngroups();
-    nmri::pores_tiles(a->ngroups - 1, &a->gpt, &a->ntiles);
+    a->gpt = nmri::pores_per_tile(a->ngroups - 1);
+    a->ntiles = (a->ngroups - 1 + a->gpt - 1) / a->gpt;
     a->amask = (c->prob.flags & NMR_F_ADVECT_MASK) ? 1 : 0;
     return NMR_OK;
+}
+
+// Steps whose partial sums are held before a reduction: at most kChunkSteps,
+// and 32 MiB of them (256^3: 160 steps).
+int64_t pore_chunk(const nmr_ctx* c, int ntiles)
+{
+    const size_t step = (size_t)ntiles * (size_t)c->nsig() * sizeof(double);
+    return (int64_t)std::min<size_t>(kChunkSteps, std::max<size_t>(8, ((size_t)32 << 20) / std::max<size_t>(1, step)));
 }
 
 // Steps on the list: any scheme, boundary rule and per-voxel data.
@@ -943,12 +965,13 @@ int run_pores(nmr_ctx* c, int64_t nsteps, const double* grad_sched, double* sign
 {
     const nmr_problem& p = c->prob;
     const int ns = c->nsig();
-    const bool mak = p.scheme == NMR_SCHEME_MACCORMACK, gen = !pore_plain(c);
+    const bool mak = p.scheme == NMR_SCHEME_MACCORMACK, gen = !pore_plain(c) || c->pl_reads_solids;
     int rc = ensure_signal(c, (size_t)(nsteps + 1) * ns);
     if (rc || (rc = state_pores(c)) || (rc = pore_data(c))) return rc;
     nmr::PoreArgs a{};
     if ((rc = pore_args(c, &a))) return rc;
-    if ((rc = ensure_partials(c, (size_t)std::min<int64_t>(nsteps, kChunkSteps) * a.ntiles * ns))) return rc;
+    const int64_t most = pore_chunk(c, a.ntiles);
+    if ((rc = ensure_partials(c, (size_t)std::min(nsteps, most) * a.ntiles * ns))) return rc;
     const bool have0 = c->sig_valid;
     double sig0[6];
     std::copy(c->sig_now, c->sig_now + 6, sig0);
@@ -957,7 +980,7 @@ int run_pores(nmr_ctx* c, int64_t nsteps, const double* grad_sched, double* sign
     if (nsteps > 0) c->home = nmri::kHomePores;
     int64_t done = 0;
     while (done < nsteps) {
-        const int chunk = (int)std::min<int64_t>(kChunkSteps, nsteps - done);
+        const int chunk = (int)std::min(most, nsteps - done);
         for (int s = 0; s < chunk; s++) {
             double g[3] = {p.grad[0], p.grad[1], p.grad[2]};
             if (grad_sched)
@@ -977,7 +1000,7 @@ int run_pores(nmr_ctx* c, int64_t nsteps, const double* grad_sched, double* sign
             } else {
                 a.f = cin;
                 a.out = cout;
-                HIP_TRY(nmr::launch_pores(c->nc, c->vel, nmr::GEN_UPWIND, c->exact && !gen, gen, c->hetero, a, c->stream));
+                HIP_TRY(nmr::launch_pores(c->nc, c->vel, nmr::GEN_UPWIND, c->exact && pore_plain(c), gen, c->hetero, a, c->stream));
             }
             c->ppar ^= 1;
         }
@@ -1007,7 +1030,7 @@ int presize_buffers(nmr_ctx* c)
     if (pores) {
         nmr::PoreArgs a{};
         if ((rc = pore_args(c, &a))) return rc;
-        need = (size_t)kChunkSteps * a.ntiles * ns;
+        need = (size_t)pore_chunk(c, a.ntiles) * a.ntiles * ns;
     } else if (c->general) {
         if (c->variant != -2) need = (size_t)kChunkSteps * general_geometry(c, c->brick_on && bricks_fit(c)).nwg * ns;
     } else {

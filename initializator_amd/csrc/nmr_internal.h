@@ -50,21 +50,21 @@ struct PoreList {
     uint32_t nslots = 0;  // slots in use, the empty group 0 among them
     size_t cap = 0;       // slots allocated
     int nc = 0;
+    bool wide = false;    // some group needs its 16-bit offsets
     nmr::PoreGroup* groups = nullptr;
-    nmr::PoreGhost* ghost = nullptr;
-    uint2* off = nullptr;
-    uint32_t* xoff = nullptr;
-    uint32_t *vox = nullptr, *xy = nullptr;
+    nmr::PoreAux* aux = nullptr;
+    uint32_t *off8 = nullptr, *xoff = nullptr, *vox = nullptr, *xy = nullptr;
+    uint2* off16 = nullptr;
     float* state[2] = {nullptr, nullptr};
     float* pred = nullptr;
-    float* vel = nullptr;
+    uint4* rec = nullptr; // offsets and velocity sums (with velocity)
     float* pv[6] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr}; // dn, r1v, r2v, bn, w[0], w[1]
     int ngroups() const { return (int)(nslots / 64); }
 };
 // What of the list a problem needs beside the state.
 struct PoreNeeds {
     int nc;
-    bool vel, ghosts, xoff, pred;
+    bool vel, aux, xoff, pred;
 };
 // Buffers for `nslots` slots, grown where they are too small or missing;
 // everything in them is cleared (the voxel numbers set to "empty").  The
@@ -74,12 +74,13 @@ void pores_free(PoreList* L);
 // Slots of one domain (b.first is set, b's temporary arrays are made here):
 // counts them and gives the slot past the last one in *end (waits for the
 // stream).  pores_link then assigns and links them in the list's arrays
-// (waits too) and releases the temporary arrays; *ok: every offset fits.
+// (waits too), notes wide groups in the list and releases the temporary
+// arrays; *ok: every offset fits.
 int pores_count(nmr::PoreBuild* b, hipStream_t s, uint64_t* end);
-int pores_link(const PoreList& L, nmr::PoreBuild* b, uint64_t end, hipStream_t s, bool* ok);
+int pores_link(PoreList* L, nmr::PoreBuild* b, uint64_t end, hipStream_t s, bool* ok);
 void pores_drop_temp(nmr::PoreBuild* b);
-// Workgroups of a sweep over `groups` groups and the groups of each.
-void pores_tiles(int groups, int* gpt, int* ntiles);
+// Groups that a workgroup takes of a list of `groups`.
+int pores_per_tile(int64_t groups);
 // Whether a list of this many slots stays inside the kernels' 32-bit byte offsets.
 bool pores_fit(uint64_t nslots);
 
@@ -138,6 +139,7 @@ struct nmr_ctx {
     // found not to fit, for the current mask and velocity.
     nmri::PoreList pl;
     bool pl_tried = false, pl_ok = false;
+    bool pl_reads_solids = false; // solids next to pores have slots
     bool pl_vel_ok = false, pl_pv_ok = false; // velocity sums and per-voxel arrays gathered
     bool pl_zeroed = false;   // a MacCormack step ran on the list: solids hold 0
     int ppar = 0;

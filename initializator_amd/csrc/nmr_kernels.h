@@ -176,24 +176,38 @@ struct FieldSumArgs {
 
 // ---- list of pores (nmr_pores.hip) ----
 // 64 slots of the list, in the grid's order and of one plane: the lowest slot
-// of its neighbours per side (x-, x+, y-, y+, z-, z+), which the 16-bit z
-// offsets count from, and 64-bit lane masks.
+// that its lanes read per side (x-, x+, y-, y+, z-, z+), which the offsets
+// count from, and 64-bit lane masks.
 struct PoreGroup {
-    int32_t base[6];
+    uint32_t base[6];
     float zc;               // plane + 1/2
-    int32_t inst;           // instance of a batch
+    uint32_t wide;          // an offset needs more than 8 bits: the 16-bit ones are read
     uint64_t pore[6];       // the neighbour on this side counts as a pore
     uint64_t active;        // the slot holds a pore (else a solid that pores read, or nothing)
     uint64_t window;        // a pore inside the signal window
     uint64_t xm, xp;        // the x neighbour is the slot before / after (else the own value is read)
-    uint64_t zm, zp;        // a z neighbour is read (else the own value)
+    uint64_t pad[2];
 };
 static_assert(sizeof(PoreGroup) == 128, "group descriptor");
 
-// Lanes whose neighbour on a side is a ghost (only with ghosts other than
-// zero-derivative ones).
-struct PoreGhost {
-    uint64_t side[6];
+// Lane masks for ghosts other than zero-derivative ones and for solids that
+// are read: the side is read through its offset, reads as 0, is a ghost.
+struct PoreAux {
+    uint64_t has[6], zero[6], ghost[6];
+};
+
+// Consecutive groups of one workgroup of a batch, all of one instance.
+struct PoreTile {
+    uint32_t first, count;
+    uint32_t inst;
+};
+
+// One instance of a batch: coefficients without the gradient, and its
+// pulsed-gradient pair (as BatchInst).
+struct PoreInst {
+    Coef c;
+    float bgz;
+    int nd, nD;
 };
 
 struct PoreArgs {
@@ -201,20 +215,27 @@ struct PoreArgs {
     const float* mavg;      // corrector stage: the state at the start of the step
     float* out;
     const PoreGroup* groups;
-    const PoreGhost* ghost; // or null
-    const uint2* off;       // 16-bit y-, y+ (distances) and z-, z+ (from the group's bases)
-    const uint32_t* xoff;   // of x-, x+ where they are not the slots next to it; or null
+    const PoreAux* aux;     // where solids are read or a ghost reads as 0; or null
+    const PoreAux* ghost;   // the same array, for per-voxel diffusivities behind ghosts; or null
+    const uint4* rec;       // with velocity: 8-bit y-, y+, z-, z+ offsets, 3 velocity sums (upwind or centred)
+    const uint32_t* off8;   // without: the offsets
+    const uint2* off16;     // the same in 16 bits
+    const uint32_t* xoff;   // 16-bit x-, x+ offsets where they are not the slots next to it; or null
     const uint32_t* xy;     // x | y << 16 (three components)
-    const float* vel;       // 3 velocity sums per slot (upwind or centred)
     const float* dn;        // per-voxel diffusivity / reference, dt/T1, dt/T2, field: or null
     const float* r1v;
     const float* r2v;
     const float* bn;
     const float* w[2];      // phase weights, or null
     double* partials;       // [ntiles][sums] of this step
-    int ngroups;            // one past the last group (group 0 is empty)
-    int gpt, ntiles;        // groups per workgroup, workgroups
+    int ntiles;             // workgroups
+    int ngroups, gpt;       // one domain: past its last group (group 0 is empty), groups per workgroup
+    int wide;               // some group needs its 16-bit offsets
     int bnax, amask;
+    const PoreTile* tiles;  // a batch: the workgroups' groups, its instances, the device step counter and
+    const PoreInst* inst;   //   the step within the chunk
+    const int* step_base;
+    int local_step;
     Coef c;
 };
 
@@ -232,11 +253,12 @@ struct PoreBuild {
     uint32_t* slotmap;      // [nz][ny][pitch] slot of a voxel, 0: none
     uint32_t* vox;          // voxel (row layout) of a slot, ~0: empty
     PoreGroup* groups;
-    PoreGhost* ghost;       // or null
-    uint2* off;
+    PoreAux* aux;           // or null
+    uint32_t* off8;
+    uint2* off16;
     uint32_t* xoff;         // or null
     uint32_t* xy;           // or null
-    int* overflow;          // set when an offset does not fit
+    int* overflow;          // [0] set when an offset does not fit, [1] when a group needs 16-bit offsets
 };
 
 hipError_t launch_pore_count(const PoreBuild& b, hipStream_t s);
@@ -244,6 +266,8 @@ hipError_t launch_pore_link(const PoreBuild& b, hipStream_t s);
 // out[stride*slot + at] = row[vox[slot]] for slots [s0, s1), 0 at empty ones
 hipError_t launch_pore_gather(const float* row, const uint32_t* vox, uint32_t s0, uint32_t s1, int stride, int at,
                               float* out, hipStream_t s);
+// rec[s].x = off8[s], s < n
+hipError_t launch_pore_record(const uint32_t* off8, uint32_t n, uint4* rec, hipStream_t s);
 // row[vox[slot]] (and row2, unless null) = f[stride*slot + at]
 hipError_t launch_pore_scatter(const float* f, const uint32_t* vox, uint32_t s0, uint32_t s1, int stride, int at,
                                float* row, float* row2, hipStream_t s);
@@ -251,7 +275,8 @@ hipError_t launch_pore_scatter(const float* f, const uint32_t* vox, uint32_t s0,
 hipError_t launch_solids_finite(const float* row, const uint8_t* mask, size_t n, int* flag, hipStream_t s);
 hipError_t launch_pore_sum(int nc, const PoreArgs& a, hipStream_t s);
 // a step (stage st) of the whole list; gen: anything but the plain problem
-// (per-voxel data, ghosts other than zero-derivative ones, masked advection)
+// (per-voxel data, ghosts other than zero-derivative ones, solids that are
+// read, masked advection)
 hipError_t launch_pores(int nc, bool vel, int st, bool exact, bool gen, bool coef, const PoreArgs& a, hipStream_t s);
 hipError_t launch_pore_pulse(const PulseArgs& a, float* f, int nc, const uint32_t* vox, uint32_t s0, uint32_t s1,
                              hipStream_t s);

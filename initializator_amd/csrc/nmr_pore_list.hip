@@ -60,15 +60,16 @@ int pores_alloc(PoreList* L, uint32_t nslots, const PoreNeeds& n, hipStream_t s,
         L->nc = n.nc;
     }
     groups(&L->groups);
-    if (n.ghosts || L->ghost) groups(&L->ghost);
-    need(&L->off, 1, 0xff);
-    if (n.xoff || L->xoff) need(&L->xoff, 1, 0xff);
+    if (n.aux || L->aux) groups(&L->aux);
+    need(&L->off8, 1, 0);
+    need(&L->off16, 1, 0);
+    if (n.xoff || L->xoff) need(&L->xoff, 1, 0);
     need(&L->vox, 1, 0xff);
     if (n.nc == 3 || L->xy) need(&L->xy, 1, 0);
     need(&L->state[0], (size_t)n.nc, 0);
     need(&L->state[1], (size_t)n.nc, 0);
     if (n.pred || L->pred) need(&L->pred, (size_t)n.nc, 0);
-    if (n.vel || L->vel) need(&L->vel, 3, 0);
+    if (n.vel || L->rec) need(&L->rec, 1, 0);
     if (more)
         for (float*& p : L->pv)
             if (p && !rc) {
@@ -80,13 +81,15 @@ int pores_alloc(PoreList* L, uint32_t nslots, const PoreNeeds& n, hipStream_t s,
     if (rc) return rc;
     L->cap = cap;
     L->nslots = nslots;
+    L->wide = false;
     return NMR_OK;
 }
 
 void pores_free(PoreList* L)
 {
-    for (void* p : {(void*)L->groups, (void*)L->ghost, (void*)L->off, (void*)L->xoff, (void*)L->vox, (void*)L->xy,
-                    (void*)L->state[0], (void*)L->state[1], (void*)L->pred, (void*)L->vel, (void*)L->pv[0],
+    for (void* p : {(void*)L->groups, (void*)L->aux, (void*)L->off8, (void*)L->off16, (void*)L->xoff, (void*)L->vox,
+                    (void*)L->xy, (void*)L->state[0], (void*)L->state[1], (void*)L->pred,
+                    (void*)L->rec, (void*)L->pv[0],
                     (void*)L->pv[1], (void*)L->pv[2], (void*)L->pv[3], (void*)L->pv[4], (void*)L->pv[5]})
         if (p) (void)hipFree(p);
     *L = PoreList{};
@@ -126,32 +129,36 @@ int pores_count(nmr::PoreBuild* b, hipStream_t s, uint64_t* end)
     return rc;
 }
 
-int pores_link(const PoreList& L, nmr::PoreBuild* b, uint64_t end, hipStream_t s, bool* ok)
+int pores_link(PoreList* L, nmr::PoreBuild* b, uint64_t end, hipStream_t s, bool* ok)
 {
-    b->vox = L.vox;
-    b->groups = L.groups;
-    b->ghost = L.ghost;
-    b->off = L.off;
-    b->xoff = L.xoff;
-    b->xy = L.xy;
+    b->vox = L->vox;
+    b->groups = L->groups;
+    b->aux = L->aux;
+    b->off8 = L->off8;
+    b->off16 = L->off16;
+    b->xoff = L->xoff;
+    b->xy = L->xy;
     b->count = (int64_t)((end - b->first) / 64);
-    int over = 0, rc = NMR_OK;
+    int over[2] = {0, 0}, rc = NMR_OK;
     hipError_t e = nmr::launch_pore_link(*b, s);
-    if (e == hipSuccess) e = hipMemcpyAsync(&over, b->overflow, sizeof(int), hipMemcpyDeviceToHost, s);
+    if (e == hipSuccess) e = hipMemcpyAsync(over, b->overflow, sizeof(over), hipMemcpyDeviceToHost, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
     if (e != hipSuccess) rc = fail(NMR_ERR_DEVICE, "pore list: %s", hipGetErrorString(e));
     pores_drop_temp(b);
-    *ok = rc == NMR_OK && over == 0;
+    *ok = rc == NMR_OK && over[0] == 0;
+    L->wide = L->wide || over[1] != 0;
     return rc;
 }
 
-void pores_tiles(int groups, int* gpt, int* ntiles)
+int pores_per_tile(int64_t groups)
 {
-    // two groups a wavefront: 256^3 (52 K groups) 21.0 / 20.6 / 21.5 / 24.7 / 25.4 us
-    // a step at 4 / 8 / 16 / 32 / 64 groups a workgroup; fewer than a few
-    // workgroups per CU: one (64^3, 1.2 K groups: 3.0 / 3.4 / 4.5 us at 4 / 8 / 16)
-    *gpt = groups <= 8192 ? 4 : 8;
-    *ntiles = std::max(1, (groups + *gpt - 1) / *gpt);
+    // one group a wavefront: 256^3, porosity 0.2 (52 K groups) 19.8 / 20.2 /
+    // 20.3 us a step at 4 / 8 / 12 groups a workgroup, 512x512x130 35.3 / 36.1
+    // at 4 / 8, 64^3 2.8 / 3.3; more where a step's partial sums, one a
+    // workgroup, would pass 64 K
+    int per = 4;
+    while (groups / per > 65536) per *= 2;
+    return per;
 }
 
 } // namespace nmri

@@ -6,23 +6,26 @@
 // costs as much as a full one.  Here the state of the pores is kept as a
 // list: 64 slots to a group, in the grid's order, so that the wavefront of a
 // group has a pore in every lane.  A slot's x neighbours are the slots next
-// to it; its y and z neighbours are given as 16-bit offsets from a base of
-// the group; which neighbours are pores, and which lanes count in the signal,
-// are 64-bit lane masks of the group's descriptor, read into scalar registers
-// and used as lane conditions directly.  A group never spans two planes, so
-// z and the precession angle of a z gradient are uniform in a wavefront.
+// to it; its y and z neighbours are given as 8-bit offsets from four bases of
+// the group (16-bit ones where a group needs them), packed with the three
+// velocity sums into one 16-byte record; which neighbours are pores, and
+// which lanes count in the signal, are 64-bit lane masks of the group's
+// descriptor, read into scalar registers and used as lane conditions
+// directly.  A group never spans two planes, so z and the precession angle of
+// a z gradient are uniform in a wavefront.
 //
-// A step moves 38 bytes a pore -- two components read and written (16), the
-// velocity sums (12), the offsets (8), the descriptor (2) -- less than half of
-// the tile sweep's traffic a voxel at 20 % porosity; a workgroup's groups are
-// consecutive and each XCD takes a contiguous run of workgroups, so the
-// planes above and below are in that XCD's L2.  256^3, porosity 0.2, flow and
-// gradient: 20.6 us a step (the tile sweep on bricks: 58.0).  What bounds it
-// there is not those bytes but the vector memory path: 200 L1 accesses a group
-// (16 for a 64-lane load of 8 bytes, ten such accesses a slot), 17 us at one
-// a cycle and CU; leaving out the gathers' spread or a third of the vector
-// instructions changed nothing.  On 512x512x130 (259 MB a step, past the
-// memory-side cache) it is the bytes: 39 us, 6.6 TB/s.
+// What bounds it: bytes past the L2.  A step moves 34 a pore -- two
+// components read and written (16), the record (16), the descriptor (2) --
+// less than half of the tile sweep's a voxel at 20 % porosity; the neighbours
+// are L1 and L2 hits (each XCD takes a contiguous run of workgroups).  256^3,
+// porosity 0.2, flow and gradient: 19.9 us a step (the tile sweep on bricks:
+// 57.9; this list with 16-bit offsets and a separate 12-byte velocity: 20.6),
+// of which about 4 are the launch's ramp and tail; 123 MB past the L2 in the
+// rest, 7.6 TB/s, what a copy inside the memory-side cache reaches (7.7-8.3).
+// 512x512x130 (231 MB a step): 35.3 us, 6.5 TB/s.  Not what bounds it: the
+// gathers (left out: the same time), the vector instructions (131 or 85 a
+// group: the same), L1 accesses (halved by staging the neighbourhood in LDS:
+// the same, and slower with three components or periodic rows).
 //
 // The arithmetic of a voxel is that of the tile sweeps (update_chunk,
 // gupdate_chunk) and of general_kernel, operation by operation, so the fields
@@ -41,17 +44,12 @@ namespace {
 
 constexpr int kThreads = 256;
 constexpr int kWaves = kThreads / 64;
-// Codes among the offsets.  y: the signed distance to the neighbour's slot, 0
-// where the slot's own value is read; z (and x, where it has offsets): the
-// distance from the group's base.
-constexpr uint32_t kOwn = 0xffffu;   // x: the own value is read
-constexpr uint32_t kZero = 0xfffeu;  // x, z: 0 is read (slot 0, which stays 0)
-constexpr uint32_t kZeroY = 0x8000u; // y: 0 is read
-
 // Group descriptors are read through the constant address space: uniform
 // loads from it go to scalar registers, also in a loop that stores.
 typedef const __attribute__((address_space(4))) PoreGroup* GroupPtr;
-typedef const __attribute__((address_space(4))) PoreGhost* GhostPtr;
+typedef const __attribute__((address_space(4))) PoreAux* AuxPtr;
+typedef const __attribute__((address_space(4))) PoreTile* TilePtr;
+typedef const __attribute__((address_space(4))) PoreInst* InstPtr;
 __device__ __forceinline__ GroupPtr group_at(const PoreGroup* g, int i) { return (GroupPtr)(uintptr_t)(g + i); }
 
 // Values that the compiler must have at this point: it would otherwise sink
@@ -86,11 +84,6 @@ template <int NC>
 using Vec = typename VecOf<NC>::type;
 
 template <int NC>
-__device__ __forceinline__ Vec<NC> ldm(const float* base, uint32_t i)
-{
-    return *reinterpret_cast<const Vec<NC>*>(reinterpret_cast<const char*>(base) + i * (uint32_t)(4 * NC));
-}
-template <int NC>
 __device__ __forceinline__ void stm(float* base, uint32_t i, const Vec<NC>& v)
 {
     *reinterpret_cast<Vec<NC>*>(reinterpret_cast<char*>(base) + i * (uint32_t)(4 * NC)) = v;
@@ -107,6 +100,7 @@ __device__ __forceinline__ T at_byte(const void* base, uint32_t o)
 {
     return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) + o);
 }
+
 // v of another lane by a DPP move of both halves (0 where the move has no source).
 template <int CTRL, int ROWS>
 __device__ __forceinline__ double dpp_add(double v)
@@ -156,14 +150,14 @@ __device__ __forceinline__ void group_reduce(double (&acc)[NS], double (*sred)[N
 
 // The descriptor of a group, in scalar registers.
 struct GroupRegs {
-    uint32_t base[6];
+    uint32_t base[6], wide;
     float zc;
-    uint64_t pore[6], active, window, xm, xp, zm, zp;
-    template <bool GEN>
+    uint64_t pore[6], active, window, xm, xp;
     __device__ __forceinline__ void load(GroupPtr G)
     {
 #pragma unroll
-        for (int s = GEN ? 0 : 4; s < 6; s++) base[s] = (uint32_t)G->base[s];
+        for (int s = 0; s < 6; s++) base[s] = G->base[s];
+        wide = G->wide;
         zc = G->zc;
 #pragma unroll
         for (int s = 0; s < 6; s++) pore[s] = G->pore[s];
@@ -171,34 +165,15 @@ struct GroupRegs {
         window = G->window;
         xm = G->xm;
         xp = G->xp;
-        zm = G->zm;
-        zp = G->zp;
+        // the compiler would sink these loads into branches around the
+        // selects that use them, one dependent wait each
 #pragma unroll
-        for (int s = GEN ? 0 : 4; s < 6; s++) have_s(base[s]);
+        for (int s = 2; s < 6; s++) have_s(base[s]);
         have_s(xm);
         have_s(xp);
-        have_s(zm);
-        have_s(zp);
     }
 };
 
-// A 16-bit half of x times K plus a, one instruction each.
-template <int K, bool HI>
-__device__ __forceinline__ uint32_t mad_i16(uint32_t x, uint32_t a)
-{
-    uint32_t r;
-    if constexpr (HI) asm("v_mad_i32_i16 %0, %1, %2, %3 op_sel:[1,0,0,0]" : "=v"(r) : "v"(x), "n"(K), "v"(a));
-    else asm("v_mad_i32_i16 %0, %1, %2, %3" : "=v"(r) : "v"(x), "n"(K), "v"(a));
-    return r;
-}
-template <int K, bool HI>
-__device__ __forceinline__ uint32_t mad_u16(uint32_t x, uint32_t a)
-{
-    uint32_t r;
-    if constexpr (HI) asm("v_mad_u32_u16 %0, %1, %2, %3 op_sel:[1,0,0,0]" : "=v"(r) : "v"(x), "n"(K), "s"(a));
-    else asm("v_mad_u32_u16 %0, %1, %2, %3" : "=v"(r) : "v"(x), "n"(K), "s"(a));
-    return r;
-}
 // max(v, 0) and min(v, 0) (0 for a NaN) without the canonicalisation that
 // fmaxf adds for signalling NaNs, which no loaded sum is.
 __device__ __forceinline__ float pos(float v)
@@ -214,37 +189,49 @@ __device__ __forceinline__ float neg(float v)
     return r;
 }
 
-// Offsets of the neighbours x-, x+, y-, y+, z-, z+ of a slot, in units of K
-// bytes a slot; a missing neighbour gives the slot itself.
-template <int K, bool GEN>
-__device__ __forceinline__ void neighbours(const PoreArgs& a, const GroupRegs& G, uint2 off, uint32_t slot,
+// Byte offsets, K bytes a slot, of the neighbours x-, x+, y-, y+, z-, z+ of a
+// slot.  A side with nothing to read gives the slot itself.
+template <int K, bool GEN, bool WIDE>
+__device__ __forceinline__ void neighbours(const PoreArgs& a, const GroupRegs& G, int g, uint32_t off8, uint32_t slot,
                                            uint32_t (&nb)[6])
 {
     const uint32_t own = slot * (uint32_t)K;
     nb[0] = lane_in(G.xm) ? own - (uint32_t)K : own;
     nb[1] = lane_in(G.xp) ? own + (uint32_t)K : own;
-    nb[2] = mad_i16<K, false>(off.x, own);
-    nb[3] = mad_i16<K, true>(off.x, own);
-    const uint32_t zm = mad_u16<K, false>(off.y, G.base[4] * (uint32_t)K);
-    const uint32_t zp = mad_u16<K, true>(off.y, G.base[5] * (uint32_t)K);
-    nb[4] = lane_in(G.zm) ? zm : own;
-    nb[5] = lane_in(G.zp) ? zp : own;
+    uint32_t o[4] = {off8 & 0xffu, (off8 >> 8) & 0xffu, (off8 >> 16) & 0xffu, off8 >> 24};
+    if (WIDE && G.wide) { // some neighbour lies more than 255 slots from its base
+        const uint2 o16 = ldw(a.off16, slot);
+        o[0] = o16.x & 0xffffu;
+        o[1] = o16.x >> 16;
+        o[2] = o16.y & 0xffffu;
+        o[3] = o16.y >> 16;
+    }
+    uint32_t v[6];
+#pragma unroll
+    for (int s = 2; s < 6; s++) {
+        v[s] = o[s - 2] * (uint32_t)K + G.base[s] * (uint32_t)K;
+        nb[s] = lane_in(G.pore[s]) ? v[s] : own; // pores and ghosts are read, solids are not
+    }
     if constexpr (GEN) {
-        if ((off.x & 0xffffu) == kZeroY) nb[2] = 0u;
-        if ((off.x >> 16) == kZeroY) nb[3] = 0u;
-        if ((off.y & 0xffffu) == kZero) nb[4] = 0u;
-        if ((off.y >> 16) == kZero) nb[5] = 0u;
         if (a.xoff) {
             const uint32_t xo = ldw(a.xoff, slot);
-            const uint32_t m = xo & 0xffffu, p = xo >> 16;
-            nb[0] = m == kOwn ? own : (m == kZero ? 0u : (G.base[0] + m) * (uint32_t)K);
-            nb[1] = p == kOwn ? own : (p == kZero ? 0u : (G.base[1] + p) * (uint32_t)K);
+            v[0] = ((xo & 0xffffu) + G.base[0]) * (uint32_t)K;
+            v[1] = ((xo >> 16) + G.base[1]) * (uint32_t)K;
+            nb[0] = lane_in(G.pore[0]) ? v[0] : own;
+            nb[1] = lane_in(G.pore[1]) ? v[1] : own;
+        }
+        if (a.aux) { // solids that are read, ghosts that read as 0 (slot 0 stays 0)
+            const AuxPtr A = (AuxPtr)(uintptr_t)(a.aux + g);
+#pragma unroll
+            for (int s = 0; s < 6; s++) {
+                if (s >= 2 || a.xoff) nb[s] = lane_in(A->has[s]) ? v[s] : own;
+                nb[s] = lane_in(A->zero[s]) ? 0u : nb[s];
+            }
         }
     }
 }
 
-// r + s0*(faces to solids on the axis of sides m and m+1): fmaf(s, n, r) with n
-// 0, 1 or 2 from the lane masks.
+// Faces to solids on the axis of sides m and m+1: 0, 1 or 2 from the lane masks.
 __device__ __forceinline__ float solid_faces(const GroupRegs& G, int m)
 {
     const uint64_t any = ~(G.pore[m] & G.pore[m + 1]), both = ~(G.pore[m] | G.pore[m + 1]);
@@ -255,20 +242,28 @@ __device__ __forceinline__ float solid_faces(const GroupRegs& G, int m)
 // One step (or MacCormack stage ST) of the 64 slots of group g, lane by lane.
 // GEN: per-voxel field, masked advection, non-zero-derivative ghosts and
 // phase weights may be present (null pointers and flags say which); COEF:
-// per-voxel diffusivity and rates.
-template <int NC, bool VEL, int ST, bool EXACT, bool GEN, bool COEF, int NS>
+// per-voxel diffusivity and rates; WIDE: some group needs its 16-bit offsets.
+template <int NC, bool VEL, int ST, bool EXACT, bool GEN, bool COEF, bool WIDE, int NS>
 __device__ __forceinline__ void pore_step(const PoreArgs& a, const Coef& cf, const int g, double (&acc)[NS])
 {
     constexpr int K = 4 * NC;
     const uint32_t slot = (uint32_t)g * 64u + (threadIdx.x & 63u);
-    const uint2 off = ldw(a.off, slot);
-    const Vec<NC> mc = ldm<NC>(a.f, slot);
+    uint32_t off8;
+    float adv[3] = {0.f, 0.f, 0.f};
+    if constexpr (VEL) {
+        const uint4 r = ldw(a.rec, slot);
+        off8 = r.x;
+        adv[0] = __uint_as_float(r.y);
+        adv[1] = __uint_as_float(r.z);
+        adv[2] = __uint_as_float(r.w);
+    } else {
+        off8 = ldw(a.off8, slot);
+    }
+    const Vec<NC> mc = at_byte<Vec<NC>>(a.f, slot * (uint32_t)K);
     GroupRegs G;
-    G.load<GEN>(group_at(a.groups, g));
-    Vec<3> adv = {0.f, 0.f, 0.f};
-    if constexpr (VEL) adv = ldm<3>(a.vel, slot);
+    G.load(group_at(a.groups, g));
     uint32_t nb[6];
-    neighbours<K, GEN>(a, G, off, slot, nb);
+    neighbours<K, GEN, WIDE>(a, G, g, off8, slot, nb);
     Vec<NC> fn[6];
 #pragma unroll
     for (int s = 0; s < 6; s++) fn[s] = at_byte<Vec<NC>>(a.f, nb[s]);
@@ -282,14 +277,14 @@ __device__ __forceinline__ void pore_step(const PoreArgs& a, const Coef& cf, con
     float w[6];
     if constexpr (COEF) {
         uint32_t nd[6];
-        neighbours<4, GEN>(a, G, off, slot, nd);
+        neighbours<4, GEN, WIDE>(a, G, g, off8, slot, nd);
         const float dc = ldw(a.dn, slot);
         const float cd[3] = {cf.cdx, cf.cdy, cf.cdz};
 #pragma unroll
         for (int s = 0; s < 6; s++) {
             float dnb = at_byte<float>(a.dn, nd[s]);
             // ghosts carry the diffusivity of the voxel they border
-            if (a.ghost && lane_in(((GhostPtr)(uintptr_t)(a.ghost + g))->side[s])) dnb = dc;
+            if (a.ghost && lane_in(((AuxPtr)(uintptr_t)(a.ghost + g))->ghost[s])) dnb = dc;
             const float hm = hmean(dc, dnb);
             w[s] = cd[s / 2] * hm * (kn[s] ? 1.f : 0.f);
         }
@@ -385,7 +380,7 @@ __device__ __forceinline__ void pore_step(const PoreArgs& a, const Coef& cf, con
     const bool act = lane_in(G.active);
     Vec<NC> out;
     if constexpr (ST == GEN_CORRECT) {
-        const Vec<NC> mav = ldm<NC>(a.mavg, slot);
+        const Vec<NC> mav = at_byte<Vec<NC>>(a.mavg, slot * (uint32_t)K);
 #pragma unroll
         for (int q = 0; q < NC; q++) {
             float v = 0.5f * (mav[q] + (mc[q] + d[q]));
@@ -418,39 +413,78 @@ __device__ __forceinline__ void pore_step(const PoreArgs& a, const Coef& cf, con
     }
 }
 
-// One domain: workgroup t takes groups [first + t*gpt, first + (t+1)*gpt),
-// its four wavefronts in turn.
-template <int NC, bool VEL, int ST, bool EXACT, bool GEN, bool COEF, bool W>
+template <bool BATCH>
+__device__ __forceinline__ void tile_range(const PoreArgs& a, int t, int& g0, int& g1, uint32_t& inst)
+{
+    inst = 0;
+    if constexpr (BATCH) {
+        const TilePtr T = (TilePtr)(uintptr_t)(a.tiles + t);
+        g0 = (int)T->first;
+        g1 = g0 + (int)T->count;
+        inst = T->inst;
+    } else {
+        g0 = 1 + t * a.gpt;
+        g1 = min(g0 + a.gpt, a.ngroups);
+    }
+}
+
+// Coefficients of the step: the launch's, or in a batch the instance's with
+// the gradient of its pulsed-gradient pair at this step (+G on steps [0, nd),
+// -G on [nD, nD + nd), the second lobe where they overlap).
+template <bool BATCH>
+__device__ __forceinline__ Coef step_coef(const PoreArgs& a, uint32_t inst)
+{
+    if constexpr (!BATCH) return a.c;
+    const InstPtr I = (InstPtr)(uintptr_t)(a.inst + inst);
+    Coef c;
+    const __attribute__((address_space(4))) float* s = (const __attribute__((address_space(4))) float*)&I->c;
+    float* d = reinterpret_cast<float*>(&c);
+#pragma unroll
+    for (unsigned k = 0; k < sizeof(Coef) / 4; k++) d[k] = s[k];
+    const int step = *a.step_base + a.local_step;
+    c.bgz = (step >= I->nD && step < I->nD + I->nd) ? -I->bgz : (step < I->nd ? I->bgz : 0.f);
+    return c;
+}
+
+// Workgroup t takes tile t's groups, its wavefronts in turn: of one domain
+// gpt consecutive groups, of a batch what the tile list says.
+template <int NC, bool VEL, int ST, bool EXACT, bool GEN, bool COEF, bool W, bool BATCH, bool WIDE>
 __global__ void __launch_bounds__(kThreads) pore_kernel(PoreArgs a)
 {
     constexpr int NS = W ? 2 * NC : NC;
     __shared__ double sred[ST == GEN_PREDICT ? 1 : kWaves - 1][NS][64];
     const int t = xcd_tile(blockIdx.x, a.ntiles);
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-    const int g0 = 1 + t * a.gpt, g1 = min(g0 + a.gpt, a.ngroups);
+    int g0, g1;
+    uint32_t inst;
+    tile_range<BATCH>(a, t, g0, g1, inst);
+    const Coef cf = step_coef<BATCH>(a, inst);
     double acc[NS];
 #pragma unroll
     for (int q = 0; q < NS; q++) acc[q] = 0.0;
-    for (int g = g0 + wave; g < g1; g += kWaves) pore_step<NC, VEL, ST, EXACT, GEN, COEF, NS>(a, a.c, g, acc);
+    for (int g = g0 + wave; g < g1; g += kWaves) pore_step<NC, VEL, ST, EXACT, GEN, COEF, WIDE, NS>(a, cf, g, acc);
     if constexpr (ST != GEN_PREDICT) group_reduce<NS>(acc, sred, a.partials + (size_t)t * NS);
 }
 
-// Pore sums of the state over the signal window (weights: phase-weighted).
-template <int NC, bool W>
+// Pore sums of the state over the signal window (weights: phase-weighted),
+// one partial a tile.
+template <int NC, bool W, bool BATCH>
 __global__ void __launch_bounds__(kThreads) pore_sum_kernel(PoreArgs a)
 {
     constexpr int NS = W ? 2 * NC : NC;
     __shared__ double sred[kWaves - 1][NS][64];
     const int t = blockIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-    const int g0 = 1 + t * a.gpt, g1 = min(g0 + a.gpt, a.ngroups);
+    int g0, g1;
+    uint32_t inst;
+    tile_range<BATCH>(a, t, g0, g1, inst);
     double acc[NS];
 #pragma unroll
     for (int q = 0; q < NS; q++) acc[q] = 0.0;
     for (int g = g0 + wave; g < g1; g += kWaves) {
         if (!lane_in(group_at(a.groups, g)->window)) continue;
         const uint32_t slot = (uint32_t)g * 64u + (threadIdx.x & 63u);
-        const Vec<NC> m = ldm<NC>(a.f, slot);
+        const Vec<NC> m = at_byte<Vec<NC>>(a.f, slot * (uint32_t)(4 * NC));
         if constexpr (W) {
             const double w1 = (double)ldw(a.w[0], slot), w2 = (double)ldw(a.w[1], slot);
 #pragma unroll
@@ -595,14 +629,13 @@ __global__ void __launch_bounds__(kThreads) pore_link_kernel(PoreBuild b)
     const int c[3] = {x, y, z}, n[3] = {b.nx, b.ny, b.nz};
     const uint32_t st[3] = {1u, P, plane};
 
-    // neighbour slots: kOwn / kZero codes, else a slot number
+    // neighbour slots; a zero-derivative ghost reads the slot itself
     uint32_t nbs[6];
-    bool own[6], zero[6], pore[6], ghost[6];
+    bool has[6], zero[6], pore[6], ghost[6];
 #pragma unroll
     for (int s = 0; s < 6; s++) {
         const int ax = s >> 1, up = s & 1;
-        own[s] = true;
-        zero[s] = pore[s] = ghost[s] = false;
+        has[s] = zero[s] = pore[s] = ghost[s] = false;
         nbs[s] = 0;
         if (!act) continue;
         const bool edge = up ? c[ax] == n[ax] - 1 : c[ax] == 0;
@@ -611,71 +644,73 @@ __global__ void __launch_bounds__(kThreads) pore_link_kernel(PoreBuild b)
             pore[s] = b.mask[v] != 0;
             if (pore[s] || b.read_solids) {
                 nbs[s] = b.slotmap[v];
-                own[s] = nbs[s] == 0;
+                has[s] = nbs[s] != 0;
             }
         } else {
             pore[s] = ghost[s] = true;
+            has[s] = b.bc[ax] != BC_DIRICHLET;
+            zero[s] = !has[s];
+            nbs[s] = slot;
             if (b.bc[ax] == BC_PERIODIC) {
                 const uint32_t d = (uint32_t)(n[ax] - 1) * st[ax];
                 nbs[s] = b.slotmap[up ? o - d : o + d];
-                own[s] = false;
-            } else if (b.bc[ax] == BC_DIRICHLET) {
-                zero[s] = true;
-                own[s] = false;
             }
         }
     }
-    uint32_t base[6], off[6];
-    bool over = false;
+    // the lowest slot read on each side, and the offsets from it
+    uint32_t lo[6];
 #pragma unroll
     for (int s = 0; s < 6; s++) {
-        const bool at = !own[s] && !zero[s];
-        uint32_t lo = at ? nbs[s] : 0xffffffffu;
-        for (int h = 32; h > 0; h >>= 1) lo = min(lo, (uint32_t)__shfl_xor((int)lo, h, 64));
-        base[s] = lo == 0xffffffffu ? 0u : lo;
-        if (s == 2 || s == 3) { // signed distance
-            const int64_t d = at ? (int64_t)nbs[s] - (int64_t)slot : 0;
-            if (d < -32767 || d > 32767) over = true;
-            off[s] = zero[s] ? kZeroY : ((uint32_t)(int32_t)d & 0xffffu);
-        } else {
-            const uint32_t d = at ? nbs[s] - base[s] : 0u;
-            const bool x_next = s < 2 && !b.xoff; // the slot next to this one
-            if (at && !x_next && d >= kZero) over = true;
-            off[s] = own[s] ? kOwn : (zero[s] ? kZero : (d & 0xffffu));
-        }
+        lo[s] = has[s] ? nbs[s] : 0xffffffffu;
+        for (int h = 32; h > 0; h >>= 1) lo[s] = min(lo[s], (uint32_t)__shfl_xor((int)lo[s], h, 64));
     }
-    if (over) *b.overflow = 1;
-    b.off[slot] = make_uint2(off[2] | (off[3] << 16), off[4] | (off[5] << 16));
-    if (b.xoff) b.xoff[slot] = off[0] | (off[1] << 16);
+    uint32_t off[6];
+    bool wide = false, over = false;
+#pragma unroll
+    for (int s = 0; s < 6; s++) {
+        off[s] = has[s] ? nbs[s] - lo[s] : 0u;
+        if (s >= 2 && off[s] > 0xffu) wide = true;
+        if ((s >= 2 || b.xoff) && off[s] > 0xffffu) over = true;
+    }
+    if (over) b.overflow[0] = 1;
+    if (wide) b.overflow[1] = 1;
+    b.off8[slot] = (off[2] & 0xffu) | (off[3] & 0xffu) << 8 | (off[4] & 0xffu) << 16 | (off[5] & 0xffu) << 24;
+    b.off16[slot] = make_uint2((off[2] & 0xffffu) | off[3] << 16, (off[4] & 0xffffu) | off[5] << 16);
+    if (b.xoff) b.xoff[slot] = (off[0] & 0xffffu) | off[1] << 16;
     if (b.xy) b.xy[slot] = (uint32_t)x | ((uint32_t)y << 16);
     const bool win = act && x >= b.w[0] && x < b.w[1] && y >= b.w[2] && y < b.w[3] && z >= b.w[4] && z < b.w[5];
     const uint64_t any = __ballot(used);
     const int first = any ? (int)__ffsll((unsigned long long)any) - 1 : 0;
     const int gz = __shfl(z, first, 64);
-    uint64_t pm[6], gm[6];
+    uint64_t pm[6], hm[6], zm[6], gm[6];
 #pragma unroll
     for (int s = 0; s < 6; s++) {
         pm[s] = __ballot(pore[s]);
+        hm[s] = __ballot(has[s]);
+        zm[s] = __ballot(zero[s]);
         gm[s] = __ballot(ghost[s]);
     }
-    const uint64_t am = __ballot(act), wm = __ballot(win), xm = __ballot(!own[0]), xp = __ballot(!own[1]);
-    const uint64_t zm = __ballot(!own[4]), zp = __ballot(!own[5]);
+    const uint64_t am = __ballot(act), wm = __ballot(win), wd = __ballot(wide);
+    const uint64_t xm = __ballot(has[0] && nbs[0] != slot), xp = __ballot(has[1] && nbs[1] != slot);
     if (lane == 0) {
         PoreGroup G{};
         for (int s = 0; s < 6; s++) {
-            G.base[s] = (int32_t)base[s];
+            G.base[s] = lo[s] == 0xffffffffu ? 0u : lo[s];
             G.pore[s] = pm[s];
         }
         G.zc = (float)gz + 0.5f;
+        G.wide = wd != 0;
         G.active = am;
         G.window = wm;
         G.xm = xm;
         G.xp = xp;
-        G.zm = zm;
-        G.zp = zp;
         b.groups[g] = G;
-        if (b.ghost)
-            for (int s = 0; s < 6; s++) b.ghost[g].side[s] = gm[s];
+        if (b.aux)
+            for (int s = 0; s < 6; s++) {
+                b.aux[g].has[s] = hm[s];
+                b.aux[g].zero[s] = zm[s];
+                b.aux[g].ghost[s] = gm[s];
+            }
     }
 }
 
@@ -689,6 +724,14 @@ __global__ void __launch_bounds__(kThreads) pore_gather_kernel(const float* __re
     if (s >= s1) return;
     const uint32_t o = vox[s];
     out[(size_t)s * stride + at] = o != 0xffffffffu ? row[o] : 0.f;
+}
+
+// The first word of every record: the packed offsets.
+__global__ void __launch_bounds__(kThreads) pore_record_kernel(const uint32_t* __restrict__ off8, uint32_t n,
+                                                               uint4* __restrict__ rec)
+{
+    const uint32_t s = blockIdx.x * (uint32_t)kThreads + threadIdx.x;
+    if (s < n) rec[s].x = off8[s];
 }
 
 // The state of the slots (nc components) back into one row array.
@@ -771,6 +814,13 @@ hipError_t launch_pore_gather(const float* row, const uint32_t* vox, uint32_t s0
     return hipGetLastError();
 }
 
+hipError_t launch_pore_record(const uint32_t* off8, uint32_t n, uint4* rec, hipStream_t s)
+{
+    if (n == 0) return hipSuccess;
+    hipLaunchKernelGGL(pore_record_kernel, dim3((n + kThreads - 1) / kThreads), dim3(kThreads), 0, s, off8, n, rec);
+    return hipGetLastError();
+}
+
 hipError_t launch_pore_scatter(const float* f, const uint32_t* vox, uint32_t s0, uint32_t s1, int stride, int at,
                                float* row, float* row2, hipStream_t s)
 {
@@ -791,10 +841,11 @@ hipError_t launch_pore_sum(int nc, const PoreArgs& a, hipStream_t s)
 {
     const dim3 grid((unsigned)a.ntiles), block(kThreads);
     const bool w = a.w[0] != nullptr;
-#define SUM(N)                                                                           \
-    case N:                                                                              \
-        if (w) hipLaunchKernelGGL((pore_sum_kernel<N, true>), grid, block, 0, s, a);     \
-        else hipLaunchKernelGGL((pore_sum_kernel<N, false>), grid, block, 0, s, a);      \
+#define SUM(N)                                                                                     \
+    case N:                                                                                        \
+        if (a.inst) hipLaunchKernelGGL((pore_sum_kernel<N, false, true>), grid, block, 0, s, a);   \
+        else if (w) hipLaunchKernelGGL((pore_sum_kernel<N, true, false>), grid, block, 0, s, a);   \
+        else hipLaunchKernelGGL((pore_sum_kernel<N, false, false>), grid, block, 0, s, a);         \
         break
     switch (nc) {
         SUM(1);
@@ -808,55 +859,68 @@ hipError_t launch_pore_sum(int nc, const PoreArgs& a, hipStream_t s)
 
 namespace {
 
-template <int NC, bool VEL, int ST, bool EXACT>
-void launch_pores_st(bool gen, bool coef, const PoreArgs& a, hipStream_t s)
+template <int NC, bool VEL, int ST, bool EXACT, bool GEN, bool COEF, bool W, bool BATCH>
+hipError_t launch_one(const PoreArgs& a, hipStream_t s)
 {
     const dim3 grid((unsigned)a.ntiles), block(kThreads);
-    if constexpr (EXACT) {
-        hipLaunchKernelGGL((pore_kernel<NC, VEL, ST, true, false, false, false>), grid, block, 0, s, a);
-    } else {
-        const bool w = a.w[0] != nullptr && ST != GEN_PREDICT;
-        if (!gen) hipLaunchKernelGGL((pore_kernel<NC, VEL, ST, false, false, false, false>), grid, block, 0, s, a);
-        else if (coef && w) hipLaunchKernelGGL((pore_kernel<NC, VEL, ST, false, true, true, ST != GEN_PREDICT>), grid, block, 0, s, a);
-        else if (coef) hipLaunchKernelGGL((pore_kernel<NC, VEL, ST, false, true, true, false>), grid, block, 0, s, a);
-        else if (w) hipLaunchKernelGGL((pore_kernel<NC, VEL, ST, false, true, false, ST != GEN_PREDICT>), grid, block, 0, s, a);
-        else hipLaunchKernelGGL((pore_kernel<NC, VEL, ST, false, true, false, false>), grid, block, 0, s, a);
+    if (a.wide) hipLaunchKernelGGL((pore_kernel<NC, VEL, ST, EXACT, GEN, COEF, W, BATCH, true>), grid, block, 0, s, a);
+    else hipLaunchKernelGGL((pore_kernel<NC, VEL, ST, EXACT, GEN, COEF, W, BATCH, false>), grid, block, 0, s, a);
+    return hipGetLastError();
+}
+
+template <int NC, bool VEL, int ST>
+hipError_t launch_st(bool exact, bool gen, bool coef, const PoreArgs& a, hipStream_t s)
+{
+    if (exact) {
+        if constexpr (NC == 2 && ST == GEN_UPWIND) {
+            if (gen) return launch_one<NC, VEL, ST, true, true, false, false, false>(a, s);
+            return launch_one<NC, VEL, ST, true, false, false, false, false>(a, s);
+        }
+        return hipErrorInvalidValue;
     }
+    constexpr bool SUMS = ST != GEN_PREDICT; // the predictor has no signal
+    const bool w = SUMS && a.w[0] != nullptr;
+    if (!gen) return launch_one<NC, VEL, ST, false, false, false, false, false>(a, s);
+    if (coef && w) return launch_one<NC, VEL, ST, false, true, true, SUMS, false>(a, s);
+    if (coef) return launch_one<NC, VEL, ST, false, true, true, false, false>(a, s);
+    if (w) return launch_one<NC, VEL, ST, false, true, false, SUMS, false>(a, s);
+    return launch_one<NC, VEL, ST, false, true, false, false, false>(a, s);
 }
 
 template <int NC, bool VEL>
-hipError_t launch_pores_nc(int st, bool exact, bool gen, bool coef, const PoreArgs& a, hipStream_t s)
+hipError_t launch_nc(int st, bool exact, bool gen, bool coef, const PoreArgs& a, hipStream_t s)
 {
-    if (exact) {
-        if constexpr (NC == 2) launch_pores_st<NC, VEL, GEN_UPWIND, true>(gen, coef, a, s);
-        else return hipErrorInvalidValue;
-    } else if (st == GEN_UPWIND) {
-        launch_pores_st<NC, VEL, GEN_UPWIND, false>(gen, coef, a, s);
-    } else if (st == GEN_PREDICT) {
-        launch_pores_st<NC, VEL, GEN_PREDICT, false>(gen, coef, a, s);
-    } else {
-        launch_pores_st<NC, VEL, GEN_CORRECT, false>(gen, coef, a, s);
+    if (a.inst) { // a batch: the plain upwind step, solids read or not
+        if constexpr (NC == 2) {
+            if (exact && gen) return launch_one<NC, VEL, GEN_UPWIND, true, true, false, false, true>(a, s);
+            if (exact) return launch_one<NC, VEL, GEN_UPWIND, true, false, false, false, true>(a, s);
+        }
+        if (exact || coef || st != GEN_UPWIND) return hipErrorInvalidValue;
+        if (gen) return launch_one<NC, VEL, GEN_UPWIND, false, true, false, false, true>(a, s);
+        return launch_one<NC, VEL, GEN_UPWIND, false, false, false, false, true>(a, s);
     }
-    return hipGetLastError();
+    switch (st) {
+    case GEN_UPWIND: return launch_st<NC, VEL, GEN_UPWIND>(exact, gen, coef, a, s);
+    case GEN_PREDICT: return launch_st<NC, VEL, GEN_PREDICT>(exact, gen, coef, a, s);
+    case GEN_CORRECT: return launch_st<NC, VEL, GEN_CORRECT>(exact, gen, coef, a, s);
+    default: return hipErrorInvalidValue;
+    }
 }
 
 } // namespace
 
 hipError_t launch_pores(int nc, bool vel, int st, bool exact, bool gen, bool coef, const PoreArgs& a, hipStream_t s)
 {
-    if (a.ntiles < 1 || a.gpt < 1) return hipErrorInvalidValue;
-#define GO(N, V) \
-    case 2 * N + V: return launch_pores_nc<N, (V) != 0>(st, exact, gen, coef, a, s)
+    if (a.ntiles < 1 || (!a.inst && a.gpt < 1)) return hipErrorInvalidValue;
     switch (nc * 2 + (vel ? 1 : 0)) {
-        GO(1, 0);
-        GO(1, 1);
-        GO(2, 0);
-        GO(2, 1);
-        GO(3, 0);
-        GO(3, 1);
+    case 2: return launch_nc<1, false>(st, exact, gen, coef, a, s);
+    case 3: return launch_nc<1, true>(st, exact, gen, coef, a, s);
+    case 4: return launch_nc<2, false>(st, exact, gen, coef, a, s);
+    case 5: return launch_nc<2, true>(st, exact, gen, coef, a, s);
+    case 6: return launch_nc<3, false>(st, exact, gen, coef, a, s);
+    case 7: return launch_nc<3, true>(st, exact, gen, coef, a, s);
     default: return hipErrorInvalidValue;
     }
-#undef GO
 }
 
 } // namespace nmr
