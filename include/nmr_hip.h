@@ -268,9 +268,11 @@ int nmr_hip_batch_upload(nmr_batch* b, int32_t i, const uint8_t* mask, const dou
                          const double* vz, const double* mx, const double* my, const double* mz);
 int nmr_hip_batch_download(nmr_batch* b, int32_t i, double* mx, double* my, double* mz);
 /* Device layout of the batch (no reference counterpart): 1 (the default)
- * keeps every instance's state and per-voxel face-velocity sums in bricks
- * of 8 x-voxels by 4 rows from run to run, as nmr_hip_set_layout does for one domain; 0 sweeps
- * the row layout.  The fields are the same bits either way. */
+ * keeps every instance's state and per-voxel face-velocity sums converted
+ * from run to run, as nmr_hip_set_layout does for one domain: with the
+ * automatic tile in one list of the pores of all instances, else in bricks of
+ * 8 x-voxels by 4 rows; 0 sweeps the row layout.  The fields are the same
+ * bits either way. */
 int nmr_hip_batch_set_layout(nmr_batch* b, int32_t brick);
 /* signal (nullable): [ninst][nsteps+1][ncomp]; step counting continues
  * across calls (the gradient schedule sees steps 0, 1, ... since create). */
@@ -284,8 +286,10 @@ int nmr_hip_batch_set_tile(nmr_batch* b, int32_t variant, int32_t lz, int32_t gr
 /* Times every one-step tile variant (and -3), z-chunk and grid kind on this batch
  * (repeated single steps from the current state, which stays unchanged),
  * times the four fastest again over three times the steps on the warm
- * device, and keeps the fastest of those; the choice is cached per set of
- * instance shapes.  Any output pointer may be NULL. */
+ * device, and keeps the fastest of those; then times the list of the pores
+ * against it.  Where the list is faster, runs take it as long as the tile
+ * that this call returned is set.  The choice is cached per set of instance
+ * shapes.  Any output pointer may be NULL. */
 int nmr_hip_batch_autotune(nmr_batch* b, int32_t trial_steps, int32_t* variant, int32_t* lz,
                            int32_t* persistent);
 /* GPU ms of the last run's steps and the voxel-steps they advanced. */

@@ -778,12 +778,9 @@ bool pore_plain(const nmr_ctx* c)
 // without flow, 0.5 / 0.8 (188 MB) / 1: 29.3 / 41.0 / 47.8 against 36.4 / 39.0 /
 // 39.2; 160^3 MacCormack, 1 (172 MB): 47.9 against 54.1; 512x512x256, 1: 511
 // against 388; 64^3, one component, 1: 2.9 against 9.4.
-bool pores_pay(const nmr_ctx* c, uint64_t slots)
+bool pores_pay(double slots, double voxels, int state_words, bool vel)
 {
-    const nmr_problem& p = c->prob;
-    const double vox = (double)p.nx * p.ny * p.nz;
-    const double words = (p.scheme == NMR_SCHEME_MACCORMACK ? 3 : 2) * c->nc + (c->vel ? 3 : 0) + 1.5;
-    return (double)slots <= 0.6 * vox || 4.0 * words * (double)slots <= 180e6;
+    return slots <= 0.6 * voxels || 4.0 * (state_words + (vel ? 3 : 0) + 1.5) * slots <= 180e6;
 }
 
 // Builds the list for the current mask and velocity.
@@ -810,20 +807,26 @@ int build_pores(nmr_ctx* c)
     b.read_solids = p.scheme == NMR_SCHEME_UPWIND && c->vel && !c->inert && !(p.flags & NMR_F_ADVECT_MASK);
     signal_window(p, b.w);
     b.first = 64;
+    const size_t rows = (size_t)p.ny * p.nz;
+    if ((rc = nmri::pores_temp(&b, rows, (size_t)p.nz, rows * c->pitch, c->stream))) return rc;
+    struct Temp {
+        nmr::PoreBuild* b;
+        ~Temp() { nmri::pores_drop_temp(b); }
+    } temp{&b};
     uint64_t end = 0;
-    if ((rc = nmri::pores_count(&b, c->stream, &end))) return rc;
-    if (!nmri::pores_fit(end) || !pores_pay(c, end)) {
-        nmri::pores_drop_temp(&b);
+    HIP_TRY(nmr::launch_pore_count(b, c->stream));
+    HIP_TRY(hipMemcpyAsync(&end, b.planes + p.nz, sizeof(end), hipMemcpyDeviceToHost, c->stream));
+    HIP_TRY(hipStreamSynchronize(c->stream));
+    if (!nmri::pores_fit(end) ||
+        !pores_pay((double)end, (double)p.nx * p.ny * p.nz, (p.scheme == NMR_SCHEME_MACCORMACK ? 3 : 2) * c->nc, c->vel))
         return NMR_OK;
-    }
     const nmri::PoreNeeds n{c->nc, c->vel, ghosts || b.read_solids, p.bc[0] != NMR_BC_NEUMANN,
                             p.scheme == NMR_SCHEME_MACCORMACK};
-    if ((rc = nmri::pores_alloc(&c->pl, (uint32_t)end, n, c->stream, &c->device_bytes))) {
-        nmri::pores_drop_temp(&b);
-        return rc;
-    }
+    if ((rc = nmri::pores_alloc(&c->pl, (uint32_t)end, n, c->stream, &c->device_bytes))) return rc;
     c->pl_reads_solids = b.read_solids != 0;
-    return nmri::pores_link(&c->pl, &b, end, c->stream, &c->pl_ok);
+    nmri::pores_into(c->pl, &b, end);
+    HIP_TRY(nmr::launch_pore_link(b, c->stream));
+    return nmri::pores_finish(&c->pl, b, c->stream, &c->pl_ok);
 }
 
 // Whether the solids' magnetization is finite: their value reaches no pore
@@ -1935,7 +1938,7 @@ int nmr_hip_run_static(nmr_ctx* ctx, int64_t nsteps, const double* grad_sched, d
 namespace {
 
 std::mutex g_tune_mu;
-struct Tuned { int variant, lz, persistent; std::array<double, 7> cost; };
+struct Tuned { int variant, lz, persistent; bool list; std::array<double, 7> cost; };
 std::map<std::vector<int>, Tuned> g_tune_cache; // shapes -> fastest launch
 
 void batch_free(nmr_batch* b)
@@ -1955,7 +1958,8 @@ void batch_free(nmr_batch* b)
         if (I.vy) (void)hipFree(I.vy);
         if (I.vz) (void)hipFree(I.vz);
     }
-    for (void* p : {(void*)b->d_inst, (void*)b->d_tiles, (void*)b->d_off, (void*)b->d_ids, (void*)b->d_step,
+    nmri::pores_free(&b->pl);
+    for (void* p : {(void*)b->d_pinst, (void*)b->d_ptiles, (void*)b->d_poff, (void*)b->d_inst, (void*)b->d_tiles, (void*)b->d_off, (void*)b->d_ids, (void*)b->d_step,
                     (void*)b->d_part, (void*)b->d_signal, (void*)b->d_fpart, (void*)b->d_flag})
         if (p) (void)hipFree(p);
     if (b->h_signal) (void)hipHostFree(b->h_signal);
@@ -2029,6 +2033,7 @@ int batch_inst_to_bricks(nmr_batch* b, int i)
 int batch_bricks(nmr_batch* b)
 {
     if (b->home & nmri::kHomeBricks) return NMR_OK;
+    if (int rc = nmri::batch_rows(b)) return rc;
     for (int i = 0; i < b->ninst; i++) {
         int rc = batch_inst_to_bricks(b, i);
         if (rc) return rc;
@@ -2056,6 +2061,194 @@ int mixed_variant(int nx, int ny, const double* cost)
         }
     }
     return best;
+}
+
+// Coefficients of an instance without the gradient, which the kernels choose
+// per step, and its pulsed-gradient pair.
+nmr::PoreInst batch_coef(const nmr_problem& p, const nmr_batch_instance& s)
+{
+    nmr::PoreInst d{};
+    nmr_problem q = p;
+    q.rho1 = s.rho1;
+    q.rho2 = s.rho2;
+    q.flags &= ~NMR_F_PRECESSION;
+    nmr_ctx tmp;
+    tmp.prob = q;
+    const double g0[3] = {0.0, 0.0, 0.0};
+    d.c = make_coef(&tmp, g0);
+    d.nd = (int)std::lround(s.delta / p.dt);
+    d.nD = (int)std::lround(s.big_delta / p.dt);
+    // same rounding as make_coef for a gradient (0, 0, G)
+    d.bgz = (p.flags & NMR_F_PRECESSION) ? (float)(p.dt * p.gamma * s.grad_amp * p.dz) : 0.f;
+    return d;
+}
+
+// ---- the list of the pores of all instances ----
+// One launch a step over consecutive groups, each workgroup in one instance:
+// no tile is padded and the launch is even.  256 instances of edge 32-128:
+// 428.6 us a step against 1018 on the fastest tile (64x16 bricks).
+
+// Builds the list for the uploaded instances.
+int build_batch_pores(nmr_batch* b)
+{
+    b->pl_tried = true;
+    b->pl_ok = b->pl_reads_solids = false;
+    const nmr_problem& p = b->prob;
+    size_t rows = 0, planes = 0, voxels = 0;
+    double grid = 0.0;
+    for (int i = 0; i < b->ninst; i++) {
+        const nmr_batch_instance& s = b->spec[i];
+        const auto& I = b->inst[i];
+        if (!I.solids_ok || (b->nc == 3 && (s.nx > 65536 || s.ny > 65536))) return NMR_OK;
+        rows = std::max(rows, (size_t)s.ny * s.nz);
+        planes = std::max(planes, (size_t)s.nz);
+        voxels = std::max(voxels, I.n_m);
+        grid += (double)s.nx * s.ny * s.nz;
+        b->pl_reads_solids = b->pl_reads_solids || (b->vel && !I.inert);
+    }
+    nmr::PoreBuild t{};
+    int rc = nmri::pores_temp(&t, rows, planes, voxels, b->stream);
+    if (rc) return rc;
+    uint64_t* ends = nullptr;
+    struct Temp {
+        nmr::PoreBuild* t;
+        uint64_t** e;
+        ~Temp()
+        {
+            nmri::pores_drop_temp(t);
+            if (*e) (void)hipFree(*e);
+        }
+    } temp{&t, &ends};
+    HIP_TRY(hipMalloc((void**)&ends, (size_t)b->ninst * sizeof(uint64_t)));
+    auto domain = [&](int i) {
+        const nmr_batch_instance& s = b->spec[i];
+        const auto& I = b->inst[i];
+        t.mask = I.mask;
+        t.nx = s.nx;
+        t.ny = s.ny;
+        t.nz = s.nz;
+        t.pitch = I.pitch;
+        t.read_solids = b->vel && !I.inert;
+        t.w[0] = p.buffer[0]; t.w[1] = s.nx - p.buffer[0];
+        t.w[2] = p.buffer[1]; t.w[3] = s.ny - p.buffer[1];
+        t.w[4] = p.buffer[2]; t.w[5] = s.nz - p.buffer[2];
+    };
+    // slots of every instance
+    for (int i = 0; i < b->ninst; i++) {
+        domain(i);
+        t.first = 0;
+        HIP_TRY(nmr::launch_pore_count(t, b->stream));
+        HIP_TRY(hipMemcpyAsync(ends + i, t.planes + t.nz, sizeof(uint64_t), hipMemcpyDeviceToDevice, b->stream));
+    }
+    std::vector<uint64_t> n(b->ninst);
+    HIP_TRY(hipMemcpyAsync(n.data(), ends, n.size() * sizeof(uint64_t), hipMemcpyDeviceToHost, b->stream));
+    HIP_TRY(hipStreamSynchronize(b->stream));
+    uint64_t end = 64;
+    for (uint64_t v : n) end += v;
+    if (!nmri::pores_fit(end) || !pores_pay((double)end, grid, 2 * b->nc, b->vel)) return NMR_OK;
+    int64_t bytes = 0;
+    const nmri::PoreNeeds needs{b->nc, b->vel, b->pl_reads_solids, false, false};
+    if ((rc = nmri::pores_alloc(&b->pl, (uint32_t)end, needs, b->stream, &bytes))) return rc;
+    // link them; tiles of whole groups, instance by instance
+    int per = nmri::pores_per_tile((int64_t)(end / 64));
+    const size_t S = (size_t)std::max(b->graph_steps, 2);
+    while ((end / 64 / per) * S * b->nc * sizeof(double) > ((size_t)128 << 20)) per *= 2; // partial sums of a chunk
+    std::vector<nmr::PoreTile> tiles;
+    std::vector<int> off(b->ninst + 1, 0);
+    std::vector<nmr::PoreInst> pi(b->ninst);
+    t.first = 64;
+    for (int i = 0; i < b->ninst; i++) {
+        domain(i);
+        HIP_TRY(nmr::launch_pore_count(t, b->stream));
+        nmri::pores_into(b->pl, &t, t.first + n[i]);
+        HIP_TRY(nmr::launch_pore_link(t, b->stream));
+        auto& I = b->inst[i];
+        I.slot0 = (uint32_t)t.first;
+        I.slot1 = (uint32_t)(t.first + n[i]);
+        if (b->vel)
+            for (int q = 0; q < 3; q++)
+                HIP_TRY(nmr::launch_pore_gather(I.adv[q], b->pl.vox, I.slot0, I.slot1, 4, 1 + q,
+                                                reinterpret_cast<float*>(b->pl.rec), b->stream));
+        for (uint32_t g = I.slot0 / 64; g < I.slot1 / 64; g += (uint32_t)per)
+            tiles.push_back({g, std::min((uint32_t)per, I.slot1 / 64 - g), (uint32_t)i});
+        off[i + 1] = (int)tiles.size();
+        pi[i] = batch_coef(p, b->spec[i]);
+        t.first += n[i];
+    }
+    if (b->vel) HIP_TRY(nmr::launch_pore_record(b->pl.off8, b->pl.nslots, b->pl.rec, b->stream));
+    bool ok = false;
+    if ((rc = nmri::pores_finish(&b->pl, t, b->stream, &ok)) || !ok) return rc;
+    for (void** q : {(void**)&b->d_pinst, (void**)&b->d_ptiles, (void**)&b->d_poff}) {
+        if (*q) HIP_TRY(hipFree(*q));
+        *q = nullptr;
+    }
+    if ((rc = balloc(b->stream, &b->d_pinst, pi.size())) || (rc = balloc(b->stream, &b->d_ptiles, tiles.size())) ||
+        (rc = balloc(b->stream, &b->d_poff, off.size())))
+        return rc;
+    HIP_TRY(hipMemcpy(b->d_pinst, pi.data(), pi.size() * sizeof(pi[0]), hipMemcpyHostToDevice));
+    HIP_TRY(hipMemcpy(b->d_ptiles, tiles.data(), tiles.size() * sizeof(tiles[0]), hipMemcpyHostToDevice));
+    HIP_TRY(hipMemcpy(b->d_poff, off.data(), off.size() * sizeof(int), hipMemcpyHostToDevice));
+    b->pl_ntiles = (int)tiles.size();
+    b->pl_ok = true;
+    return NMR_OK;
+}
+
+// Whether the next run sweeps the list: the layout switch on, no tile set
+// (or the autotuner's, where the list was faster), and a list that fits.
+int batch_use_pores(nmr_batch* b, bool* yes)
+{
+    *yes = false;
+    if (!b->brick_on) return NMR_OK;
+    const bool chosen = b->tuned && b->variant == b->tuned_variant && b->lz == b->tuned_lz &&
+                        b->persistent == b->tuned_persistent;
+    if (chosen ? !b->tuned_list : b->variant != -1) return NMR_OK;
+    if (!b->pl_tried)
+        if (int rc = build_batch_pores(b)) return rc;
+    *yes = b->pl_ok;
+    return NMR_OK;
+}
+
+// Every instance's state into the list unless it is there.
+int batch_state_pores(nmr_batch* b)
+{
+    if (b->home & nmri::kHomePores) return NMR_OK;
+    if (int rc = nmri::batch_rows(b)) return rc;
+    for (int i = 0; i < b->ninst; i++)
+        for (int q = 0; q < b->nc; q++)
+            HIP_TRY(nmr::launch_pore_gather(b->inst[i].m[b->parity][q], b->pl.vox, b->inst[i].slot0, b->inst[i].slot1,
+                                            b->nc, q, b->pl.state[0], b->stream));
+    b->ppar = 0;
+    b->home |= nmri::kHomePores;
+    return NMR_OK;
+}
+
+nmr::PoreArgs batch_pore_args(const nmr_batch* b, int parity, int local, double* part)
+{
+    nmr::PoreArgs a{};
+    a.f = b->pl.state[parity];
+    a.out = b->pl.state[parity ^ 1];
+    a.groups = b->pl.groups;
+    a.aux = b->pl_reads_solids ? b->pl.aux : nullptr;
+    a.rec = b->pl.rec;
+    a.off8 = b->pl.off8;
+    a.off16 = b->pl.off16;
+    a.xy = b->pl.xy;
+    a.partials = part;
+    a.ntiles = b->pl_ntiles;
+    a.ngroups = b->pl.ngroups();
+    a.wide = b->pl.wide ? 1 : 0;
+    a.tiles = b->d_ptiles;
+    a.inst = b->d_pinst;
+    a.step_base = b->d_step;
+    a.local_step = local;
+    return a;
+}
+
+int batch_pore_step(nmr_batch* b, int local, int parity, double* part)
+{
+    HIP_TRY(nmr::launch_pores(b->nc, b->vel, nmr::GEN_UPWIND, b->exact, b->pl_reads_solids, false,
+                              batch_pore_args(b, parity, local, part), b->stream));
+    return NMR_OK;
 }
 
 // Tile list, descriptors and grid for (variant, lz, grid kind); variant -3
@@ -2098,18 +2291,11 @@ int batch_prepare(nmr_batch* b, int variant, int lz, int persistent, bool brick)
         d.by0 = p.buffer[1]; d.by1 = s.ny - p.buffer[1];
         d.bz0 = p.buffer[2]; d.bz1 = s.nz - p.buffer[2];
         d.inert = I.inert;
-        nmr_problem q = p;
-        q.rho1 = s.rho1;
-        q.rho2 = s.rho2;
-        q.flags &= ~NMR_F_PRECESSION; // the gradient is chosen per step in the kernel
-        nmr_ctx tmp;
-        tmp.prob = q;
-        const double g0[3] = {0.0, 0.0, 0.0};
-        d.c = make_coef(&tmp, g0);
-        d.nd = (int)std::lround(s.delta / p.dt);
-        d.nD = (int)std::lround(s.big_delta / p.dt);
-        // same rounding as make_coef for a gradient (0, 0, G)
-        d.bgz = (p.flags & NMR_F_PRECESSION) ? (float)(p.dt * p.gamma * s.grad_amp * p.dz) : 0.f;
+        const nmr::PoreInst pi = batch_coef(p, s);
+        d.c = pi.c;
+        d.nd = pi.nd;
+        d.nD = pi.nD;
+        d.bgz = pi.bgz;
         const int n = d.ntx * d.nty * d.ntz;
         for (int t = 0; t < n; t++) {
             const int tz = t / (d.ntx * d.nty);
@@ -2191,9 +2377,9 @@ int batch_prepare(nmr_batch* b, int variant, int lz, int persistent, bool brick)
     return NMR_OK;
 }
 
-int batch_partials(nmr_batch* b, size_t steps)
+int batch_partials(nmr_batch* b, size_t steps, int ntiles)
 {
-    const size_t need = steps * (size_t)b->ntiles * b->nc;
+    const size_t need = steps * (size_t)ntiles * b->nc;
     if (need <= b->part_cap) return NMR_OK;
     if (b->d_part) HIP_TRY(hipFree(b->d_part));
     b->d_part = nullptr;
@@ -2227,9 +2413,18 @@ void batch_auto(const nmr_batch* b, int* variant, int* lz)
     *lz = 8;
 }
 
+// Remembers the autotuner's tile: while it is set, tuned_list decides.
+void set_tuned(nmr_batch* b)
+{
+    b->tuned = true;
+    b->tuned_variant = b->variant;
+    b->tuned_lz = b->lz;
+    b->tuned_persistent = b->persistent;
+}
+
 std::vector<int> batch_key(const nmr_batch* b)
 {
-    std::vector<int> k = {b->nc, (int)b->vel, (int)b->exact};
+    std::vector<int> k = {b->nc, (int)b->vel, (int)b->exact, (int)b->brick_on};
     for (const auto& s : b->spec) {
         k.push_back(s.nx);
         k.push_back(s.ny);
@@ -2339,6 +2534,12 @@ int nmr_hip_batch_upload(nmr_batch* b, int32_t i, const uint8_t* mask, const dou
     auto& I = b->inst[i];
     const int P = I.pitch, P1 = I.pitch1;
     int rc = NMR_OK;
+    if (b->home & nmri::kHomePores) { // the other instances' states leave the list, which the new mask ends
+        if ((rc = nmri::batch_rows(b))) return rc;
+        HIP_TRY(hipStreamSynchronize(b->stream));
+        b->home &= ~nmri::kHomePores;
+    }
+    b->pl_tried = b->pl_ok = false;
     {
         std::vector<uint8_t> h(I.n_m, 0);
         int64_t np = 0;
@@ -2388,11 +2589,12 @@ int nmr_hip_batch_upload(nmr_batch* b, int32_t i, const uint8_t* mask, const dou
                         (float)src[q][(size_t)x + (size_t)s.nx * ((size_t)j + (size_t)s.ny * k)];
         for (int par = 0; par < 2; par++) HIP_TRY(hipMemcpy(I.m[par][q], h.data(), h.size() * 4, hipMemcpyHostToDevice));
     }
-    // inertness of this instance (no velocity on faces touching solid)
-    if (!b->vel) {
-        I.inert = 1;
-    } else {
-        HIP_TRY(hipMemsetAsync(b->d_flag, 0, sizeof(int), b->stream));
+    // inertness of this instance (no velocity on faces touching solid), and
+    // whether its solids' magnetization is finite
+    HIP_TRY(hipMemsetAsync(b->d_flag, 0, 2 * sizeof(int), b->stream));
+    for (int q = 0; q < b->nc; q++)
+        HIP_TRY(nmr::launch_solids_finite(I.m[b->parity][q], I.mask, I.n_m, b->d_flag + 1, b->stream));
+    if (b->vel) {
         nmr::InertArgs a{};
         a.mask = I.mask;
         a.vx = I.vx;
@@ -2416,11 +2618,12 @@ int nmr_hip_batch_upload(nmr_batch* b, int32_t i, const uint8_t* mask, const dou
         v.pitch = P;
         v.pitch1 = P1;
         HIP_TRY(nmr::launch_adv(v, b->stream));
-        int f = 0;
-        HIP_TRY(hipMemcpyAsync(&f, b->d_flag, sizeof(int), hipMemcpyDeviceToHost, b->stream));
-        HIP_TRY(hipStreamSynchronize(b->stream));
-        I.inert = f == 0;
     }
+    int f[2] = {0, 0};
+    HIP_TRY(hipMemcpyAsync(f, b->d_flag, sizeof(f), hipMemcpyDeviceToHost, b->stream));
+    HIP_TRY(hipStreamSynchronize(b->stream));
+    I.inert = f[0] == 0;
+    I.solids_ok = f[1] == 0;
     I.uploaded = true;
     I.adv_bricks = false;
     // the rows hold the new state (both buffers); so do the bricks if they
@@ -2439,10 +2642,17 @@ int nmr_hip_batch_download(nmr_batch* b, int32_t i, double* mx, double* my, doub
     double* dst[3] = {mx, my, mz};
     const nmr_batch_instance& s = b->spec[i];
     auto& I = b->inst[i];
-    if (!(b->home & nmri::kHomeRows)) // the instance's current buffer from the bricks
-        for (int q = 0; q < b->nc; q++)
+    if (!(b->home & nmri::kHomeRows)) { // the instance's current buffer from the list or the bricks
+        for (int q = 0; q < b->nc; q++) {
+            if (b->home & nmri::kHomePores) {
+                HIP_TRY(nmr::launch_pore_scatter(b->pl.state[b->ppar], b->pl.vox, I.slot0, I.slot1, b->nc, q,
+                                                 I.m[b->parity][q], nullptr, b->stream));
+                continue;
+            }
             HIP_TRY(nmr::launch_brick(I.mb[b->parity][q], I.m[b->parity][q], I.pitch / 4, s.ny, s.nz, false,
                                       b->stream));
+        }
+    }
     HIP_TRY(hipStreamSynchronize(b->stream));
     std::vector<float> h(I.n_m);
     for (int q = 0; q < b->nc; q++) {
@@ -2494,6 +2704,8 @@ int nmr_hip_batch_autotune(nmr_batch* b, int32_t trial_steps, int32_t* variant, 
             b->variant = it->second.variant;
             b->lz = it->second.lz;
             b->persistent = it->second.persistent;
+            b->tuned_list = it->second.list;
+            set_tuned(b);
             b->tile_cost = it->second.cost;
             b->cur_variant = -2; // the per-instance shapes may have changed
             if (variant) *variant = b->variant;
@@ -2515,7 +2727,7 @@ int nmr_hip_batch_autotune(nmr_batch* b, int32_t trial_steps, int32_t* variant, 
     auto time_cfg = [&](int v, int l, int per, int n, double* ms_out) -> int {
         int rc = batch_prepare(b, v, l, per, brick);
         if (rc) return rc;
-        if ((rc = batch_partials(b, 1))) return rc;
+        if ((rc = batch_partials(b, 1, b->ntiles))) return rc;
         if ((rc = batch_launch_step(b, 0, b->parity, b->d_part))) return rc;
         HIP_TRY(hipEventRecord(b->ev0, b->stream));
         for (int r = 0; r < n; r++)
@@ -2585,9 +2797,31 @@ int nmr_hip_batch_autotune(nmr_batch* b, int32_t trial_steps, int32_t* variant, 
     b->variant = bv;
     b->lz = bl;
     b->persistent = bp;
+    // the list of the pores against the fastest tile
+    b->tuned = b->tuned_list = false;
+    if (b->brick_on) {
+        b->variant = -1;
+        bool list = false;
+        int rc = batch_use_pores(b, &list);
+        b->variant = bv;
+        if (rc) return rc;
+        if (list) {
+            if ((rc = batch_state_pores(b)) || (rc = batch_partials(b, 1, b->pl_ntiles))) return rc;
+            if ((rc = batch_pore_step(b, 0, b->ppar, b->d_part))) return rc;
+            HIP_TRY(hipEventRecord(b->ev0, b->stream));
+            for (int r = 0; r < 3 * trials; r++)
+                if ((rc = batch_pore_step(b, 0, b->ppar, b->d_part))) return rc;
+            HIP_TRY(hipEventRecord(b->ev1, b->stream));
+            HIP_TRY(hipEventSynchronize(b->ev1));
+            float ms = 0.f;
+            HIP_TRY(hipEventElapsedTime(&ms, b->ev0, b->ev1));
+            b->tuned_list = ms / (3 * trials) < best;
+        }
+    }
+    set_tuned(b);
     {
         std::lock_guard<std::mutex> g(g_tune_mu);
-        g_tune_cache[key] = {bv, bl, bp, b->tile_cost};
+        g_tune_cache[key] = {bv, bl, bp, b->tuned_list, b->tile_cost};
     }
     if (variant) *variant = bv;
     if (lz) *lz = bl;
@@ -2616,15 +2850,23 @@ int nmr_hip_batch_run(nmr_batch* b, int64_t nsteps, double* signal)
         if (v < 0) v = av;
         if (l <= 0) l = al;
     }
-    // the state stays in bricks from run to run when the layout allows
-    const bool brick = b->brick_on && batch_bricks_fit(b);
-    int rc = brick ? batch_bricks(b) : nmri::batch_rows(b);
+    // the state stays in the list of the pores or in bricks from run to run
+    // when the layout allows
+    bool list = false;
+    int rc = batch_use_pores(b, &list);
     if (rc) return rc;
-    if ((rc = batch_prepare(b, v, l, b->persistent, brick))) return rc;
+    const bool brick = !list && b->brick_on && batch_bricks_fit(b);
+    if (list) {
+        if ((rc = batch_state_pores(b))) return rc;
+    } else {
+        if ((rc = brick ? batch_bricks(b) : nmri::batch_rows(b))) return rc;
+        if ((rc = batch_prepare(b, v, l, b->persistent, brick))) return rc;
+    }
+    const int ntiles = list ? b->pl_ntiles : b->ntiles;
     const int nc = b->nc;
     const int64_t rows = nsteps + 1;
     const int S = b->graph_steps;
-    if ((rc = batch_partials(b, (size_t)std::max(S, 2)))) return rc;
+    if ((rc = batch_partials(b, (size_t)std::max(S, 2), ntiles))) return rc;
     const size_t need = (size_t)b->ninst * rows * nc;
     if (need > b->signal_cap) {
         // room for runs of up to kChunkSteps steps, so that a short warm-up
@@ -2642,7 +2884,17 @@ int nmr_hip_batch_run(nmr_batch* b, int64_t nsteps, double* signal)
     b->sig_now.resize((size_t)b->ninst * nc, 0.0);
     const std::vector<uint8_t> have0 = b->sig_ok;
     const std::vector<double> sig0 = b->sig_now;
-    for (int i = 0; i < b->ninst; i++) {
+    const int step0 = (int)b->steps_done;
+    // the device step counter holds the global step (the gradient schedule
+    // reads it); signal rows count from this run's first step
+    HIP_TRY(hipMemcpyAsync(b->d_step, &step0, sizeof(int), hipMemcpyHostToDevice, b->stream));
+    if (list && std::find(have0.begin(), have0.end(), 0) != have0.end()) {
+        // row 0 of every instance at once
+        HIP_TRY(nmr::launch_pore_sum(nc, batch_pore_args(b, b->ppar, 0, b->d_part), b->stream));
+        HIP_TRY(nmr::launch_batch_reduce(b->d_part, ntiles, nc, b->d_poff, nullptr, b->d_step, step0 + 1, rows, b->d_signal,
+                                         1, b->ninst, b->stream));
+    }
+    for (int i = 0; i < b->ninst && !list; i++) {
         if (have0[i]) continue;
         const nmr_batch_instance& s = b->spec[i];
         nmr::FieldSumArgs a{};
@@ -2664,10 +2916,6 @@ int nmr_hip_batch_run(nmr_batch* b, int64_t nsteps, double* signal)
         HIP_TRY(nmr::launch_field_sum(nc, a, b->stream));
         HIP_TRY(nmr::launch_reduce_partials(b->d_fpart, 1, nfb, nc, b->d_signal + (size_t)i * rows * nc, b->stream));
     }
-    // the device step counter holds the global step (the gradient schedule
-    // reads it); signal rows count from this run's first step
-    const int step0 = (int)b->steps_done;
-    HIP_TRY(hipMemcpyAsync(b->d_step, &step0, sizeof(int), hipMemcpyHostToDevice, b->stream));
     HIP_TRY(hipStreamSynchronize(b->stream));
     int64_t done = 0;
     hipGraphExec_t exec = nullptr;
@@ -2675,11 +2923,13 @@ int nmr_hip_batch_run(nmr_batch* b, int64_t nsteps, double* signal)
     HIP_TRY(hipEventRecord(b->ev0, b->stream));
     auto enqueue_chunk = [&](int n) -> int {
         for (int s = 0; s < n; s++) {
-            int r = batch_launch_step(b, s, (b->parity + s) & 1, b->d_part + (size_t)s * b->ntiles * nc);
+            double* part = b->d_part + (size_t)s * ntiles * nc;
+            int r = list ? batch_pore_step(b, s, (b->ppar + s) & 1, part)
+                         : batch_launch_step(b, s, (b->parity + s) & 1, part);
             if (r) return r;
         }
-        HIP_TRY(nmr::launch_batch_reduce(b->d_part, b->ntiles, nc, b->d_off, b->d_ids, b->d_step, step0, rows,
-                                         b->d_signal, n, b->ninst, b->stream));
+        HIP_TRY(nmr::launch_batch_reduce(b->d_part, ntiles, nc, list ? b->d_poff : b->d_off, list ? nullptr : b->d_ids,
+                                         b->d_step, step0, rows, b->d_signal, n, b->ninst, b->stream));
         HIP_TRY(nmr::launch_step_advance(b->d_step, n, b->stream));
         return NMR_OK;
     };
@@ -2703,11 +2953,11 @@ int nmr_hip_batch_run(nmr_batch* b, int64_t nsteps, double* signal)
     while (done < nsteps) {
         const int n = (int)std::min<int64_t>(std::max(S, 2), nsteps - done);
         if ((rc = enqueue_chunk(n))) return rc;
-        b->parity = (b->parity + n) & 1;
+        (list ? b->ppar : b->parity) ^= n & 1;
         done += n;
     }
     HIP_TRY(hipEventRecord(b->ev1, b->stream));
-    b->home = brick ? nmri::kHomeBricks : nmri::kHomeRows;
+    if (nsteps > 0) b->home = list ? nmri::kHomePores : (brick ? nmri::kHomeBricks : nmri::kHomeRows);
     // The signal rows go to the host in one copy of the whole
     // [ninst][rows][nc] block: into the caller's buffer, else into pinned
     // staging (up to kBatchStage doubles), and the last row of every
@@ -2770,6 +3020,12 @@ int batch_rows(nmr_batch* b)
     for (int i = 0; i < b->ninst; i++) {
         const auto& s = b->spec[i];
         auto& I = b->inst[i];
+        if (b->home & kHomePores) { // both row buffers still hold the solids' values
+            for (int q = 0; q < b->nc; q++)
+                HIP_TRY(nmr::launch_pore_scatter(b->pl.state[b->ppar], b->pl.vox, I.slot0, I.slot1, b->nc, q, I.m[0][q],
+                                                 I.m[1][q], b->stream));
+            continue;
+        }
         for (int p = 0; p < 2; p++)
             for (int q = 0; q < b->nc; q++)
                 HIP_TRY(nmr::launch_brick(I.mb[b->parity][q], I.m[p][q], I.pitch / 4, s.ny, s.nz, false, b->stream));

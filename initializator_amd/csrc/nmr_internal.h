@@ -71,14 +71,15 @@ struct PoreNeeds {
 // per-voxel arrays pv are made by who gathers them; they go when the list grows.
 int pores_alloc(PoreList* L, uint32_t nslots, const PoreNeeds& n, hipStream_t s, int64_t* bytes);
 void pores_free(PoreList* L);
-// Slots of one domain (b.first is set, b's temporary arrays are made here):
-// counts them and gives the slot past the last one in *end (waits for the
-// stream).  pores_link then assigns and links them in the list's arrays
-// (waits too), notes wide groups in the list and releases the temporary
-// arrays; *ok: every offset fits.
-int pores_count(nmr::PoreBuild* b, hipStream_t s, uint64_t* end);
-int pores_link(PoreList* L, nmr::PoreBuild* b, uint64_t end, hipStream_t s, bool* ok);
+// Building: temporary arrays for domains of up to `rows` rows, `planes` planes
+// and `voxels` voxels (row layout); per domain, with first set,
+// launch_pore_count (planes[nz] is then the slot past its last one) and, with
+// the list's arrays taken by pores_into, launch_pore_link.
+int pores_temp(nmr::PoreBuild* b, size_t rows, size_t planes, size_t voxels, hipStream_t s);
 void pores_drop_temp(nmr::PoreBuild* b);
+void pores_into(const PoreList& L, nmr::PoreBuild* b, uint64_t end);
+// Waits for the stream; notes wide groups in the list; *ok: every offset fits.
+int pores_finish(PoreList* L, const nmr::PoreBuild& b, hipStream_t s, bool* ok);
 // Groups that a workgroup takes of a list of `groups`.
 int pores_per_tile(int64_t groups);
 // Whether a list of this many slots stays inside the kernels' 32-bit byte offsets.
@@ -190,7 +191,9 @@ struct nmr_batch {
         float *vx = nullptr, *vy = nullptr, *vz = nullptr;
         bool uploaded = false;
         int inert = 0;
+        bool solids_ok = false; // every solid's magnetization is finite
         int64_t npore = 0;
+        uint32_t slot0 = 0, slot1 = 0; // its slots in the list of pores
         // upwind velocity sums of the plain sweep (rows), computed at upload
         float* adv[3] = {nullptr, nullptr, nullptr};
         // brick copies (8 x-voxels by 4 rows) of the state and the velocity sums
@@ -208,6 +211,19 @@ struct nmr_batch {
     // conversion writes both buffers of its target layout)
     bool brick_on = true;
     int home = 1;
+    // the list of the pores of all instances (one launch a step, no padding),
+    // built before its first run after an upload; state[ppar] is current when
+    // home says so
+    nmri::PoreList pl;
+    bool pl_tried = false, pl_ok = false, pl_reads_solids = false;
+    int ppar = 0;
+    nmr::PoreInst* d_pinst = nullptr;
+    nmr::PoreTile* d_ptiles = nullptr;
+    int* d_poff = nullptr; // first tile of every instance
+    int pl_ntiles = 0;
+    // the autotuner's choice: its tile, and whether the list was faster
+    int tuned_variant = -1, tuned_lz = 0, tuned_persistent = 0;
+    bool tuned = false, tuned_list = false;
     // signal of every instance's current state ([ninst][nc], host copy of the
     // last rows of the last run) and, per instance, whether it is still the
     // signal of that state (an upload clears it)

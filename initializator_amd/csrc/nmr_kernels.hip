@@ -1187,7 +1187,8 @@ __global__ void __launch_bounds__(256) batch_kernel(BatchArgs b)
 }
 
 // Per-instance signal rows of a chunk of batched steps: block (s, i) sums the
-// partials of instance i's tiles (fixed order) into signal[i][row][q],
+// partials of instance i's tiles (fixed order; ids null: tiles off[i] ..
+// off[i+1] - 1) into signal[i][row][q],
 // row = *step_base - row0 + s + 1 (row0: the step counter at the run's start).
 __global__ void __launch_bounds__(64) batch_reduce_kernel(const double* __restrict__ part, int ntiles, int nc,
                                                           const int* __restrict__ off, const int* __restrict__ ids,
@@ -1200,7 +1201,7 @@ __global__ void __launch_bounds__(64) batch_reduce_kernel(const double* __restri
     const int64_t row = (int64_t)(*step_base - row0) + s + 1;
     for (int q = 0; q < nc; q++) {
         double v = 0.0;
-        for (int k = off[i] + (int)threadIdx.x; k < off[i + 1]; k += 64) v += p[(size_t)ids[k] * nc + q];
+        for (int k = off[i] + (int)threadIdx.x; k < off[i + 1]; k += 64) v += p[(size_t)(ids ? ids[k] : k) * nc + q];
         sh[threadIdx.x] = v;
         __syncthreads();
         for (int h = 32; h > 0; h >>= 1) {

@@ -105,9 +105,8 @@ void pores_drop_temp(nmr::PoreBuild* b)
     b->overflow = nullptr;
 }
 
-int pores_count(nmr::PoreBuild* b, hipStream_t s, uint64_t* end)
+int pores_temp(nmr::PoreBuild* b, size_t rows, size_t planes, size_t voxels, hipStream_t s)
 {
-    const size_t rows = (size_t)b->ny * (size_t)b->nz;
     b->rows = nullptr;
     b->planes = nullptr;
     b->slotmap = nullptr;
@@ -119,35 +118,34 @@ int pores_count(nmr::PoreBuild* b, hipStream_t s, uint64_t* end)
         return !rc;
     };
     if (check(hipMalloc((void**)&b->rows, rows * sizeof(uint32_t))) &&
-        check(hipMalloc((void**)&b->planes, ((size_t)b->nz + 1) * sizeof(uint64_t))) &&
-        check(hipMalloc((void**)&b->slotmap, rows * (size_t)b->pitch * sizeof(uint32_t))) &&
-        check(hipMalloc((void**)&b->overflow, 256)) && check(hipMemsetAsync(b->overflow, 0, 256, s)) &&
-        check(nmr::launch_pore_count(*b, s)) &&
-        check(hipMemcpyAsync(end, b->planes + b->nz, sizeof(uint64_t), hipMemcpyDeviceToHost, s)))
-        check(hipStreamSynchronize(s));
+        check(hipMalloc((void**)&b->planes, (planes + 1) * sizeof(uint64_t))) &&
+        check(hipMalloc((void**)&b->slotmap, voxels * sizeof(uint32_t))) &&
+        check(hipMalloc((void**)&b->overflow, 256)))
+        check(hipMemsetAsync(b->overflow, 0, 256, s));
     if (rc) pores_drop_temp(b);
     return rc;
 }
 
-int pores_link(PoreList* L, nmr::PoreBuild* b, uint64_t end, hipStream_t s, bool* ok)
+void pores_into(const PoreList& L, nmr::PoreBuild* b, uint64_t end)
 {
-    b->vox = L->vox;
-    b->groups = L->groups;
-    b->aux = L->aux;
-    b->off8 = L->off8;
-    b->off16 = L->off16;
-    b->xoff = L->xoff;
-    b->xy = L->xy;
+    b->vox = L.vox;
+    b->groups = L.groups;
+    b->aux = L.aux;
+    b->off8 = L.off8;
+    b->off16 = L.off16;
+    b->xoff = L.xoff;
+    b->xy = L.xy;
     b->count = (int64_t)((end - b->first) / 64);
-    int over[2] = {0, 0}, rc = NMR_OK;
-    hipError_t e = nmr::launch_pore_link(*b, s);
-    if (e == hipSuccess) e = hipMemcpyAsync(over, b->overflow, sizeof(over), hipMemcpyDeviceToHost, s);
-    if (e == hipSuccess) e = hipStreamSynchronize(s);
-    if (e != hipSuccess) rc = fail(NMR_ERR_DEVICE, "pore list: %s", hipGetErrorString(e));
-    pores_drop_temp(b);
-    *ok = rc == NMR_OK && over[0] == 0;
-    L->wide = L->wide || over[1] != 0;
-    return rc;
+}
+
+int pores_finish(PoreList* L, const nmr::PoreBuild& b, hipStream_t s, bool* ok)
+{
+    int over[2] = {0, 0};
+    HIP_TRY(hipMemcpyAsync(over, b.overflow, sizeof(over), hipMemcpyDeviceToHost, s));
+    HIP_TRY(hipStreamSynchronize(s));
+    *ok = over[0] == 0;
+    L->wide = over[1] != 0;
+    return NMR_OK;
 }
 
 int pores_per_tile(int64_t groups)

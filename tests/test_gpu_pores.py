@@ -9,7 +9,7 @@ import numpy as np
 import pytest
 
 from initializator_amd import generators
-from initializator_amd.solver import HipSolver
+from initializator_amd.solver import BatchSolver, HipSolver
 
 pytestmark = pytest.mark.gpu
 
@@ -107,3 +107,39 @@ def test_solids_that_are_not_finite_leave_it_to_the_tiles():
             s.upload_magnetization(*m0)
             outs.append((s.run(5), s.download_magnetization()))
     _same([outs[0]], [outs[1]])
+
+
+@pytest.mark.parametrize("exact,graph", [(False, 0), (True, 4)])
+def test_batch_list_equals_tiles(exact, graph):
+    """The batch on the list of the pores (the automatic choice) against a tile of the batch: uneven
+    instances, one of them without pores, one with velocity on pore-solid faces, solids that hold values;
+    runs, a download between them, and an instance uploaded again."""
+    kinds = [63, "gaps", "none", "full", "one", 129]
+    rng = np.random.default_rng(11)
+    specs = []
+    for i, k in enumerate(kinds):
+        m = _mask(k)
+        nz, ny, nx = m.shape
+        vel = generators.velocity(m, seed=i, sigma=1.0)
+        if k == "gaps":
+            vel = [rng.uniform(-1e-3, 1e-3, s) for s in ((nz, ny, nx + 1), (nz, ny + 1, nx), (nz + 1, ny, nx))]
+        specs.append(dict(shape=m.shape, mask=m, vel=vel, m0=[rng.random(m.shape), rng.random(m.shape) - 0.4],
+                          rho1=(i + 1) * 1e-6, rho2=(i + 2) * 1e-6, grad_amp=0.1 * (i + 1), delta=3 * DT,
+                          big_delta=(4 + i) * DT))
+    again = [rng.random(specs[1]["shape"]) for _ in range(2)]
+    outs = []
+    for variant in (-1, 4):
+        b = BatchSolver(specs, 2, DX, DT, D, 0.5, velocity=True, precession=True, phase_exact=exact, buffer=(0, 1, 0))
+        b.set_tile(variant, 0, graph, True)
+        for i, s in enumerate(specs):
+            b.upload(i, s["mask"], s["m0"], s["vel"])
+        out = [(b.run(9), b.download(1))]
+        out.append((b.run(5), b.download(3)))
+        b.upload(1, specs[1]["mask"], again, specs[1]["vel"])
+        out.append((b.run(8), sum((b.download(i) for i in range(len(specs))), [])))
+        outs.append(out)
+        b.close()
+    for (sa, fa), (sb, fb) in zip(*outs):
+        for x, y in zip(fa, fb):
+            assert np.array_equal(x, y)
+        np.testing.assert_allclose(sa, sb, rtol=1e-11, atol=1e-13)
