@@ -283,7 +283,7 @@ hipError_t launch_pore_pulse(const PulseArgs& a, float* f, int nc, const uint32_
 
 // ---- learned corrector (nmr_learn_kernels.hip) ----
 // Tensors: BF16 channels-last on the grid padded by one zero voxel per side.
-constexpr int kWgradPart = 27 * 256 + 16; // floats per wavefront partial of wgrad
+constexpr int kWgradPart = 27 * 256 + 16; // floats per partial of wgrad
 
 struct ConvArgs {
     const uint16_t* in;     // [(nz+2)(ny+2)(nx+2)][cin]
@@ -304,7 +304,7 @@ struct ConvArgs {
 struct WgradArgs {
     const uint16_t* in;     // layer input [..][cin]
     const uint16_t* gout;   // output gradient [..][16]
-    float* part;            // [waves][kWgradPart]
+    float* part;            // [npart][kWgradPart]
     int nx, ny, nz;
 };
 
@@ -350,7 +350,8 @@ hipError_t launch_conv_tiled(int cin, int mode, const ConvArgs& a, int grid, hip
 // columns of 16 x 16 output rows by zc planes of the z-marching convolution
 int conv_columns(int nx, int ny, int nz, int zc);
 hipError_t launch_conv_zm(int cin, int mode, const ConvArgs& a, int grid, hipStream_t s);
-hipError_t launch_wgrad(int cin, const WgradArgs& a, int grid, hipStream_t s);
+// npart partial sums
+hipError_t launch_wgrad(int cin, const WgradArgs& a, int npart, hipStream_t s);
 hipError_t launch_wreduce(const float* part, int nwaves, int cin_real, int cout_real, float* grad, hipStream_t s);
 hipError_t launch_pack(const float* w, int cin_real, int cout_real, int cin_store, int backward, uint16_t* frag,
                        hipStream_t s);

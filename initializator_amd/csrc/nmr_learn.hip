@@ -32,7 +32,7 @@ constexpr int kParams = 10402;
 // canonical layout: W1 [16][6][27], b1 [16], W2 [16][16][27], b2 [16], W3 [2][16][27], b3 [2]
 constexpr int kW1 = 0, kB1 = 2592, kW2 = 2608, kB2 = 9520, kW3 = 9536, kB3 = 10400;
 constexpr int kFragF1 = 7 * 512, kFragF = 14 * 512; // uint16 per fragment set (cin 8 / 16)
-constexpr int kWgradGrid = 128;                     // workgroups of the weight-gradient kernel
+constexpr int kWgradParts = 512;                    // partial sums of the weight-gradient kernel
 
 struct Tensors {
     int nx = 0, ny = 0, nz = 0;
@@ -292,18 +292,18 @@ int backward(nmr_corrector* c)
     w.ny = t.ny;
     w.nz = t.nz;
     w.part = c->wpart;
-    const int nw = kWgradGrid * 4;
+    const int nw = kWgradParts;
     w.in = t.a2;
     w.gout = t.g3;
-    HIP_TRY(nmr::launch_wgrad(16, w, kWgradGrid, c->stream));
+    HIP_TRY(nmr::launch_wgrad(16, w, nw, c->stream));
     HIP_TRY(nmr::launch_wreduce(c->wpart, nw, 16, 2, c->grad + kW3, c->stream));
     w.in = t.a1;
     w.gout = t.g2;
-    HIP_TRY(nmr::launch_wgrad(16, w, kWgradGrid, c->stream));
+    HIP_TRY(nmr::launch_wgrad(16, w, nw, c->stream));
     HIP_TRY(nmr::launch_wreduce(c->wpart, nw, 16, 16, c->grad + kW2, c->stream));
     w.in = t.x;
     w.gout = t.g1;
-    HIP_TRY(nmr::launch_wgrad(8, w, kWgradGrid, c->stream));
+    HIP_TRY(nmr::launch_wgrad(8, w, nw, c->stream));
     HIP_TRY(nmr::launch_wreduce(c->wpart, nw, 6, 16, c->grad + kW1, c->stream));
     return NMR_OK;
 }
@@ -398,7 +398,7 @@ int nmr_hip_corrector_create(uint64_t seed, nmr_corrector** out)
     if ((rc = dalloc(s, &c->w, kParams)) || (rc = dalloc(s, &c->m, kParams)) || (rc = dalloc(s, &c->v, kParams)) ||
         (rc = dalloc(s, &c->grad, kParams)) || (rc = dalloc(s, &c->f1, kFragF1)) || (rc = dalloc(s, &c->f2, kFragF)) ||
         (rc = dalloc(s, &c->f3, kFragF)) || (rc = dalloc(s, &c->d2, kFragF)) || (rc = dalloc(s, &c->d3, kFragF)) ||
-        (rc = dalloc(s, &c->wpart, (size_t)kWgradGrid * 4 * nmr::kWgradPart)) || (rc = dalloc(s, &c->dstat, 8)))
+        (rc = dalloc(s, &c->wpart, (size_t)kWgradParts * nmr::kWgradPart)) || (rc = dalloc(s, &c->dstat, 8)))
         return bail(rc);
     // He-normal weights (last layer scaled by 0.1), zero biases
     std::mt19937_64 gen(seed);

@@ -398,76 +398,120 @@ __global__ void __launch_bounds__(256, 3) conv_zm_kernel(ConvArgs a)
 }
 
 // Weight gradient dW[t][ci][co] = sum_v in[v + off(t)][ci] * gout[v][co] and
-// bias gradient sum_v gout[v][co], per wavefront over 32-voxel x segments,
-// into part[wave][27*256 + 16].  MFMA: A = input (16 ci x 32 voxels), B =
-// output gradient (32 voxels x 16 co), both gathered per lane.
+// bias gradient sum_v gout[v][co], as partials over 32-voxel x segments:
+// partial w takes segments w, w + npart, ..., into part[w][27*256 + 16].
+// MFMA: A = input (16 ci x 32 voxels), B = output gradient (32 voxels x 16
+// co), both gathered per lane.
+//
+// Bound by the gathers' latency: the operands want eight voxels of one channel
+// a lane from channels-last tensors, 2-byte loads.  A wavefront therefore
+// takes three of the 27 taps, those of one (dz, dy), whose operands are the
+// same ten voxels shifted by one: 18 loads for three MFMAs instead of 224 for
+// 27, and nine wavefronts in place of one on each partial (512 wavefronts
+// alone leave half of the CUs idle).  Each tap's sum runs over the same
+// segments in the same order as with one wavefront for all taps, so the
+// gradients keep their bits.  96x80x64: 31.9 us at 16 channels and 38.1 at 8,
+// 97.2 and 264 with one wavefront for all taps.
 template <int CIN>
-__global__ void __launch_bounds__(256) wgrad_kernel(WgradArgs a)
+__global__ void __launch_bounds__(256) wgrad_kernel(WgradArgs a, int npart)
 {
     const int lane = threadIdx.x & 63;
     const int g = lane >> 4, n = lane & 15;
-    const long px = a.nx + 2, plane = px * (long)(a.ny + 2);
-    const int wave = blockIdx.x * 4 + (threadIdx.x >> 6);
-    const int nwaves = gridDim.x * 4;
-    fl4 acc[27];
+    const int px = a.nx + 2, plane = px * (a.ny + 2); // (the padded grid has fewer than 2^31 voxels)
+    const int job = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * 4 + (threadIdx.x >> 6)));
+    const int w = job / 9, d = job % 9; // partial; (dz, dy) = (d / 3 - 1, d % 3 - 1)
+    if (w >= npart) return;
+    const int shift = (d / 3 - 1) * plane + (d % 3 - 1) * px;
+    fl4 acc[3];
 #pragma unroll
-    for (int t = 0; t < 27; t++) acc[t] = fl4{0.f, 0.f, 0.f, 0.f};
+    for (int t = 0; t < 3; t++) acc[t] = fl4{0.f, 0.f, 0.f, 0.f};
     float bsum = 0.f;
     const int nseg32 = (a.nx + 31) / 32;
     const int nrows = nseg32 * a.ny * a.nz;
     const bool chan = n < CIN;
-    for (int r = wave; r < nrows; r += nwaves) {
+    for (int r = w; r < nrows; r += npart) {
         const int seg = r % nseg32, yz = r / nseg32;
         const int y = yz % a.ny, z = yz / a.ny;
-        const long rowb = ((long)(z + 1) * (a.ny + 2) + (y + 1)) * px;
-        // B: gout[x0 + 8g + j][co = n]
-        uint16_t bv[8];
-        long vb[8];
+        const int rowb = (z + 1) * plane + (y + 1) * px;
+        const int x0 = seg * 32 + 8 * g;
+        uint16_t bv[8], av[3][8];
+        if (seg * 32 + 32 <= a.nx) {
+            const uint16_t* go = a.gout + ((size_t)(rowb + x0 + 1) * 16 + n);
+            const uint16_t* in = a.in + ((long)(rowb + shift + x0) * CIN + n);
+            uint16_t v[10]; // voxels x0 - 1 .. x0 + 8
 #pragma unroll
-        for (int j = 0; j < 8; j++) {
-            const int x = seg * 32 + 8 * g + j;
-            const bool ok = x < a.nx;
-            vb[j] = rowb + (ok ? x : a.nx - 1) + 1;
-            bv[j] = ok ? a.gout[vb[j] * 16 + n] : (uint16_t)0;
-            bsum += bf2f(bv[j]);
+            for (int j = 0; j < 8; j++) bv[j] = go[j * 16];
+#pragma unroll
+            for (int j = 0; j < 10; j++) v[j] = chan ? in[j * CIN] : (uint16_t)0;
+#pragma unroll
+            for (int t = 0; t < 3; t++)
+#pragma unroll
+                for (int j = 0; j < 8; j++) av[t][j] = v[j + t];
+        } else { // the row's end: voxels past it read the last one's, with a zero gradient
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                const bool ok = x0 + j < a.nx;
+                const int vb = rowb + (ok ? x0 + j : a.nx - 1) + 1;
+                bv[j] = ok ? a.gout[(size_t)vb * 16 + n] : (uint16_t)0;
+#pragma unroll
+                for (int t = 0; t < 3; t++)
+                    av[t][j] = chan ? a.in[(long)(vb + shift + t - 1) * CIN + n] : (uint16_t)0;
+            }
         }
+#pragma unroll
+        for (int j = 0; j < 8; j++) bsum += bf2f(bv[j]);
         const uint4 B = make_uint4((uint32_t)bv[0] | ((uint32_t)bv[1] << 16), (uint32_t)bv[2] | ((uint32_t)bv[3] << 16),
                                    (uint32_t)bv[4] | ((uint32_t)bv[5] << 16), (uint32_t)bv[6] | ((uint32_t)bv[7] << 16));
 #pragma unroll
-        for (int t = 0; t < 27; t++) {
-            const long o = tap_off(t, px, plane);
-            uint16_t av[8];
-#pragma unroll
-            for (int j = 0; j < 8; j++) av[j] = chan ? a.in[(vb[j] + o) * CIN + n] : (uint16_t)0;
-            const uint4 Av = make_uint4((uint32_t)av[0] | ((uint32_t)av[1] << 16),
-                                        (uint32_t)av[2] | ((uint32_t)av[3] << 16),
-                                        (uint32_t)av[4] | ((uint32_t)av[5] << 16),
-                                        (uint32_t)av[6] | ((uint32_t)av[7] << 16));
+        for (int t = 0; t < 3; t++) {
+            const uint4 Av = make_uint4((uint32_t)av[t][0] | ((uint32_t)av[t][1] << 16),
+                                        (uint32_t)av[t][2] | ((uint32_t)av[t][3] << 16),
+                                        (uint32_t)av[t][4] | ((uint32_t)av[t][5] << 16),
+                                        (uint32_t)av[t][6] | ((uint32_t)av[t][7] << 16));
             acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf8(Av), as_bf8(B), acc[t], 0, 0, 0);
         }
     }
-    float* dst = a.part + (size_t)wave * kWgradPart;
+    float* dst = a.part + (size_t)w * kWgradPart;
     // D[i = ci = 4g + j][col = co = n]
 #pragma unroll
-    for (int t = 0; t < 27; t++)
+    for (int t = 0; t < 3; t++)
 #pragma unroll
-        for (int j = 0; j < 4; j++) dst[t * 256 + (4 * g + j) * 16 + n] = acc[t][j];
+        for (int j = 0; j < 4; j++) dst[(3 * d + t) * 256 + (4 * g + j) * 16 + n] = acc[t][j];
     // bias: lanes n, n+16, n+32, n+48 hold the same co
     bsum += __shfl_xor(bsum, 16);
     bsum += __shfl_xor(bsum, 32);
-    if (g == 0) dst[27 * 256 + n] = bsum;
+    if (d == 0 && g == 0) dst[27 * 256 + n] = bsum;
 }
 
-// Sum of the wavefront partials in a fixed order, scattered to the
-// canonical gradient layout W[co][ci][t] (cout_real x cin_real x 27) followed
-// by the bias.
+// Sum of the partials in a fixed order (FP64, partial 0 first), scattered to
+// the canonical gradient layout W[co][ci][t] (cout_real x cin_real x 27)
+// followed by the bias.  A workgroup takes kRedEl elements: all threads bring
+// kRedRows partials of them into LDS at once, then one thread an element adds
+// them up in order -- the order is the serial chain that bounds it (512 FP64
+// additions), not a load behind every addition: 10.7 us against 125.
+constexpr int kRedEl = 16, kRedRows = 512;
 __global__ void __launch_bounds__(256) wreduce_kernel(const float* __restrict__ part, int nwaves, int cin_real,
                                                       int cout_real, float* __restrict__ grad)
 {
-    const int e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= kWgradPart) return;
+    __shared__ float sh[kRedRows * kRedEl];
+    const int e0 = blockIdx.x * kRedEl, col = threadIdx.x % kRedEl;
+    const int e = e0 + col;
     double s = 0.0;
-    for (int w = 0; w < nwaves; w++) s += (double)part[(size_t)w * kWgradPart + e];
+    for (int w0 = 0; w0 < nwaves; w0 += kRedRows) {
+        const int rows = min(kRedRows, nwaves - w0);
+        if (e < kWgradPart) {
+#pragma unroll 8
+            for (int w = threadIdx.x / kRedEl; w < rows; w += 256 / kRedEl)
+                sh[w * kRedEl + col] = part[(size_t)(w0 + w) * kWgradPart + e];
+        }
+        __syncthreads();
+        if (threadIdx.x < kRedEl && e < kWgradPart) {
+#pragma unroll 16
+            for (int w = 0; w < rows; w++) s += (double)sh[w * kRedEl + col];
+        }
+        __syncthreads();
+    }
+    if (threadIdx.x >= kRedEl || e >= kWgradPart) return;
     if (e < 27 * 256) {
         const int t = e / 256, ci = (e / 16) % 16, co = e % 16;
         if (ci < cin_real && co < cout_real) grad[((size_t)co * cin_real + ci) * 27 + t] = (float)s;
@@ -770,17 +814,18 @@ hipError_t launch_conv_zm(int cin, int mode, const ConvArgs& a, int grid, hipStr
     return hipGetLastError();
 }
 
-hipError_t launch_wgrad(int cin, const WgradArgs& a, int grid, hipStream_t s)
+hipError_t launch_wgrad(int cin, const WgradArgs& a, int npart, hipStream_t s)
 {
-    if (cin == 8) hipLaunchKernelGGL((wgrad_kernel<8>), dim3(grid), dim3(256), 0, s, a);
-    else if (cin == 16) hipLaunchKernelGGL((wgrad_kernel<16>), dim3(grid), dim3(256), 0, s, a);
+    const dim3 grid((unsigned)((npart * 9 + 3) / 4)), block(256);
+    if (cin == 8) hipLaunchKernelGGL((wgrad_kernel<8>), grid, block, 0, s, a, npart);
+    else if (cin == 16) hipLaunchKernelGGL((wgrad_kernel<16>), grid, block, 0, s, a, npart);
     else return hipErrorInvalidValue;
     return hipGetLastError();
 }
 
 hipError_t launch_wreduce(const float* part, int nwaves, int cin_real, int cout_real, float* grad, hipStream_t s)
 {
-    hipLaunchKernelGGL(wreduce_kernel, dim3((kWgradPart + 255) / 256), dim3(256), 0, s, part, nwaves, cin_real,
+    hipLaunchKernelGGL(wreduce_kernel, dim3((kWgradPart + kRedEl - 1) / kRedEl), dim3(256), 0, s, part, nwaves, cin_real,
                        cout_real, grad);
     return hipGetLastError();
 }
