@@ -331,7 +331,7 @@ int nmr_hip_corrector_set_scales(nmr_corrector* net, double vscale, double out_s
 int nmr_hip_corrector_get_scales(nmr_corrector* net, double* vscale, double* out_scale);
 /* Convolution kernel of the corrector (all give the same bits):
  * NMR_CONV_ZMARCH (default) marches columns of 16 x 16 output rows along z
- * through a ring of LDS planes, zc planes per column (0: 16);
+ * through a ring of LDS planes, zc planes per column (0: by the grid);
  * NMR_CONV_TILES stages 16 x 8 x 4-voxel tiles; NMR_CONV_ROWS gathers each
  * row's operands from memory; NMR_CONV_ZMARCH_SPARSE is NMR_CONV_ZMARCH with
  * the learned solve's last layer computed only on rows that hold a pore

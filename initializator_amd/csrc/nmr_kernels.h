@@ -295,7 +295,7 @@ struct ConvArgs {
     const int* rows;        // row list, row = (z*ny + y)*nseg + seg; null = all rows
     int nrows;
     int nx, ny, nz, nseg;   // nseg = ceil(nx/16)
-    int zc;                 // output planes per column of the z-marching kernel (0 = 16)
+    int zc;                 // output planes per column of the z-marching kernel
     const float* smx;       // mode 4: input channels 0, 1 from this state (Mx, My times the pore
     const float* smy;       //   channel), compact with pitch spitch
     int spitch;

@@ -20,6 +20,7 @@
 // correction larger than tol times the largest |M| of the previous state --
 // and otherwise replaced by factor plain steps from the kept state.  The net
 // computes only the rows its pore outputs depend on.
+#include <climits>
 #include <random>
 
 #include "nmr_internal.h"
@@ -64,7 +65,7 @@ struct nmr_corrector {
     int nrows[3] = {0, 0, 0};
     // convolution kernel (NMR_CONV_*) and planes per z-marching column
     int conv = 0;
-    int zc = 16;
+    int zc = 0; // 0: by the grid (zm_planes)
 };
 
 namespace {
@@ -135,26 +136,49 @@ int conv_grid(int nrows) { return std::max(1, std::min(2048, (nrows + 3) / 4)); 
 // persistent grid of the tiled convolution: 4 resident workgroups per CU
 // (34.6 KB of LDS each at 16 channels) on 256 CUs
 int tile_grid(const Tensors& t) { return std::max(1, std::min(1024, nmr::conv_tiles(t.nx, t.ny, t.nz))); }
-// persistent grid of the z-marching convolution: 3 resident workgroups per
-// CU at 16 input channels (41.5 KB of LDS each), 4 at 8
-int zm_grid(const Tensors& t, int cin, int zc)
+// Planes per column of the z-marching convolution: two workgroups fit a CU
+// (their weights and open accumulators take up to 256 registers a lane), and
+// a column costs its planes and about three more (two planes of halo, the
+// start).  Measured (16 -> 16 layer), 16 planes and the choice: 96x80x64
+// (4 planes) 22.0 and 14.6 us, 50x60x40 (2) 22.5 and 8.8, 64^3 (2) 21.5 and 9.4,
+// 128x128x96 (12) 33.0 and 28.2, 128^3 (16) 36.
+constexpr int kZmResident = 512;
+int zm_planes(const nmr_corrector* c)
 {
-    return std::max(1, std::min(cin == 8 ? 1024 : 768, nmr::conv_columns(t.nx, t.ny, t.nz, zc)));
+    if (c->zc > 0) return c->zc;
+    const Tensors& t = c->t;
+    int best = 1;
+    long least = LONG_MAX;
+    for (int zc = std::min(t.nz, 32); zc >= 1; zc--) {
+        const long cols = nmr::conv_columns(t.nx, t.ny, t.nz, zc);
+        const long cost = (cols + kZmResident - 1) / kZmResident * (zc + 3);
+        if (cost < least) {
+            least = cost;
+            best = zc;
+        }
+    }
+    return best;
 }
+int zm_grid(const Tensors& t, int zc)
+{
+    return std::max(1, std::min(kZmResident, nmr::conv_columns(t.nx, t.ny, t.nz, zc)));
+}
+// Its offsets within a plane are 32-bit byte offsets.
+bool zm_fits(const Tensors& t) { return (double)(t.nx + 2) * (t.ny + 2) * 32.0 < 4294967296.0; }
 
 // One dense convolution layer with the context's kernel choice.
 int conv_dense(nmr_corrector* c, int cin, int mode, nmr::ConvArgs a)
 {
     const Tensors& t = c->t;
-    if (c->conv == NMR_CONV_TILES) {
+    if (c->conv == NMR_CONV_TILES || (c->conv != NMR_CONV_ROWS && !zm_fits(t))) {
         HIP_TRY(nmr::launch_conv_tiled(cin, mode, a, tile_grid(t), c->stream));
     } else if (c->conv == NMR_CONV_ROWS) {
         a.rows = nullptr;
         a.nrows = a.nseg * t.ny * t.nz;
         HIP_TRY(nmr::launch_conv(cin, mode, a, conv_grid(a.nrows), c->stream));
     } else {
-        a.zc = c->zc;
-        HIP_TRY(nmr::launch_conv_zm(cin, mode, a, zm_grid(t, cin, c->zc), c->stream));
+        a.zc = zm_planes(c);
+        HIP_TRY(nmr::launch_conv_zm(cin, mode, a, zm_grid(t, a.zc), c->stream));
     }
     return NMR_OK;
 }
@@ -188,8 +212,8 @@ int forward(nmr_corrector* c, bool sparse = false, const float* smx = nullptr, c
         a.smx = smx;
         a.smy = smy;
         a.spitch = spitch;
-        a.zc = c->zc;
-        HIP_TRY(nmr::launch_conv_zm(8, 4, a, zm_grid(t, 8, c->zc), c->stream));
+        a.zc = zm_planes(c);
+        HIP_TRY(nmr::launch_conv_zm(8, 4, a, zm_grid(t, a.zc), c->stream));
         a.smx = a.smy = nullptr;
     } else if ((rc = conv_dense(c, 8, 0, a))) {
         return rc;
@@ -469,7 +493,7 @@ int nmr_hip_corrector_set_conv(nmr_corrector* c, int32_t kind, int32_t zc)
         return fail(NMR_ERR_INVALID, "nmr_hip_corrector_set_conv: kind %d", kind);
     if (zc < 0 || zc > 4096) return fail(NMR_ERR_INVALID, "nmr_hip_corrector_set_conv: zc %d", zc);
     c->conv = kind;
-    c->zc = zc > 0 ? zc : 16;
+    c->zc = zc;
     return NMR_OK;
 }
 
@@ -777,7 +801,7 @@ int nmr_hip_run_learned(nmr_ctx* ctx, nmr_corrector* c, int64_t ncoarse, int32_t
     const float vinv = (float)(1.0 / c->vscale);
     // the z-marching kernels stage (Mx, My) from the state: the feature
     // tensor's other channels (pore, velocity) are written once per run
-    const bool state_fed = c->conv == NMR_CONV_ZMARCH || c->conv == NMR_CONV_ZMARCH_SPARSE;
+    const bool state_fed = (c->conv == NMR_CONV_ZMARCH || c->conv == NMR_CONV_ZMARCH_SPARSE) && zm_fits(c->t);
     auto features = [&](int buf) -> int {
         nmr::FeatureArgs f{};
         f.mx = ctx->m[buf][0];

@@ -24,6 +24,7 @@
 #include <algorithm>
 #include <type_traits>
 
+#include "nmr_device.h"
 #include "nmr_kernels.h"
 
 namespace nmr {
@@ -40,10 +41,26 @@ __device__ __forceinline__ uint16_t f2bf(float f)
     u += 0x7fffu + ((u >> 16) & 1u);
     return (uint16_t)(u >> 16);
 }
+// The same of two values, b in the upper half (one v_cvt_pk_bf16_f32; the same
+// bits as f2bf for every value).
+__device__ __forceinline__ uint32_t f2bf2(float a, float b)
+{
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    const bf16x2 v = {(__bf16)a, (__bf16)b};
+    return __builtin_bit_cast(uint32_t, v);
+}
 __device__ __forceinline__ float bf2f(uint16_t h) { return __uint_as_float((uint32_t)h << 16); }
 __device__ __forceinline__ bool bf_pos(uint16_t h) { return h != 0 && (h & 0x8000u) == 0; }
 
 __device__ __forceinline__ bf16x8 as_bf8(uint4 v) { return __builtin_bit_cast(bf16x8, v); }
+
+// A barrier that orders LDS accesses only: global loads stay in flight across it.
+__device__ __forceinline__ void lds_barrier()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
 
 // tap t = kz*9 + ky*3 + kx, offsets -1..1 on each axis
 __device__ __forceinline__ long tap_off(int t, long px, long plane)
@@ -197,23 +214,36 @@ __global__ void __launch_bounds__(256) conv_tile_kernel(ConvArgs a)
 
 // The same convolution marching along z through columns of 16 x 16 output
 // rows: the input planes of the column (18 x 18 voxels, all channels) pass
-// through a ring of four LDS slots, so that each is loaded once per column
+// through a ring of three LDS slots, so that each is loaded once per column
 // instead of once per 16 x 8 x 4 tile (1.27 input reads per output voxel
-// instead of 2.1), and the next plane's global loads are in flight while the
-// current output plane is computed.  Output plane z reads padded input
-// planes z, z + 1, z + 2 (slots z & 3, ...); plane z + 3 goes into slot
-// (z + 3) & 3, which no wavefront reads during plane z, and the barrier at
-// the end of each plane orders it before its first read.  Wavefront w
-// computes rows w, w + 4, w + 8, w + 12 of a plane as four independent
-// accumulators that share each weight fragment; per row the MFMA sequence is
-// the row kernel's (same operands, same chunk order), so the bits equal
-// those of conv_kernel and conv_tile_kernel.  Persistent: workgroup b takes
-// columns b, b + gridDim.x, ...; a column is a.zc output planes (the last
-// one what is left).  MODE 4 (8 input channels) is MODE 0 with the input's
-// channels 0 and 1 staged from the FP32 state a.smx/smy times the pore
-// channel, rounded as feature_kernel rounds them, so that the feature
-// tensor's other channels (pore, velocity), which do not change during a
-// run, are written once.
+// instead of 2.1).  A plane is used for all three output planes that read it
+// while it is there: output z takes its taps of plane z, then of z + 1, then
+// of z + 2, which is the order of the reduction, so three planes of
+// accumulators are open at a time and the bits equal those of conv_kernel and
+// conv_tile_kernel (same operands, same chunk order).
+//
+// Bound by LDS reads where every chunk reads its own operand (56 of 16 bytes a
+// lane for the 56 MFMAs of four rows at 16 channels: 1800 cycles a plane of
+// one workgroup, against 900 of the matrix cores).  A wavefront therefore
+// takes four consecutive rows, whose chunks share operands: those of one plane
+// are runs of taps that recur at another row offset (kx 0,1 | kx 1,2 | kx 2 and
+// the next row's 0), so 22 reads serve the 56 MFMAs (22 for 28 at 8 channels).
+// The channel halves of a plane lie apart in LDS, so that 16 lanes read 256
+// consecutive bytes.  Two planes of global loads are in flight behind the one
+// that is computed (the barrier orders LDS only), and BF16 results are rounded
+// two at a time in one instruction (a branch on NaN for each value cost 15 %).
+// What is left is the chain of a plane -- reads, MFMAs, store, barrier -- with
+// two workgroups a CU.  96x80x64, with one read an MFMA and columns of 16
+// planes before: 34.4 -> 14.6 us at 16 -> 16, 26.7 -> 11.3 at 16 -> 2, 39.5 ->
+// 15.1 the input gradient, 25.9 -> 9.7 at 8 -> 16.  128^3: 41.6 -> 36.0, 31.6 ->
+// 30.7 (the MFMAs of 18 planes take 27 us at 2.4 GHz), 53.3 the gradient, 24.7.
+//
+// Persistent: workgroup b takes columns b, b + gridDim.x, ...; a column is
+// a.zc output planes (the last one what is left).  MODE 4 (8 input channels)
+// is MODE 0 with the input's channels 0 and 1 staged from the FP32 state
+// a.smx/smy times the pore channel, rounded as feature_kernel rounds them, so
+// that the feature tensor's other channels (pore, velocity), which do not
+// change during a run, are written once.
 constexpr int kZmY = 16;
 template <int N>
 struct Plane {
@@ -225,39 +255,53 @@ struct PlaneS {
     float fx[N], fy[N];
 };
 template <int CIN, int MODE>
-__global__ void __launch_bounds__(256, 3) conv_zm_kernel(ConvArgs a)
+__global__ void __launch_bounds__(256, 2) conv_zm_kernel(ConvArgs a)
 {
     constexpr int TPC = 32 / CIN;
     constexpr int NCH = (27 + TPC - 1) / TPC;
-    constexpr int HX = 18, HY = kZmY + 2;
+    constexpr int HX = 18, HY = kZmY + 2, HV = HX * HY;
     constexpr int V16 = CIN / 8;
-    constexpr int PV = HX * HY * V16;          // uint4 per staged plane
+    constexpr int PV = HV * V16;               // uint4 per staged plane
     constexpr int NLD = (PV + 255) / 256;
-    constexpr int ROWB = HX * V16 * 16;         // bytes per staged row
-    __shared__ uint4 sin[4 * PV];
+    constexpr int ROWB = HX * 16, SLOTB = PV * 16; // bytes per staged row and per slot
+    __shared__ uint4 sin[3 * PV + HX + 16];    // (the zeroed half of the last row's last chunk reads past the plane)
     const int lane = threadIdx.x & 63;
     const int g = lane >> 4, n = lane & 15;
-    const int wave = threadIdx.x >> 6;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     bf16x8 A[NCH];
     const uint4* wa4 = reinterpret_cast<const uint4*>(a.wa);
 #pragma unroll
     for (int c = 0; c < NCH; c++) A[c] = as_bf8(wa4[c * 64 + lane]);
-    // this lane's B element of chunk c within a staged plane, in bytes from
-    // the wavefront's first row; hi bit c: the lane's tap lies in the later
-    // of the two planes a chunk spans; `last`: the lane's tap of the last
-    // chunk exists (t < 27)
-    int inner[NCH];
-    uint32_t hi = 0;
-    const int tg = (8 * g) / CIN, part0 = ((8 * g) % CIN) / 8;
-#pragma unroll
-    for (int c = 0; c < NCH; c++) {
-        const int t = min(c * TPC + tg, 26);
-        const int kz = t / 9, ky = (t / 3) % 3, kx = t % 3;
-        inner[c] = ((ky * HX + n + kx) * V16 + part0) * 16;
-        if (kz != (c * TPC) / 9) hi |= 1u << c;
-    }
-    const bool last = (NCH - 1) * TPC + tg < 27;
     static_assert(MODE != 4 || CIN == 8, "state-fed input is the first layer's");
+    // Byte offset of this lane's part of an operand within a plane: (row, x)
+    // of the lane's tap from the operand's row of this wavefront.
+    auto at = [&](int row, int dx) {
+        return ((CIN == 16 ? (g & 1) * HV : 0) + (wave * 4 + row) * HX + n + dx) * 16;
+    };
+    const int tg = CIN == 16 ? g >> 1 : g; // the lane's tap in a chunk
+    // operands of one plane: 16 channels: kx 0,1 | kx 1,2 | kx 2 and the next
+    // row's kx 0; 8 channels: kx 0,1,2 and the next row's 0 | kx 1,2 and the
+    // next row's 0,1 | kx 2 and the next row's 0,1,2
+    int o0, o1, o2;
+    if constexpr (CIN == 16) {
+        o0 = at(0, tg);
+        o1 = at(0, 1 + tg);
+        o2 = tg ? at(1, 0) : at(0, 2);
+    } else {
+        o0 = tg < 3 ? at(0, tg) : at(1, 0);
+        o1 = tg < 2 ? at(0, 1 + tg) : at(1, tg - 2);
+        o2 = tg ? at(1, tg - 1) : at(0, 2);
+    }
+    // operands that span two planes: ky 2, kx 2 (8 channels: or kx 1,2) of the
+    // plane before and the first taps of this one; by slot of this plane
+    int m0[3], m1[3];
+#pragma unroll
+    for (int s = 0; s < 3; s++) {
+        const int before = (s + 2) % 3 * SLOTB, here = s * SLOTB;
+        m0[s] = tg == 0 ? before + at(2, 2) : here + at(0, tg - 1);
+        m1[s] = tg < 2 ? before + at(2, 1 + tg) : here + at(0, tg - 2);
+    }
+    const bool last = (NCH - 1) * TPC + tg < 27; // the lane's tap of the last chunk exists
     float bias[4] = {0.f, 0.f, 0.f, 0.f};
     if constexpr (MODE == 0 || MODE == 4) {
 #pragma unroll
@@ -266,13 +310,16 @@ __global__ void __launch_bounds__(256, 3) conv_zm_kernel(ConvArgs a)
         bias[0] = a.bias[0];
         bias[1] = a.bias[1];
     }
-    const long px = a.nx + 2;
-    const long pstride = (long)(a.ny + 2) * px * CIN; // elements per padded plane
-    const int zc = a.zc > 0 ? a.zc : 16;
+    const int px = a.nx + 2, plane = (a.ny + 2) * px; // (the padded grid has fewer than 2^31 voxels)
+    const int zc = a.zc;
     const int nyb = (a.ny + kZmY - 1) / kZmY, nzb = (a.nz + zc - 1) / zc;
     const int ncol = a.nseg * nyb * nzb;
-    const char* lds = reinterpret_cast<const char*>(sin);
-    for (int col = blockIdx.x; col < ncol; col += gridDim.x) {
+    char* lds = reinterpret_cast<char*>(sin);
+    auto read = [&](int o) { return *reinterpret_cast<const uint4*>(lds + o); };
+    auto mfma = [&](int c, const uint4& b, fl4& d) {
+        d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[c], as_bf8(b), d, 0, 0, 0);
+    };
+    for (int col = xcd_tile(blockIdx.x, (int)gridDim.x); col < ncol; col += gridDim.x) {
         const int seg = col % a.nseg, r2 = col / a.nseg;
         const int x0 = seg * 16, y0 = (r2 % nyb) * kZmY, zs = (r2 / nyb) * zc;
         const int ze = min(zs + zc, a.nz);
@@ -280,36 +327,35 @@ __global__ void __launch_bounds__(256, 3) conv_zm_kernel(ConvArgs a)
         // padded (x0 + xx, y0 + yy), clamped to the padded grid (clamped ones
         // feed only outputs that are not stored); a thread's element past the
         // plane loads element 0 again and is not stored
-        long goff[NLD];
-        long sidx[NLD]; // MODE 4: the state index of an interior voxel in its plane, else -1
+        uint32_t goff[NLD]; // bytes in a plane (below 4 GiB)
+        int sidx[NLD]; // MODE 4: the state index of an interior voxel in its plane, else -1
 #pragma unroll
         for (int j = 0; j < NLD; j++) {
             const int i = threadIdx.x + 256 * j < PV ? threadIdx.x + 256 * j : 0;
-            const int v = i / V16, pt = i % V16;
-            const long gx = min(x0 + v % HX, a.nx + 1), gy = min(y0 + v / HX, a.ny + 1);
-            goff[j] = (gy * px + gx) * CIN + pt * 8;
+            const int v = i / V16;
+            const int gx = min(x0 + v % HX, a.nx + 1), gy = min(y0 + v / HX, a.ny + 1);
+            goff[j] = (uint32_t)(gy * px + gx) * (uint32_t)(2 * CIN) + (uint32_t)(i % V16) * 16u;
             sidx[j] = (gx >= 1 && gx <= a.nx && gy >= 1 && gy <= a.ny) ? (gy - 1) * a.spitch + gx - 1 : -1;
         }
         using PL = typename std::conditional<MODE == 4, PlaneS<NLD>, Plane<NLD>>::type;
-        const long splane = (long)a.ny * a.spitch;
-        auto load = [&](int pz) {
-            PL r;
+        auto load = [&](int pz, PL& r) {
+            const char* in = reinterpret_cast<const char*>(a.in + (size_t)pz * plane * CIN);
+            const size_t c0 = (size_t)max(pz - 1, 0) * a.ny * a.spitch;
 #pragma unroll
             for (int j = 0; j < NLD; j++) {
-                r.v[j] = *reinterpret_cast<const uint4*>(a.in + (long)pz * pstride + goff[j]);
+                r.v[j] = *reinterpret_cast<const uint4*>(in + goff[j]);
                 if constexpr (MODE == 4) {
-                    const bool in = sidx[j] >= 0 && pz >= 1 && pz <= a.nz;
-                    const long c = in ? (long)(pz - 1) * splane + sidx[j] : 0;
-                    r.fx[j] = in ? a.smx[c] : 0.f;
-                    r.fy[j] = in ? a.smy[c] : 0.f;
+                    const bool ok = sidx[j] >= 0 && pz >= 1 && pz <= a.nz;
+                    r.fx[j] = ok ? a.smx[c0 + sidx[j]] : 0.f;
+                    r.fy[j] = ok ? a.smy[c0 + sidx[j]] : 0.f;
                 }
             }
-            return r;
         };
-        auto stash = [&](int pz, const PL& r) {
+        auto stash = [&](int pz, int slot, const PL& r) {
 #pragma unroll
-            for (int j = 0; j < NLD; j++)
-                if (threadIdx.x + 256 * j < PV) {
+            for (int j = 0; j < NLD; j++) {
+                const int i = threadIdx.x + 256 * j;
+                if (i < PV) {
                     uint4 w = r.v[j];
                     if constexpr (MODE == 4) {
                         if (sidx[j] >= 0 && pz >= 1 && pz <= a.nz) {
@@ -318,81 +364,159 @@ __global__ void __launch_bounds__(256, 3) conv_zm_kernel(ConvArgs a)
                             w.x = (uint32_t)f2bf(r.fx[j] * pore) | ((uint32_t)f2bf(r.fy[j] * pore) << 16);
                         }
                     }
-                    sin[(pz & 3) * PV + threadIdx.x + 256 * j] = w;
+                    sin[slot * PV + (i % V16) * HV + i / V16] = w;
                 }
+            }
         };
-        {
-            const PL r0 = load(zs), r1 = load(zs + 1), r2v = load(zs + 2);
-            stash(zs, r0);
-            stash(zs + 1, r1);
-            stash(zs + 2, r2v);
-        }
-        __syncthreads();
-        const int x = x0 + n;
-        for (int z = zs; z < ze; z++) {
-            // output voxel of row i of this wavefront
-            long base[4];
-            bool store[4];
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int y = y0 + wave + 4 * i;
-                store[i] = x < a.nx && y < a.ny;
-                base[i] = ((long)(z + 1) * (a.ny + 2) + (min(y, a.ny - 1) + 1)) * px + (min(x, a.nx - 1) + 1);
-            }
+        const int x = x0 + n, yw = y0 + wave * 4;
+        const bool live = yw < a.ny; // this wavefront has rows
+        // this lane's first output in its plane, in bytes
+        const uint32_t oo = (uint32_t)((yw + 1) * px + x + 1) * (MODE == 1 ? 8u : 32u) + (MODE == 1 ? 0u : 8u * g);
+        PL pl[3];
+        // Plane p in slot s (p - zs modulo 3): opens output plane p in `first`,
+        // goes on with p - 1 in `mid` and completes p - 2 in `fin`.
+        auto step = [&](const int p, auto S, fl4 (&first)[4], fl4 (&mid)[4], fl4 (&fin)[4]) {
+            constexpr int s = decltype(S)::value;
+            constexpr int sb = s * SLOTB;
+            const int z = p - 2;
+            const bool out = z >= zs;
+            if (p + 2 <= ze + 1) load(p + 2, pl[(s + 2) % 3]);
+            const size_t zb = (size_t)(z + 1) * plane; // (z + 1 = p - 1 < 0 only where nothing is stored)
             uint2 gate[4];
-            if constexpr (MODE == 2) {
+            if (live) {
+                uint4 P[6], Q[6], X[6];
 #pragma unroll
-                for (int i = 0; i < 4; i++) gate[i] = *reinterpret_cast<const uint2*>(a.ref + base[i] * 16 + 4 * g);
+                for (int r = 0; r < 6; r++) {
+                    P[r] = read(o0 + sb + r * ROWB);
+                    if (CIN == 16 || (r >= 1 && r < 5)) Q[r] = read(o1 + sb + r * ROWB);
+                    if (CIN == 16 || r < 4) X[r] = read(o2 + sb + r * ROWB);
+                }
+                if (p < ze) {
+#pragma unroll
+                    for (int i = 0; i < 4; i++) first[i] = fl4{0.f, 0.f, 0.f, 0.f};
+                    if constexpr (CIN == 16) {
+#pragma unroll
+                        for (int i = 0; i < 4; i++) mfma(0, P[i], first[i]);
+#pragma unroll
+                        for (int i = 0; i < 4; i++) mfma(1, X[i], first[i]);
+#pragma unroll
+                        for (int i = 0; i < 4; i++) mfma(2, Q[i + 1], first[i]);
+#pragma unroll
+                        for (int i = 0; i < 4; i++) mfma(3, P[i + 2], first[i]);
+                    } else {
+#pragma unroll
+                        for (int i = 0; i < 4; i++) mfma(0, P[i], first[i]);
+#pragma unroll
+                        for (int i = 0; i < 4; i++) mfma(1, Q[i + 1], first[i]);
+                    }
+                }
+                if (p - 1 >= zs && p - 1 < ze) {
+                    uint4 M[4];
+#pragma unroll
+                    for (int i = 0; i < 4; i++) M[i] = read(m0[s] + i * ROWB);
+                    if constexpr (CIN == 16) {
+#pragma unroll
+                        for (int i = 0; i < 4; i++) mfma(4, M[i], mid[i]);
+#pragma unroll
+                        for (int i = 0; i < 4; i++) mfma(5, Q[i], mid[i]);
+#pragma unroll
+                        for (int i = 0; i < 4; i++) mfma(6, P[i + 1], mid[i]);
+#pragma unroll
+                        for (int i = 0; i < 4; i++) mfma(7, X[i + 1], mid[i]);
+#pragma unroll
+                        for (int i = 0; i < 4; i++) mfma(8, Q[i + 2], mid[i]);
+                    } else {
+#pragma unroll
+                        for (int i = 0; i < 4; i++) mfma(2, M[i], mid[i]);
+#pragma unroll
+                        for (int i = 0; i < 4; i++) mfma(3, P[i + 1], mid[i]);
+                    }
+                }
+                if (out) {
+                    const uint4 none = make_uint4(0u, 0u, 0u, 0u);
+                    if constexpr (MODE == 2) {
+#pragma unroll
+                        for (int i = 0; i < 4; i++) {
+                            gate[i] = make_uint2(0u, 0u);
+                            if (x < a.nx && yw + i < a.ny)
+                                gate[i] = *reinterpret_cast<const uint2*>(
+                                    reinterpret_cast<const char*>(a.ref + (zb + (size_t)i * px) * 16) + oo);
+                        }
+                    }
+                    if constexpr (CIN == 16) {
+#pragma unroll
+                        for (int i = 0; i < 4; i++) mfma(9, P[i], fin[i]);
+#pragma unroll
+                        for (int i = 0; i < 4; i++) mfma(10, X[i], fin[i]);
+#pragma unroll
+                        for (int i = 0; i < 4; i++) mfma(11, Q[i + 1], fin[i]);
+#pragma unroll
+                        for (int i = 0; i < 4; i++) mfma(12, P[i + 2], fin[i]);
+#pragma unroll
+                        for (int i = 0; i < 4; i++) mfma(13, last ? X[i + 2] : none, fin[i]);
+                    } else {
+                        uint4 M[4];
+#pragma unroll
+                        for (int i = 0; i < 4; i++) M[i] = read(m1[s] + i * ROWB);
+#pragma unroll
+                        for (int i = 0; i < 4; i++) mfma(4, M[i], fin[i]);
+#pragma unroll
+                        for (int i = 0; i < 4; i++) mfma(5, X[i], fin[i]);
+#pragma unroll
+                        for (int i = 0; i < 4; i++) mfma(6, last ? P[i + 2] : none, fin[i]);
+                    }
+                }
             }
-            const bool more = z + 3 <= ze + 1;
-            PL nx4{};
-            if (more) nx4 = load(z + 3);
-            int sb[3];
-#pragma unroll
-            for (int kz = 0; kz < 3; kz++) sb[kz] = ((z + kz) & 3) * PV * 16 + wave * ROWB;
-            fl4 acc[4];
-#pragma unroll
-            for (int i = 0; i < 4; i++) acc[i] = fl4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int c = 0; c < NCH; c++) {
-                const int kzl = (c * TPC) / 9, kzh = min(c * TPC + TPC - 1, 26) / 9;
-                const int ad = ((kzl == kzh || !((hi >> c) & 1u)) ? sb[kzl] : sb[kzh]) + inner[c];
-                uint4 B[4];
+            // the next plane goes into the slot of plane p - 2, last read in the step before
+            if (p + 1 <= ze + 1) stash(p + 1, (s + 1) % 3, pl[(s + 1) % 3]);
+            if (live && out) {
+                // lane holds output channels 4g..4g+3 of voxel n
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
-                    B[i] = *reinterpret_cast<const uint4*>(lds + ad + i * 4 * ROWB);
-                    if (c == NCH - 1 && !last) B[i] = make_uint4(0u, 0u, 0u, 0u);
-                }
-#pragma unroll
-                for (int i = 0; i < 4; i++)
-                    acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[c], as_bf8(B[i]), acc[i], 0, 0, 0);
-            }
-            // lane holds output channels 4g..4g+3 of voxel n
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                if (!store[i]) continue;
-                if constexpr (MODE == 1) {
-                    if (g == 0) {
-                        a.outf[base[i] * 2 + 0] = acc[i][0] + bias[0];
-                        a.outf[base[i] * 2 + 1] = acc[i][1] + bias[1];
-                    }
-                } else {
-                    uint16_t h[4];
-                    if constexpr (MODE == 0 || MODE == 4) {
-#pragma unroll
-                        for (int j = 0; j < 4; j++) h[j] = f2bf(fmaxf(acc[i][j] + bias[j], 0.f));
+                    if (x >= a.nx || yw + i >= a.ny) continue;
+                    if constexpr (MODE == 1) {
+                        if (g == 0)
+                            *reinterpret_cast<float2*>(reinterpret_cast<char*>(a.outf + (zb + (size_t)i * px) * 2) + oo) =
+                                make_float2(fin[i][0] + bias[0], fin[i][1] + bias[1]);
                     } else {
-                        const uint16_t rr4[4] = {(uint16_t)(gate[i].x & 0xffffu), (uint16_t)(gate[i].x >> 16),
-                                                 (uint16_t)(gate[i].y & 0xffffu), (uint16_t)(gate[i].y >> 16)};
+                        uint32_t h[2];
+                        if constexpr (MODE == 0 || MODE == 4) {
+                            float v[4];
 #pragma unroll
-                        for (int j = 0; j < 4; j++) h[j] = bf_pos(rr4[j]) ? f2bf(acc[i][j]) : (uint16_t)0;
+                            for (int j = 0; j < 4; j++) v[j] = fmaxf(fin[i][j] + bias[j], 0.f);
+                            h[0] = f2bf2(v[0], v[1]);
+                            h[1] = f2bf2(v[2], v[3]);
+                        } else {
+                            const uint32_t gt[2] = {gate[i].x, gate[i].y};
+#pragma unroll
+                            for (int j = 0; j < 2; j++) {
+                                const uint32_t lo = bf_pos((uint16_t)(gt[j] & 0xffffu)) ? 0xffffu : 0u;
+                                const uint32_t hi = bf_pos((uint16_t)(gt[j] >> 16)) ? 0xffff0000u : 0u;
+                                h[j] = f2bf2(fin[i][2 * j], fin[i][2 * j + 1]) & (lo | hi);
+                            }
+                        }
+                        *reinterpret_cast<uint2*>(reinterpret_cast<char*>(a.out + (zb + (size_t)i * px) * 16) + oo) =
+                            make_uint2(h[0], h[1]);
                     }
-                    *reinterpret_cast<uint2*>(a.out + base[i] * 16 + 4 * g) =
-                        make_uint2((uint32_t)h[0] | ((uint32_t)h[1] << 16), (uint32_t)h[2] | ((uint32_t)h[3] << 16));
                 }
             }
-            if (more) stash(z + 3, nx4);
-            __syncthreads();
+            lds_barrier();
+        };
+        load(zs, pl[0]);
+        load(zs + 1, pl[1]);
+        stash(zs, 0, pl[0]);
+        lds_barrier();
+        fl4 acc[3][4];
+#pragma unroll
+        for (int k = 0; k < 3; k++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) acc[k][i] = fl4{0.f, 0.f, 0.f, 0.f};
+        for (int p = zs; p <= ze + 1; p += 3) {
+            step(p, std::integral_constant<int, 0>{}, acc[0], acc[2], acc[1]);
+            if (p + 1 > ze + 1) break;
+            step(p + 1, std::integral_constant<int, 1>{}, acc[1], acc[0], acc[2]);
+            if (p + 2 > ze + 1) break;
+            step(p + 2, std::integral_constant<int, 2>{}, acc[2], acc[1], acc[0]);
         }
     }
 }

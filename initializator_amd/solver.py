@@ -364,7 +364,7 @@ class Corrector:
     def set_conv(self, kind: int = 0, zc: int = 0) -> None:
         """Convolution kernel (0 z-marching columns, 1 tiles, 2 row gathers,
         3 z-marching with the learned solve's last layer on pore rows only);
-        zc: output planes per z-marching column (0: 16).  Same bits for all."""
+        zc: output planes per z-marching column (0: by the grid).  Same bits for all."""
         check(self.lib.nmr_hip_corrector_set_conv(self.h, int(kind), int(zc)), "nmr_hip_corrector_set_conv")
 
     def scales(self):
