@@ -3062,6 +3062,31 @@ nmr::Coef make_coef(const nmr_ctx* c, const double g[3]) { return ::make_coef(c,
 
 int ensure_partials(nmr_ctx* c, size_t doubles) { return ::ensure_partials(c, doubles); }
 
+int learned_list(nmr_ctx* c, bool* yes)
+{
+    int rc = use_pores(c, yes);
+    if (rc) return rc;
+    *yes = *yes && pore_plain(c);
+    if (!*yes) return NMR_OK;
+    if ((rc = state_pores(c)) || (rc = pore_data(c))) return rc;
+    nmr::PoreArgs a{};
+    if ((rc = pore_args(c, &a))) return rc;
+    return ::ensure_partials(c, (size_t)a.ntiles * c->nc);
+}
+
+int list_step(nmr_ctx* c, const nmr::Coef& cf)
+{
+    nmr::PoreArgs a{};
+    int rc = pore_args(c, &a);
+    if (rc) return rc;
+    a.c = cf;
+    a.partials = c->partials;
+    a.f = c->pl.state[c->ppar];
+    a.out = c->pl.state[c->ppar ^ 1];
+    HIP_TRY(nmr::launch_pores(c->nc, c->vel, nmr::GEN_UPWIND, true, c->pl_reads_solids, false, a, c->stream));
+    return NMR_OK;
+}
+
 int sweep_step(nmr_ctx* c, const nmr::Coef& cf, bool exact, int in, int out)
 {
     const nmr_problem& p = c->prob;

@@ -264,6 +264,12 @@ int ensure_partials(nmr_ctx* c, size_t doubles);
 // of the context (the automatic one-step tile), on its stream; the step's
 // signal partials go to the context's partial buffer.
 int sweep_step(nmr_ctx* c, const nmr::Coef& cf, bool exact, int in, int out);
+// Whether the learned solve steps on the list of the pores (plain problems
+// for which a run would); the state is then in it.
+int learned_list(nmr_ctx* c, bool* yes);
+// One exact-phase step with coefficients cf from the list's current state
+// into its other state buffer.
+int list_step(nmr_ctx* c, const nmr::Coef& cf);
 // Make the row buffers hold the current state (both of them, converted from
 // the bricks when only those hold it).
 int state_rows(nmr_ctx* c);

@@ -296,9 +296,6 @@ struct ConvArgs {
     int nrows;
     int nx, ny, nz, nseg;   // nseg = ceil(nx/16)
     int zc;                 // output planes per column of the z-marching kernel
-    const float* smx;       // mode 4: input channels 0, 1 from this state (Mx, My times the pore
-    const float* smy;       //   channel), compact with pitch spitch
-    int spitch;
 };
 
 struct WgradArgs {
@@ -333,8 +330,12 @@ struct LossArgs {
 };
 
 struct ApplyArgs {
-    float* mx;
+    float* mx;              // the state in rows, or
     float* my;
+    float* slots;           //   in the list of the pores: (Mx, My) of the slots [s0, s1), whose voxels
+    const uint32_t* vox;    //   vox[] gives; null: rows
+    uint32_t s0, s1;
+    uint16_t* x;            // the net's input, whose channels 0 and 1 take the state at the pores
     const uint8_t* mask;
     const float* pred;      // [..][2] or null (statistics only)
     double* part;           // [blocks][6]
@@ -364,8 +365,10 @@ hipError_t launch_adam(float* p, float* m, float* v, const float* g, int n, floa
                        float c1, float c2, hipStream_t s);
 hipError_t launch_diff(const float* ax, const float* ay, const float* bx, const float* by, float* ox, float* oy,
                        long n, hipStream_t s);
-int apply_blocks(int nx, int ny, int nz);
-hipError_t launch_apply(const ApplyArgs& a, hipStream_t s);
+// workgroups for n voxels or slots
+int apply_blocks(uint64_t n);
+hipError_t launch_apply(const ApplyArgs& a, int blocks, hipStream_t s);
+// out: six doubles, in host memory that the device sees
 hipError_t launch_stats_reduce(const double* part, int nblocks, double* out, hipStream_t s);
 hipError_t launch_row_flags(const uint8_t* mask, int nx, int ny, int nz, int pitch, uint8_t* flag, hipStream_t s);
 // grid workgroups of 256 threads, each wave `iters` x 8 MFMA 16x16x32 BF16; out: grid*256 floats

@@ -56,7 +56,7 @@ struct nmr_corrector {
     size_t lpart_cap = 0;
     double* apart = nullptr; // apply partials
     size_t apart_cap = 0;
-    double* dstat = nullptr; // reduced statistics [6]
+    double* hstat = nullptr; // reduced statistics [6], pinned host memory that the reduction writes
     bool train_ws = false;
     // rows of the three layers that the pores of one context need
     const nmr_ctx* rows_ctx = nullptr;
@@ -140,8 +140,8 @@ int tile_grid(const Tensors& t) { return std::max(1, std::min(1024, nmr::conv_ti
 // (their weights and open accumulators take up to 256 registers a lane), and
 // a column costs its planes and about three more (two planes of halo, the
 // start).  Measured (16 -> 16 layer), 16 planes and the choice: 96x80x64
-// (4 planes) 22.0 and 14.6 us, 50x60x40 (2) 22.5 and 8.8, 64^3 (2) 21.5 and 9.4,
-// 128x128x96 (12) 33.0 and 28.2, 128^3 (16) 36.
+// (4 planes) 21.8 and 14.2 us, 50x60x40 (2) 21.8 and 8.7, 64^3 (2) 20.8 and 10.4,
+// 128x128x96 (12) 32.7 and 27.8, 128^3 (16) 35.
 constexpr int kZmResident = 512;
 int zm_planes(const nmr_corrector* c)
 {
@@ -186,10 +186,8 @@ int conv_dense(nmr_corrector* c, int cin, int mode, nmr::ConvArgs a)
 // Forward pass on the tensors (x already filled): a1, a2, p.  Layers 1 and
 // 2 run over every row; with row lists (sparse = true) layer 3 computes
 // only the rows c->rows[2] (those holding a pore) unless the z-marching
-// kernel runs it over every row.  With a state (smx, smy; z-marching kernels
-// only) layer 1 takes input channels 0 and 1 from it instead of from x.
-int forward(nmr_corrector* c, bool sparse = false, const float* smx = nullptr, const float* smy = nullptr,
-            int spitch = 0)
+// kernel runs it over every row.
+int forward(nmr_corrector* c, bool sparse = false)
 {
     const Tensors& t = c->t;
     nmr::ConvArgs a{};
@@ -208,16 +206,7 @@ int forward(nmr_corrector* c, bool sparse = false, const float* smx = nullptr, c
     a.bias = c->w + kB1;
     a.out = t.a1;
     int rc = NMR_OK;
-    if (smx) {
-        a.smx = smx;
-        a.smy = smy;
-        a.spitch = spitch;
-        a.zc = zm_planes(c);
-        HIP_TRY(nmr::launch_conv_zm(8, 4, a, zm_grid(t, a.zc), c->stream));
-        a.smx = a.smy = nullptr;
-    } else if ((rc = conv_dense(c, 8, 0, a))) {
-        return rc;
-    }
+    if ((rc = conv_dense(c, 8, 0, a))) return rc;
     a.in = t.a1;
     a.wa = c->f2;
     a.bias = c->w + kB2;
@@ -422,8 +411,10 @@ int nmr_hip_corrector_create(uint64_t seed, nmr_corrector** out)
     if ((rc = dalloc(s, &c->w, kParams)) || (rc = dalloc(s, &c->m, kParams)) || (rc = dalloc(s, &c->v, kParams)) ||
         (rc = dalloc(s, &c->grad, kParams)) || (rc = dalloc(s, &c->f1, kFragF1)) || (rc = dalloc(s, &c->f2, kFragF)) ||
         (rc = dalloc(s, &c->f3, kFragF)) || (rc = dalloc(s, &c->d2, kFragF)) || (rc = dalloc(s, &c->d3, kFragF)) ||
-        (rc = dalloc(s, &c->wpart, (size_t)kWgradParts * nmr::kWgradPart)) || (rc = dalloc(s, &c->dstat, 8)))
+        (rc = dalloc(s, &c->wpart, (size_t)kWgradParts * nmr::kWgradPart)))
         return bail(rc);
+    if (hipHostMalloc((void**)&c->hstat, 8 * sizeof(double), hipHostMallocDefault) != hipSuccess)
+        return bail(fail(NMR_ERR_NOMEM, "pinned host allocation"));
     // He-normal weights (last layer scaled by 0.1), zero biases
     std::mt19937_64 gen(seed);
     std::vector<float> h(kParams, 0.f);
@@ -448,9 +439,9 @@ int nmr_hip_corrector_destroy(nmr_corrector* c)
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     tfree(c->t);
     for (void* q : {(void*)c->w, (void*)c->m, (void*)c->v, (void*)c->grad, (void*)c->f1, (void*)c->f2, (void*)c->f3,
-                    (void*)c->d2, (void*)c->d3, (void*)c->wpart, (void*)c->lpart, (void*)c->apart, (void*)c->dstat,
-                    (void*)c->rows[0], (void*)c->rows[1], (void*)c->rows[2]})
+                    (void*)c->d2, (void*)c->d3, (void*)c->wpart, (void*)c->lpart, (void*)c->apart, (void*)c->rows[0], (void*)c->rows[1], (void*)c->rows[2]})
         if (q) (void)hipFree(q);
+    if (c->hstat) (void)hipHostFree(c->hstat);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
     return NMR_OK;
@@ -746,27 +737,35 @@ int nmr_hip_run_learned(nmr_ctx* ctx, nmr_corrector* c, int64_t ncoarse, int32_t
     if (!(c->out_scale > 0)) return fail(NMR_ERR_STATE, "the corrector has no output scale (train or set it)");
     int rc = ensure_tensors(c, p.nx, p.ny, p.nz, false);
     if (rc) return rc;
-    const int nab = nmr::apply_blocks(p.nx, p.ny, p.nz);
-    if ((rc = ensure_dev_doubles(c, &c->apart, &c->apart_cap, (size_t)nab * 6))) return rc;
-    if ((rc = build_rows(c, ctx))) return rc;
-    // The loop works on the row buffers (the coarse step, the net, the
-    // statistics and the fallback runs); it leaves the state there and the
-    // context's layout switch as it found it.
-    if ((rc = nmri::state_rows(ctx))) return rc;
-    struct RowsOnly {
+    if (c->conv != NMR_CONV_ZMARCH && (rc = build_rows(c, ctx))) return rc;
+    // The loop works where a run would: on the list of the pores, or on the
+    // row buffers (the coarse step, the statistics and the fallback runs),
+    // where it leaves the state, the context's layout switch as it found it.
+    bool list = false;
+    if ((rc = nmri::learned_list(ctx, &list))) return rc;
+    if (!list && (rc = nmri::state_rows(ctx))) return rc;
+    struct Home {
         nmr_ctx* c;
-        bool keep;
-        ~RowsOnly()
+        bool keep, list;
+        ~Home()
         {
             c->brick_on = keep;
-            c->home = nmri::kHomeRows;
+            c->home = list ? nmri::kHomePores : nmri::kHomeRows;
             c->sig_valid = false;
         }
-    } guard{ctx, ctx->brick_on};
-    ctx->brick_on = false;
-    ctx->home = nmri::kHomeRows;
+    } guard{ctx, ctx->brick_on, list};
+    if (!list) ctx->brick_on = false;
+    ctx->home = list ? nmri::kHomePores : nmri::kHomeRows;
     ctx->sig_valid = false;
     nmr::ApplyArgs ap{};
+    if (list) {
+        ap.vox = ctx->pl.vox;
+        ap.s0 = 64; // (group 0 is empty)
+        ap.s1 = ctx->pl.nslots;
+    }
+    const int nab = nmr::apply_blocks(list ? (uint64_t)(ap.s1 - ap.s0) : (uint64_t)p.nx * p.ny * p.nz);
+    if ((rc = ensure_dev_doubles(c, &c->apart, &c->apart_cap, (size_t)nab * 6))) return rc;
+    ap.x = c->t.x;
     ap.mask = ctx->mask;
     ap.part = c->apart;
     ap.nx = p.nx;
@@ -777,52 +776,49 @@ int nmr_hip_run_learned(nmr_ctx* ctx, nmr_corrector* c, int64_t ncoarse, int32_t
     ap.by0 = p.buffer[1]; ap.by1 = p.ny - p.buffer[1];
     ap.bz0 = p.buffer[2]; ap.bz1 = p.nz - p.buffer[2];
     ap.scale = (float)c->out_scale;
+    // which of the two state buffers is current
+    int& cur_buf = list ? ctx->ppar : ctx->cur;
     // stats: [energy, max |correction|, max |M| before, non-finite, sum Mx, sum My]
     auto stats = [&](int buf, const float* pred, double st[6]) -> int {
         ap.mx = ctx->m[buf][0];
         ap.my = ctx->m[buf][1];
+        ap.slots = list ? ctx->pl.state[buf] : nullptr;
         ap.pred = pred;
-        HIP_TRY(nmr::launch_apply(ap, ctx->stream));
-        HIP_TRY(nmr::launch_stats_reduce(c->apart, nab, c->dstat, ctx->stream));
-        HIP_TRY(hipMemcpyAsync(st, c->dstat, 6 * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
+        HIP_TRY(nmr::launch_apply(ap, nab, ctx->stream));
+        HIP_TRY(nmr::launch_stats_reduce(c->apart, nab, c->hstat, ctx->stream));
         HIP_TRY(hipStreamSynchronize(ctx->stream));
+        std::copy(c->hstat, c->hstat + 6, st);
         return NMR_OK;
     };
     // the net's stream waits on the context's stream through explicit syncs
     HIP_TRY(hipStreamSynchronize(c->stream));
+    // the net's input: its pore and velocity channels once per run, its first
+    // two by every pass of the statistics
+    nmr::FeatureArgs f{};
+    f.mx = ctx->m[ctx->cur][0];
+    f.my = ctx->m[ctx->cur][1];
+    f.mask = ctx->mask;
+    f.vx = ctx->vx;
+    f.vy = ctx->vy;
+    f.vz = ctx->vz;
+    f.out = c->t.x;
+    f.nx = p.nx;
+    f.ny = p.ny;
+    f.nz = p.nz;
+    f.pitch = ctx->pitch;
+    f.pitch1 = ctx->pitch1;
+    f.vinv = ctx->vel ? (float)(1.0 / c->vscale) : 0.f;
+    HIP_TRY(nmr::launch_features(f, ctx->stream));
     double cur[6];
-    if ((rc = stats(ctx->cur, nullptr, cur))) return rc;
+    if ((rc = stats(cur_buf, nullptr, cur))) return rc;
     if (signal) {
         signal[0] = cur[4];
         signal[1] = cur[5];
     }
     int64_t nfall = 0, why[3] = {0, 0, 0};
     std::vector<double> sig8((size_t)(factor + 1) * 2);
-    const float vinv = (float)(1.0 / c->vscale);
-    // the z-marching kernels stage (Mx, My) from the state: the feature
-    // tensor's other channels (pore, velocity) are written once per run
-    const bool state_fed = (c->conv == NMR_CONV_ZMARCH || c->conv == NMR_CONV_ZMARCH_SPARSE) && zm_fits(c->t);
-    auto features = [&](int buf) -> int {
-        nmr::FeatureArgs f{};
-        f.mx = ctx->m[buf][0];
-        f.my = ctx->m[buf][1];
-        f.mask = ctx->mask;
-        f.vx = ctx->vx;
-        f.vy = ctx->vy;
-        f.vz = ctx->vz;
-        f.out = c->t.x;
-        f.nx = p.nx;
-        f.ny = p.ny;
-        f.nz = p.nz;
-        f.pitch = ctx->pitch;
-        f.pitch1 = ctx->pitch1;
-        f.vinv = ctx->vel ? vinv : 0.f;
-        HIP_TRY(nmr::launch_features(f, ctx->stream));
-        return NMR_OK;
-    };
-    if (state_fed && ncoarse > 0 && (rc = features(ctx->cur))) return rc;
     for (int64_t k = 0; k < ncoarse; k++) {
-        const int in = ctx->cur, out = in ^ 1;
+        const int in = cur_buf, out = in ^ 1;
         double gsum = 0.0;
         for (int s = 0; s < factor; s++) gsum += grad_sched ? grad_sched[3 * (k * factor + s) + 2] : p.grad[2];
         if (!(p.flags & NMR_F_PRECESSION)) gsum = 0.0;
@@ -833,19 +829,19 @@ int nmr_hip_run_learned(nmr_ctx* ctx, nmr_corrector* c, int64_t ncoarse, int32_t
                     return fail(NMR_ERR_UNSUPPORTED, "ncomp 2 takes a finite z gradient only");
             }
         // coarse step into the other buffer
-        if ((rc = nmri::sweep_step(ctx, coarse_coef(p, factor, &gsum), true, in, out))) return rc;
-        if (!state_fed && (rc = features(in))) return rc;
+        const nmr::Coef cf = coarse_coef(p, factor, &gsum);
+        if ((rc = list ? nmri::list_step(ctx, cf) : nmri::sweep_step(ctx, cf, true, in, out))) return rc;
         // the net runs on the context's stream
         hipStream_t keep_stream = c->stream;
         c->stream = ctx->stream;
-        rc = state_fed ? forward(c, true, ctx->m[in][0], ctx->m[in][1], ctx->pitch) : forward(c, true);
+        rc = forward(c, true);
         c->stream = keep_stream;
         if (rc) return rc;
         double nxt[6];
         if ((rc = stats(out, c->t.p, nxt))) return rc;
         const bool finite = nxt[3] == 0.0, energy = nxt[0] <= cur[0] * (1.0 + tol), size = nxt[1] <= tol * cur[2];
         if (finite && energy && size) {
-            ctx->cur = out;
+            cur_buf = out;
             std::copy(nxt, nxt + 6, cur);
         } else {
             nfall += 1;
@@ -855,7 +851,7 @@ int nmr_hip_run_learned(nmr_ctx* ctx, nmr_corrector* c, int64_t ncoarse, int32_t
             if (grad_sched) gs.assign(grad_sched + 3 * k * factor, grad_sched + 3 * (k + 1) * factor);
             ctx->sig_valid = false; // accepted coarse steps changed the state
             if ((rc = nmr_hip_run(ctx, factor, grad_sched ? gs.data() : nullptr, sig8.data()))) return rc;
-            if ((rc = stats(ctx->cur, nullptr, cur))) return rc;
+            if ((rc = stats(cur_buf, nullptr, cur))) return rc;
         }
         if (signal) {
             signal[2 * (k + 1)] = cur[4];

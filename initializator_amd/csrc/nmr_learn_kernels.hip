@@ -32,6 +32,7 @@ namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float fl4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4))); // (arrays of uint4 end up in scratch memory)
 
 // Round to nearest even (NaN kept quiet), and back.
 __device__ __forceinline__ uint16_t f2bf(float f)
@@ -234,26 +235,14 @@ __global__ void __launch_bounds__(256) conv_tile_kernel(ConvArgs a)
 // two at a time in one instruction (a branch on NaN for each value cost 15 %).
 // What is left is the chain of a plane -- reads, MFMAs, store, barrier -- with
 // two workgroups a CU.  96x80x64, with one read an MFMA and columns of 16
-// planes before: 34.4 -> 14.6 us at 16 -> 16, 26.7 -> 11.3 at 16 -> 2, 39.5 ->
-// 15.1 the input gradient, 25.9 -> 9.7 at 8 -> 16.  128^3: 41.6 -> 36.0, 31.6 ->
-// 30.7 (the MFMAs of 18 planes take 27 us at 2.4 GHz), 53.3 the gradient, 24.7.
+// planes before: 34.4 -> 14.2 us at 16 -> 16, 26.7 -> 11.3 at 16 -> 2, 39.5 ->
+// 14.8 the input gradient, 25.9 -> 10.1 at 8 -> 16.  128^3: 41.6 -> 33.2, 31.6 ->
+// 28.5 (the MFMAs of 18 planes take 13.4 a SIMD's wavefront, two of them 27 us
+// at 2.4 GHz), 45.2 the gradient, 23.2 at 8 -> 16.
 //
 // Persistent: workgroup b takes columns b, b + gridDim.x, ...; a column is
-// a.zc output planes (the last one what is left).  MODE 4 (8 input channels)
-// is MODE 0 with the input's channels 0 and 1 staged from the FP32 state
-// a.smx/smy times the pore channel, rounded as feature_kernel rounds them, so
-// that the feature tensor's other channels (pore, velocity), which do not
-// change during a run, are written once.
+// a.zc output planes (the last one what is left).
 constexpr int kZmY = 16;
-template <int N>
-struct Plane {
-    uint4 v[N];
-};
-template <int N>
-struct PlaneS {
-    uint4 v[N];
-    float fx[N], fy[N];
-};
 template <int CIN, int MODE>
 __global__ void __launch_bounds__(256, 2) conv_zm_kernel(ConvArgs a)
 {
@@ -264,7 +253,7 @@ __global__ void __launch_bounds__(256, 2) conv_zm_kernel(ConvArgs a)
     constexpr int PV = HV * V16;               // uint4 per staged plane
     constexpr int NLD = (PV + 255) / 256;
     constexpr int ROWB = HX * 16, SLOTB = PV * 16; // bytes per staged row and per slot
-    __shared__ uint4 sin[3 * PV + HX + 16];    // (the zeroed half of the last row's last chunk reads past the plane)
+    __shared__ u32x4 sin[3 * PV + HX + 16];    // (the zeroed half of the last row's last chunk reads past the plane)
     const int lane = threadIdx.x & 63;
     const int g = lane >> 4, n = lane & 15;
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
@@ -272,7 +261,6 @@ __global__ void __launch_bounds__(256, 2) conv_zm_kernel(ConvArgs a)
     const uint4* wa4 = reinterpret_cast<const uint4*>(a.wa);
 #pragma unroll
     for (int c = 0; c < NCH; c++) A[c] = as_bf8(wa4[c * 64 + lane]);
-    static_assert(MODE != 4 || CIN == 8, "state-fed input is the first layer's");
     // Byte offset of this lane's part of an operand within a plane: (row, x)
     // of the lane's tap from the operand's row of this wavefront.
     auto at = [&](int row, int dx) {
@@ -303,7 +291,7 @@ __global__ void __launch_bounds__(256, 2) conv_zm_kernel(ConvArgs a)
     }
     const bool last = (NCH - 1) * TPC + tg < 27; // the lane's tap of the last chunk exists
     float bias[4] = {0.f, 0.f, 0.f, 0.f};
-    if constexpr (MODE == 0 || MODE == 4) {
+    if constexpr (MODE == 0) {
 #pragma unroll
         for (int j = 0; j < 4; j++) bias[j] = a.bias[4 * g + j];
     } else if constexpr (MODE == 1) {
@@ -315,9 +303,9 @@ __global__ void __launch_bounds__(256, 2) conv_zm_kernel(ConvArgs a)
     const int nyb = (a.ny + kZmY - 1) / kZmY, nzb = (a.nz + zc - 1) / zc;
     const int ncol = a.nseg * nyb * nzb;
     char* lds = reinterpret_cast<char*>(sin);
-    auto read = [&](int o) { return *reinterpret_cast<const uint4*>(lds + o); };
-    auto mfma = [&](int c, const uint4& b, fl4& d) {
-        d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[c], as_bf8(b), d, 0, 0, 0);
+    auto read = [&](int o) { return *reinterpret_cast<const u32x4*>(lds + o); };
+    auto mfma = [&](int c, const u32x4& b, fl4& d) {
+        d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[c], __builtin_bit_cast(bf16x8, b), d, 0, 0, 0);
     };
     for (int col = xcd_tile(blockIdx.x, (int)gridDim.x); col < ncol; col += gridDim.x) {
         const int seg = col % a.nseg, r2 = col / a.nseg;
@@ -328,63 +316,44 @@ __global__ void __launch_bounds__(256, 2) conv_zm_kernel(ConvArgs a)
         // feed only outputs that are not stored); a thread's element past the
         // plane loads element 0 again and is not stored
         uint32_t goff[NLD]; // bytes in a plane (below 4 GiB)
-        int sidx[NLD]; // MODE 4: the state index of an interior voxel in its plane, else -1
 #pragma unroll
         for (int j = 0; j < NLD; j++) {
             const int i = threadIdx.x + 256 * j < PV ? threadIdx.x + 256 * j : 0;
             const int v = i / V16;
             const int gx = min(x0 + v % HX, a.nx + 1), gy = min(y0 + v / HX, a.ny + 1);
             goff[j] = (uint32_t)(gy * px + gx) * (uint32_t)(2 * CIN) + (uint32_t)(i % V16) * 16u;
-            sidx[j] = (gx >= 1 && gx <= a.nx && gy >= 1 && gy <= a.ny) ? (gy - 1) * a.spitch + gx - 1 : -1;
         }
-        using PL = typename std::conditional<MODE == 4, PlaneS<NLD>, Plane<NLD>>::type;
-        auto load = [&](int pz, PL& r) {
+        auto load = [&](int pz, u32x4 (&r)[NLD]) {
             const char* in = reinterpret_cast<const char*>(a.in + (size_t)pz * plane * CIN);
-            const size_t c0 = (size_t)max(pz - 1, 0) * a.ny * a.spitch;
 #pragma unroll
-            for (int j = 0; j < NLD; j++) {
-                r.v[j] = *reinterpret_cast<const uint4*>(in + goff[j]);
-                if constexpr (MODE == 4) {
-                    const bool ok = sidx[j] >= 0 && pz >= 1 && pz <= a.nz;
-                    r.fx[j] = ok ? a.smx[c0 + sidx[j]] : 0.f;
-                    r.fy[j] = ok ? a.smy[c0 + sidx[j]] : 0.f;
-                }
-            }
+            for (int j = 0; j < NLD; j++) r[j] = *reinterpret_cast<const u32x4*>(in + goff[j]);
         };
-        auto stash = [&](int pz, int slot, const PL& r) {
+        auto stash = [&](int slot, const u32x4 (&r)[NLD]) {
 #pragma unroll
             for (int j = 0; j < NLD; j++) {
                 const int i = threadIdx.x + 256 * j;
-                if (i < PV) {
-                    uint4 w = r.v[j];
-                    if constexpr (MODE == 4) {
-                        if (sidx[j] >= 0 && pz >= 1 && pz <= a.nz) {
-                            // feature_kernel's channels 0, 1: (Mx, My) * pore
-                            const float pore = (w.y & 0xffffu) != 0u ? 1.f : 0.f;
-                            w.x = (uint32_t)f2bf(r.fx[j] * pore) | ((uint32_t)f2bf(r.fy[j] * pore) << 16);
-                        }
-                    }
-                    sin[slot * PV + (i % V16) * HV + i / V16] = w;
-                }
+                if (i < PV) sin[slot * PV + (i % V16) * HV + i / V16] = r[j];
             }
         };
         const int x = x0 + n, yw = y0 + wave * 4;
         const bool live = yw < a.ny; // this wavefront has rows
         // this lane's first output in its plane, in bytes
         const uint32_t oo = (uint32_t)((yw + 1) * px + x + 1) * (MODE == 1 ? 8u : 32u) + (MODE == 1 ? 0u : 8u * g);
-        PL pl[3];
+        u32x4 l0[NLD], l1[NLD], l2[NLD];
         // Plane p in slot s (p - zs modulo 3): opens output plane p in `first`,
-        // goes on with p - 1 in `mid` and completes p - 2 in `fin`.
-        auto step = [&](const int p, auto S, fl4 (&first)[4], fl4 (&mid)[4], fl4 (&fin)[4]) {
+        // goes on with p - 1 in `mid` and completes p - 2 in `fin`; plane p + 1 is
+        // on its way in `next`, and p + 2 sets out into `ahead`.
+        auto step = [&](const int p, auto S, const u32x4 (&next)[NLD], u32x4 (&ahead)[NLD], fl4 (&first)[4], fl4 (&mid)[4],
+                        fl4 (&fin)[4]) {
             constexpr int s = decltype(S)::value;
             constexpr int sb = s * SLOTB;
             const int z = p - 2;
             const bool out = z >= zs;
-            if (p + 2 <= ze + 1) load(p + 2, pl[(s + 2) % 3]);
+            load(min(p + 2, ze + 1), ahead); // (without a branch, whose join would wait for the loads)
             const size_t zb = (size_t)(z + 1) * plane; // (z + 1 = p - 1 < 0 only where nothing is stored)
             uint2 gate[4];
             if (live) {
-                uint4 P[6], Q[6], X[6];
+                u32x4 P[6], Q[6], X[6];
 #pragma unroll
                 for (int r = 0; r < 6; r++) {
                     P[r] = read(o0 + sb + r * ROWB);
@@ -411,7 +380,7 @@ __global__ void __launch_bounds__(256, 2) conv_zm_kernel(ConvArgs a)
                     }
                 }
                 if (p - 1 >= zs && p - 1 < ze) {
-                    uint4 M[4];
+                    u32x4 M[4];
 #pragma unroll
                     for (int i = 0; i < 4; i++) M[i] = read(m0[s] + i * ROWB);
                     if constexpr (CIN == 16) {
@@ -433,7 +402,7 @@ __global__ void __launch_bounds__(256, 2) conv_zm_kernel(ConvArgs a)
                     }
                 }
                 if (out) {
-                    const uint4 none = make_uint4(0u, 0u, 0u, 0u);
+                    const u32x4 none = {0u, 0u, 0u, 0u};
                     if constexpr (MODE == 2) {
 #pragma unroll
                         for (int i = 0; i < 4; i++) {
@@ -455,7 +424,7 @@ __global__ void __launch_bounds__(256, 2) conv_zm_kernel(ConvArgs a)
 #pragma unroll
                         for (int i = 0; i < 4; i++) mfma(13, last ? X[i + 2] : none, fin[i]);
                     } else {
-                        uint4 M[4];
+                        u32x4 M[4];
 #pragma unroll
                         for (int i = 0; i < 4; i++) M[i] = read(m1[s] + i * ROWB);
 #pragma unroll
@@ -468,7 +437,7 @@ __global__ void __launch_bounds__(256, 2) conv_zm_kernel(ConvArgs a)
                 }
             }
             // the next plane goes into the slot of plane p - 2, last read in the step before
-            if (p + 1 <= ze + 1) stash(p + 1, (s + 1) % 3, pl[(s + 1) % 3]);
+            stash((s + 1) % 3, next);
             if (live && out) {
                 // lane holds output channels 4g..4g+3 of voxel n
 #pragma unroll
@@ -480,7 +449,7 @@ __global__ void __launch_bounds__(256, 2) conv_zm_kernel(ConvArgs a)
                                 make_float2(fin[i][0] + bias[0], fin[i][1] + bias[1]);
                     } else {
                         uint32_t h[2];
-                        if constexpr (MODE == 0 || MODE == 4) {
+                        if constexpr (MODE == 0) {
                             float v[4];
 #pragma unroll
                             for (int j = 0; j < 4; j++) v[j] = fmaxf(fin[i][j] + bias[j], 0.f);
@@ -502,9 +471,9 @@ __global__ void __launch_bounds__(256, 2) conv_zm_kernel(ConvArgs a)
             }
             lds_barrier();
         };
-        load(zs, pl[0]);
-        load(zs + 1, pl[1]);
-        stash(zs, 0, pl[0]);
+        load(zs, l0);
+        load(zs + 1, l1);
+        stash(0, l0);
         lds_barrier();
         fl4 acc[3][4];
 #pragma unroll
@@ -512,11 +481,11 @@ __global__ void __launch_bounds__(256, 2) conv_zm_kernel(ConvArgs a)
 #pragma unroll
             for (int i = 0; i < 4; i++) acc[k][i] = fl4{0.f, 0.f, 0.f, 0.f};
         for (int p = zs; p <= ze + 1; p += 3) {
-            step(p, std::integral_constant<int, 0>{}, acc[0], acc[2], acc[1]);
+            step(p, std::integral_constant<int, 0>{}, l1, l2, acc[0], acc[2], acc[1]);
             if (p + 1 > ze + 1) break;
-            step(p + 1, std::integral_constant<int, 1>{}, acc[1], acc[0], acc[2]);
+            step(p + 1, std::integral_constant<int, 1>{}, l2, l0, acc[1], acc[0], acc[2]);
             if (p + 2 > ze + 1) break;
-            step(p + 2, std::integral_constant<int, 2>{}, acc[2], acc[1], acc[0]);
+            step(p + 2, std::integral_constant<int, 2>{}, l0, l1, acc[2], acc[1], acc[0]);
         }
     }
 }
@@ -790,32 +759,55 @@ __global__ void __launch_bounds__(256) diff_kernel(const float* __restrict__ ax,
     oy[i] = ay[i] - by[i];
 }
 
-// Adds scale * pred to the pores of (mx, my) and reduces, per block, the
-// state's pore energy sum(Mx^2 + My^2), the largest |correction|, the
-// largest |M| of the state before the correction, a non-finite count, and
-// the signal sums over the trim window: part[block][6].
-constexpr int kApplyBlocks = 2048; // workgroups (= partials) of the apply pass
+// Adds scale * pred to the pores of the state, brings the result into the
+// net's input (channels 0 and 1, what feature_kernel writes there: the other
+// channels do not change during a run, and solids hold 0), and reduces, per
+// block, the state's pore energy sum(Mx^2 + My^2), the largest |correction|,
+// the largest |M| of the state before the correction, a non-finite count, and
+// the signal sums over the trim window: part[block][6].  LIST: the state is
+// in the list of the pores.  128^3, porosity 0.2: 9.8 us on the list, 16.2 over
+// the rows (every voxel's mask, 64-bit indices).
+constexpr int kApplyBlocks = 1024; // workgroups (= partials) of the apply pass
+template <bool LIST>
 __global__ void __launch_bounds__(256) apply_kernel(ApplyArgs a)
 {
     __shared__ double sh[4][6];
-    const long n = (long)a.nx * a.ny * a.nz;
+    // (the padded grid has fewer than 2^31 voxels)
+    const uint32_t n = LIST ? a.s1 - a.s0 : (uint32_t)a.nx * (uint32_t)a.ny * (uint32_t)a.nz;
     double st[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0}; // energy, max |d|, max |M|, non-finite, sum Mx, sum My
-    for (long v = (long)blockIdx.x * 256 + threadIdx.x; v < n; v += (long)gridDim.x * 256) {
-        const int x = (int)(v % a.nx), y = (int)((v / a.nx) % a.ny), z = (int)(v / ((long)a.nx * a.ny));
+    for (uint32_t v = blockIdx.x * 256u + threadIdx.x; v < n; v += gridDim.x * 256u) {
+        const uint32_t row = LIST ? (uint32_t)a.pitch : (uint32_t)a.nx, plane = (uint32_t)a.ny * row;
+        const uint32_t o = LIST ? a.vox[a.s0 + v] : v;
+        if (LIST && o == 0xffffffffu) continue;
+        const int x = (int)(o % plane % row), y = (int)(o % plane / row), z = (int)(o / plane);
         const size_t c = ((size_t)z * a.ny + y) * a.pitch + x;
         if (!a.mask[c]) continue;
-        float mx = a.mx[c], my = a.my[c];
+        const size_t pv = ((size_t)(z + 1) * (a.ny + 2) + (y + 1)) * (a.nx + 2) + (x + 1);
+        float mx, my;
+        if constexpr (LIST) {
+            const float2 m = *reinterpret_cast<const float2*>(a.slots + 2 * (size_t)(a.s0 + v));
+            mx = m.x;
+            my = m.y;
+        } else {
+            mx = a.mx[c];
+            my = a.my[c];
+        }
         st[2] = fmax(st[2], (double)fmaxf(fabsf(mx), fabsf(my)));
         if (a.pred) {
-            const long pv = ((long)(z + 1) * (a.ny + 2) + (y + 1)) * (a.nx + 2) + (x + 1);
-            const float d0 = a.scale * a.pred[pv * 2], d1 = a.scale * a.pred[pv * 2 + 1];
+            const float2 p = *reinterpret_cast<const float2*>(a.pred + pv * 2);
+            const float d0 = a.scale * p.x, d1 = a.scale * p.y;
             mx += d0;
             my += d1;
-            a.mx[c] = mx;
-            a.my[c] = my;
+            if constexpr (LIST) {
+                *reinterpret_cast<float2*>(a.slots + 2 * (size_t)(a.s0 + v)) = make_float2(mx, my);
+            } else {
+                a.mx[c] = mx;
+                a.my[c] = my;
+            }
             st[1] = fmax(st[1], (double)fmaxf(fabsf(d0), fabsf(d1)));
             if (!(fabsf(d0) <= 3.0e38f) || !(fabsf(d1) <= 3.0e38f)) st[3] += 1.0;
         }
+        *reinterpret_cast<uint32_t*>(a.x + pv * 8) = f2bf2(mx, my);
         if (!(fabsf(mx) <= 3.0e38f) || !(fabsf(my) <= 3.0e38f)) st[3] += 1.0;
         st[0] += (double)mx * mx + (double)my * my;
         if (x >= a.bx0 && x < a.bx1 && y >= a.by0 && y < a.by1 && z >= a.bz0 && z < a.bz1) {
@@ -930,7 +922,6 @@ hipError_t launch_conv_zm(int cin, int mode, const ConvArgs& a, int grid, hipStr
 {
     const dim3 g(grid), b(256);
     if (cin == 8 && mode == 0) hipLaunchKernelGGL((conv_zm_kernel<8, 0>), g, b, 0, s, a);
-    else if (cin == 8 && mode == 4) hipLaunchKernelGGL((conv_zm_kernel<8, 4>), g, b, 0, s, a);
     else if (cin == 16 && mode == 0) hipLaunchKernelGGL((conv_zm_kernel<16, 0>), g, b, 0, s, a);
     else if (cin == 16 && mode == 1) hipLaunchKernelGGL((conv_zm_kernel<16, 1>), g, b, 0, s, a);
     else if (cin == 16 && mode == 2) hipLaunchKernelGGL((conv_zm_kernel<16, 2>), g, b, 0, s, a);
@@ -1009,11 +1000,12 @@ hipError_t launch_diff(const float* ax, const float* ay, const float* bx, const 
     return hipGetLastError();
 }
 
-int apply_blocks(int nx, int ny, int nz) { return (int)std::max<long>(1, std::min<long>(kApplyBlocks, blocks_for((long)nx * ny * nz))); }
+int apply_blocks(uint64_t n) { return (int)std::max<uint64_t>(1, std::min<uint64_t>(kApplyBlocks, (n + 255) / 256)); }
 
-hipError_t launch_apply(const ApplyArgs& a, hipStream_t s)
+hipError_t launch_apply(const ApplyArgs& a, int blocks, hipStream_t s)
 {
-    hipLaunchKernelGGL(apply_kernel, dim3(apply_blocks(a.nx, a.ny, a.nz)), dim3(256), 0, s, a);
+    if (a.vox) hipLaunchKernelGGL(apply_kernel<true>, dim3(blocks), dim3(256), 0, s, a);
+    else hipLaunchKernelGGL(apply_kernel<false>, dim3(blocks), dim3(256), 0, s, a);
     return hipGetLastError();
 }
 

@@ -276,3 +276,50 @@ def test_matrix_core_rate_is_measured():
     assert lib.nmr_hip_mfma_rate(256, 2, ctypes.byref(tf)) == 0, lib.nmr_hip_last_error().decode()
     print(f"[mfma] {tf.value:.0f} TFLOP/s dense BF16 (v_mfma_f32_16x16x32_bf16)", flush=True)
     assert 0.0 < tf.value <= 2750.0
+
+
+@pytest.mark.parametrize("kind", ["smooth", "ragged", "one", "none", "read solids", "trim"])
+def test_learned_solve_on_the_list_of_pores_equals_the_rows(kind):
+    """The learned solve steps on the list of the pores where a run would, on
+    the row buffers otherwise: the same operations on the same values, so the
+    fields agree bit for bit and the signal to the order of its FP64 sums.
+    Some steps are accepted and some redone (a bound on the corrections that
+    splits them), on grids off every tile's edge, with one pore and none, with
+    solids that pores read, and with a trimmed signal window."""
+    shape = {"ragged": (7, 19, 37), "one": (3, 4, 5), "none": (3, 4, 5)}.get(kind, (20, 18, 33))
+    if kind in ("one", "none"):
+        mask = np.zeros(shape, np.uint8)
+        mask[1, 2, 3] = kind == "one"
+    else:
+        mask = generators.porosity(shape, 0.3, 31, sigma=1.5)
+    vel = generators.velocity(mask, 32, sigma=1.5, vmax=1e-3, d=(DX, DX, DX))
+    if kind == "read solids":
+        vel = generators.velocity(np.ones(shape, np.uint8), 33, sigma=1.5, vmax=1e-3, d=(DX, DX, DX))
+    rng = np.random.default_rng(34)
+    m0 = [rng.normal(0.5, 0.2, shape), rng.normal(0.0, 0.2, shape)]
+    if kind != "read solids":
+        m0 = [m * mask for m in m0]
+    ncoarse, factor = 6, 4
+    sched = generators.pgse_schedule(ncoarse * factor, DT, 0.2, 2e-4, 4e-4)
+    out = {}
+    with Corrector(8) as net:
+        net.set_scales(1e-3, 1e-3)
+        for rows in (False, True):
+            for tol in (1e30, 4e-4):
+                with HipSolver(shape, 2, DX, DT, D, 0.5, r1_bulk=1 / 2.5e10, rho1=20e-6, rho2=20e-6, velocity=True,
+                               precession=True, phase_exact=True, buffer=(1, 2, 0) if kind == "trim" else (0, 0, 0)) as s:
+                    s.set_layout(not rows)
+                    s.upload_mask(mask)
+                    s.upload_velocity(*vel)
+                    s.upload_magnetization(*m0)
+                    a, na = net.run_learned(s, ncoarse, factor, sched, tol=tol, reasons=True)
+                    b = s.run(3)  # a run continues from where the learned solve left off
+                    c, nb = net.run_learned(s, 2, factor, None, tol=tol, reasons=True)
+                    out[rows, tol] = (np.concatenate([a, b, c]), na + nb, s.download_magnetization())
+    for tol in (1e30, 4e-4):
+        (sig, nf, f), (sig_r, nf_r, f_r) = out[False, tol], out[True, tol]
+        print(f"[learned] {kind} tol {tol:g}: {nf}", flush=True)
+        assert nf == nf_r
+        for a, b in zip(f, f_r):
+            np.testing.assert_array_equal(a, b)
+        np.testing.assert_allclose(sig, sig_r, rtol=1e-12, atol=1e-12 * max(1e-30, np.abs(sig_r).max()))
