@@ -1494,19 +1494,16 @@ int nmr_hip_download_magnetization(nmr_ctx* ctx, double* mx, double* my, double*
     double* dst[3] = {mx, my, mz};
     const nmr_problem& p = ctx->prob;
     if ((rc = nmri::state_rows(ctx))) return rc;
-    std::vector<float> h(ctx->n_m);
+    std::vector<float> h(layout == NMR_LAYOUT_COMPACT ? 0 : ctx->n_m);
     for (int q = 0; q < ctx->nc; q++) {
         if (!dst[q]) continue;
-        HIP_TRY(hipMemcpyAsync(h.data(), ctx->m[ctx->cur][q], h.size() * sizeof(float), hipMemcpyDeviceToHost,
-                               ctx->stream));
-        HIP_TRY(hipStreamSynchronize(ctx->stream));
         if (layout == NMR_LAYOUT_COMPACT) {
-            for (int k = 0; k < p.nz; k++)
-                for (int j = 0; j < p.ny; j++)
-                    for (int i = 0; i < p.nx; i++)
-                        dst[q][(size_t)i + (size_t)p.nx * ((size_t)j + (size_t)p.ny * k)] =
-                            h[(size_t)k * p.ny * ctx->pitch + (size_t)j * ctx->pitch + i];
+            rc = ctx->stage.down_rows(ctx->stream, ctx->m[ctx->cur][q], p.nx, (size_t)p.ny * p.nz, ctx->pitch, dst[q]);
+            if (rc) return rc;
         } else {
+            HIP_TRY(hipMemcpyAsync(h.data(), ctx->m[ctx->cur][q], h.size() * sizeof(float), hipMemcpyDeviceToHost,
+                                   ctx->stream));
+            HIP_TRY(hipStreamSynchronize(ctx->stream));
             // interior plus the ghost layer each axis's boundary condition
             // leaves (copy of the adjacent cell, opposite cell, or 0)
             auto ghost = [](int i, int n, int bc, bool* zero) {
@@ -2653,16 +2650,10 @@ int nmr_hip_batch_download(nmr_batch* b, int32_t i, double* mx, double* my, doub
                                       b->stream));
         }
     }
-    HIP_TRY(hipStreamSynchronize(b->stream));
-    std::vector<float> h(I.n_m);
     for (int q = 0; q < b->nc; q++) {
         if (!dst[q]) continue;
-        HIP_TRY(hipMemcpy(h.data(), I.m[b->parity][q], h.size() * 4, hipMemcpyDeviceToHost));
-        for (int k = 0; k < s.nz; k++)
-            for (int j = 0; j < s.ny; j++)
-                for (int x = 0; x < s.nx; x++)
-                    dst[q][(size_t)x + (size_t)s.nx * ((size_t)j + (size_t)s.ny * k)] =
-                        h[(size_t)k * s.ny * I.pitch + (size_t)j * I.pitch + x];
+        const int rc = b->stage.down_rows(b->stream, I.m[b->parity][q], s.nx, (size_t)s.ny * s.nz, I.pitch, dst[q]);
+        if (rc) return rc;
     }
     return NMR_OK;
 }

@@ -11,6 +11,7 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <functional>
 #include <new>
 #include <string>
 #include <vector>
@@ -43,6 +44,28 @@ inline size_t biggest_array_bytes(int nx, int ny, int nz)
     } while (0)
 
 namespace nmri {
+
+// Pinned staging of one object's large copies (nmr_stage.hip): a ring of up to
+// kSlots slots, made when first needed.  A copy returns when it has ended and
+// its threads have.
+struct HostStage {
+    static constexpr size_t kSlotBytes = (size_t)1 << 20;
+    static constexpr int kSlots = 12;
+    char* buf = nullptr;
+    int have = 0;
+    std::array<hipEvent_t, kSlots> ev{};
+    HostStage() = default;
+    HostStage(const HostStage&) = delete;
+    HostStage& operator=(const HostStage&) = delete;
+    ~HostStage();
+    int open(int slots);
+    // n floats at src, in pieces of any length and order, to use(first, count, values).
+    int down(hipStream_t s, const float* src, size_t n, const std::function<void(size_t, size_t, const float*)>& use);
+    // n floats from host memory.
+    int up(hipStream_t s, float* dst, const float* src, size_t n);
+    // Rows of nx of `pitch` floats into a compact array of doubles.
+    int down_rows(hipStream_t s, const float* src, int nx, size_t rows, int pitch, double* dst);
+};
 
 // A list of the pores of one domain or of all instances of a batch
 // (nmr_pores.hip), its state and its per-slot data, in device memory.
@@ -162,6 +185,7 @@ struct nmr_ctx {
     size_t dsignal_cap = 0;  // doubles
     double* hsignal = nullptr; // pinned host staging of a run's signal rows (at most kPinnedSignal doubles)
     size_t hsignal_cap = 0;    // doubles
+    nmri::HostStage stage;     // downloads
     int cur = 0;
     bool has_mask = false, has_mag = false;
     int64_t mask_version = 0; // bumped by every mask upload
@@ -248,6 +272,7 @@ struct nmr_batch {
     double* d_signal = nullptr;
     double* h_signal = nullptr; // pinned host staging of a run's signal block
     size_t h_signal_cap = 0;    // doubles
+    nmri::HostStage stage;      // downloads
     size_t signal_cap = 0;
     double* d_fpart = nullptr; // field-sum partials (max nz)
     int* d_flag = nullptr;

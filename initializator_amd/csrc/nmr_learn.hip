@@ -63,6 +63,10 @@ struct nmr_corrector {
     int64_t rows_version = -1;
     int* rows[3] = {nullptr, nullptr, nullptr};
     int nrows[3] = {0, 0, 0};
+    // features and output gradients that a caller gives or takes: staging and device copies
+    nmri::HostStage stage;
+    float *io = nullptr, *io2 = nullptr;
+    size_t io_cap = 0, io2_cap = 0; // floats
     // convolution kernel (NMR_CONV_*) and planes per z-marching column
     int conv = 0;
     int zc = 0; // 0: by the grid (zm_planes)
@@ -342,31 +346,45 @@ int ensure_dev_doubles(nmr_corrector* c, double** p, size_t* cap, size_t n)
     return NMR_OK;
 }
 
+int ensure_io(nmr_corrector* c, float** p, size_t* cap, size_t n)
+{
+    if (n <= *cap) return NMR_OK;
+    if (*p) {
+        HIP_TRY(hipStreamSynchronize(c->stream));
+        HIP_TRY(hipFree(*p));
+    }
+    *p = nullptr;
+    *cap = 0;
+    HIP_TRY(hipMalloc((void**)p, std::max<size_t>(n * sizeof(float), 256)));
+    *cap = n;
+    return NMR_OK;
+}
+
 // Interior of a padded FP32 2-channel tensor to host [nz][ny][nx][2].
 int download_p(nmr_corrector* c, float* out)
 {
     const Tensors& t = c->t;
-    const size_t nv = (size_t)(t.nx + 2) * (t.ny + 2) * (t.nz + 2);
-    std::vector<float> h(nv * 2);
-    HIP_TRY(hipMemcpyAsync(h.data(), t.p, h.size() * 4, hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
-    for (int z = 0; z < t.nz; z++)
-        for (int y = 0; y < t.ny; y++)
-            for (int x = 0; x < t.nx; x++) {
-                const size_t pv = ((size_t)(z + 1) * (t.ny + 2) + (y + 1)) * (t.nx + 2) + (x + 1);
-                const size_t v = ((size_t)z * t.ny + y) * t.nx + x;
-                out[2 * v] = h[2 * pv];
-                out[2 * v + 1] = h[2 * pv + 1];
-            }
-    return NMR_OK;
+    const size_t px = 2 * (size_t)(t.nx + 2), py = (size_t)(t.ny + 2); // floats a padded row, rows a padded plane
+    const size_t nx = 2 * (size_t)t.nx, ny = (size_t)t.ny;
+    // planes 1 .. nz; a row gives what of it lies in 2 .. px - 2
+    return c->stage.down(c->stream, t.p + px * py, px * py * (size_t)t.nz, [=](size_t i, size_t n, const float* p) {
+        for (size_t e = i + n; i < e;) {
+            const size_t r = i / px, y = r % py, z = r / py, end = std::min(e, (r + 1) * px);
+            const size_t from = std::max(i, r * px + 2), to = std::min(end, r * px + px - 2);
+            if (y >= 1 && y <= ny && from < to)
+                std::memcpy(out + (z * ny + y - 1) * nx + (from - r * px - 2), p + (from - i), (to - from) * sizeof(float));
+            p += end - i;
+            i = end;
+        }
+    });
 }
 
-int upload_features(nmr_corrector* c, int nx, int ny, int nz, const float* f6, float** dev)
+int upload_features(nmr_corrector* c, int nx, int ny, int nz, const float* f6)
 {
     const size_t n = (size_t)nx * ny * nz * 6;
-    HIP_TRY(hipMalloc((void**)dev, std::max<size_t>(n * 4, 256)));
-    HIP_TRY(hipMemcpyAsync(*dev, f6, n * 4, hipMemcpyHostToDevice, c->stream));
-    HIP_TRY(nmr::launch_feature_copy(*dev, nx, ny, nz, c->t.x, c->stream));
+    int rc = ensure_io(c, &c->io, &c->io_cap, n);
+    if (rc || (rc = c->stage.up(c->stream, c->io, f6, n))) return rc;
+    HIP_TRY(nmr::launch_feature_copy(c->io, nx, ny, nz, c->t.x, c->stream));
     return NMR_OK;
 }
 
@@ -439,7 +457,7 @@ int nmr_hip_corrector_destroy(nmr_corrector* c)
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     tfree(c->t);
     for (void* q : {(void*)c->w, (void*)c->m, (void*)c->v, (void*)c->grad, (void*)c->f1, (void*)c->f2, (void*)c->f3,
-                    (void*)c->d2, (void*)c->d3, (void*)c->wpart, (void*)c->lpart, (void*)c->apart, (void*)c->rows[0], (void*)c->rows[1], (void*)c->rows[2]})
+                    (void*)c->d2, (void*)c->d3, (void*)c->wpart, (void*)c->lpart, (void*)c->apart, (void*)c->io, (void*)c->io2, (void*)c->rows[0], (void*)c->rows[1], (void*)c->rows[2]})
         if (q) (void)hipFree(q);
     if (c->hstat) (void)hipHostFree(c->hstat);
     if (c->stream) (void)hipStreamDestroy(c->stream);
@@ -501,12 +519,10 @@ int nmr_hip_corrector_forward(nmr_corrector* c, int32_t nx, int32_t ny, int32_t 
     if (!c || !features || !out) return fail(NMR_ERR_NULL, "nmr_hip_corrector_forward: null argument");
     int rc = check_dims(nx, ny, nz);
     if (rc || (rc = ensure_tensors(c, nx, ny, nz, false))) return rc;
-    float* dev = nullptr;
-    rc = upload_features(c, nx, ny, nz, features, &dev);
+    rc = upload_features(c, nx, ny, nz, features);
     if (!rc) rc = forward(c);
     if (!rc) rc = download_p(c, out);
     (void)hipStreamSynchronize(c->stream);
-    if (dev) (void)hipFree(dev);
     return rc;
 }
 
@@ -517,24 +533,18 @@ int nmr_hip_corrector_backward(nmr_corrector* c, int32_t nx, int32_t ny, int32_t
         return fail(NMR_ERR_NULL, "nmr_hip_corrector_backward: null argument");
     int rc = check_dims(nx, ny, nz);
     if (rc || (rc = ensure_tensors(c, nx, ny, nz, true))) return rc;
-    float* dev = nullptr;
-    float* dg = nullptr;
     const size_t n = (size_t)nx * ny * nz;
-    rc = upload_features(c, nx, ny, nz, features, &dev);
+    rc = ensure_io(c, &c->io2, &c->io2_cap, n * 2);
+    if (!rc) rc = upload_features(c, nx, ny, nz, features);
     if (!rc) rc = forward(c);
-    if (!rc) {
-        if (hipMalloc((void**)&dg, std::max<size_t>(n * 8, 256)) != hipSuccess ||
-            hipMemcpyAsync(dg, grad_out, n * 8, hipMemcpyHostToDevice, c->stream) != hipSuccess ||
-            nmr::launch_gout_copy(dg, nx, ny, nz, c->t.g3, c->stream) != hipSuccess)
-            rc = fail(NMR_ERR_DEVICE, "output gradient upload failed");
-    }
+    if (!rc) rc = c->stage.up(c->stream, c->io2, grad_out, n * 2);
+    if (!rc && nmr::launch_gout_copy(c->io2, nx, ny, nz, c->t.g3, c->stream) != hipSuccess)
+        rc = fail(NMR_ERR_DEVICE, "output gradient upload failed");
     if (!rc) rc = backward(c);
     if (!rc && (hipMemcpyAsync(grad_params, c->grad, kParams * 4, hipMemcpyDeviceToHost, c->stream) != hipSuccess ||
                 hipStreamSynchronize(c->stream) != hipSuccess))
         rc = fail(NMR_ERR_DEVICE, "gradient download failed");
     (void)hipStreamSynchronize(c->stream);
-    if (dev) (void)hipFree(dev);
-    if (dg) (void)hipFree(dg);
     return rc;
 }
 

@@ -7,7 +7,7 @@ import pytest
 
 import oracle
 from initializator_amd import _lib, generators
-from initializator_amd.solver import HipSolver
+from initializator_amd.solver import BatchSolver, Corrector, HipSolver
 
 pytestmark = pytest.mark.gpu
 
@@ -100,3 +100,44 @@ def test_zero_steps(mode):
         np.testing.assert_array_equal(f[q], np.asarray(m0[q], dtype=np.float32))
         np.testing.assert_allclose(sig[0, q], np.sum(np.asarray(m0[q], dtype=np.float32) * mask, dtype=np.float64),
                                    rtol=1e-12)
+
+
+@pytest.mark.parametrize("shape", [(1, 1, 1), (3, 5, 7), (2, 3, 300001), (5, 401, 203), (67, 128, 255), (65, 256, 256)])
+def test_download_returns_every_voxel_through_the_staging(shape):
+    """Downloads pass through 1 MiB pinned slots, converted by several threads:
+    one slot and less, a slot's edge inside a row, rows longer than a slot, more
+    slots than the ring has; rows of whole and of padded length."""
+    rng = np.random.default_rng(list(shape))
+    mask = (rng.random(shape) < 0.4).astype(np.uint8)
+    m = [rng.standard_normal(shape).astype(np.float32).astype(np.float64) for _ in range(2)]
+    with HipSolver(shape, 2, 1e-6, 1e-5, 2.3e-9, 0.5) as s:
+        s.upload_mask(mask)
+        s.upload_magnetization(*m)
+        for _ in range(2):
+            for a, b in zip(s.download_magnetization(), m):
+                np.testing.assert_array_equal(a, b)
+    with BatchSolver([dict(shape=shape), dict(shape=(2, 2, 3))], 2, 1e-6, 1e-5, 2.3e-9, 0.5) as b:
+        b.upload(1, np.ones((2, 2, 3), np.uint8), [np.ones((2, 2, 3)), np.zeros((2, 2, 3))])
+        b.upload(0, mask, m)
+        for x, y in zip(b.download(0), m):
+            np.testing.assert_array_equal(x, y)
+
+
+@pytest.mark.parametrize("shape", [(1, 1, 1), (4, 9, 1213), (40, 61, 47), (50, 128, 130)])
+def test_net_arrays_pass_through_the_staging_whole(shape):
+    """Features up and outputs down in pieces (outputs are the interior of a
+    padded tensor): a net that hands on one feature returns it everywhere."""
+    p = np.zeros(10402, np.float32)
+    p[13] = 1.0                                  # W1[0][0][13]: the centre tap of feature 0
+    p[2608 + 13] = 1.0                           # W2[0][0][13]
+    p[9536 + 13], p[9536 + 432 + 13] = 1.0, 2.0  # W3[0][0][13], W3[1][0][13]
+    f = np.random.default_rng(5).integers(0, 200, shape + (6,)).astype(np.float32)  # exact in bfloat16
+    with Corrector() as net:
+        net.params = p
+        for _ in range(2):
+            out = net.forward(f)
+            np.testing.assert_array_equal(out[..., 0], f[..., 0])
+            np.testing.assert_array_equal(out[..., 1], 2.0 * f[..., 0])
+        g = net.backward(f, np.ones(shape + (2,), np.float32))
+        want = 3.0 * (f[..., 0].astype(np.float64).sum())  # d/dW2[0][0][13] of the sum of both outputs
+        assert abs(g[2608 + 13] - want) <= 1e-5 * max(1.0, want)
