@@ -824,8 +824,12 @@ int build_pores(nmr_ctx* c)
                             p.scheme == NMR_SCHEME_MACCORMACK};
     if ((rc = nmri::pores_alloc(&c->pl, (uint32_t)end, n, c->stream, &c->device_bytes))) return rc;
     c->pl_reads_solids = b.read_solids != 0;
+    if (pore_plain(c) && !b.read_solids && p.scheme == NMR_SCHEME_UPWIND &&
+        (rc = nmri::pores_blocks(&c->pl, &b, c->stream, &c->device_bytes)))
+        return rc;
     nmri::pores_into(c->pl, &b, end);
     HIP_TRY(nmr::launch_pore_link(b, c->stream));
+    if (b.blocks) HIP_TRY(nmr::launch_block_build(b, c->stream));
     return nmri::pores_finish(&c->pl, b, c->stream, &c->pl_ok);
 }
 
@@ -955,6 +959,16 @@ int pore_args(nmr_ctx* c, nmr::PoreArgs* a)
     return NMR_OK;
 }
 
+// Whether a run takes several steps a launch (the problem may have got
+// per-voxel data since the list was built).
+bool pore_blocks(const nmr_ctx* c)
+{
+    return c->pl.blocks_ok && pore_plain(c) && !c->pl_reads_solids && c->prob.scheme == NMR_SCHEME_UPWIND;
+}
+
+// Partial sums of a step, in rows of nsig(): one a workgroup.
+int pore_tiles(const nmr_ctx* c, const nmr::PoreArgs& a) { return pore_blocks(c) ? c->pl.nblocks() : a.ntiles; }
+
 // Steps whose partial sums are held before a reduction: at most kChunkSteps,
 // and 32 MiB of them (256^3: 160 steps).
 int64_t pore_chunk(const nmr_ctx* c, int ntiles)
@@ -973,8 +987,10 @@ int run_pores(nmr_ctx* c, int64_t nsteps, const double* grad_sched, double* sign
     if (rc || (rc = state_pores(c)) || (rc = pore_data(c))) return rc;
     nmr::PoreArgs a{};
     if ((rc = pore_args(c, &a))) return rc;
-    const int64_t most = pore_chunk(c, a.ntiles);
-    if ((rc = ensure_partials(c, (size_t)std::min(nsteps, most) * a.ntiles * ns))) return rc;
+    const bool blocks = pore_blocks(c);
+    const int ntiles = pore_tiles(c, a);
+    const int64_t most = pore_chunk(c, ntiles);
+    if ((rc = ensure_partials(c, (size_t)std::min(nsteps, most) * ntiles * ns))) return rc;
     const bool have0 = c->sig_valid;
     double sig0[6];
     std::copy(c->sig_now, c->sig_now + 6, sig0);
@@ -984,12 +1000,32 @@ int run_pores(nmr_ctx* c, int64_t nsteps, const double* grad_sched, double* sign
     int64_t done = 0;
     while (done < nsteps) {
         const int chunk = (int)std::min(most, nsteps - done);
-        for (int s = 0; s < chunk; s++) {
+        auto coef_of = [&](int s) {
             double g[3] = {p.grad[0], p.grad[1], p.grad[2]};
             if (grad_sched)
                 for (int q = 0; q < 3; q++) g[q] = grad_sched[3 * (done + s) + q];
-            a.c = make_coef(c, g);
-            a.partials = c->partials + (size_t)s * a.ntiles * ns;
+            return make_coef(c, g);
+        };
+        for (int s = 0; blocks && s < chunk;) {
+            nmr::BlockArgs k{};
+            k.f = c->pl.state[c->ppar];
+            k.out = c->pl.state[c->ppar ^ 1];
+            k.rec = c->pl.rec;
+            k.blocks = c->pl.blocks;
+            k.bcount = c->pl.bcount;
+            k.partials = c->partials + (size_t)s * ntiles * ns;
+            k.nblocks = ntiles;
+            k.nbx = c->pl.nbx;
+            k.nby = c->pl.nby;
+            k.steps = std::min(chunk - s, nmr::kBlockSteps);
+            for (int i = 0; i < k.steps; i++) k.c[i] = coef_of(s + i);
+            HIP_TRY(nmr::launch_blocks(c->nc, c->vel, c->exact, k, c->stream));
+            c->ppar ^= 1;
+            s += k.steps;
+        }
+        for (int s = 0; !blocks && s < chunk; s++) {
+            a.c = coef_of(s);
+            a.partials = c->partials + (size_t)s * ntiles * ns;
             float *cin = c->pl.state[c->ppar], *cout = c->pl.state[c->ppar ^ 1];
             if (mak) {
                 a.f = cin;
@@ -1007,7 +1043,7 @@ int run_pores(nmr_ctx* c, int64_t nsteps, const double* grad_sched, double* sign
             }
             c->ppar ^= 1;
         }
-        HIP_TRY(nmr::launch_reduce_partials(c->partials, chunk, a.ntiles, ns, c->dsignal + (size_t)(done + 1) * ns,
+        HIP_TRY(nmr::launch_reduce_partials(c->partials, chunk, ntiles, ns, c->dsignal + (size_t)(done + 1) * ns,
                                             c->stream));
         done += chunk;
     }
@@ -1033,7 +1069,7 @@ int presize_buffers(nmr_ctx* c)
     if (pores) {
         nmr::PoreArgs a{};
         if ((rc = pore_args(c, &a))) return rc;
-        need = (size_t)pore_chunk(c, a.ntiles) * a.ntiles * ns;
+        need = std::max<size_t>((size_t)pore_chunk(c, pore_tiles(c, a)) * pore_tiles(c, a), a.ntiles) * ns;
     } else if (c->general) {
         if (c->variant != -2) need = (size_t)kChunkSteps * general_geometry(c, c->brick_on && bricks_fit(c)).nwg * ns;
     } else {
@@ -1875,7 +1911,7 @@ int nmr_hip_run_static(nmr_ctx* ctx, int64_t nsteps, const double* grad_sched, d
     if (pores) {
         nmr::PoreArgs pa{};
         if ((rc = pore_args(ctx, &pa))) return rc;
-        per_step = (size_t)pa.ntiles * ns;
+        per_step = (size_t)std::max(pore_tiles(ctx, pa), pa.ntiles) * ns; // (a step's, and a field sum's)
     } else if (ctx->general) {
         if (ctx->variant != -2) per_step = (size_t)general_geometry(ctx, ctx->brick_on && bricks_fit(ctx)).nwg * ns;
     } else {

@@ -82,6 +82,14 @@ struct PoreList {
     float* pred = nullptr;
     uint4* rec = nullptr; // offsets and velocity sums (with velocity)
     float* pv[6] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr}; // dn, r1v, r2v, bn, w[0], w[1]
+    // boxes that take several steps a launch (nmr_pore_blocks.hip), where the
+    // list is small and they fit
+    nmr::u32x4* blocks = nullptr;
+    uint32_t* bcount = nullptr;
+    size_t bcap = 0, ncap = 0; // slots of blocks, and boxes, allocated
+    int nbx = 0, nby = 0, nbz = 0;
+    bool blocks_ok = false;
+    int nblocks() const { return nbx * nby * nbz; }
     int ngroups() const { return (int)(nslots / 64); }
 };
 // What of the list a problem needs beside the state.
@@ -101,6 +109,9 @@ void pores_free(PoreList* L);
 int pores_temp(nmr::PoreBuild* b, size_t rows, size_t planes, size_t voxels, hipStream_t s);
 void pores_drop_temp(nmr::PoreBuild* b);
 void pores_into(const PoreList& L, nmr::PoreBuild* b, uint64_t end);
+// Counts the boxes' pores of the domain b and makes their buffers, where the
+// list is small enough for them; launch_block_build then fills them.
+int pores_blocks(PoreList* L, nmr::PoreBuild* b, hipStream_t s, int64_t* bytes);
 // Waits for the stream; notes wide groups in the list; *ok: every offset fits.
 int pores_finish(PoreList* L, const nmr::PoreBuild& b, hipStream_t s, bool* ok);
 // Groups that a workgroup takes of a list of `groups`.

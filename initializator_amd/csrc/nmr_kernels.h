@@ -7,6 +7,9 @@
 
 namespace nmr {
 
+// (local arrays of uint4 end up in scratch memory where those of this type do not)
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
 // Per-step coefficients of the update, all pre-multiplied by dt (FP32).
 struct Coef {
     float cdx, cdy, cdz;    // dt*D/d^2 per axis (0 when diffusion is off)
@@ -258,11 +261,35 @@ struct PoreBuild {
     uint2* off16;
     uint32_t* xoff;         // or null
     uint32_t* xy;           // or null
-    int* overflow;          // [0] set when an offset does not fit, [1] when a group needs 16-bit offsets
+    int* overflow;          // [0] set when an offset does not fit, [1] when a group needs 16-bit offsets,
+                            // [2] slots of all blocks
+    u32x4* blocks;          // the blocks' slots, or null
+    uint32_t* bcount;       // [nblocks][8]: slots within 0 .. kBlockSteps faces of the box, the first one's place
+    int nbx, nby, nbz;      // boxes per axis
+};
+
+// Several steps of the pores of one box of kBlockEdge^3 voxels in one
+// workgroup (nmr_pore_blocks.hip): its pores and those within kBlockSteps
+// faces of it, by distance.
+constexpr int kBlockEdge = 8, kBlockSteps = 4, kBlockThreads = 1024;
+struct BlockArgs {
+    const float* f;         // the list's state, nc floats per slot
+    float* out;
+    const uint4* rec;       // with velocity: the list's records
+    const u32x4* blocks;
+    const uint32_t* bcount;
+    double* partials;       // [steps][nblocks][nc]
+    int nblocks, nbx, nby;
+    int steps;              // 1 .. kBlockSteps
+    Coef c[kBlockSteps];
 };
 
 hipError_t launch_pore_count(const PoreBuild& b, hipStream_t s);
 hipError_t launch_pore_link(const PoreBuild& b, hipStream_t s);
+hipError_t launch_block_count(const PoreBuild& b, hipStream_t s);
+hipError_t launch_block_build(const PoreBuild& b, hipStream_t s);
+// a.steps plain upwind steps (exact: with the exact phase)
+hipError_t launch_blocks(int nc, bool vel, bool exact, const BlockArgs& a, hipStream_t s);
 // out[stride*slot + at] = row[vox[slot]] for slots [s0, s1), 0 at empty ones
 hipError_t launch_pore_gather(const float* row, const uint32_t* vox, uint32_t s0, uint32_t s1, int stride, int at,
                               float* out, hipStream_t s);

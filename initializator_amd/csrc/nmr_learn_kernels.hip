@@ -32,7 +32,6 @@ namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float fl4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4))); // (arrays of uint4 end up in scratch memory)
 
 // Round to nearest even (NaN kept quiet), and back.
 __device__ __forceinline__ uint16_t f2bf(float f)

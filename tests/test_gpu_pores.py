@@ -143,3 +143,48 @@ def test_batch_list_equals_tiles(exact, graph):
         for x, y in zip(fa, fb):
             assert np.array_equal(x, y)
         np.testing.assert_allclose(sa, sb, rtol=1e-11, atol=1e-13)
+
+
+@pytest.mark.parametrize("shape,phi", [((8, 8, 8), 1.0), ((9, 17, 7), 0.5), ((16, 24, 8), 0.3), ((1, 1, 1), 1.0),
+                                       ((3, 2, 100), 0.6), ((24, 24, 24), 1.0), ((64, 64, 64), 0.25),
+                                       ((64, 64, 65), 0.25)])
+@pytest.mark.parametrize("nc,vel,exact", [(1, False, False), (1, True, False), (2, False, False), (2, True, True),
+                                          (2, False, True), (2, True, False), (3, False, False), (3, True, False)])
+def test_several_steps_a_launch_equal_single_steps(shape, phi, nc, vel, exact):
+    """Small grids take up to four steps a launch, box by box (64 x 64 x 65: one layer of boxes too many,
+    single steps); against the row layout.  Boxes full of pores, off the grid's edge, without a pore; runs of
+    1 to 11 steps, so of every remainder; a gradient that changes from step to step; a trimmed window; a field
+    map that takes the problem to the general kernels and back."""
+    mask = (np.ones(shape, np.uint8) if phi == 1.0 else generators.porosity(shape, phi, 3, sigma=2.0 if shape[0] > 8 else 0.7))
+    if shape == (64, 64, 64):
+        mask[:24, :24, :24] = 0
+    rng = np.random.default_rng(4)
+    v = generators.velocity(mask, 5, sigma=1.5, vmax=1e-3, d=(DX, DX, DX)) if vel else None
+    m0 = [rng.random(shape) - 0.3 for _ in range(nc)]
+    kw = dict(buffer=tuple(1 if n > 4 else 0 for n in shape[::-1]), phase_exact=exact)
+    if nc == 3:
+        kw.update(p_eq=0.1, **(dict(b0_dir=(0.2, -0.3, 0.9)) if vel else {}))
+    field = rng.standard_normal(shape) * 1e-5
+    outs = []
+    for rows in (False, True):
+        with HipSolver(shape, nc, DX, DT, D, 0.5, r1_bulk=0.4, rho1=4e-6, rho2=9e-6, velocity=vel, precession=nc > 1,
+                       **kw) as s:
+            s.set_layout(not rows)
+            s.upload_mask(mask)
+            if vel:
+                s.upload_velocity(*v)
+            s.upload_magnetization(*m0)
+            out = []
+            for steps in (1, 2, 3, 4, 11):
+                g = None
+                if nc > 1:
+                    g = np.zeros((steps, 3))
+                    g[:, 2] = np.arange(steps) % 3 * 0.1
+                    g[:, :2] = 0.0 if nc == 2 else 0.03
+                out.append((s.run(steps, g), s.download_magnetization()))
+            if nc == 3 and not vel:
+                for b in (field, None):
+                    s.upload_field(b)
+                    out.append((s.run(6), s.download_magnetization()))
+            outs.append(out)
+    _same(*outs)
