@@ -1091,23 +1091,27 @@ int presize_buffers(nmr_ctx* c)
 }
 
 // The one-time work of a solve, done by the uploads so that runs start at
-// once: the inert check, the brick buffers with the velocity and per-voxel
-// arrays converted, the partial-sum and signal buffers.
+// once: the inert check, then the list of the pores with its data, or where
+// the next run takes the tiles the brick buffers with the velocity and
+// per-voxel arrays converted, and the partial-sum and signal buffers.  Which
+// of them is known once there is magnetization; a tile or layout that is set
+// later prepares for itself.
 int prepare(nmr_ctx* c)
 {
     if (!c->has_mask) return NMR_OK;
     int rc = refresh_inert(c);
-    if (rc) return rc;
-    if (c->brick_on && bricks_fit(c)) {
-        if ((rc = ensure_bricks(c))) return rc;
-        if ((rc = ensure_pv_bricks(c))) return rc;
-    }
-    // the per-voxel velocity sums the sweeps read: upwind (the plain sweep,
-    // the general sweep's upwind stage) or centred (MacCormack)
-    if ((rc = velocity_sums(c, c->brick_on && bricks_fit(c), c->prob.scheme == NMR_SCHEME_MACCORMACK))) return rc;
+    if (rc || !c->has_mag) return rc;
     bool pores = false;
     if ((rc = use_pores(c, &pores))) return rc;
-    if (pores && ((rc = state_pores(c)) || (rc = pore_data(c)))) return rc;
+    if (pores) {
+        if ((rc = state_pores(c)) || (rc = pore_data(c))) return rc;
+    } else {
+        const bool brick = c->brick_on && bricks_fit(c);
+        if (brick && ((rc = ensure_bricks(c)) || (rc = ensure_pv_bricks(c)))) return rc;
+        // the per-voxel velocity sums the sweeps read: upwind (the plain sweep,
+        // the general sweep's upwind stage) or centred (MacCormack)
+        if ((rc = velocity_sums(c, brick, c->prob.scheme == NMR_SCHEME_MACCORMACK))) return rc;
+    }
     if ((rc = presize_buffers(c))) return rc;
     HIP_TRY(hipStreamSynchronize(c->stream));
     return NMR_OK;
@@ -1567,8 +1571,9 @@ int nmr_hip_set_layout(nmr_ctx* ctx, int32_t brick)
 {
     if (!ctx) return fail(NMR_ERR_NULL, "nmr_hip_set_layout: null context");
     if (brick != 0 && brick != 1) return fail(NMR_ERR_INVALID, "layout %d", (int)brick);
+    if (ctx->brick_on == (brick != 0)) return NMR_OK;
     ctx->brick_on = brick != 0;
-    return NMR_OK;
+    return prepare(ctx);
 }
 
 int nmr_hip_set_tile(nmr_ctx* ctx, int32_t variant, int32_t lz)
@@ -1577,9 +1582,10 @@ int nmr_hip_set_tile(nmr_ctx* ctx, int32_t variant, int32_t lz)
     if (variant < -2 || variant >= nmr::num_variants()) return fail(NMR_ERR_INVALID, "variant %d", (int)variant);
     if (variant == -2 && ctx->exact) return fail(NMR_ERR_UNSUPPORTED, "the per-voxel kernel has no exact phase");
     if (lz < 0) return fail(NMR_ERR_INVALID, "lz %d", (int)lz);
+    if (ctx->variant == variant && ctx->lz == lz) return NMR_OK;
     ctx->variant = variant;
     ctx->lz = lz;
-    return NMR_OK;
+    return prepare(ctx);
 }
 
 int nmr_hip_signal(nmr_ctx* ctx, double* out)
