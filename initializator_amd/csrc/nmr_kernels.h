@@ -344,6 +344,30 @@ struct FeatureArgs {
     float vinv;             // 1 / velocity scale
 };
 
+struct WreduceArgs {
+    const float* part[3];   // [npart][kWgradPart] of each layer
+    float* grad[3];
+    int cin[3], cout[3];    // real channels
+    int npart;
+};
+
+// A layer's weights, and the fragments to make of them.
+struct PackJob {
+    const float* w;
+    uint16_t* frag;
+    int cin_real, cout_real, cin_store, backward;
+};
+constexpr int kPackJobs = 5;
+struct PackArgs {
+    PackJob job[kPackJobs];
+};
+
+struct HaloArgs {
+    uint16_t* x;            // [..][8]
+    uint16_t* t[5];         // [..][16], or null
+    int nx, ny, nz;
+};
+
 struct LossArgs {
     const float* pred;      // [..][2]
     const float* tx;        // target, compact with pitch
@@ -380,9 +404,9 @@ int conv_columns(int nx, int ny, int nz, int zc);
 hipError_t launch_conv_zm(int cin, int mode, const ConvArgs& a, int grid, hipStream_t s);
 // npart partial sums
 hipError_t launch_wgrad(int cin, const WgradArgs& a, int npart, hipStream_t s);
-hipError_t launch_wreduce(const float* part, int nwaves, int cin_real, int cout_real, float* grad, hipStream_t s);
-hipError_t launch_pack(const float* w, int cin_real, int cout_real, int cin_store, int backward, uint16_t* frag,
-                       hipStream_t s);
+hipError_t launch_wreduce(const WreduceArgs& a, hipStream_t s);
+hipError_t launch_pack(const PackArgs& a, hipStream_t s);
+hipError_t launch_halo(const HaloArgs& a, hipStream_t s);
 hipError_t launch_features(const FeatureArgs& a, hipStream_t s);
 hipError_t launch_feature_copy(const float* f6, int nx, int ny, int nz, uint16_t* out, hipStream_t s);
 hipError_t launch_gout_copy(const float* g2, int nx, int ny, int nz, uint16_t* out, hipStream_t s);

@@ -51,7 +51,7 @@ struct nmr_corrector {
     int64_t adam_t = 0;
     double vscale = 1e-3, out_scale = 0.0;
     Tensors t;
-    float* wpart = nullptr; // wgrad partials
+    float* wpart = nullptr; // wgrad partials of the three layers
     double* lpart = nullptr;
     size_t lpart_cap = 0;
     double* apart = nullptr; // apply partials
@@ -116,9 +116,8 @@ int ensure_tensors(nmr_corrector* c, int nx, int ny, int nz, bool train)
         t.cap = cap;
     } else if (t.nx != nx || t.ny != ny || t.nz != nz) {
         // a different padded shape: old interiors would sit in the new halos
-        HIP_TRY(hipMemsetAsync(t.x, 0, nv * 8 * 2, c->stream));
-        for (uint16_t* q : {t.a1, t.a2, t.g3, t.g2, t.g1})
-            if (q) HIP_TRY(hipMemsetAsync(q, 0, nv * 16 * 2, c->stream));
+        // (every kernel that fills a tensor writes its whole interior)
+        HIP_TRY(nmr::launch_halo({t.x, {t.a1, t.a2, t.g3, t.g2, t.g1}, nx, ny, nz}, c->stream));
     }
     t.nx = nx;
     t.ny = ny;
@@ -128,11 +127,12 @@ int ensure_tensors(nmr_corrector* c, int nx, int ny, int nz, bool train)
 
 int repack(nmr_corrector* c)
 {
-    HIP_TRY(nmr::launch_pack(c->w + kW1, 6, 16, 8, 0, c->f1, c->stream));
-    HIP_TRY(nmr::launch_pack(c->w + kW2, 16, 16, 16, 0, c->f2, c->stream));
-    HIP_TRY(nmr::launch_pack(c->w + kW3, 16, 2, 16, 0, c->f3, c->stream));
-    HIP_TRY(nmr::launch_pack(c->w + kW2, 16, 16, 16, 1, c->d2, c->stream));
-    HIP_TRY(nmr::launch_pack(c->w + kW3, 16, 2, 16, 1, c->d3, c->stream));
+    HIP_TRY(nmr::launch_pack({{{c->w + kW1, c->f1, 6, 16, 8, 0},
+                               {c->w + kW2, c->f2, 16, 16, 16, 0},
+                               {c->w + kW3, c->f3, 16, 2, 16, 0},
+                               {c->w + kW2, c->d2, 16, 16, 16, 1},
+                               {c->w + kW3, c->d3, 16, 2, 16, 1}}},
+                             c->stream));
     return NMR_OK;
 }
 
@@ -308,20 +308,22 @@ int backward(nmr_corrector* c)
     w.nx = t.nx;
     w.ny = t.ny;
     w.nz = t.nz;
-    w.part = c->wpart;
-    const int nw = kWgradParts;
+    const size_t layer = (size_t)kWgradParts * nmr::kWgradPart;
+    nmr::WreduceArgs red{{c->wpart, c->wpart + layer, c->wpart + 2 * layer},
+                         {c->grad + kW3, c->grad + kW2, c->grad + kW1}, {16, 16, 6}, {2, 16, 16}, kWgradParts};
     w.in = t.a2;
     w.gout = t.g3;
-    HIP_TRY(nmr::launch_wgrad(16, w, nw, c->stream));
-    HIP_TRY(nmr::launch_wreduce(c->wpart, nw, 16, 2, c->grad + kW3, c->stream));
+    w.part = c->wpart;
+    HIP_TRY(nmr::launch_wgrad(16, w, kWgradParts, c->stream));
     w.in = t.a1;
     w.gout = t.g2;
-    HIP_TRY(nmr::launch_wgrad(16, w, nw, c->stream));
-    HIP_TRY(nmr::launch_wreduce(c->wpart, nw, 16, 16, c->grad + kW2, c->stream));
+    w.part = c->wpart + layer;
+    HIP_TRY(nmr::launch_wgrad(16, w, kWgradParts, c->stream));
     w.in = t.x;
     w.gout = t.g1;
-    HIP_TRY(nmr::launch_wgrad(8, w, nw, c->stream));
-    HIP_TRY(nmr::launch_wreduce(c->wpart, nw, 6, 16, c->grad + kW1, c->stream));
+    w.part = c->wpart + 2 * layer;
+    HIP_TRY(nmr::launch_wgrad(8, w, kWgradParts, c->stream));
+    HIP_TRY(nmr::launch_wreduce(red, c->stream));
     return NMR_OK;
 }
 
@@ -429,7 +431,7 @@ int nmr_hip_corrector_create(uint64_t seed, nmr_corrector** out)
     if ((rc = dalloc(s, &c->w, kParams)) || (rc = dalloc(s, &c->m, kParams)) || (rc = dalloc(s, &c->v, kParams)) ||
         (rc = dalloc(s, &c->grad, kParams)) || (rc = dalloc(s, &c->f1, kFragF1)) || (rc = dalloc(s, &c->f2, kFragF)) ||
         (rc = dalloc(s, &c->f3, kFragF)) || (rc = dalloc(s, &c->d2, kFragF)) || (rc = dalloc(s, &c->d3, kFragF)) ||
-        (rc = dalloc(s, &c->wpart, (size_t)kWgradParts * nmr::kWgradPart)))
+        (rc = dalloc(s, &c->wpart, (size_t)3 * kWgradParts * nmr::kWgradPart)))
         return bail(rc);
     if (hipHostMalloc((void**)&c->hstat, 8 * sizeof(double), hipHostMallocDefault) != hipSuccess)
         return bail(fail(NMR_ERR_NOMEM, "pinned host allocation"));

@@ -493,134 +493,234 @@ __global__ void __launch_bounds__(256, 2) conv_zm_kernel(ConvArgs a)
 // bias gradient sum_v gout[v][co], as partials over 32-voxel x segments:
 // partial w takes segments w, w + npart, ..., into part[w][27*256 + 16].
 // MFMA: A = input (16 ci x 32 voxels), B = output gradient (32 voxels x 16
-// co), both gathered per lane.
+// co): eight voxels of one channel a lane, from channels-last tensors.
 //
-// Bound by the gathers' latency: the operands want eight voxels of one channel
-// a lane from channels-last tensors, 2-byte loads.  A wavefront therefore
-// takes three of the 27 taps, those of one (dz, dy), whose operands are the
-// same ten voxels shifted by one: 18 loads for three MFMAs instead of 224 for
-// 27, and nine wavefronts in place of one on each partial (512 wavefronts
-// alone leave half of the CUs idle).  Each tap's sum runs over the same
-// segments in the same order as with one wavefront for all taps, so the
-// gradients keep their bits.  96x80x64: 31.9 us at 16 channels and 38.1 at 8,
-// 97.2 and 264 with one wavefront for all taps.
+// A workgroup takes a partial, its nine wavefronts the nine (dz, dy) of the
+// taps.  The segment's nine input rows and its gradient are loaded 16 bytes a
+// thread in the tensors' order and turned into channel-major rows in LDS,
+// where a lane's eight voxels are 16 bytes and the taps of kx 0 and 2 the same
+// shifted by half a word; two segments are on their way meanwhile.  Rows of 56
+// halfwords (28 words): 16 lanes' 16-byte reads and a wavefront's writes cover
+// all banks.  What bounds it is the instructions around three MFMAs: gathering
+// the operands from the tensors takes 18 two-byte loads for them (31.9 us at
+// 96x80x64 and 16 channels, 38.1 at 8; this: 27.1 and 22.5; 32^3 to 96^3 in turns,
+// where the gathers miss the caches, 47.5 -> 27.3 and 71.0 -> 21.6).  Tried: two
+// voxels' pieces a thread in voxel order (each 16 bytes from a line of its own):
+// 38; partials of neighbouring segments on one L2: no different; four segments
+// on their way: 68 (their registers leave one workgroup a CU).
+// Each tap's sum runs over the same voxels in the same order as a gather's, so
+// the gradients keep their bits.
+constexpr int kWgradThreads = 9 * 64, kWgradPitch = 56;
 template <int CIN>
-__global__ void __launch_bounds__(256) wgrad_kernel(WgradArgs a, int npart)
+__global__ void __launch_bounds__(kWgradThreads) wgrad_kernel(WgradArgs a, int npart)
 {
-    const int lane = threadIdx.x & 63;
+    // pieces of a segment: eight channels of a voxel, loaded in the tensors'
+    // order; of two voxels that share a word in LDS each thread writes four channels
+    constexpr int V16 = CIN / 8, NIN = 9 * V16 * 36, NP = NIN + 64;
+    constexpr int NLD = (NP + kWgradThreads - 1) / kWgradThreads;
+    constexpr int kSwap = V16 == 2 ? 0x4e : 0xb1; // quad_perm to the other voxel's thread
+    constexpr int ROWS = 9 * CIN + 16;
+    __shared__ __align__(16) uint16_t sh[2][(ROWS + 1) * kWgradPitch]; // the last row: zeros, for lanes past 8 channels
+    const int t = threadIdx.x, lane = t & 63;
     const int g = lane >> 4, n = lane & 15;
+    const int d = __builtin_amdgcn_readfirstlane(t >> 6); // (dz, dy) = (d / 3 - 1, d % 3 - 1)
     const int px = a.nx + 2, plane = px * (a.ny + 2); // (the padded grid has fewer than 2^31 voxels)
-    const int job = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * 4 + (threadIdx.x >> 6)));
-    const int w = job / 9, d = job % 9; // partial; (dz, dy) = (d / 3 - 1, d % 3 - 1)
-    if (w >= npart) return;
-    const int shift = (d / 3 - 1) * plane + (d % 3 - 1) * px;
-    fl4 acc[3];
-#pragma unroll
-    for (int t = 0; t < 3; t++) acc[t] = fl4{0.f, 0.f, 0.f, 0.f};
-    float bsum = 0.f;
+    const int w = blockIdx.x;
     const int nseg32 = (a.nx + 31) / 32;
     const int nrows = nseg32 * a.ny * a.nz;
-    const bool chan = n < CIN;
-    for (int r = w; r < nrows; r += npart) {
-        const int seg = r % nseg32, yz = r / nseg32;
-        const int y = yz % a.ny, z = yz / a.ny;
-        const int rowb = (z + 1) * plane + (y + 1) * px;
-        const int x0 = seg * 32 + 8 * g;
-        uint16_t bv[8], av[3][8];
-        if (seg * 32 + 32 <= a.nx) {
-            const uint16_t* go = a.gout + ((size_t)(rowb + x0 + 1) * 16 + n);
-            const uint16_t* in = a.in + ((long)(rowb + shift + x0) * CIN + n);
-            uint16_t v[10]; // voxels x0 - 1 .. x0 + 8
+    const uint32_t second = (t & V16) != 0 ? 0xffffffffu : 0u; // of its two voxels
+    // this thread's pieces: voxel xv of input row (dz, dy), counted from the
+    // segment's first (two that only fill their words repeat -1 and 32), or of
+    // the gradient
+    const char* from[NLD]; // of the segment of the grid's first padded voxel
+    int xv[NLD], dst[NLD];
+    bool grad[NLD];
 #pragma unroll
-            for (int j = 0; j < 8; j++) bv[j] = go[j * 16];
+    for (int k = 0; k < NLD; k++) {
+        const int p = min(t + k * kWgradThreads, NP - 1); // (threads past the last piece load it too: no branch, whose
+                                                          // join would wait for every load on its way)
+        grad[k] = p >= NIN;
+        if (!grad[k]) {
+            const int row = p / (36 * V16), part = p % V16;
+            xv[k] = min(max(p / V16 % 36 - 2, -1), 32);
+            from[k] = reinterpret_cast<const char*>(a.in) +
+                      ((long)((row / 3 - 1) * plane + (row % 3 - 1) * px + xv[k]) * V16 + part) * 16;
+            dst[k] = (row * CIN + part * 8) * kWgradPitch + p / V16 % 36 + 6;
+        } else {
+            const int q = p - NIN, part = V16 == 2 ? q % 2 : q / 32;
+            xv[k] = V16 == 2 ? q / 2 : q % 32;
+            from[k] = reinterpret_cast<const char*>(a.gout) + (xv[k] * 2 + part) * 16;
+            dst[k] = (9 * CIN + part * 8) * kWgradPitch + xv[k] + 8;
+        }
+        if (second) dst[k] += 4 * kWgradPitch - 1;
+    }
+    // Position of the segment to load next, and how far npart segments on is.
+    int ls = w % nseg32, ly = w / nseg32 % a.ny, lz = w / nseg32 / a.ny;
+    const int ds = npart % nseg32, dy = npart / nseg32 % a.ny, dz = npart / nseg32 / a.ny;
+    auto load = [&](u32x4 (&v)[NLD]) { // (past the last segment: some voxel of the last plane)
+        const int x0 = ls * 32;
+        const int vox = (min(lz, a.nz - 1) + 1) * plane + (ly + 1) * px + x0 + 1;
 #pragma unroll
-            for (int j = 0; j < 10; j++) v[j] = chan ? in[j * CIN] : (uint16_t)0;
+        for (int k = 0; k < NLD; k++) { // (past the padded row's end: its last voxel)
+            const int bytes = V16 == 2 || grad[k] ? 32 : 16;
+            const int at = vox - max(x0 + xv[k] - a.nx, 0); // (below 0 on the smallest grids; from[k] adds xv back)
+            v[k] = *reinterpret_cast<const u32x4*>(from[k] + (long)at * bytes);
+        }
+        const int was = x0;
+        ls += ds;
+        ly += dy;
+        lz += dz;
+        if (ls >= nseg32) {
+            ls -= nseg32;
+            ly++;
+        }
+        if (ly >= a.ny) {
+            ly -= a.ny;
+            lz++;
+        }
+        return was;
+    };
+    auto stash = [&](uint16_t* to, u32x4 (&v)[NLD], int x0) {
+        if (x0 + 32 > a.nx) // past the row's end: no gradient
 #pragma unroll
-            for (int t = 0; t < 3; t++)
+            for (int k = 0; k < NLD; k++)
+                if (grad[k] && x0 + xv[k] >= a.nx) v[k] = u32x4{0u, 0u, 0u, 0u};
 #pragma unroll
-                for (int j = 0; j < 8; j++) av[t][j] = v[j + t];
-        } else { // the row's end: voxels past it read the last one's, with a zero gradient
+        for (int k = 0; k < NLD; k++) {
+            if (t + k * kWgradThreads >= NP) continue;
+            uint32_t own[2], other[2];
 #pragma unroll
-            for (int j = 0; j < 8; j++) {
-                const bool ok = x0 + j < a.nx;
-                const int vb = rowb + (ok ? x0 + j : a.nx - 1) + 1;
-                bv[j] = ok ? a.gout[(size_t)vb * 16 + n] : (uint16_t)0;
-#pragma unroll
-                for (int t = 0; t < 3; t++)
-                    av[t][j] = chan ? a.in[(long)(vb + shift + t - 1) * CIN + n] : (uint16_t)0;
+            for (int h = 0; h < 2; h++) {
+                // (masks: a select of two elements becomes an indexed one)
+                own[h] = (second & v[k][2 + h]) | (~second & v[k][h]);
+                const uint32_t give = (second & v[k][h]) | (~second & v[k][2 + h]);
+                other[h] = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)give, kSwap, 0xf, 0xf, false);
+                const uint32_t lo = (second & other[h]) | (~second & own[h]), hi = (second & own[h]) | (~second & other[h]);
+                uint32_t* w = reinterpret_cast<uint32_t*>(to + dst[k] + 2 * h * kWgradPitch);
+                w[0] = (lo & 0xffffu) | (hi << 16);
+                w[kWgradPitch / 2] = (lo >> 16) | (hi & 0xffff0000u);
             }
         }
+    };
+    fl4 acc[3];
 #pragma unroll
-        for (int j = 0; j < 8; j++) bsum += bf2f(bv[j]);
-        const uint4 B = make_uint4((uint32_t)bv[0] | ((uint32_t)bv[1] << 16), (uint32_t)bv[2] | ((uint32_t)bv[3] << 16),
-                                   (uint32_t)bv[4] | ((uint32_t)bv[5] << 16), (uint32_t)bv[6] | ((uint32_t)bv[7] << 16));
+    for (int k = 0; k < 3; k++) acc[k] = fl4{0.f, 0.f, 0.f, 0.f};
+    float bsum = 0.f;
+    const bool chan = n < CIN;
+    auto segment = [&](const int b) {
+        const uint16_t* in = sh[b] + (chan ? d * CIN + n : ROWS) * kWgradPitch + 8 + 8 * g;
+        const u32x4 B = *reinterpret_cast<const u32x4*>(sh[b] + (9 * CIN + n) * kWgradPitch + 8 + 8 * g);
+        const u32x4 c = *reinterpret_cast<const u32x4*>(in);
+        const uint32_t before = *reinterpret_cast<const uint32_t*>(in - 2), after = *reinterpret_cast<const uint32_t*>(in + 8);
+        if (d == 0) {
 #pragma unroll
-        for (int t = 0; t < 3; t++) {
-            const uint4 Av = make_uint4((uint32_t)av[t][0] | ((uint32_t)av[t][1] << 16),
-                                        (uint32_t)av[t][2] | ((uint32_t)av[t][3] << 16),
-                                        (uint32_t)av[t][4] | ((uint32_t)av[t][5] << 16),
-                                        (uint32_t)av[t][6] | ((uint32_t)av[t][7] << 16));
-            acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf8(Av), as_bf8(B), acc[t], 0, 0, 0);
+            for (int j = 0; j < 8; j++) bsum += bf2f((uint16_t)(B[j / 2] >> (16 * (j & 1))));
         }
+        uint32_t m[5]; // voxels -1 0, 1 2, 3 4, 5 6, 7 8 of the lane's eight
+        m[0] = __builtin_amdgcn_alignbit(c[0], before, 16);
+        m[1] = __builtin_amdgcn_alignbit(c[1], c[0], 16);
+        m[2] = __builtin_amdgcn_alignbit(c[2], c[1], 16);
+        m[3] = __builtin_amdgcn_alignbit(c[3], c[2], 16);
+        m[4] = __builtin_amdgcn_alignbit(after, c[3], 16);
+        const u32x4 av[3] = {u32x4{m[0], m[1], m[2], m[3]}, c, u32x4{m[1], m[2], m[3], m[4]}};
+#pragma unroll
+        for (int k = 0; k < 3; k++)
+            acc[k] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, av[k]),
+                                                             __builtin_bit_cast(bf16x8, B), acc[k], 0, 0, 0);
+    };
+    // two segments on their way
+    if (t < kWgradPitch) sh[0][ROWS * kWgradPitch + t] = sh[1][ROWS * kWgradPitch + t] = 0;
+    u32x4 n0[NLD], n1[NLD];
+    int x0 = 0, x1 = 0;
+    if (w < nrows) {
+        x0 = load(n0);
+        x1 = load(n1);
     }
-    float* dst = a.part + (size_t)w * kWgradPart;
+    for (int r = w; r < nrows; r += 2 * npart) {
+        stash(sh[0], n0, x0); // (read two segments ago)
+        x0 = load(n0);
+        lds_barrier();
+        segment(0);
+        if (r + npart >= nrows) break;
+        stash(sh[1], n1, x1);
+        x1 = load(n1);
+        lds_barrier();
+        segment(1);
+    }
+    float* to = a.part + (size_t)w * kWgradPart;
     // D[i = ci = 4g + j][col = co = n]
 #pragma unroll
-    for (int t = 0; t < 3; t++)
+    for (int k = 0; k < 3; k++)
 #pragma unroll
-        for (int j = 0; j < 4; j++) dst[(3 * d + t) * 256 + (4 * g + j) * 16 + n] = acc[t][j];
+        for (int j = 0; j < 4; j++) to[(3 * d + k) * 256 + (4 * g + j) * 16 + n] = acc[k][j];
     // bias: lanes n, n+16, n+32, n+48 hold the same co
     bsum += __shfl_xor(bsum, 16);
     bsum += __shfl_xor(bsum, 32);
-    if (d == 0 && g == 0) dst[27 * 256 + n] = bsum;
+    if (d == 0 && g == 0) to[27 * 256 + n] = bsum;
 }
 
-// Sum of the partials in a fixed order (FP64, partial 0 first), scattered to
-// the canonical gradient layout W[co][ci][t] (cout_real x cin_real x 27)
-// followed by the bias.  A workgroup takes kRedEl elements: all threads bring
-// kRedRows partials of them into LDS at once, then one thread an element adds
-// them up in order -- the order is the serial chain that bounds it (512 FP64
-// additions), not a load behind every addition: 10.7 us against 125.
-constexpr int kRedEl = 16, kRedRows = 512;
-__global__ void __launch_bounds__(256) wreduce_kernel(const float* __restrict__ part, int nwaves, int cin_real,
-                                                      int cout_real, float* __restrict__ grad)
+// Sums of the partials (FP64), scattered to the canonical gradient layout
+// W[co][ci][t] (cout_real x cin_real x 27) followed by the bias; blockIdx.y is
+// the layer.  A workgroup takes 16 elements, 16 threads each: a thread adds
+// every sixteenth partial, so that its loads are all on their way at once and
+// the chain of additions is 32 long instead of 512: 13.4 us for the three
+// layers in one launch, 10.7 a layer with one thread an element.
+constexpr int kRedEl = 16, kRedSlices = 16;
+__global__ void __launch_bounds__(256) wreduce_kernel(WreduceArgs a)
 {
-    __shared__ float sh[kRedRows * kRedEl];
-    const int e0 = blockIdx.x * kRedEl, col = threadIdx.x % kRedEl;
-    const int e = e0 + col;
+    __shared__ double sh[kRedSlices][kRedEl];
+    const int l = blockIdx.y, col = threadIdx.x % kRedEl, slice = threadIdx.x / kRedEl;
+    const int e = blockIdx.x * kRedEl + col;
+    const float* part = a.part[l];
     double s = 0.0;
-    for (int w0 = 0; w0 < nwaves; w0 += kRedRows) {
-        const int rows = min(kRedRows, nwaves - w0);
-        if (e < kWgradPart) {
+    if (e < kWgradPart) {
 #pragma unroll 8
-            for (int w = threadIdx.x / kRedEl; w < rows; w += 256 / kRedEl)
-                sh[w * kRedEl + col] = part[(size_t)(w0 + w) * kWgradPart + e];
-        }
-        __syncthreads();
-        if (threadIdx.x < kRedEl && e < kWgradPart) {
-#pragma unroll 16
-            for (int w = 0; w < rows; w++) s += (double)sh[w * kRedEl + col];
-        }
-        __syncthreads();
+        for (int w = slice; w < a.npart; w += kRedSlices) s += (double)part[(size_t)w * kWgradPart + e];
     }
-    if (threadIdx.x >= kRedEl || e >= kWgradPart) return;
+    sh[slice][col] = s;
+    __syncthreads();
+    if (slice != 0 || e >= kWgradPart) return;
+    for (int k = 1; k < kRedSlices; k++) s += sh[k][col];
+    float* grad = a.grad[l];
+    const int cin = a.cin[l], cout = a.cout[l];
     if (e < 27 * 256) {
         const int t = e / 256, ci = (e / 16) % 16, co = e % 16;
-        if (ci < cin_real && co < cout_real) grad[((size_t)co * cin_real + ci) * 27 + t] = (float)s;
+        if (ci < cin && co < cout) grad[((size_t)co * cin + ci) * 27 + t] = (float)s;
     } else {
         const int co = e - 27 * 256;
-        if (co < cout_real) grad[(size_t)cout_real * cin_real * 27 + co] = (float)s;
+        if (co < cout) grad[(size_t)cout * cin * 27 + co] = (float)s;
     }
+}
+
+// Zeroes the halo of a grid's tensors (x of 8 channels, the others of 16 or
+// null): what another grid left there.
+__global__ void __launch_bounds__(256) halo_kernel(HaloArgs a)
+{
+    const int px = a.nx + 2, py = a.ny + 2, plane = px * py;
+    const uint32_t v = blockIdx.x * 256u + threadIdx.x;
+    if (v >= (uint32_t)plane * (uint32_t)(a.nz + 2)) return;
+    const int x = (int)(v % (uint32_t)px), y = (int)(v / (uint32_t)px % (uint32_t)py), z = (int)(v / (uint32_t)plane);
+    if (x >= 1 && x <= a.nx && y >= 1 && y <= a.ny && z >= 1 && z <= a.nz) return;
+    const uint4 none = make_uint4(0u, 0u, 0u, 0u);
+    reinterpret_cast<uint4*>(a.x)[v] = none;
+#pragma unroll
+    for (int k = 0; k < 5; k++)
+        if (a.t[k]) {
+            uint4* p = reinterpret_cast<uint4*>(a.t[k]) + (size_t)v * 2;
+            p[0] = none;
+            p[1] = none;
+        }
 }
 
 // Packs the canonical FP32 weights of one layer, W[co][ci][t], into the A
 // fragments of conv_kernel: forward (rows = output channels co, reduction
 // (t, ci) with cin_store channels per tap) or input gradient (rows = ci,
 // reduction (t', co) over 16 stored channels, W'[t'][co][ci] = W[26-t'][ci][co]).
-__global__ void __launch_bounds__(256) pack_kernel(const float* __restrict__ w, int cin_real, int cout_real,
-                                                   int cin_store, int backward, uint16_t* __restrict__ frag)
+// blockIdx.y is the set of fragments.
+__global__ void __launch_bounds__(256) pack_kernel(PackArgs a)
 {
-    const int cin = backward ? 16 : cin_store;
+    const PackJob& p = a.job[blockIdx.y];
+    const int cin = p.backward ? 16 : p.cin_store;
     const int tpc = 32 / cin, nch = (27 + tpc - 1) / tpc;
     const int e = blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= nch * 64 * 8) return;
@@ -630,13 +730,13 @@ __global__ void __launch_bounds__(256) pack_kernel(const float* __restrict__ w, 
     const int t = c * tpc + k / cin, ch = k % cin;
     float v = 0.f;
     if (t < 27) {
-        if (!backward) {
-            if (ch < cin_real && row < cout_real) v = w[((size_t)row * cin_real + ch) * 27 + t];
+        if (!p.backward) {
+            if (ch < p.cin_real && row < p.cout_real) v = p.w[((size_t)row * p.cin_real + ch) * 27 + t];
         } else {
-            if (ch < cout_real && row < cin_real) v = w[((size_t)ch * cin_real + row) * 27 + (26 - t)];
+            if (ch < p.cout_real && row < p.cin_real) v = p.w[((size_t)ch * p.cin_real + row) * 27 + (26 - t)];
         }
     }
-    frag[e] = f2bf(v);
+    p.frag[e] = f2bf(v);
 }
 
 // Input tensor of the net: (Mx, My) * pore, pore, cell-centred velocity /
@@ -930,28 +1030,30 @@ hipError_t launch_conv_zm(int cin, int mode, const ConvArgs& a, int grid, hipStr
 
 hipError_t launch_wgrad(int cin, const WgradArgs& a, int npart, hipStream_t s)
 {
-    const dim3 grid((unsigned)((npart * 9 + 3) / 4)), block(256);
+    const dim3 grid((unsigned)npart), block(kWgradThreads);
     if (cin == 8) hipLaunchKernelGGL((wgrad_kernel<8>), grid, block, 0, s, a, npart);
     else if (cin == 16) hipLaunchKernelGGL((wgrad_kernel<16>), grid, block, 0, s, a, npart);
     else return hipErrorInvalidValue;
     return hipGetLastError();
 }
 
-hipError_t launch_wreduce(const float* part, int nwaves, int cin_real, int cout_real, float* grad, hipStream_t s)
+hipError_t launch_wreduce(const WreduceArgs& a, hipStream_t s)
 {
-    hipLaunchKernelGGL(wreduce_kernel, dim3((kWgradPart + kRedEl - 1) / kRedEl), dim3(256), 0, s, part, nwaves, cin_real,
-                       cout_real, grad);
+    hipLaunchKernelGGL(wreduce_kernel, dim3((kWgradPart + kRedEl - 1) / kRedEl, 3), dim3(256), 0, s, a);
     return hipGetLastError();
 }
 
-hipError_t launch_pack(const float* w, int cin_real, int cout_real, int cin_store, int backward, uint16_t* frag,
-                       hipStream_t s)
+hipError_t launch_pack(const PackArgs& a, hipStream_t s)
 {
-    const int cin = backward ? 16 : cin_store;
-    const int tpc = 32 / cin, nch = (27 + tpc - 1) / tpc;
-    const int n = nch * 64 * 8;
-    hipLaunchKernelGGL(pack_kernel, dim3((n + 255) / 256), dim3(256), 0, s, w, cin_real, cout_real, cin_store,
-                       backward, frag);
+    constexpr int n = 14 * 64 * 8; // of the largest set
+    hipLaunchKernelGGL(pack_kernel, dim3((n + 255) / 256, kPackJobs), dim3(256), 0, s, a);
+    return hipGetLastError();
+}
+
+hipError_t launch_halo(const HaloArgs& a, hipStream_t s)
+{
+    const uint64_t n = (uint64_t)(a.nx + 2) * (a.ny + 2) * (a.nz + 2);
+    hipLaunchKernelGGL(halo_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, a);
     return hipGetLastError();
 }
 

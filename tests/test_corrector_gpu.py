@@ -323,3 +323,45 @@ def test_learned_solve_on_the_list_of_pores_equals_the_rows(kind):
         for a, b in zip(f, f_r):
             np.testing.assert_array_equal(a, b)
         np.testing.assert_allclose(sig, sig_r, rtol=1e-12, atol=1e-12 * max(1e-30, np.abs(sig_r).max()))
+
+
+@pytest.mark.parametrize("shape", [(1, 1, 1), (2, 3, 31), (3, 2, 32), (2, 2, 33), (5, 4, 63), (1, 7, 65), (9, 40, 96),
+                                   (33, 17, 34)])
+def test_weight_gradient_at_the_edges_of_segments(shape):
+    """The weight gradient runs over x segments of 32 voxels, 512 partials of
+    them: rows that end on a segment's edge and next to it, fewer segments than
+    partials and more, against the convolution gradients in FP64 of the BF16
+    tensors (exact inputs, positive weights and activations, so that only the
+    FP32 sums round).  Then another grid on the same net and back: what one
+    leaves in the halo is not seen by the other."""
+    rng = np.random.default_rng(list(shape))
+    p = np.zeros(10402, np.float32)
+    for c in range(6):  # layer 1: channel c hands on feature c; layer 2: the same; layer 3: sums of them
+        p[(c * 6 + c) * 27 + 13] = 1.0
+        p[2608 + (c * 16 + c) * 27 + 13] = 1.0
+        p[9536 + c * 27 + 13], p[9536 + (16 + c) * 27 + 13] = 1.0, 0.5
+    f = rng.integers(1, 64, shape + (6,)).astype(np.float32)
+    g = rng.integers(-8, 9, shape + (2,)).astype(np.float32)
+
+    def taps(x, y):  # dW[t] = sum_v x[v + off(t)] y[v]
+        q = np.pad(x.astype(np.float64), 1)
+        nz, ny, nx = y.shape
+        return np.array([(q[k // 9:k // 9 + nz, k // 3 % 3:k // 3 % 3 + ny, k % 3:k % 3 + nx] * y).sum() for k in range(27)])
+
+    with Corrector() as net:
+        net.params = p
+        got = net.backward(f, g)
+        net.backward(rng.random((4, 5, 6, 6)).astype(np.float32), np.ones((4, 5, 6, 2), np.float32))
+        again = net.backward(f, g)
+    np.testing.assert_array_equal(got, again)
+    back = g[..., 0].astype(np.float64) + 0.5 * g[..., 1]  # exact in BF16: the gradient at channels 0..5 of layers 2 and 1
+    scale = 64.0 * 12.0 * np.prod(shape)
+    for c in range(6):
+        for o in range(2):
+            e = np.abs(got[9536 + (16 * o + c) * 27:][:27] - taps(f[..., c], g[..., o].astype(np.float64)))
+            assert e.max() <= 2.0 ** -22 * scale, (c, o)
+        e = np.abs(got[2608 + (16 * 2 + c) * 27:][:27] - taps(f[..., c], back))
+        assert e.max() <= 2.0 ** -22 * scale, c
+        e = np.abs(got[(6 * 3 + c) * 27:][:27] - taps(f[..., c], back))
+        assert e.max() <= 2.0 ** -22 * scale, c
+    np.testing.assert_allclose(got[10400:], g.reshape(-1, 2).sum(0), atol=2.0 ** -22 * scale)
