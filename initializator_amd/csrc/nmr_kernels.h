@@ -370,8 +370,8 @@ struct HaloArgs {
 
 struct LossArgs {
     const float* pred;      // [..][2]
-    const float* tx;        // target, compact with pitch
-    const float* ty;
+    const float *ax, *ay;   // target: a - b, compact with pitch
+    const float *bx, *by;
     const uint8_t* mask;
     uint16_t* gout;         // [..][16]
     double* lpart;          // [blocks]
@@ -414,8 +414,6 @@ int loss_blocks(int nx, int ny, int nz);
 hipError_t launch_loss(const LossArgs& a, hipStream_t s);
 hipError_t launch_adam(float* p, float* m, float* v, const float* g, int n, float lr, float b1, float b2, float eps,
                        float c1, float c2, hipStream_t s);
-hipError_t launch_diff(const float* ax, const float* ay, const float* bx, const float* by, float* ox, float* oy,
-                       long n, hipStream_t s);
 // workgroups for n voxels or slots
 int apply_blocks(uint64_t n);
 hipError_t launch_apply(const ApplyArgs& a, int blocks, hipStream_t s);

@@ -33,6 +33,9 @@ constexpr int kParams = 10402;
 // canonical layout: W1 [16][6][27], b1 [16], W2 [16][16][27], b2 [16], W3 [2][16][27], b3 [2]
 constexpr int kW1 = 0, kB1 = 2592, kW2 = 2608, kB2 = 9520, kW3 = 9536, kB3 = 10400;
 constexpr int kFragF1 = 7 * 512, kFragF = 14 * 512; // uint16 per fragment set (cin 8 / 16)
+// Planes of a coarse training step's z-chunks: small grids need the workgroups
+// (a sample of 32^3 to 96^3: 20.2 us at 8 planes, 9.2 at 2).
+constexpr int kCoarseLz = 2;
 constexpr int kWgradParts = 512;                    // partial sums of the weight-gradient kernel
 
 struct Tensors {
@@ -52,8 +55,6 @@ struct nmr_corrector {
     double vscale = 1e-3, out_scale = 0.0;
     Tensors t;
     float* wpart = nullptr; // wgrad partials of the three layers
-    double* lpart = nullptr;
-    size_t lpart_cap = 0;
     double* apart = nullptr; // apply partials
     size_t apart_cap = 0;
     double* hstat = nullptr; // reduced statistics [6], pinned host memory that the reduction writes
@@ -459,7 +460,7 @@ int nmr_hip_corrector_destroy(nmr_corrector* c)
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     tfree(c->t);
     for (void* q : {(void*)c->w, (void*)c->m, (void*)c->v, (void*)c->grad, (void*)c->f1, (void*)c->f2, (void*)c->f3,
-                    (void*)c->d2, (void*)c->d3, (void*)c->wpart, (void*)c->lpart, (void*)c->apart, (void*)c->io, (void*)c->io2, (void*)c->rows[0], (void*)c->rows[1], (void*)c->rows[2]})
+                    (void*)c->d2, (void*)c->d3, (void*)c->wpart, (void*)c->apart, (void*)c->io, (void*)c->io2, (void*)c->rows[0], (void*)c->rows[1], (void*)c->rows[2]})
         if (q) (void)hipFree(q);
     if (c->hstat) (void)hipHostFree(c->hstat);
     if (c->stream) (void)hipStreamDestroy(c->stream);
@@ -559,20 +560,10 @@ int nmr_hip_corrector_train(nmr_corrector* c, nmr_batch* b, const nmr_train_opts
         return fail(NMR_ERR_INVALID, "training options");
     for (const auto& I : b->inst)
         if (!I.uploaded) return fail(NMR_ERR_STATE, "train before every instance is uploaded");
-    // the samples are read from the instances' row buffers: the batch runs
-    // on rows while training and leaves its state there
+    // The batch steps where its runs do (the list of the pores, bricks or rows);
+    // the samples are read from the instances' row buffers, and the batch
+    // leaves its state there.
     if (int rc0 = nmri::batch_rows(b)) return rc0;
-    struct RowsOnly {
-        nmr_batch* b;
-        bool keep;
-        ~RowsOnly()
-        {
-            b->brick_on = keep;
-            b->home = nmri::kHomeRows;
-        }
-    } guard{b, b->brick_on};
-    b->brick_on = false;
-    b->home = nmri::kHomeRows;
     const nmr_problem& P = b->prob;
     size_t nmax = 0;
     int mx = 1, my = 1, mz = 1;
@@ -585,34 +576,38 @@ int nmr_hip_corrector_train(nmr_corrector* c, nmr_batch* b, const nmr_train_opts
     // allocate for the largest instance first so that later shapes only clear
     int rc = ensure_tensors(c, mx, my, mz, true);
     if (rc) return rc;
-    float *coarse[2] = {nullptr, nullptr}, *tgt[2] = {nullptr, nullptr};
-    double* spart = nullptr;
+    float* coarse[2] = {nullptr, nullptr};
+    double *spart = nullptr, *lparts = nullptr;
     std::vector<float*> kept((size_t)b->ninst * 2, nullptr); // state of every instance before the plain steps
     auto cleanup = [&]() {
         (void)hipStreamSynchronize(c->stream);
-        for (float* q : {coarse[0], coarse[1], tgt[0], tgt[1]})
+        for (float* q : {coarse[0], coarse[1]})
             if (q) (void)hipFree(q);
         for (float* q : kept)
             if (q) (void)hipFree(q);
-        if (spart) (void)hipFree(spart);
+        for (double* q : {spart, lparts})
+            if (q) (void)hipFree(q);
     };
     for (int q = 0; q < 2 && !rc; q++)
-        if ((rc = dalloc(c->stream, &coarse[q], nmax)) || (rc = dalloc(c->stream, &tgt[q], nmax))) break;
+        rc = dalloc(c->stream, &coarse[q], nmax);
     for (int i = 0; i < b->ninst && !rc; i++)
         for (int q = 0; q < 2 && !rc; q++) rc = dalloc(c->stream, &kept[2 * i + q], b->inst[i].n_m);
     const int nlb = nmr::loss_blocks(mx, my, mz);
-    if (!rc) rc = ensure_dev_doubles(c, &c->lpart, &c->lpart_cap, (size_t)nlb);
-    // partials of the coarse sweep (tile 32 x 32, z-chunks of 8)
-    const size_t nswp = (size_t)((mx + 31) / 32) * ((my + 31) / 32) * ((mz + 7) / 8);
+    // loss partials of every sample of a round: read once, after its last one
+    if (!rc) rc = dalloc(c->stream, &lparts, (size_t)nlb * b->ninst);
+    // partials of the coarse sweep (tile 32 x 32, z-chunks of kCoarseLz)
+    const size_t nswp = (size_t)((mx + 31) / 32) * ((my + 31) / 32) * ((mz + kCoarseLz - 1) / kCoarseLz);
     if (!rc) rc = dalloc(c->stream, &spart, nswp * 2);
     if (rc) {
         cleanup();
         return rc;
     }
-    std::vector<double> hl(nlb);
+    std::vector<double> hl((size_t)nlb * b->ninst);
     const float vinv = (float)(1.0 / c->vscale);
     for (int r = 0; r < o->rounds && !rc; r++) {
         if (o->stride > 0 && (rc = nmr_hip_batch_run(b, o->stride, nullptr))) break;
+        if ((rc = nmri::batch_rows(b))) break;
+        HIP_TRY(hipStreamSynchronize(b->stream));
         const int p0 = b->parity;
         const int64_t step0 = b->steps_done;
         for (int i = 0; i < b->ninst && !rc; i++)
@@ -622,7 +617,8 @@ int nmr_hip_corrector_train(nmr_corrector* c, nmr_batch* b, const nmr_train_opts
                     rc = fail(NMR_ERR_DEVICE, "state copy failed");
         if (rc) break;
         HIP_TRY(hipStreamSynchronize(c->stream));
-        if ((rc = nmr_hip_batch_run(b, o->factor, nullptr))) break;
+        if ((rc = nmr_hip_batch_run(b, o->factor, nullptr)) || (rc = nmri::batch_rows(b))) break;
+        HIP_TRY(hipStreamSynchronize(b->stream));
         const int p1 = b->parity;
         for (int i = 0; i < b->ninst && !rc; i++) {
             const nmr_batch_instance& s = b->spec[i];
@@ -654,8 +650,8 @@ int nmr_hip_corrector_train(nmr_corrector* c, nmr_batch* b, const nmr_train_opts
             a.nz = s.nz;
             a.pitch = I.pitch;
             a.pitch1 = I.pitch1;
-            // variant 6: tile 32 x 32, lz 8
-            a.lz = std::min(8, s.nz);
+            // variant 6: tile 32 x 32
+            a.lz = std::min(kCoarseLz, s.nz);
             a.ntx = (s.nx + 31) / 32;
             a.nty = (s.ny + 31) / 32;
             a.ntz = (s.nz + a.lz - 1) / a.lz;
@@ -667,12 +663,7 @@ int nmr_hip_corrector_train(nmr_corrector* c, nmr_batch* b, const nmr_train_opts
             a.bx0 = 0; a.bx1 = s.nx; a.by0 = 0; a.by1 = s.ny; a.bz0 = 0; a.bz1 = s.nz;
             a.inert = I.inert;
             a.c = coarse_coef(q, o->factor, &gsum);
-            // coarse output: solids keep their value
-            for (int qq = 0; qq < 2; qq++)
-                HIP_TRY(hipMemcpyAsync(coarse[qq], kept[2 * i + qq], I.n_m * 4, hipMemcpyDeviceToDevice, c->stream));
             HIP_TRY(nmr::launch_sweep(2, b->vel, true, 6, a, c->stream));
-            HIP_TRY(nmr::launch_diff(I.m[p1][0], I.m[p1][1], coarse[0], coarse[1], tgt[0], tgt[1], (long)I.n_m,
-                                     c->stream));
             if ((rc = ensure_tensors(c, s.nx, s.ny, s.nz, true))) break;
             nmr::FeatureArgs f{};
             f.mx = kept[2 * i];
@@ -692,11 +683,16 @@ int nmr_hip_corrector_train(nmr_corrector* c, nmr_batch* b, const nmr_train_opts
             if ((rc = forward(c))) break;
             nmr::LossArgs la{};
             la.pred = c->t.p;
-            la.tx = tgt[0];
-            la.ty = tgt[1];
+            // (only the pores' values are read: the coarse step leaves the
+            // solids of its output as they are)
+            la.ax = I.m[p1][0];
+            la.ay = I.m[p1][1];
+            la.bx = coarse[0];
+            la.by = coarse[1];
             la.mask = I.mask;
             la.gout = c->t.g3;
-            la.lpart = c->lpart;
+            double* const lpart = lparts + (size_t)i * nlb;
+            la.lpart = lpart;
             la.nx = s.nx;
             la.ny = s.ny;
             la.nz = s.nz;
@@ -708,7 +704,7 @@ int nmr_hip_corrector_train(nmr_corrector* c, nmr_batch* b, const nmr_train_opts
                 HIP_TRY(hipMemsetAsync(c->t.p, 0, (size_t)(s.nx + 2) * (s.ny + 2) * (s.nz + 2) * 8, c->stream));
                 HIP_TRY(nmr::launch_loss(la, c->stream));
                 const int nb = nmr::loss_blocks(s.nx, s.ny, s.nz);
-                HIP_TRY(hipMemcpyAsync(hl.data(), c->lpart, nb * 8, hipMemcpyDeviceToHost, c->stream));
+                HIP_TRY(hipMemcpyAsync(hl.data(), lpart, nb * 8, hipMemcpyDeviceToHost, c->stream));
                 HIP_TRY(hipStreamSynchronize(c->stream));
                 double ss = 0.0;
                 for (int k = 0; k < nb; k++) ss += hl[k];
@@ -720,16 +716,18 @@ int nmr_hip_corrector_train(nmr_corrector* c, nmr_batch* b, const nmr_train_opts
             HIP_TRY(nmr::launch_loss(la, c->stream));
             if ((rc = backward(c))) break;
             if ((rc = adam_step(c, o->lr))) break;
-            if (losses) {
-                const int nb = nmr::loss_blocks(s.nx, s.ny, s.nz);
-                HIP_TRY(hipMemcpyAsync(hl.data(), c->lpart, nb * 8, hipMemcpyDeviceToHost, c->stream));
-                HIP_TRY(hipStreamSynchronize(c->stream));
-                double ss = 0.0;
-                for (int k = 0; k < nb; k++) ss += hl[k];
-                losses[(size_t)r * b->ninst + i] = ss / std::max<int64_t>(1, I.npore);
-            }
         }
+        if (rc) break;
+        if (losses)
+            HIP_TRY(hipMemcpyAsync(hl.data(), lparts, hl.size() * 8, hipMemcpyDeviceToHost, c->stream));
         HIP_TRY(hipStreamSynchronize(c->stream));
+        for (int i = 0; losses && i < b->ninst; i++) {
+            const auto& s = b->spec[i];
+            const int nb = nmr::loss_blocks(s.nx, s.ny, s.nz);
+            double ss = 0.0;
+            for (int k = 0; k < nb; k++) ss += hl[(size_t)i * nlb + k];
+            losses[(size_t)r * b->ninst + i] = ss / std::max<int64_t>(1, b->inst[i].npore);
+        }
     }
     cleanup();
     return rc;

@@ -798,7 +798,8 @@ __global__ void __launch_bounds__(256) gout_copy_kernel(const float* __restrict_
     o[1] = make_uint4(0u, 0u, 0u, 0u);
 }
 
-// Squared-error loss over pores of (pred - target/scale) and its gradient
+// Squared-error loss over pores of (pred - target/scale), the target being the
+// plain steps' result less the coarse step's, and its gradient
 // 2 (pred - t) / npore as the BF16 16-channel output gradient; per-block
 // partial loss sums.
 __global__ void __launch_bounds__(256) loss_kernel(LossArgs a)
@@ -813,8 +814,8 @@ __global__ void __launch_bounds__(256) loss_kernel(LossArgs a)
         const long pv = ((long)(z + 1) * (a.ny + 2) + (y + 1)) * (a.nx + 2) + (x + 1);
         float g0 = 0.f, g1 = 0.f;
         if (a.mask[c]) {
-            const float d0 = a.pred[pv * 2] - a.tx[c] * a.tinv;
-            const float d1 = a.pred[pv * 2 + 1] - a.ty[c] * a.tinv;
+            const float d0 = a.pred[pv * 2] - (a.ax[c] - a.bx[c]) * a.tinv;
+            const float d1 = a.pred[pv * 2 + 1] - (a.ay[c] - a.by[c]) * a.tinv;
             l = (double)d0 * d0 + (double)d1 * d1;
             g0 = 2.f * d0 * a.winv;
             g1 = 2.f * d1 * a.winv;
@@ -845,17 +846,6 @@ __global__ void __launch_bounds__(256) adam_kernel(float* __restrict__ p, float*
     m[i] = mi;
     v[i] = vi;
     p[i] -= lr * (mi / c1) / (sqrtf(vi / c2) + eps);
-}
-
-// target = after - coarse over both components (compact layout).
-__global__ void __launch_bounds__(256) diff_kernel(const float* __restrict__ ax, const float* __restrict__ ay,
-                                                   const float* __restrict__ bx, const float* __restrict__ by,
-                                                   float* __restrict__ ox, float* __restrict__ oy, long n)
-{
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    ox[i] = ax[i] - bx[i];
-    oy[i] = ay[i] - by[i];
 }
 
 // Adds scale * pred to the pores of the state, brings the result into the
@@ -1091,13 +1081,6 @@ hipError_t launch_adam(float* p, float* m, float* v, const float* g, int n, floa
                        float c1, float c2, hipStream_t s)
 {
     hipLaunchKernelGGL(adam_kernel, dim3(blocks_for(n)), dim3(256), 0, s, p, m, v, g, n, lr, b1, b2, eps, c1, c2);
-    return hipGetLastError();
-}
-
-hipError_t launch_diff(const float* ax, const float* ay, const float* bx, const float* by, float* ox, float* oy,
-                       long n, hipStream_t s)
-{
-    hipLaunchKernelGGL(diff_kernel, dim3(blocks_for(n)), dim3(256), 0, s, ax, ay, bx, by, ox, oy, n);
     return hipGetLastError();
 }
 

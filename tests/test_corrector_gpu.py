@@ -365,3 +365,20 @@ def test_weight_gradient_at_the_edges_of_segments(shape):
         e = np.abs(got[(6 * 3 + c) * 27:][:27] - taps(f[..., c], back))
         assert e.max() <= 2.0 ** -22 * scale, c
     np.testing.assert_allclose(got[10400:], g.reshape(-1, 2).sum(0), atol=2.0 ** -22 * scale)
+
+
+def test_training_gives_the_same_net_whatever_the_batch_steps_on():
+    """The batch steps on the list of the pores, on a tile in bricks or in rows
+    while it trains: the same samples, so the same losses and parameters, and
+    the same state left behind."""
+    specs, out = _instances(4), []
+    for layout, variant in ((True, -1), (True, 4), (False, -1)):
+        with _batch(specs) as b, Corrector(3) as net:
+            b.set_layout(layout)
+            b.set_tile(variant)
+            losses = net.train(b, factor=4, rounds=3, stride=3)
+            out.append([losses, net.params] + sum((b.download(i) for i in range(4)), []) + [b.run(2)])
+    for o in out[1:]:
+        for x, y in zip(o[:-1], out[0][:-1]):
+            np.testing.assert_array_equal(x, y)
+        np.testing.assert_allclose(o[-1], out[0][-1], rtol=1e-11, atol=1e-12)
