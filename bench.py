@@ -8,9 +8,10 @@ in FP32, D = 2.3e-9 m^2/s, T2 = 2 s, rho = 10 um/s, dt = 0.4 x the explicit
 limit.  A step is one time step of the whole grid (update + per-step signal
 reduction); inputs are resident in HBM before the timed region.
 
-Prints one JSON line.  The roofline object prices the sweep kernel at its
-compulsory traffic, 29 bytes per voxel-step (read Mx, My: 8; write Mx, My:
-8; uint8 mask: 1; Vx, Vy, Vz faces: 12), against 8 TB/s.  cpu_baseline
+Prints one JSON line.  The roofline object prices a step at what it cannot do
+without, against 8 TB/s: 28 bytes a pore (read Mx, My: 8; write Mx, My: 8;
+three velocity sums: 12) and the pore map at one bit a voxel -- solids never
+change, and the sweeps over the list of the pores do not touch them.  cpu_baseline
 times the FP64 CPU oracle on this host on a bounded number of steps of the
 same grid.
 """
@@ -28,21 +29,25 @@ sys.path.insert(0, ROOT)
 
 METRIC = "voxel-steps/s & %HBM roofline @256³; learned vs plain time-to-signal @1e-3"
 HBM_PEAK_GBS = 8000.0
-BYTES_PER_VOXEL_STEP = 29.0  # read Mx,My (8) + write Mx,My (8) + mask (1) + velocity (12)
-# MacCormack (--scheme maccormack): predictor pass 29 B (as above, writing the
-# predictor) + corrector pass 37 B (reads the predictor and the state, 8 each)
-BYTES_PER_VOXEL_STEP_MAK = 66.0
-# Bytes past the L2 per sweep launch of the default workload (256^3, phi
-# 0.20, automatic tile, brick layout): rocprofv3 --pmc FETCH_SIZE (x2.0) +
-# WRITE_SIZE (x1.0) per dispatch, scaled by what the same counters read for a
-# plain 1 GiB copy (summary under profiles/, sweep_kernel_256cube_flow_pgse.md).
-# The device's memory-side cache serves part of these requests; the counters
-# at the L2 do not tell which.
-DEFAULT_TRAFFIC = 226.1e6 + 52.5e6
-# The same for --scheme maccormack at 256^3, phi 0.20 (brick layout): the
-# predictor and the corrector launch of one step together (summary under
-# profiles/, gsweep_maccormack_256cube_flow_pgse.md).
-MAK_TRAFFIC = (219.2e6 + 50.4e6) + (286.7e6 + 50.4e6)
+BYTES_PER_PORE_STEP = 28.0  # read Mx,My (8) + write Mx,My (8) + velocity sums (12)
+# MacCormack (--scheme maccormack): predictor pass 28 B (as above, writing the
+# predictor) + corrector pass 36 B (reads the predictor and the state, 8 each)
+BYTES_PER_PORE_STEP_MAK = 64.0
+# Bytes past the L2 per step of the default workload (256^3, phi 0.20, the list
+# of the pores): rocprofv3 --pmc FETCH_SIZE (x2.0) + WRITE_SIZE (x1.0) per
+# dispatch, scaled by what the same counters read for a plain 1 GiB copy
+# (summary under profiles/, pore_kernel_256cube_flow_pgse.md).  The device's
+# memory-side cache serves part of these requests; the counters at the L2 do
+# not tell which.
+DEFAULT_TRAFFIC = 95.7e6 + 27.1e6
+# The same for --scheme maccormack at 256^3, phi 0.20: the predictor and the
+# corrector launch of one step together.
+MAK_TRAFFIC = (95.7e6 + 26.9e6) + (122.6e6 + 27.1e6)
+
+
+def compulsory_bytes(npore: int, nvox: int, per_pore: float, passes: int = 1) -> float:
+    """Bytes a step cannot do without: per_pore at the pores, the pore map once a pass."""
+    return per_pore * npore + passes * nvox / 8.0
 
 
 def _cpu_model() -> str:
@@ -231,7 +236,8 @@ def batch_main(args) -> int:
         loop = {"value": nvox * args.single_steps / (loop_ms * 1e-3), "unit": "voxel-steps/s",
                 "steps": args.single_steps, "gpu_ms": loop_ms}
     kernel_s = gpu_ms * 1e-3 / args.steps
-    achieved = BYTES_PER_VOXEL_STEP * nvox / kernel_s / 1e9
+    step_bytes = compulsory_bytes(sum(int(np.count_nonzero(sp["mask"])) for sp in specs), nvox, BYTES_PER_PORE_STEP)
+    achieved = step_bytes / kernel_s / 1e9
     err = instance_errors(specs, args.error_instances, args.error_steps, dx, dt, D) if args.error_instances else None
     out = {
         "metric": "voxel-steps/s (batched uneven instances)",
@@ -254,7 +260,7 @@ def batch_main(args) -> int:
             "lz": lz,
             "persistent_grid": per,
             "graph_steps": args.graph_steps,
-            "bytes_per_voxel_step": BYTES_PER_VOXEL_STEP,
+            "bytes_per_voxel_step": step_bytes / nvox,
         },
         "roofline": {
             "bound": "hbm",
@@ -439,10 +445,10 @@ def main() -> int:
     from initializator_amd import _lib
 
     mak = args.scheme == "maccormack"
-    bpv = BYTES_PER_VOXEL_STEP_MAK if mak else BYTES_PER_VOXEL_STEP
-    # per-voxel inputs each pass reads: the field 4 B, D and 1/T2 8 B
-    extra = (4.0 if args.field else 0.0) + (8.0 if args.coef else 0.0)
-    bpv += extra * (2 if mak else 1)
+    passes = 2 if mak else 1
+    # per-voxel inputs each pass reads at the pores: the field 4 B, D and 1/T2 8 B
+    per_pore = (BYTES_PER_PORE_STEP_MAK if mak else BYTES_PER_PORE_STEP) + passes * (
+        (4.0 if args.field else 0.0) + (8.0 if args.coef else 0.0))
     bc = {"neumann": _lib.NMR_BC_NEUMANN, "periodic": _lib.NMR_BC_PERIODIC,
           "dirichlet": _lib.NMR_BC_DIRICHLET}[args.bc]
     total = args.warmup + args.steps
@@ -460,8 +466,8 @@ def main() -> int:
         s.upload_field(rng.uniform(-2e-5, 2e-5, case.shape))
     if args.coef:
         s.upload_coefficients(np.where(case.mask != 0, case.diffusivity, 0.0), rng.uniform(0.5, 5.0, case.shape))
-    # the upload converts the state to the sweep's brick layout and sizes its
-    # buffers; the state then stays on the device, in bricks, from run to run
+    # the upload brings the state into the list of the pores (or bricks) and sizes
+    # the buffers; it then stays there from run to run
     s.upload_magnetization(case.mask.astype("float64"), np.zeros(case.shape))
     # the warm-up takes the same path as the timed run (signal rows copied
     # back), so that no first call of it falls inside the timed region
@@ -478,6 +484,7 @@ def main() -> int:
     nvox = case.nvox
     value = nvox * args.steps / wall
     kernel_s = gpu_ms * 1e-3 / args.steps
+    bpv = compulsory_bytes(int(np.count_nonzero(case.mask)), nvox, per_pore, passes) / nvox
     achieved = bpv * nvox / kernel_s / 1e9
     plain_physics = args.bc == "neumann" and not args.field and not args.coef
     default = (shape, args.phi, args.variant, args.lz, args.rho) == ((256, 256, 256), 0.20, -1, 0, 10e-6) \
@@ -515,8 +522,7 @@ def main() -> int:
             "traffic": traffic,
             # traffic is not measured by this run: rocprofv3 --pmc FETCH_SIZE /
             # WRITE_SIZE of the same command, scaled by a plain copy's counters
-            "traffic_source": (f"profiles/{'gsweep_maccormack' if mak else 'sweep_kernel'}_256cube_flow_pgse.md"
-                               if traffic else None),
+            "traffic_source": "profiles/pore_kernel_256cube_flow_pgse.md" if traffic else None,
             # measured DRAM bytes over the same kernel time, against 8 TB/s
             "dram_frac": traffic / kernel_s / (HBM_PEAK_GBS * 1e9) if traffic else None,
             "kernel_us": kernel_s * 1e6,
