@@ -221,9 +221,12 @@ int nmr_hip_last_run_ms(nmr_ctx* ctx, double* ms, int64_t* sweeps);
  * list's offsets); with a tile variant set, or where the list does not pay,
  * bricks of 128 bytes (8 x-voxels by 4 rows of one plane), so that all-solid
  * bricks are never fetched.  The uploads convert their arrays once; the state
- * stays converted from run to run (pulses rotate it there) and is converted
- * back only for a download or a learned solve.  0 always sweeps the row
- * layout.  The fields are the same bits either way. */
+ * stays converted from run to run (pulses rotate it there; a learned solve
+ * steps on the list too) and is converted back only for a download, or for a
+ * learned solve that the list does not take.  Small grids take several plain
+ * upwind steps a launch.  0 always sweeps the row layout.  The fields are the
+ * same bits either way.  Once mask and magnetization are uploaded, this and
+ * nmr_hip_set_tile prepare (and allocate) what the next run takes. */
 int nmr_hip_set_layout(nmr_ctx* ctx, int32_t brick);
 /* Tile shape of the sweep kernel: variant index (-1 = automatic, -2 = a
  * one-thread-per-voxel kernel with the arithmetic of the sweeps, a

@@ -70,8 +70,14 @@ int HostStage::down(hipStream_t s, const float* src, size_t n, const std::functi
     constexpr size_t per = kSlotBytes / sizeof(float);
     const size_t chunks = (n + per - 1) / per;
     if (chunks == 0) return NMR_OK;
-    int rc = open((int)std::min<size_t>(chunks, kSlots));
-    if (rc) return rc;
+    if (open((int)std::min<size_t>(chunks, kSlots)) != NMR_OK) { // no pinned memory: through pageable memory
+        (void)hipGetLastError();
+        std::vector<float> h(n);
+        HIP_TRY(hipMemcpyAsync(h.data(), src, n * sizeof(float), hipMemcpyDeviceToHost, s));
+        HIP_TRY(hipStreamSynchronize(s));
+        use(0, n, h.data());
+        return NMR_OK;
+    }
     auto slot = [&](size_t c) { return reinterpret_cast<float*>(buf + (c % have) * kSlotBytes); };
     if (chunks == 1) {
         HIP_TRY(hipMemcpyAsync(slot(0), src, n * sizeof(float), hipMemcpyDeviceToHost, s));
@@ -149,8 +155,12 @@ int HostStage::up(hipStream_t s, float* dst, const float* src, size_t n)
     constexpr size_t per = kSlotBytes / sizeof(float);
     const size_t chunks = (n + per - 1) / per;
     if (chunks == 0) return NMR_OK;
-    int rc = open((int)std::min<size_t>(chunks, kSlots));
-    if (rc) return rc;
+    if (open((int)std::min<size_t>(chunks, kSlots)) != NMR_OK) {
+        (void)hipGetLastError();
+        HIP_TRY(hipMemcpyAsync(dst, src, n * sizeof(float), hipMemcpyHostToDevice, s));
+        HIP_TRY(hipStreamSynchronize(s));
+        return NMR_OK;
+    }
     auto slot = [&](size_t c) { return buf + (c % have) * kSlotBytes; };
     auto count = [&](size_t c) { return std::min(per, n - c * per) * sizeof(float); };
     std::mutex mu;
