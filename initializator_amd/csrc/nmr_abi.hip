@@ -1534,35 +1534,41 @@ int nmr_hip_download_magnetization(nmr_ctx* ctx, double* mx, double* my, double*
     double* dst[3] = {mx, my, mz};
     const nmr_problem& p = ctx->prob;
     if ((rc = nmri::state_rows(ctx))) return rc;
-    std::vector<float> h(layout == NMR_LAYOUT_COMPACT ? 0 : ctx->n_m);
+    if (layout == NMR_LAYOUT_COMPACT) {
+        const float* from[3];
+        double* to[3];
+        int n = 0;
+        for (int q = 0; q < ctx->nc; q++) {
+            if (!dst[q]) continue;
+            from[n] = ctx->m[ctx->cur][q];
+            to[n++] = dst[q];
+        }
+        return ctx->stage.down_rows(ctx->stream, from, n, p.nx, (size_t)p.ny * p.nz, ctx->pitch, to);
+    }
+    std::vector<float> h(ctx->n_m);
     for (int q = 0; q < ctx->nc; q++) {
         if (!dst[q]) continue;
-        if (layout == NMR_LAYOUT_COMPACT) {
-            rc = ctx->stage.down_rows(ctx->stream, ctx->m[ctx->cur][q], p.nx, (size_t)p.ny * p.nz, ctx->pitch, dst[q]);
-            if (rc) return rc;
-        } else {
-            HIP_TRY(hipMemcpyAsync(h.data(), ctx->m[ctx->cur][q], h.size() * sizeof(float), hipMemcpyDeviceToHost,
-                                   ctx->stream));
-            HIP_TRY(hipStreamSynchronize(ctx->stream));
-            // interior plus the ghost layer each axis's boundary condition
-            // leaves (copy of the adjacent cell, opposite cell, or 0)
-            auto ghost = [](int i, int n, int bc, bool* zero) {
-                if (i >= 1 && i <= n) return i - 1;
-                if (bc == NMR_BC_DIRICHLET) *zero = true;
-                if (bc == NMR_BC_PERIODIC) return i == 0 ? n - 1 : 0;
-                return i == 0 ? 0 : n - 1;
-            };
-            for (int k = 0; k < p.nz + 2; k++)
-                for (int j = 0; j < p.ny + 2; j++)
-                    for (int i = 0; i < p.nx + 2; i++) {
-                        bool zero = false;
-                        const int ii = ghost(i, p.nx, p.bc[0], &zero);
-                        const int jj = ghost(j, p.ny, p.bc[1], &zero);
-                        const int kk = ghost(k, p.nz, p.bc[2], &zero);
-                        dst[q][pidx(p, i, j, k)] =
-                            zero ? 0.0 : h[(size_t)kk * p.ny * ctx->pitch + (size_t)jj * ctx->pitch + ii];
-                    }
-        }
+        HIP_TRY(hipMemcpyAsync(h.data(), ctx->m[ctx->cur][q], h.size() * sizeof(float), hipMemcpyDeviceToHost,
+                               ctx->stream));
+        HIP_TRY(hipStreamSynchronize(ctx->stream));
+        // interior plus the ghost layer each axis's boundary condition
+        // leaves (copy of the adjacent cell, opposite cell, or 0)
+        auto ghost = [](int i, int n, int bc, bool* zero) {
+            if (i >= 1 && i <= n) return i - 1;
+            if (bc == NMR_BC_DIRICHLET) *zero = true;
+            if (bc == NMR_BC_PERIODIC) return i == 0 ? n - 1 : 0;
+            return i == 0 ? 0 : n - 1;
+        };
+        for (int k = 0; k < p.nz + 2; k++)
+            for (int j = 0; j < p.ny + 2; j++)
+                for (int i = 0; i < p.nx + 2; i++) {
+                    bool zero = false;
+                    const int ii = ghost(i, p.nx, p.bc[0], &zero);
+                    const int jj = ghost(j, p.ny, p.bc[1], &zero);
+                    const int kk = ghost(k, p.nz, p.bc[2], &zero);
+                    dst[q][pidx(p, i, j, k)] =
+                        zero ? 0.0 : h[(size_t)kk * p.ny * ctx->pitch + (size_t)jj * ctx->pitch + ii];
+                }
     }
     return NMR_OK;
 }
@@ -2692,12 +2698,15 @@ int nmr_hip_batch_download(nmr_batch* b, int32_t i, double* mx, double* my, doub
                                       b->stream));
         }
     }
+    const float* from[3];
+    double* to[3];
+    int n = 0;
     for (int q = 0; q < b->nc; q++) {
         if (!dst[q]) continue;
-        const int rc = b->stage.down_rows(b->stream, I.m[b->parity][q], s.nx, (size_t)s.ny * s.nz, I.pitch, dst[q]);
-        if (rc) return rc;
+        from[n] = I.m[b->parity][q];
+        to[n++] = dst[q];
     }
-    return NMR_OK;
+    return b->stage.down_rows(b->stream, from, n, s.nx, (size_t)s.ny * s.nz, I.pitch, to);
 }
 
 int nmr_hip_batch_set_layout(nmr_batch* b, int32_t brick)

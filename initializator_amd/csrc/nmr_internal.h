@@ -59,12 +59,13 @@ struct HostStage {
     HostStage& operator=(const HostStage&) = delete;
     ~HostStage();
     int open(int slots);
-    // n floats at src, in pieces of any length and order, to use(first, count, values).
-    int down(hipStream_t s, const float* src, size_t n, const std::function<void(size_t, size_t, const float*)>& use);
+    // n floats of each array, in pieces of any length and order, to use(array, first, count, values).
+    int down(hipStream_t s, const float* const* src, int arrays, size_t n,
+             const std::function<void(int, size_t, size_t, const float*)>& use);
     // n floats from host memory.
     int up(hipStream_t s, float* dst, const float* src, size_t n);
-    // Rows of nx of `pitch` floats into a compact array of doubles.
-    int down_rows(hipStream_t s, const float* src, int nx, size_t rows, int pitch, double* dst);
+    // Rows of nx of `pitch` floats into compact arrays of doubles.
+    int down_rows(hipStream_t s, const float* const* src, int arrays, int nx, size_t rows, int pitch, double* const* dst);
 };
 
 // A list of the pores of one domain or of all instances of a batch

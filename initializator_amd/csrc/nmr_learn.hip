@@ -370,7 +370,8 @@ int download_p(nmr_corrector* c, float* out)
     const size_t px = 2 * (size_t)(t.nx + 2), py = (size_t)(t.ny + 2); // floats a padded row, rows a padded plane
     const size_t nx = 2 * (size_t)t.nx, ny = (size_t)t.ny;
     // planes 1 .. nz; a row gives what of it lies in 2 .. px - 2
-    return c->stage.down(c->stream, t.p + px * py, px * py * (size_t)t.nz, [=](size_t i, size_t n, const float* p) {
+    const float* const planes = t.p + px * py;
+    return c->stage.down(c->stream, &planes, 1, px * py * (size_t)t.nz, [=](int, size_t i, size_t n, const float* p) {
         for (size_t e = i + n; i < e;) {
             const size_t r = i / px, y = r % py, z = r / py, end = std::min(e, (r + 1) * px);
             const size_t from = std::max(i, r * px + 2), to = std::min(end, r * px + px - 2);

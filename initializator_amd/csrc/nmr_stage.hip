@@ -5,8 +5,8 @@
 // What bounds a large download is the host: FP32 rows become FP64 arrays whose
 // pages the caller has just allocated, so the kernel clears each on its first
 // touch, and one thread does 7 GB/s of that behind pageable copies: 256^3, two
-// components, 268 MB: 37.3 ms; eight threads on 1 MiB slots: 6.2 (43 GB/s).
-// 512x512x130 76 -> 12 ms, 203x97x151 3.6-6.6 -> 1.4, 64^3 0.24 -> 0.14.  Up:
+// components, 268 MB: 37.3 ms; eight threads on 1 MiB slots: 5.6 (48 GB/s).
+// 512x512x130 76 -> 10.5 ms, 203x97x151 3.6-6.6 -> 1.1, 64^3 0.24 -> 0.11.  Up:
 // the net's 11.8 MB of features at 96x80x64 (with its pass and the result)
 // 0.93 -> 0.73 ms.
 #include "nmr_internal.h"
@@ -65,29 +65,40 @@ int HostStage::open(int slots)
     return NMR_OK;
 }
 
-int HostStage::down(hipStream_t s, const float* src, size_t n, const std::function<void(size_t, size_t, const float*)>& use)
+int HostStage::down(hipStream_t s, const float* const* src, int arrays, size_t n,
+                    const std::function<void(int, size_t, size_t, const float*)>& use)
 {
-    constexpr size_t per = kSlotBytes / sizeof(float);
-    const size_t chunks = (n + per - 1) / per;
-    if (chunks == 0) return NMR_OK;
+    if (arrays < 1 || n == 0) {
+        HIP_TRY(hipStreamSynchronize(s));
+        return NMR_OK;
+    }
+    // a thread for each 768 KiB (starting one costs 20 us), and pieces of up to
+    // a slot that give every thread one
+    const size_t total = n * (size_t)arrays;
+    const int threads = (int)std::min<size_t>(kWorkers, std::max<size_t>(1, total / ((size_t)3 << 16)));
+    const size_t per = std::min(kSlotBytes / sizeof(float), (total + threads - 1) / threads);
+    const size_t each = (n + per - 1) / per, chunks = each * (size_t)arrays; // pieces of an array, of all
     if (open((int)std::min<size_t>(chunks, kSlots)) != NMR_OK) { // no pinned memory: through pageable memory
         (void)hipGetLastError();
         std::vector<float> h(n);
-        HIP_TRY(hipMemcpyAsync(h.data(), src, n * sizeof(float), hipMemcpyDeviceToHost, s));
-        HIP_TRY(hipStreamSynchronize(s));
-        use(0, n, h.data());
+        for (int q = 0; q < arrays; q++) {
+            HIP_TRY(hipMemcpyAsync(h.data(), src[q], n * sizeof(float), hipMemcpyDeviceToHost, s));
+            HIP_TRY(hipStreamSynchronize(s));
+            use(q, 0, n, h.data());
+        }
         return NMR_OK;
     }
     auto slot = [&](size_t c) { return reinterpret_cast<float*>(buf + (c % have) * kSlotBytes); };
     if (chunks == 1) {
-        HIP_TRY(hipMemcpyAsync(slot(0), src, n * sizeof(float), hipMemcpyDeviceToHost, s));
+        HIP_TRY(hipMemcpyAsync(slot(0), src[0], n * sizeof(float), hipMemcpyDeviceToHost, s));
         HIP_TRY(hipStreamSynchronize(s));
-        use(0, n, slot(0));
+        use(0, 0, n, slot(0));
         return NMR_OK;
     }
-    auto count = [&](size_t c) { return std::min(per, n - c * per); };
+    auto first = [&](size_t c) { return c % each * per; };
+    auto count = [&](size_t c) { return std::min(per, n - first(c)); };
     auto issue = [&](size_t c) -> hipError_t {
-        hipError_t e = hipMemcpyAsync(slot(c), src + c * per, count(c) * sizeof(float), hipMemcpyDeviceToHost, s);
+        hipError_t e = hipMemcpyAsync(slot(c), src[c / each] + first(c), count(c) * sizeof(float), hipMemcpyDeviceToHost, s);
         return e != hipSuccess ? e : hipEventRecord(ev[c % have], s);
     };
     std::mutex mu;
@@ -105,7 +116,7 @@ int HostStage::down(hipStream_t s, const float* src, size_t n, const std::functi
             if (stop || next >= here) return false;
             c = next++;
         }
-        use(c * per, count(c), slot(c));
+        use((int)(c / each), first(c), count(c), slot(c));
         {
             std::lock_guard<std::mutex> l(mu);
             done[c] = 1;
@@ -117,10 +128,12 @@ int HostStage::down(hipStream_t s, const float* src, size_t n, const std::functi
     hipError_t e = hipSuccess;
     {
         Team team;
-        team.start((int)std::min<size_t>(kWorkers, chunks) - 1, [&] {
-            while (work(true)) {}
-        });
         size_t sent = 0;
+        while (e == hipSuccess && sent < std::min<size_t>(chunks, have)) e = issue(sent++);
+        if (e == hipSuccess)
+            team.start(threads - 1, [&] {
+                while (work(true)) {}
+            });
         for (size_t c = 0; c < chunks && e == hipSuccess; c++) {
             for (;;) { // copies on their way into every free slot
                 size_t free_to;
@@ -223,13 +236,14 @@ int HostStage::up(hipStream_t s, float* dst, const float* src, size_t n)
     return NMR_OK;
 }
 
-int HostStage::down_rows(hipStream_t s, const float* src, int nx, size_t rows, int pitch, double* dst)
+int HostStage::down_rows(hipStream_t s, const float* const* src, int arrays, int nx, size_t rows, int pitch,
+                         double* const* dst)
 {
-    return down(s, src, rows * (size_t)pitch, [=](size_t i, size_t n, const float* p) {
-        for (size_t e = i + n; i < e;) { // one row, or what of it the chunk holds
+    return down(s, src, arrays, rows * (size_t)pitch, [=](int q, size_t i, size_t n, const float* p) {
+        for (size_t e = i + n; i < e;) { // one row, or what of it the piece holds
             const size_t r = i / (size_t)pitch, x = i % (size_t)pitch, end = std::min(e, (r + 1) * (size_t)pitch);
             const size_t stop = std::min(end, r * (size_t)pitch + (size_t)nx);
-            double* d = dst + r * (size_t)nx + x;
+            double* d = dst[q] + r * (size_t)nx + x;
             for (size_t k = 0; i + k < stop; k++) d[k] = (double)p[k];
             p += end - i;
             i = end;
