@@ -817,7 +817,7 @@ int build_pores(nmr_ctx* c)
     HIP_TRY(nmr::launch_pore_count(b, c->stream));
     HIP_TRY(hipMemcpyAsync(&end, b.planes + p.nz, sizeof(end), hipMemcpyDeviceToHost, c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));
-    if (!nmri::pores_fit(end) ||
+    if (!nmri::pores_fit(end, c->vel) ||
         !pores_pay((double)end, (double)p.nx * p.ny * p.nz, (p.scheme == NMR_SCHEME_MACCORMACK ? 3 : 2) * c->nc, c->vel))
         return NMR_OK;
     const nmri::PoreNeeds n{c->nc, c->vel, ghosts || b.read_solids, p.bc[0] != NMR_BC_NEUMANN,
@@ -2190,7 +2190,7 @@ int build_batch_pores(nmr_batch* b)
     HIP_TRY(hipStreamSynchronize(b->stream));
     uint64_t end = 64;
     for (uint64_t v : n) end += v;
-    if (!nmri::pores_fit(end) || !pores_pay((double)end, grid, 2 * b->nc, b->vel)) return NMR_OK;
+    if (!nmri::pores_fit(end, b->vel) || !pores_pay((double)end, grid, 2 * b->nc, b->vel)) return NMR_OK;
     int64_t bytes = 0;
     const nmri::PoreNeeds needs{b->nc, b->vel, b->pl_reads_solids, false, false};
     if ((rc = nmri::pores_alloc(&b->pl, (uint32_t)end, needs, b->stream, &bytes))) return rc;

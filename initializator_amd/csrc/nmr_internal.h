@@ -117,8 +117,10 @@ int pores_blocks(PoreList* L, nmr::PoreBuild* b, hipStream_t s, int64_t* bytes);
 int pores_finish(PoreList* L, const nmr::PoreBuild& b, hipStream_t s, bool* ok);
 // Groups that a workgroup takes of a list of `groups`.
 int pores_per_tile(int64_t groups);
-// Whether a list of this many slots stays inside the kernels' 32-bit byte offsets.
-bool pores_fit(uint64_t nslots);
+// Whether a list of this many slots stays inside the kernels' 32-bit byte
+// offsets: slot * size of its widest array, the records with velocity, else
+// three components.
+bool pores_fit(uint64_t nslots, bool vel);
 
 } // namespace nmri
 

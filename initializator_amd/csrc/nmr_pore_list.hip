@@ -26,9 +26,11 @@ int grow(T** p, size_t count, int fill, hipStream_t s, int64_t* bytes, size_t ol
 
 } // namespace
 
-bool pores_fit(uint64_t nslots)
+bool pores_fit(uint64_t nslots, bool vel)
 {
-    return nslots > 64 && (nslots + 64) * 12 < ((uint64_t)1 << 32) - 256;
+    constexpr uint64_t state = 3 * sizeof(float), rec = sizeof(*PoreList::rec);
+    static_assert(rec >= state && state >= sizeof(*PoreList::off16) && state >= sizeof(*PoreList::vox), "widest arrays");
+    return nslots > 64 && (nslots + 64) * (vel ? rec : state) < ((uint64_t)1 << 32) - 256;
 }
 
 int pores_alloc(PoreList* L, uint32_t nslots, const PoreNeeds& n, hipStream_t s, int64_t* bytes)
