@@ -309,6 +309,7 @@ int ensure_signal(nmr_ctx* c, size_t doubles)
 }
 
 int pore_args(nmr_ctx* c, nmr::PoreArgs* a);
+int pore_data(nmr_ctx* c);
 
 // Signal of the current state into dsignal[row*nc ...] (enqueued on the stream).
 int enqueue_field_sum(nmr_ctx* c, size_t row)
@@ -319,8 +320,8 @@ int enqueue_field_sum(nmr_ctx* c, size_t row)
                     (row + 1) * (size_t)c->nsig());
     if (c->home == nmri::kHomePores) { // the state is only in the list
         nmr::PoreArgs a{};
-        int rc = pore_args(c, &a);
-        if (rc) return rc;
+        int rc = pore_data(c); // (weights may have come while another sweep was set)
+        if (rc || (rc = pore_args(c, &a))) return rc;
         if ((rc = ensure_partials(c, (size_t)a.ntiles * c->nsig()))) return rc;
         a.f = c->pl.state[c->ppar];
         a.partials = c->partials;
@@ -369,7 +370,6 @@ int state_bricks(nmr_ctx* c);
 int use_pores(nmr_ctx* c, bool* yes);
 int drop_pores(nmr_ctx* c);
 int state_pores(nmr_ctx* c);
-int pore_data(nmr_ctx* c);
 
 // Launch geometry of the general sweep: 256 threads, tiles of 4*lanes x
 // (256/lanes) voxels, z-chunks of lz planes (the round model unless set).

@@ -1,0 +1,49 @@
+"""Calls that change which sweep the next run takes while the state lives in the
+list of the pores: what they return equals a solver that never leaves the rows."""
+import numpy as np
+import pytest
+
+from initializator_amd import generators
+from initializator_amd.solver import HipSolver
+
+pytestmark = pytest.mark.gpu
+
+DX, D = 1e-6, 2.3e-9
+DT = generators.stable_dt(DX, D)
+
+
+def _solver(shape, mask, m0, nc, rows=False, **kw):
+    s = HipSolver(shape, nc, DX, DT, D, 0.5, r1_bulk=0.4, rho1=4e-6, rho2=9e-6, **kw)
+    s.set_layout(not rows)
+    s.upload_mask(mask)
+    s.upload_magnetization(*m0[:nc])
+    return s
+
+
+@pytest.mark.parametrize("leave", ["layout", "tile", "per voxel"])
+@pytest.mark.parametrize("before", [False, True])
+def test_signal_after_weights_that_come_while_another_sweep_is_set(leave, before):
+    """A run leaves the state in the list only; then another sweep is set and
+    phase weights are uploaded (the first ones, or others in place of them):
+    the signal is that of the new weights, here and in row 0 of the next run."""
+    shape, nc = (14, 11, 37), 2
+    mask = generators.porosity(shape, 0.3, 5, sigma=1.0)
+    rng = np.random.default_rng(6)
+    m0 = [rng.random(shape) - 0.3 for _ in range(nc)]
+    w = [rng.random(shape) for _ in range(4)]
+    outs = []
+    for rows in (False, True):
+        with _solver(shape, mask, m0, nc, rows) as s:
+            if before:
+                s.upload_phase_weights(w[0], w[1])
+            s.run(5)
+            if not rows:
+                s.set_layout(False) if leave == "layout" else s.set_tile(4 if leave == "tile" else -2)
+            s.upload_phase_weights(w[2], w[3])
+            outs.append([s.signal(), s.run(4), *s.download_magnetization()])
+    for a, b in zip(*outs):
+        np.testing.assert_allclose(a, b, rtol=1e-12, atol=1e-14)
+    for a, b in zip(outs[0][2:], outs[1][2:]):
+        np.testing.assert_array_equal(a, b)
+    f = outs[0][2:]
+    assert np.isfinite(f[0]).all() and outs[0][0].shape == (2 * nc,)
