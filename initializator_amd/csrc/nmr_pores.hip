@@ -440,45 +440,49 @@ __device__ __forceinline__ bool has_slot(const PoreBuild& b, int x, int y, int z
     return false;
 }
 
-// Slots per row (y, z): one wavefront a row.
+// Slots per row (y, z): one wavefront a row, rows in turn where there are more
+// than a launch may have threads for.
 __global__ void __launch_bounds__(kThreads) pore_count_kernel(PoreBuild b)
 {
-    const int64_t row = (int64_t)blockIdx.x * kWaves + (threadIdx.x >> 6);
-    if (row >= (int64_t)b.ny * b.nz) return;
+    const int64_t nrows = (int64_t)b.ny * b.nz;
     const int lane = threadIdx.x & 63;
-    const int y = (int)(row % b.ny), z = (int)(row / b.ny);
-    int n = 0;
-    for (int x0 = 0; x0 < b.nx; x0 += 64) {
-        const int x = x0 + lane;
-        n += __popcll(__ballot(x < b.nx && has_slot(b, x, y, z)));
+    for (int64_t row = (int64_t)blockIdx.x * kWaves + (threadIdx.x >> 6); row < nrows; row += (int64_t)gridDim.x * kWaves) {
+        const int y = (int)(row % b.ny), z = (int)(row / b.ny);
+        int n = 0;
+        for (int x0 = 0; x0 < b.nx; x0 += 64) {
+            const int x = x0 + lane;
+            n += __popcll(__ballot(x < b.nx && has_slot(b, x, y, z)));
+        }
+        if (lane == 0) b.rows[row] = (uint32_t)n;
     }
-    if (lane == 0) b.rows[row] = (uint32_t)n;
 }
 
 // rows[] of each plane -> exclusive prefix within the plane; planes[z] =
-// its slots rounded up to whole groups.  One workgroup a plane.
+// its slots rounded up to whole groups.  One workgroup a plane (planes in turn).
 __global__ void __launch_bounds__(kThreads) pore_plane_kernel(PoreBuild b)
 {
     __shared__ uint32_t sh[kThreads];
-    const int z = blockIdx.x, t = threadIdx.x;
-    uint32_t* r = b.rows + (size_t)z * b.ny;
-    uint32_t carry = 0;
-    for (int y0 = 0; y0 < b.ny; y0 += kThreads) {
-        const int y = y0 + t;
-        const uint32_t v = y < b.ny ? r[y] : 0u;
-        sh[t] = v;
-        __syncthreads();
-        for (int h = 1; h < kThreads; h <<= 1) {
-            const uint32_t u = t >= h ? sh[t - h] : 0u;
+    const int t = threadIdx.x;
+    for (int z = blockIdx.x; z < b.nz; z += (int)gridDim.x) {
+        uint32_t* r = b.rows + (size_t)z * b.ny;
+        uint32_t carry = 0;
+        for (int y0 = 0; y0 < b.ny; y0 += kThreads) {
+            const int y = y0 + t;
+            const uint32_t v = y < b.ny ? r[y] : 0u;
+            sh[t] = v;
             __syncthreads();
-            sh[t] += u;
+            for (int h = 1; h < kThreads; h <<= 1) {
+                const uint32_t u = t >= h ? sh[t - h] : 0u;
+                __syncthreads();
+                sh[t] += u;
+                __syncthreads();
+            }
+            if (y < b.ny) r[y] = carry + sh[t] - v;
+            carry += sh[kThreads - 1];
             __syncthreads();
         }
-        if (y < b.ny) r[y] = carry + sh[t] - v;
-        carry += sh[kThreads - 1];
-        __syncthreads();
+        if (t == 0) b.planes[z] = ((uint64_t)carry + 63u) & ~(uint64_t)63u;
     }
-    if (t == 0) b.planes[z] = ((uint64_t)carry + 63u) & ~(uint64_t)63u;
 }
 
 // planes[] -> exclusive prefix starting at `first`; planes[nz] = the end.
@@ -509,20 +513,21 @@ __global__ void __launch_bounds__(kThreads) pore_base_kernel(PoreBuild b)
 // Slot of every voxel (slotmap, 0: none) and voxel of every slot (vox).
 __global__ void __launch_bounds__(kThreads) pore_assign_kernel(PoreBuild b)
 {
-    const int64_t row = (int64_t)blockIdx.x * kWaves + (threadIdx.x >> 6);
-    if (row >= (int64_t)b.ny * b.nz) return;
+    const int64_t nrows = (int64_t)b.ny * b.nz;
     const int lane = threadIdx.x & 63;
-    const int y = (int)(row % b.ny), z = (int)(row / b.ny);
-    uint32_t s0 = (uint32_t)b.planes[z] + b.rows[row];
-    for (int x0 = 0; x0 < b.nx; x0 += 64) {
-        const int x = x0 + lane;
-        const bool in = x < b.nx && has_slot(b, x, y, z);
-        const uint64_t m = __ballot(in);
-        const uint32_t s = s0 + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
-        const size_t o = (size_t)row * (size_t)b.pitch + (size_t)x;
-        if (x < b.nx) b.slotmap[o] = in ? s : 0u;
-        if (in) b.vox[s] = (uint32_t)o;
-        s0 += (uint32_t)__popcll(m);
+    for (int64_t row = (int64_t)blockIdx.x * kWaves + (threadIdx.x >> 6); row < nrows; row += (int64_t)gridDim.x * kWaves) {
+        const int y = (int)(row % b.ny), z = (int)(row / b.ny);
+        uint32_t s0 = (uint32_t)b.planes[z] + b.rows[row];
+        for (int x0 = 0; x0 < b.nx; x0 += 64) {
+            const int x = x0 + lane;
+            const bool in = x < b.nx && has_slot(b, x, y, z);
+            const uint64_t m = __ballot(in);
+            const uint32_t s = s0 + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
+            const size_t o = (size_t)row * (size_t)b.pitch + (size_t)x;
+            if (x < b.nx) b.slotmap[o] = in ? s : 0u;
+            if (in) b.vox[s] = (uint32_t)o;
+            s0 += (uint32_t)__popcll(m);
+        }
     }
 }
 
@@ -701,19 +706,25 @@ hipError_t launch_pore_pulse(const PulseArgs& a, float* f, int nc, const uint32_
     return hipGetLastError();
 }
 
+// Workgroups that take a wavefront a row: a launch's threads number below 2^32,
+// and a grid within the 4 GiB of its arrays may have 2^28 rows.
+constexpr int64_t kMostGroups = (int64_t)1 << 22;
+static unsigned row_groups(const PoreBuild& b)
+{
+    return (unsigned)std::min(kMostGroups, ((int64_t)b.ny * b.nz + kWaves - 1) / kWaves);
+}
+
 hipError_t launch_pore_count(const PoreBuild& b, hipStream_t s)
 {
-    const int64_t nrows = (int64_t)b.ny * b.nz;
-    hipLaunchKernelGGL(pore_count_kernel, dim3((unsigned)((nrows + kWaves - 1) / kWaves)), dim3(kThreads), 0, s, b);
-    hipLaunchKernelGGL(pore_plane_kernel, dim3((unsigned)b.nz), dim3(kThreads), 0, s, b);
+    hipLaunchKernelGGL(pore_count_kernel, dim3(row_groups(b)), dim3(kThreads), 0, s, b);
+    hipLaunchKernelGGL(pore_plane_kernel, dim3((unsigned)std::min<int64_t>(kMostGroups, b.nz)), dim3(kThreads), 0, s, b);
     hipLaunchKernelGGL(pore_base_kernel, dim3(1), dim3(kThreads), 0, s, b);
     return hipGetLastError();
 }
 
 hipError_t launch_pore_link(const PoreBuild& b, hipStream_t s)
 {
-    const int64_t nrows = (int64_t)b.ny * b.nz;
-    hipLaunchKernelGGL(pore_assign_kernel, dim3((unsigned)((nrows + kWaves - 1) / kWaves)), dim3(kThreads), 0, s, b);
+    hipLaunchKernelGGL(pore_assign_kernel, dim3(row_groups(b)), dim3(kThreads), 0, s, b);
     if (b.count > 0)
         hipLaunchKernelGGL(pore_link_kernel, dim3((unsigned)((b.count + kWaves - 1) / kWaves)), dim3(kThreads), 0, s,
                            b);

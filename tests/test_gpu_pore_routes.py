@@ -47,3 +47,20 @@ def test_signal_after_weights_that_come_while_another_sweep_is_set(leave, before
         np.testing.assert_array_equal(a, b)
     f = outs[0][2:]
     assert np.isfinite(f[0]).all() and outs[0][0].shape == (2 * nc,)
+
+
+def test_a_grid_of_more_rows_than_a_launch_has_wavefronts_for():
+    """2^26 rows of one voxel and some more: a wavefront each would pass the
+    2^32 threads of a launch.  The steps equal those over the rows."""
+    shape = (8193, 8192, 1)
+    rng = np.random.default_rng(8)
+    mask = (rng.random(shape, dtype=np.float32) < 0.3).astype(np.uint8)
+    m0 = rng.random(shape)
+    outs = []
+    for rows in (False, True):
+        with _solver(shape, mask, [m0], 1, rows) as s:
+            sig = s.run(3)
+            outs.append((sig, s.download_magnetization()[0]))
+        print(f"[rows] {shape} rows={rows}", flush=True)
+    np.testing.assert_allclose(outs[0][0], outs[1][0], rtol=1e-12)
+    assert np.array_equal(outs[0][1], outs[1][1])
