@@ -769,18 +769,26 @@ bool pore_plain(const nmr_ctx* c)
            !c->weighted && !((p.flags & NMR_F_ADVECT_MASK) && c->vel);
 }
 
-// Whether the list beats the tiles: where at most 0.6 of the voxels are pores,
-// or the list's data (the state's two buffers, the predictor, the velocity
-// sums, offsets and descriptors) stay well inside the memory-side cache.
-// Measured per step, list against tiles on bricks: 256^3 flow, two components,
-// porosity 0.2 / 0.35 / 0.5 / 0.65 / 0.8 / 1: 19.9 / 31.2 / 61.2 / 81.9 / 101 /
-// 124 against 57.9 / 66.2 / 74.1 / 80.1 / 84.0 / 84.2 us; 256^3, one component
-// without flow, 0.5 / 0.8 (188 MB) / 1: 29.3 / 41.0 / 47.8 against 36.4 / 39.0 /
-// 39.2; 160^3 MacCormack, 1 (172 MB): 47.9 against 54.1; 512x512x256, 1: 511
-// against 388; 64^3, one component, 1: 2.9 against 9.4.
-bool pores_pay(double slots, double voxels, int state_words, bool vel)
+// What of the problem the choice between the list and the tiles looks at.
+nmri::PoreProblem pore_problem(const nmr_ctx* c)
 {
-    return slots <= 0.6 * voxels || 4.0 * (state_words + (vel ? 3 : 0) + 1.5) * slots <= 180e6;
+    const nmr_problem& p = c->prob;
+    nmri::PoreProblem q{};
+    q.voxels = (double)p.nx * p.ny * p.nz;
+    q.padded = nmri::pores_padded(p.nx, p.ny, p.nz);
+    q.nc = c->nc;
+    q.vel = c->vel;
+    q.mak = p.scheme == NMR_SCHEME_MACCORMACK;
+    q.ghost_x = p.bc[0] != NMR_BC_NEUMANN;
+    for (int a = 0; a < 3; a++) {
+        q.zeros = q.zeros || p.bc[a] == NMR_BC_DIRICHLET;
+        if (a > 0 && p.bc[a] == NMR_BC_PERIODIC) q.wraps++;
+    }
+    q.coef = c->hetero;
+    q.field = c->bn != nullptr;
+    q.weights = c->weighted;
+    q.solids = c->pl_reads_solids;
+    return q;
 }
 
 // Builds the list for the current mask and velocity.
@@ -789,7 +797,7 @@ int build_pores(nmr_ctx* c)
     const nmr_problem& p = c->prob;
     c->pl_tried = true;
     c->pl_ok = c->pl_vel_ok = c->pl_pv_ok = false;
-    c->pl_reads_solids = false;
+    c->pl_reads_solids = c->pl_unpaid = false;
     if (c->nc == 3 && (p.nx > 65536 || p.ny > 65536)) return NMR_OK; // positions are 16 + 16 bits
     int rc = refresh_inert(c);
     if (rc) return rc;
@@ -817,13 +825,14 @@ int build_pores(nmr_ctx* c)
     HIP_TRY(nmr::launch_pore_count(b, c->stream));
     HIP_TRY(hipMemcpyAsync(&end, b.planes + p.nz, sizeof(end), hipMemcpyDeviceToHost, c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));
-    if (!nmri::pores_fit(end, c->vel) ||
-        !pores_pay((double)end, (double)p.nx * p.ny * p.nz, (p.scheme == NMR_SCHEME_MACCORMACK ? 3 : 2) * c->nc, c->vel))
-        return NMR_OK;
+    c->pl_reads_solids = b.read_solids != 0;
+    c->pl_slots = end;
+    if (!nmri::pores_fit(end, c->vel)) return NMR_OK;
+    c->pl_unpaid = !nmri::pores_pay((double)end, pore_problem(c));
+    if (c->pl_unpaid) return NMR_OK;
     const nmri::PoreNeeds n{c->nc, c->vel, ghosts || b.read_solids, p.bc[0] != NMR_BC_NEUMANN,
                             p.scheme == NMR_SCHEME_MACCORMACK};
     if ((rc = nmri::pores_alloc(&c->pl, (uint32_t)end, n, c->stream, &c->device_bytes))) return rc;
-    c->pl_reads_solids = b.read_solids != 0;
     if (pore_plain(c) && !b.read_solids && p.scheme == NMR_SCHEME_UPWIND &&
         (rc = nmri::pores_blocks(&c->pl, &b, c->stream, &c->device_bytes)))
         return rc;
@@ -850,8 +859,9 @@ int check_solids(nmr_ctx* c)
 }
 
 // Whether the next run sweeps the list: the automatic tile, the layout
-// switch on, finite solids, and a list that fits.  Builds it when needed
-// (never under the no-allocation entry point: the uploads have).
+// switch on, finite solids, and a list that fits and pays (per-voxel data may
+// have come since it was built).  Builds it when needed (never under the
+// no-allocation entry point: the uploads have).
 int use_pores(nmr_ctx* c, bool* yes)
 {
     *yes = false;
@@ -862,7 +872,7 @@ int use_pores(nmr_ctx* c, bool* yes)
         if ((c->home & nmri::kHomePores) && (rc = drop_pores(c))) return rc;
         if ((rc = build_pores(c))) return rc;
     }
-    if (!c->pl_ok) return NMR_OK;
+    if (!c->pl_ok || !nmri::pores_pay((double)c->pl_slots, pore_problem(c))) return NMR_OK;
     if (!c->solids_tried) {
         if ((rc = nmri::state_rows(c)) || (rc = check_solids(c))) return rc;
     }
@@ -1491,6 +1501,7 @@ int nmr_hip_upload_field(nmr_ctx* ctx, const double* b, int32_t layout)
         if (ctx->bn) (void)hipFree(ctx->bn);
         ctx->bn = nullptr;
         ctx->bnax = -1;
+        if (ctx->pl_unpaid) ctx->pl_tried = false; // (the list may pay without it)
         return NMR_OK;
     }
     if (ctx->exact) return fail(NMR_ERR_UNSUPPORTED, "per-voxel fields use the linear phase");
@@ -2140,7 +2151,9 @@ int build_batch_pores(nmr_batch* b)
     b->pl_ok = b->pl_reads_solids = false;
     const nmr_problem& p = b->prob;
     size_t rows = 0, planes = 0, voxels = 0;
-    double grid = 0.0;
+    nmri::PoreProblem q{};
+    q.nc = b->nc;
+    q.vel = b->vel;
     for (int i = 0; i < b->ninst; i++) {
         const nmr_batch_instance& s = b->spec[i];
         const auto& I = b->inst[i];
@@ -2148,7 +2161,8 @@ int build_batch_pores(nmr_batch* b)
         rows = std::max(rows, (size_t)s.ny * s.nz);
         planes = std::max(planes, (size_t)s.nz);
         voxels = std::max(voxels, I.n_m);
-        grid += (double)s.nx * s.ny * s.nz;
+        q.voxels += (double)s.nx * s.ny * s.nz;
+        q.padded += nmri::pores_padded(s.nx, s.ny, s.nz);
         b->pl_reads_solids = b->pl_reads_solids || (b->vel && !I.inert);
     }
     nmr::PoreBuild t{};
@@ -2190,7 +2204,8 @@ int build_batch_pores(nmr_batch* b)
     HIP_TRY(hipStreamSynchronize(b->stream));
     uint64_t end = 64;
     for (uint64_t v : n) end += v;
-    if (!nmri::pores_fit(end, b->vel) || !pores_pay((double)end, grid, 2 * b->nc, b->vel)) return NMR_OK;
+    q.solids = b->pl_reads_solids;
+    if (!nmri::pores_fit(end, b->vel) || !nmri::pores_pay((double)end, q)) return NMR_OK;
     int64_t bytes = 0;
     const nmri::PoreNeeds needs{b->nc, b->vel, b->pl_reads_solids, false, false};
     if ((rc = nmri::pores_alloc(&b->pl, (uint32_t)end, needs, b->stream, &bytes))) return rc;

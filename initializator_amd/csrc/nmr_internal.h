@@ -121,6 +121,20 @@ int pores_per_tile(int64_t groups);
 // offsets: slot * size of its widest array, the records with velocity, else
 // three components.
 bool pores_fit(uint64_t nslots, bool vel);
+// What the choice between the list and the tiles looks at.
+struct PoreProblem {
+    double voxels, padded;  // of the grid, and of the tiles that cover it
+    int nc;
+    int wraps;              // periodic y and z axes
+    bool vel, mak;          // velocity, MacCormack
+    bool ghost_x, zeros;    // x ghosts other than zero-derivative ones; ghosts that read as 0
+    bool coef, field, weights; // per-voxel coefficients, field, phase weights
+    bool solids;            // solids that pores read have slots
+};
+// Voxels of the 64 x 16 tiles that cover a grid.
+double pores_padded(int nx, int ny, int nz);
+// Whether a list of so many slots beats the tiles.
+bool pores_pay(double slots, const PoreProblem& p);
 
 } // namespace nmri
 
@@ -177,6 +191,8 @@ struct nmr_ctx {
     // found not to fit, for the current mask and velocity.
     nmri::PoreList pl;
     bool pl_tried = false, pl_ok = false;
+    bool pl_unpaid = false;   // it fits, but the tiles beat it
+    uint64_t pl_slots = 0;
     bool pl_reads_solids = false; // solids next to pores have slots
     bool pl_vel_ok = false, pl_pv_ok = false; // velocity sums and per-voxel arrays gathered
     bool pl_zeroed = false;   // a MacCormack step ran on the list: solids hold 0

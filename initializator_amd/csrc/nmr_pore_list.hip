@@ -33,6 +33,49 @@ bool pores_fit(uint64_t nslots, bool vel)
     return nslots > 64 && (nslots + 64) * (vel ? rec : state) < ((uint64_t)1 << 32) - 256;
 }
 
+double pores_padded(int nx, int ny, int nz)
+{
+    return (((int64_t)nx + 63) / 64 * 64) * (double)(((int64_t)ny + 15) / 16 * 16) * nz;
+}
+
+bool pores_pay(double slots, const PoreProblem& p)
+{
+    // The plain problem: where at most 0.6 of the voxels are pores, or the
+    // list's data stay well inside the memory-side cache.  Measured per step,
+    // list against tiles on bricks: 256^3 flow, two components, porosity 0.2 /
+    // 0.35 / 0.5 / 0.65 / 0.8 / 1: 19.9 / 31.2 / 61.2 / 81.9 / 101 / 124 against
+    // 57.9 / 66.2 / 74.1 / 80.1 / 84.0 / 84.2 us; 256^3, one component without
+    // flow, 0.5 / 0.8 (188 MB) / 1: 29.3 / 41.0 / 47.8 against 36.4 / 39.0 / 39.2;
+    // 160^3 MacCormack, 1 (172 MB): 47.9 against 54.1; 512x512x256, 1: 511
+    // against 388; 64^3, one component, 1: 2.9 against 9.4.
+    if (slots > 0.6 * p.voxels && 4.0 * ((p.mak ? 3 : 2) * p.nc + (p.vel ? 3 : 0) + 1.5) * slots > 180e6) return false;
+    // Ghosts, per-voxel data and solids that are read cost the list, which
+    // loads offsets and masks for them, more than the tiles, and the less the
+    // more components share them.  So the voxels that the tiles work on (whole
+    // 64 x 16 tiles) are compared with the slots weighed by what they load more;
+    // the factors are fitted to 36 kinds of problem on 128^3 to 320^3 at
+    // porosities 0.3 to 1.  Time of a step on tiles over that on the list: one
+    // component, zero-value ghosts, 200^3, porosity 0.4 / 0.6 / 1: 1.14 / 0.87 /
+    // 0.58; periodic, 256^3, 0.3 / 0.5 / 0.7: 1.28 / 0.90 / 0.65; two components
+    // with flow, periodic, 200^3, 0.8 / 1: 1.32 / 0.82; MacCormack, periodic,
+    // per-voxel coefficients and weights, 160^3, 0.6 / 0.8 / 1: 1.13 / 0.87 / 0.71.
+    // (On seven other grids, 612 problems, the choice costs more than 5 % in
+    // five, 14 % at most.)
+    const bool ghosts = p.ghost_x || p.zeros || p.wraps > 0;
+    const double more = (p.ghost_x ? 0.6 : 0.0) + (p.zeros ? 0.55 : 0.0) + 0.15 * p.wraps +
+                        (p.coef && ghosts ? 0.5 : 0.0) + (p.weights ? 0.12 : 0.0) + (p.solids ? 0.17 : 0.0);
+    // words a slot: state (predictor), record or offsets, descriptor, lane
+    // masks, x and 16-bit offsets, positions, per-voxel data
+    const double words = (p.mak ? 3 : 2) * p.nc + (p.vel ? 4 : 1) + 0.5 +
+                         (p.zeros || p.solids || (p.coef && ghosts) ? 0.56 : 0.0) + (p.ghost_x ? 1 : 0) +
+                         (p.wraps > 0 ? 2 : 0) + (p.nc == 3 ? 1 : 0) + (p.coef ? 2 + (p.nc == 3) : 0) + (p.field ? 1 : 0) +
+                         (p.weights ? 2 : 0);
+    static const double in_cache[3] = {0.85, 1.05, 1.25}, past[3] = {0.65, 0.75, 1.0}; // by components
+    double most = 4.0 * words * slots <= 225e6 ? in_cache[p.nc - 1] : past[p.nc - 1];
+    if (p.voxels <= 2.2e6) most *= 2.0; // (up to 128^3: the tiles do not fill the chip; 128^3 all pores 0.9-1.5)
+    return slots * (1.0 + more / (p.nc * p.nc)) <= most * p.padded;
+}
+
 int pores_alloc(PoreList* L, uint32_t nslots, const PoreNeeds& n, hipStream_t s, int64_t* bytes)
 {
     const bool more = nslots > L->cap || n.nc != L->nc;

@@ -1,10 +1,12 @@
 """Calls that change which sweep the next run takes while the state lives in the
 list of the pores: what they return equals a solver that never leaves the rows."""
+import ctypes
+
 import numpy as np
 import pytest
 
 from initializator_amd import generators
-from initializator_amd.solver import HipSolver
+from initializator_amd.solver import HipSolver, check
 
 pytestmark = pytest.mark.gpu
 
@@ -64,3 +66,36 @@ def test_a_grid_of_more_rows_than_a_launch_has_wavefronts_for():
         print(f"[rows] {shape} rows={rows}", flush=True)
     np.testing.assert_allclose(outs[0][0], outs[1][0], rtol=1e-12)
     assert np.array_equal(outs[0][1], outs[1][1])
+
+
+def _us(s, steps):
+    """Device time of a step, the least of three runs."""
+    ms, n, best = ctypes.c_double(), ctypes.c_int64(), 1e30
+    s.run(steps)
+    for _ in range(3):
+        s.run(steps)
+        check(s.lib.nmr_hip_last_run_ms(s.ctx, ctypes.byref(ms), ctypes.byref(n)), "nmr_hip_last_run_ms")
+        best = min(best, ms.value / steps * 1e3)
+    return best
+
+
+# Measured, tiles over list: 0.58, 0.71, 0.71, 1.85 and 1.88.
+@pytest.mark.parametrize("n,phi,nc,bc,scheme,data,at_most", [
+    (200, 1.0, 1, (2, 2, 2), 0, False, 1.15), (200, 1.0, 1, (1, 1, 1), 0, False, 1.15),
+    (160, 1.0, 2, (1, 1, 1), 1, True, 1.15), (160, 0.4, 2, (1, 1, 1), 0, False, 0.75),
+    (160, 0.4, 1, (0, 0, 0), 0, False, 0.75)])
+def test_the_automatic_sweep_is_the_faster_one(n, phi, nc, bc, scheme, data, at_most):
+    """The automatic choice against the tiles: no slower where ghosts and
+    per-voxel data (uploaded last) make the list dearer, and the list where it
+    is faster by far."""
+    shape = (n, n, n)
+    mask = generators.porosity(shape, phi, 3, sigma=2.0) if phi < 1 else np.ones(shape, np.uint8)
+    with _solver(shape, mask, [mask.astype(float)] * 3, nc, bc=bc, scheme=scheme) as s:
+        if data:
+            s.upload_coefficients(np.full(shape, D), np.full(shape, 0.5), np.full(shape, 0.4))
+            s.upload_phase_weights(0.5 * mask, 0.5 * mask)
+        auto = _us(s, 40)
+        s.set_tile(4)
+        tile = _us(s, 40)
+    print(f"[choice] {n} {phi} nc {nc} bc {bc}: automatic {auto:.1f}, tiles {tile:.1f} us a step", flush=True)
+    assert auto <= at_most * tile
