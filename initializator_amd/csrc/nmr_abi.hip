@@ -119,7 +119,7 @@ void free_all(nmr_ctx* c)
             if (c->mb[b][q]) (void)hipFree(c->mb[b][q]);
     for (int q = 0; q < 3; q++)
         if (c->pb[q]) (void)hipFree(c->pb[q]);
-    nmri::pores_free(&c->pl);
+    nmri::pores_free(&c->pl, &c->device_bytes);
     if (c->mask) (void)hipFree(c->mask);
     if (c->vx) (void)hipFree(c->vx);
     if (c->vy) (void)hipFree(c->vy);
@@ -791,16 +791,22 @@ nmri::PoreProblem pore_problem(const nmr_ctx* c)
     return q;
 }
 
-// Builds the list for the current mask and velocity.
+// Whether solids next to pores get slots: an upwind flow reads them.
+bool pores_read_solids(const nmr_ctx* c)
+{
+    return c->prob.scheme == NMR_SCHEME_UPWIND && c->vel && !c->inert && !(c->prob.flags & NMR_F_ADVECT_MASK);
+}
+
+// Builds the list for the current mask and velocity, and finds whether the
+// solids are finite.
 int build_pores(nmr_ctx* c)
 {
     const nmr_problem& p = c->prob;
     c->pl_tried = true;
     c->pl_ok = c->pl_vel_ok = c->pl_pv_ok = false;
-    c->pl_reads_solids = c->pl_unpaid = false;
+    c->pl_unpaid = false;
+    c->pl_reads_solids = pores_read_solids(c);
     if (c->nc == 3 && (p.nx > 65536 || p.ny > 65536)) return NMR_OK; // positions are 16 + 16 bits
-    int rc = refresh_inert(c);
-    if (rc) return rc;
     nmr::PoreBuild b{};
     b.mask = c->mask;
     b.nx = p.nx;
@@ -812,34 +818,51 @@ int build_pores(nmr_ctx* c)
         b.bc[q] = p.bc[q];
         ghosts = ghosts || p.bc[q] != NMR_BC_NEUMANN;
     }
-    b.read_solids = p.scheme == NMR_SCHEME_UPWIND && c->vel && !c->inert && !(p.flags & NMR_F_ADVECT_MASK);
+    b.read_solids = c->pl_reads_solids;
     signal_window(p, b.w);
     b.first = 64;
+    if (pore_plain(c) && !b.read_solids && p.scheme == NMR_SCHEME_UPWIND) nmri::pores_boxes(&b);
     const size_t rows = (size_t)p.ny * p.nz;
-    if ((rc = nmri::pores_temp(&b, rows, (size_t)p.nz, rows * c->pitch, c->stream))) return rc;
+    int rc = nmri::pores_temp(&b, rows, (size_t)p.nz, rows * c->pitch, c->stream);
+    if (rc) return rc;
     struct Temp {
         nmr::PoreBuild* b;
         ~Temp() { nmri::pores_drop_temp(b); }
     } temp{&b};
-    uint64_t end = 0;
+    struct Counted {
+        uint64_t end;
+        nmri::PoreFound found;
+    };
+    // (through the signal's pinned staging: no copy into pageable memory)
+    if ((rc = ensure_host_signal(c, (size_t)(kChunkSteps + 1) * c->nsig()))) return rc;
+    Counted& h = *reinterpret_cast<Counted*>(c->hsignal);
     HIP_TRY(nmr::launch_pore_count(b, c->stream));
-    HIP_TRY(hipMemcpyAsync(&end, b.planes + p.nz, sizeof(end), hipMemcpyDeviceToHost, c->stream));
+    if (b.nbx) HIP_TRY(nmr::launch_block_count(b, c->stream));
+    HIP_TRY(hipMemcpyAsync(&h, b.planes + p.nz, sizeof(h), hipMemcpyDeviceToHost, c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));
-    c->pl_reads_solids = b.read_solids != 0;
+    const uint64_t end = h.end;
     c->pl_slots = end;
     if (!nmri::pores_fit(end, c->vel)) return NMR_OK;
     c->pl_unpaid = !nmri::pores_pay((double)end, pore_problem(c));
     if (c->pl_unpaid) return NMR_OK;
     const nmri::PoreNeeds n{c->nc, c->vel, ghosts || b.read_solids, p.bc[0] != NMR_BC_NEUMANN,
-                            p.scheme == NMR_SCHEME_MACCORMACK};
+                            p.scheme == NMR_SCHEME_MACCORMACK, b.nbx * b.nby * b.nbz, h.found.block_slots};
     if ((rc = nmri::pores_alloc(&c->pl, (uint32_t)end, n, c->stream, &c->device_bytes))) return rc;
-    if (pore_plain(c) && !b.read_solids && p.scheme == NMR_SCHEME_UPWIND &&
-        (rc = nmri::pores_blocks(&c->pl, &b, c->stream, &c->device_bytes)))
-        return rc;
     nmri::pores_into(c->pl, &b, end);
     HIP_TRY(nmr::launch_pore_link(b, c->stream));
     if (b.blocks) HIP_TRY(nmr::launch_block_build(b, c->stream));
-    return nmri::pores_finish(&c->pl, b, c->stream, &c->pl_ok);
+    if (!c->solids_tried) {
+        if ((rc = nmri::state_rows(c))) return rc;
+        for (int q = 0; q < c->nc; q++)
+            HIP_TRY(nmr::launch_solids_finite(c->m[c->cur][q], c->mask, c->n_m, b.found + 3, c->stream));
+    }
+    if ((rc = nmri::pores_finish(&c->pl, b, c->stream, &h.found))) return rc;
+    c->pl_ok = !h.found.overflow;
+    if (!c->solids_tried) {
+        c->solids_ok = !h.found.solids;
+        c->solids_tried = true;
+    }
+    return NMR_OK;
 }
 
 // Whether the solids' magnetization is finite: their value reaches no pore
@@ -866,10 +889,10 @@ int use_pores(nmr_ctx* c, bool* yes)
 {
     *yes = false;
     if (!c->brick_on || c->variant != -1 || !c->has_mask || !c->has_mag) return NMR_OK;
-    int rc = NMR_OK;
+    int rc = refresh_inert(c);
+    if (rc) return rc;
     if (!c->pl_tried) {
         if (c->no_alloc) return NMR_OK;
-        if ((c->home & nmri::kHomePores) && (rc = drop_pores(c))) return rc;
         if ((rc = build_pores(c))) return rc;
     }
     if (!c->pl_ok || !nmri::pores_pay((double)c->pl_slots, pore_problem(c))) return NMR_OK;
@@ -2014,7 +2037,8 @@ void batch_free(nmr_batch* b)
         if (I.vy) (void)hipFree(I.vy);
         if (I.vz) (void)hipFree(I.vz);
     }
-    nmri::pores_free(&b->pl);
+    int64_t bytes = 0;
+    nmri::pores_free(&b->pl, &bytes);
     for (void* p : {(void*)b->d_pinst, (void*)b->d_ptiles, (void*)b->d_poff, (void*)b->d_inst, (void*)b->d_tiles, (void*)b->d_off, (void*)b->d_ids, (void*)b->d_step,
                     (void*)b->d_part, (void*)b->d_signal, (void*)b->d_fpart, (void*)b->d_flag})
         if (p) (void)hipFree(p);
@@ -2236,8 +2260,8 @@ int build_batch_pores(nmr_batch* b)
         t.first += n[i];
     }
     if (b->vel) HIP_TRY(nmr::launch_pore_record(b->pl.off8, b->pl.nslots, b->pl.rec, b->stream));
-    bool ok = false;
-    if ((rc = nmri::pores_finish(&b->pl, t, b->stream, &ok)) || !ok) return rc;
+    nmri::PoreFound found{};
+    if ((rc = nmri::pores_finish(&b->pl, t, b->stream, &found)) || found.overflow) return rc;
     for (void** q : {(void**)&b->d_pinst, (void**)&b->d_ptiles, (void**)&b->d_poff}) {
         if (*q) HIP_TRY(hipFree(*q));
         *q = nullptr;

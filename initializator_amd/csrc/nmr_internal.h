@@ -69,11 +69,12 @@ struct HostStage {
 };
 
 // A list of the pores of one domain or of all instances of a batch
-// (nmr_pores.hip), its state and its per-slot data, in device memory.
+// (nmr_pores.hip), its state and its per-slot data, in device memory: one
+// allocation, but for the per-voxel arrays.
 struct PoreList {
     uint32_t nslots = 0;  // slots in use, the empty group 0 among them
-    size_t cap = 0;       // slots allocated
-    int nc = 0;
+    char* mem = nullptr;  // what the arrays below lie in
+    size_t mem_bytes = 0;
     bool wide = false;    // some group needs its 16-bit offsets
     nmr::PoreGroup* groups = nullptr;
     nmr::PoreAux* aux = nullptr;
@@ -83,11 +84,11 @@ struct PoreList {
     float* pred = nullptr;
     uint4* rec = nullptr; // offsets and velocity sums (with velocity)
     float* pv[6] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr}; // dn, r1v, r2v, bn, w[0], w[1]
+    size_t cap = 0;       // slots of those of them that are there
     // boxes that take several steps a launch (nmr_pore_blocks.hip), where the
     // list is small and they fit
     nmr::u32x4* blocks = nullptr;
     uint32_t* bcount = nullptr;
-    size_t bcap = 0, ncap = 0; // slots of blocks, and boxes, allocated
     int nbx = 0, nby = 0, nbz = 0;
     bool blocks_ok = false;
     int nblocks() const { return nbx * nby * nbz; }
@@ -97,12 +98,18 @@ struct PoreList {
 struct PoreNeeds {
     int nc;
     bool vel, aux, xoff, pred;
+    int boxes = 0, block_slots = 0;
 };
-// Buffers for `nslots` slots, grown where they are too small or missing;
-// everything in them is cleared (the voxel numbers set to "empty").  The
-// per-voxel arrays pv are made by who gathers them; they go when the list grows.
+// What the building kernels find: an offset that does not fit, a group that
+// needs 16-bit offsets, slots of all blocks, a solid that is not finite.
+struct PoreFound {
+    int overflow, wide, block_slots, solids;
+};
+// Memory for `nslots` slots, grown where it is too small; everything in it is
+// cleared (the voxel numbers set to "empty").  The per-voxel arrays pv are made
+// by who gathers them; they go when the list outgrows them.
 int pores_alloc(PoreList* L, uint32_t nslots, const PoreNeeds& n, hipStream_t s, int64_t* bytes);
-void pores_free(PoreList* L);
+void pores_free(PoreList* L, int64_t* bytes);
 // Building: temporary arrays for domains of up to `rows` rows, `planes` planes
 // and `voxels` voxels (row layout); per domain, with first set,
 // launch_pore_count (planes[nz] is then the slot past its last one) and, with
@@ -110,11 +117,11 @@ void pores_free(PoreList* L);
 int pores_temp(nmr::PoreBuild* b, size_t rows, size_t planes, size_t voxels, hipStream_t s);
 void pores_drop_temp(nmr::PoreBuild* b);
 void pores_into(const PoreList& L, nmr::PoreBuild* b, uint64_t end);
-// Counts the boxes' pores of the domain b and makes their buffers, where the
-// list is small enough for them; launch_block_build then fills them.
-int pores_blocks(PoreList* L, nmr::PoreBuild* b, hipStream_t s, int64_t* bytes);
-// Waits for the stream; notes wide groups in the list; *ok: every offset fits.
-int pores_finish(PoreList* L, const nmr::PoreBuild& b, hipStream_t s, bool* ok);
+// Gives the domain b its boxes, where the grid is small enough for them:
+// launch_block_count counts their pores, launch_block_build fills them.
+void pores_boxes(nmr::PoreBuild* b);
+// Waits for the stream; notes wide groups and the boxes in the list.
+int pores_finish(PoreList* L, const nmr::PoreBuild& b, hipStream_t s, PoreFound* found);
 // Groups that a workgroup takes of a list of `groups`.
 int pores_per_tile(int64_t groups);
 // Whether a list of this many slots stays inside the kernels' 32-bit byte

@@ -261,10 +261,12 @@ struct PoreBuild {
     uint2* off16;
     uint32_t* xoff;         // or null
     uint32_t* xy;           // or null
-    int* overflow;          // [0] set when an offset does not fit, [1] when a group needs 16-bit offsets,
-                            // [2] slots of all blocks
+    int* found;             // what is found on the way: [0] an offset that does not fit, [1] a group that needs
+                            // 16-bit offsets, [2] slots of all blocks, [3] a solid that is not finite
+    void* temp;             // what rows, planes, slotmap, bcount and found lie in
     u32x4* blocks;          // the blocks' slots, or null
     uint32_t* bcount;       // [nblocks][8]: slots within 0 .. kBlockSteps faces of the box, the first one's place
+    uint32_t* bcount_to;    // the same in the list
     int nbx, nby, nbz;      // boxes per axis
 };
 

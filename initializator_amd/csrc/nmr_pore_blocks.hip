@@ -75,13 +75,13 @@ struct Box {
 };
 
 // Pores by distance, and a place for them.
-__global__ void __launch_bounds__(256) block_count_kernel(PoreBuild b)
+__global__ void __launch_bounds__(kThreads) block_count_kernel(PoreBuild b)
 {
     __shared__ uint32_t n[kBlockSteps + 1];
     const Box box(blockIdx.x, b.nbx, b.nby);
     if (threadIdx.x <= kBlockSteps) n[threadIdx.x] = 0;
     __syncthreads();
-    for (int c = threadIdx.x; c < kExt * kExt * kExt; c += 256) {
+    for (int c = threadIdx.x; c < kExt * kExt * kExt; c += kThreads) {
         int x, y, z;
         size_t o;
         const int d = away(c & 15) + away((c >> 4) & 15) + away(c >> 8);
@@ -92,45 +92,70 @@ __global__ void __launch_bounds__(256) block_count_kernel(PoreBuild b)
         uint32_t* out = b.bcount + (size_t)blockIdx.x * 8;
         uint32_t sum = 0;
         for (int d = 0; d <= kBlockSteps; d++) out[d] = sum += n[d];
-        out[kBlockSteps + 1] = (uint32_t)atomicAdd(&b.overflow[2], (int)sum);
+        out[kBlockSteps + 1] = (uint32_t)atomicAdd(&b.found[2], (int)sum);
     }
 }
 
-__global__ void __launch_bounds__(256) block_build_kernel(PoreBuild b)
+// The slots of a block, by distance and then by position.  Built with every
+// mask upload, so its barriers count: one pass over the surroundings finds the
+// pores of all distances (64^3: 14 us; a pass a distance, with two barriers for
+// every 256 voxels: 52).
+__global__ void __launch_bounds__(kThreads) block_build_kernel(PoreBuild b)
 {
-    __shared__ uint16_t at[kExt * kExt * kExt]; // slot in the block of a voxel
-    __shared__ uint32_t wsum[4];
+    constexpr int kVox = kExt * kExt * kExt, kRuns = kVox / 64; // runs of 64 voxels: a wavefront's
+    constexpr uint16_t kNone = 0xffffu;
+    __shared__ uint16_t at[kVox];                    // slot in the block of a voxel
+    __shared__ uint32_t runs[(kBlockSteps + 1) * kRuns]; // pores of a run at a distance, then the slots before them
+    static_assert(kVox % kThreads == 0 && kRuns == 64 && kThreads >= 64 * (kBlockSteps + 1));
+    constexpr int kEach = kVox / kThreads;
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const Box box(blockIdx.x, b.nbx, b.nby);
-    u32x4* out = b.blocks + b.bcount[(size_t)blockIdx.x * 8 + kBlockSteps + 1];
-    uint32_t n = 0;
-    for (int d = 0; d <= kBlockSteps; d++) {
-        for (int c0 = 0; c0 < kExt * kExt * kExt; c0 += 256) {
-            const int c = c0 + t;
-            int x, y, z;
-            size_t o;
-            const bool in = away(c & 15) + away((c >> 4) & 15) + away(c >> 8) == d && box.voxel(b, c, x, y, z, o);
-            const uint64_t m = __ballot(in);
-            if (lane == 0) wsum[wave] = (uint32_t)__popcll(m);
-            __syncthreads();
-            uint32_t before = n + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
-            for (int w = 0; w < 4; w++) {
-                if (w < wave) before += wsum[w];
-                n += wsum[w];
-            }
-            if (in) at[c] = (uint16_t)before;
-            __syncthreads();
-        }
-    }
-    for (int c = t; c < kExt * kExt * kExt; c += 256) {
-        const int lx = c & 15, ly = (c >> 4) & 15, lz = c >> 8;
-        const int d = away(lx) + away(ly) + away(lz);
+    const uint32_t* cnt = b.bcount + (size_t)blockIdx.x * 8;
+    u32x4* out = b.blocks + cnt[kBlockSteps + 1];
+    if (t < 8) b.bcount_to[(size_t)blockIdx.x * 8 + t] = cnt[t];
+    int dist[kEach];
+    uint32_t lower[kEach]; // pores of its distance before a voxel in its run
+#pragma unroll
+    for (int k = 0; k < kEach; k++) {
+        const int c = t + k * kThreads;
         int x, y, z;
         size_t o;
-        if (d > kBlockSteps || !box.voxel(b, c, x, y, z, o)) continue;
+        const int d = away(c & 15) + away((c >> 4) & 15) + away(c >> 8);
+        dist[k] = d <= kBlockSteps && box.voxel(b, c, x, y, z, o) ? d : -1;
+        lower[k] = 0;
+        for (int q = 0; q <= kBlockSteps; q++) {
+            const uint64_t m = __ballot(dist[k] == q);
+            if (dist[k] == q) lower[k] = (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
+            if (lane == 0) runs[q * kRuns + k * kWaves + wave] = (uint32_t)__popcll(m);
+        }
+    }
+    __syncthreads();
+    if (wave <= kBlockSteps) { // a wavefront takes the runs of a distance
+        const uint32_t own = runs[t];
+        uint32_t sum = own;
+        for (int h = 1; h < 64; h <<= 1) {
+            const uint32_t u = (uint32_t)__shfl_up((int)sum, h, 64);
+            if (lane >= h) sum += u;
+        }
+        runs[t] = sum - own + (wave > 0 ? cnt[wave - 1] : 0u);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kEach; k++)
+        at[t + k * kThreads] =
+            dist[k] < 0 ? kNone : (uint16_t)(runs[dist[k] * kRuns + k * kWaves + wave] + lower[k]);
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kEach; k++) {
+        const int c = t + k * kThreads, d = dist[k];
+        if (d < 0) continue;
+        const int lx = c & 15, ly = (c >> 4) & 15, lz = c >> 8;
+        const int x = box.x0 + lx, y = box.y0 + ly, z = box.z0 + lz;
+        const size_t o = ((size_t)z * b.ny + y) * b.pitch + x;
         const uint32_t own = at[c];
         const int p[3] = {x, y, z}, size[3] = {b.nx, b.ny, b.nz}, step[3] = {1, 16, 256};
         uint32_t w[6];
+#pragma unroll
         for (int s = 0; s < 6; s++) {
             const int ax = s >> 1, up = s & 1;
             w[s] = own;
@@ -139,10 +164,8 @@ __global__ void __launch_bounds__(256) block_build_kernel(PoreBuild b)
                 w[s] = own | 0x8000u;
                 continue;
             }
-            const int nc = up ? c + step[ax] : c - step[ax];
-            int u, v, q;
-            size_t no;
-            if (box.voxel(b, nc, u, v, q, no)) w[s] = at[nc] | 0x8000u;
+            const uint16_t nb = at[up ? c + step[ax] : c - step[ax]]; // (at most one face further)
+            if (nb != kNone) w[s] = nb | 0x8000u;
         }
         const bool win = x >= b.w[0] && x < b.w[1] && y >= b.w[2] && y < b.w[3] && z >= b.w[4] && z < b.w[5];
         w[0] |= (uint32_t)(lz & 7) << 12;
@@ -326,13 +349,13 @@ __global__ void __launch_bounds__(kThreads) block_kernel(BlockArgs a)
 
 hipError_t launch_block_count(const PoreBuild& b, hipStream_t s)
 {
-    hipLaunchKernelGGL(block_count_kernel, dim3((unsigned)(b.nbx * b.nby * b.nbz)), dim3(256), 0, s, b);
+    hipLaunchKernelGGL(block_count_kernel, dim3((unsigned)(b.nbx * b.nby * b.nbz)), dim3(kThreads), 0, s, b);
     return hipGetLastError();
 }
 
 hipError_t launch_block_build(const PoreBuild& b, hipStream_t s)
 {
-    hipLaunchKernelGGL(block_build_kernel, dim3((unsigned)(b.nbx * b.nby * b.nbz)), dim3(256), 0, s, b);
+    hipLaunchKernelGGL(block_build_kernel, dim3((unsigned)(b.nbx * b.nby * b.nbz)), dim3(kThreads), 0, s, b);
     return hipGetLastError();
 }
 

@@ -6,26 +6,6 @@ using nmri::fail;
 
 namespace nmri {
 
-namespace {
-
-template <typename T>
-int grow(T** p, size_t count, int fill, hipStream_t s, int64_t* bytes, size_t old_count)
-{
-    const size_t n = std::max<size_t>(count * sizeof(T), 256);
-    if (*p) {
-        HIP_TRY(hipStreamSynchronize(s));
-        HIP_TRY(hipFree(*p));
-        *p = nullptr;
-        *bytes -= (int64_t)std::max<size_t>(old_count * sizeof(T), 256);
-    }
-    HIP_TRY(hipMalloc((void**)p, n));
-    *bytes += (int64_t)n;
-    HIP_TRY(hipMemsetAsync(*p, fill, n, s));
-    return NMR_OK;
-}
-
-} // namespace
-
 bool pores_fit(uint64_t nslots, bool vel)
 {
     constexpr uint64_t state = 3 * sizeof(float), rec = sizeof(*PoreList::rec);
@@ -76,55 +56,80 @@ bool pores_pay(double slots, const PoreProblem& p)
     return slots * (1.0 + more / (p.nc * p.nc)) <= most * p.padded;
 }
 
+namespace {
+
+// Consecutive arrays of one allocation, each on its own 256 bytes.
+struct Carver {
+    char* base;
+    size_t used = 0;
+    template <typename T>
+    void take(T** p, size_t count)
+    {
+        *p = base && count ? reinterpret_cast<T*>(base + used) : nullptr;
+        used += (count * sizeof(T) + 255) / 256 * 256;
+    }
+};
+
+} // namespace
+
+void pores_free(PoreList* L, int64_t* bytes)
+{
+    if (L->mem) (void)hipFree(L->mem);
+    *bytes -= (int64_t)L->mem_bytes;
+    for (float* p : L->pv)
+        if (p) {
+            (void)hipFree(p);
+            *bytes -= (int64_t)((L->cap + 64) * sizeof(float));
+        }
+    *L = PoreList{};
+}
+
 int pores_alloc(PoreList* L, uint32_t nslots, const PoreNeeds& n, hipStream_t s, int64_t* bytes)
 {
-    const bool more = nslots > L->cap || n.nc != L->nc;
-    const size_t old = L->cap, cap = more ? (size_t)nslots : L->cap;
-    const size_t all = cap + 64, was = old + 64; // a spare group past the end: the last slot reads the one after it
-    int rc = NMR_OK;
-    auto need = [&](auto** p, size_t per, int fill) {
-        if (rc) return;
-        if (more || !*p) rc = grow(p, all * per, fill, s, bytes, was * per);
-        else if (hipMemsetAsync(*p, fill, all * per * sizeof(**p), s) != hipSuccess)
-            rc = fail(NMR_ERR_DEVICE, "pore list: clearing a buffer failed");
+    const size_t all = (size_t)nslots + 64; // a spare group past the end: the last slot reads the one after it
+    auto carve = [&](char* base) {
+        Carver c{base};
+        c.take(&L->groups, all / 64);
+        c.take(&L->aux, n.aux ? all / 64 : 0);
+        c.take(&L->off8, all);
+        c.take(&L->off16, all);
+        c.take(&L->xoff, n.xoff ? all : 0);
+        c.take(&L->xy, n.nc == 3 ? all : 0);
+        for (float*& f : L->state) c.take(&f, all * n.nc);
+        c.take(&L->pred, n.pred ? all * n.nc : 0);
+        c.take(&L->rec, n.vel ? all : 0);
+        c.take(&L->bcount, (size_t)n.boxes * 8);
+        // (a block's first load is a whole workgroup's)
+        c.take(&L->blocks, n.boxes ? (size_t)n.block_slots + nmr::kBlockThreads : 0);
+        c.take(&L->vox, all); // last: the others are cleared in one go
+        return c.used;
     };
-    auto groups = [&](auto** p) {
-        if (rc) return;
-        if (more || !*p) rc = grow(p, all / 64, 0, s, bytes, was / 64);
-        else if (hipMemsetAsync(*p, 0, all / 64 * sizeof(**p), s) != hipSuccess)
-            rc = fail(NMR_ERR_DEVICE, "pore list: clearing a buffer failed");
-    };
-    if (L->nc != n.nc) { // sizes below are in slots of nc words
-        for (float** p : {&L->state[0], &L->state[1], &L->pred})
-            if (*p) {
-                HIP_TRY(hipStreamSynchronize(s));
-                HIP_TRY(hipFree(*p));
-                *p = nullptr;
-                *bytes -= (int64_t)(was * 4 * (size_t)L->nc);
-            }
-        L->nc = n.nc;
+    const size_t need = carve(nullptr);
+    if (need > L->mem_bytes) {
+        if (L->mem) {
+            HIP_TRY(hipStreamSynchronize(s));
+            HIP_TRY(hipFree(L->mem));
+            *bytes -= (int64_t)L->mem_bytes;
+            L->mem = nullptr;
+            L->mem_bytes = 0;
+        }
+        HIP_TRY(hipMalloc((void**)&L->mem, need));
+        L->mem_bytes = need;
+        *bytes += (int64_t)need;
     }
-    groups(&L->groups);
-    if (n.aux || L->aux) groups(&L->aux);
-    need(&L->off8, 1, 0);
-    need(&L->off16, 1, 0);
-    if (n.xoff || L->xoff) need(&L->xoff, 1, 0);
-    need(&L->vox, 1, 0xff);
-    if (n.nc == 3 || L->xy) need(&L->xy, 1, 0);
-    need(&L->state[0], (size_t)n.nc, 0);
-    need(&L->state[1], (size_t)n.nc, 0);
-    if (n.pred || L->pred) need(&L->pred, (size_t)n.nc, 0);
-    if (n.vel || L->rec) need(&L->rec, 1, 0);
-    if (more)
-        for (float*& p : L->pv)
-            if (p && !rc) {
-                if (hipStreamSynchronize(s) != hipSuccess || hipFree(p) != hipSuccess)
-                    rc = fail(NMR_ERR_DEVICE, "pore list: freeing a buffer failed");
-                p = nullptr;
-                *bytes -= (int64_t)(was * 4);
-            }
-    if (rc) return rc;
-    L->cap = cap;
+    carve(L->mem);
+    HIP_TRY(hipMemsetAsync(L->mem, 0, (size_t)(reinterpret_cast<char*>(L->vox) - L->mem), s));
+    HIP_TRY(hipMemsetAsync(L->vox, 0xff, all * sizeof(*L->vox), s));
+    if (nslots > L->cap) { // the per-voxel arrays have become too small
+        for (float*& p : L->pv) {
+            if (!p) continue;
+            HIP_TRY(hipStreamSynchronize(s));
+            HIP_TRY(hipFree(p));
+            p = nullptr;
+            *bytes -= (int64_t)((L->cap + 64) * sizeof(float));
+        }
+        L->cap = nslots;
+    }
     L->nslots = nslots;
     L->wide = false;
     L->nbx = L->nby = L->nbz = 0;
@@ -132,45 +137,33 @@ int pores_alloc(PoreList* L, uint32_t nslots, const PoreNeeds& n, hipStream_t s,
     return NMR_OK;
 }
 
-void pores_free(PoreList* L)
-{
-    for (void* p : {(void*)L->groups, (void*)L->aux, (void*)L->off8, (void*)L->off16, (void*)L->xoff, (void*)L->vox,
-                    (void*)L->xy, (void*)L->state[0], (void*)L->state[1], (void*)L->pred,
-                    (void*)L->rec, (void*)L->blocks, (void*)L->bcount, (void*)L->pv[0],
-                    (void*)L->pv[1], (void*)L->pv[2], (void*)L->pv[3], (void*)L->pv[4], (void*)L->pv[5]})
-        if (p) (void)hipFree(p);
-    *L = PoreList{};
-}
-
 void pores_drop_temp(nmr::PoreBuild* b)
 {
-    for (void* p : {(void*)b->rows, (void*)b->planes, (void*)b->slotmap, (void*)b->overflow})
-        if (p) (void)hipFree(p);
-    b->rows = nullptr;
-    b->planes = nullptr;
-    b->slotmap = nullptr;
-    b->overflow = nullptr;
+    if (b->temp) (void)hipFree(b->temp);
+    b->temp = nullptr;
 }
 
 int pores_temp(nmr::PoreBuild* b, size_t rows, size_t planes, size_t voxels, hipStream_t s)
 {
-    b->rows = nullptr;
-    b->planes = nullptr;
-    b->slotmap = nullptr;
-    b->overflow = nullptr;
-    int rc = NMR_OK;
-    auto check = [&](hipError_t e) {
-        if (!rc && e != hipSuccess)
-            rc = fail(e == hipErrorOutOfMemory ? NMR_ERR_NOMEM : NMR_ERR_DEVICE, "pore list: %s", hipGetErrorString(e));
-        return !rc;
+    const int boxes = b->nbx * b->nby * b->nbz;
+    auto carve = [&](char* base) {
+        Carver c{base};
+        c.take(&b->rows, rows);
+        c.take(&b->slotmap, voxels);
+        c.take(&b->bcount, (size_t)boxes * 8);
+        // the domain's end and what the kernels found lie side by side, for one copy
+        c.take(&b->planes, planes + 1 + sizeof(PoreFound) / sizeof(*b->planes));
+        return c.used;
     };
-    if (check(hipMalloc((void**)&b->rows, rows * sizeof(uint32_t))) &&
-        check(hipMalloc((void**)&b->planes, (planes + 1) * sizeof(uint64_t))) &&
-        check(hipMalloc((void**)&b->slotmap, voxels * sizeof(uint32_t))) &&
-        check(hipMalloc((void**)&b->overflow, 256)))
-        check(hipMemsetAsync(b->overflow, 0, 256, s));
-    if (rc) pores_drop_temp(b);
-    return rc;
+    const size_t need = carve(nullptr);
+    b->temp = nullptr;
+    HIP_TRY(hipMalloc(&b->temp, need));
+    carve(static_cast<char*>(b->temp));
+    b->found = reinterpret_cast<int*>(b->planes + planes + 1);
+    const hipError_t e = hipMemsetAsync(b->found, 0, sizeof(PoreFound), s);
+    if (e != hipSuccess) pores_drop_temp(b);
+    HIP_TRY(e);
+    return NMR_OK;
 }
 
 void pores_into(const PoreList& L, nmr::PoreBuild* b, uint64_t end)
@@ -182,21 +175,24 @@ void pores_into(const PoreList& L, nmr::PoreBuild* b, uint64_t end)
     b->off16 = L.off16;
     b->xoff = L.xoff;
     b->xy = L.xy;
+    b->blocks = L.blocks;
+    b->bcount_to = L.bcount;
     b->count = (int64_t)((end - b->first) / 64);
 }
 
-int pores_finish(PoreList* L, const nmr::PoreBuild& b, hipStream_t s, bool* ok)
+int pores_finish(PoreList* L, const nmr::PoreBuild& b, hipStream_t s, PoreFound* found)
 {
-    int over[2] = {0, 0};
-    HIP_TRY(hipMemcpyAsync(over, b.overflow, sizeof(over), hipMemcpyDeviceToHost, s));
+    HIP_TRY(hipMemcpyAsync(found, b.found, sizeof(*found), hipMemcpyDeviceToHost, s));
     HIP_TRY(hipStreamSynchronize(s));
-    *ok = over[0] == 0;
-    L->wide = over[1] != 0;
-    L->blocks_ok = *ok && b.blocks;
+    L->wide = found->wide != 0;
+    L->nbx = b.nbx;
+    L->nby = b.nby;
+    L->nbz = b.nbz;
+    L->blocks_ok = !found->overflow && b.blocks;
     return NMR_OK;
 }
 
-int pores_blocks(PoreList* L, nmr::PoreBuild* b, hipStream_t s, int64_t* bytes)
+void pores_boxes(nmr::PoreBuild* b)
 {
     // up to two boxes a CU: past one a CU they run in turns.  us a step, blocks
     // against single steps, at 1 component / 2 with velocity / 3 / 3 with
@@ -206,31 +202,11 @@ int pores_blocks(PoreList* L, nmr::PoreBuild* b, hipStream_t s, int64_t* bytes)
     // 4.5; the porosity (0.15, 0.3, 0.5 at 64^3) hardly matters.
     constexpr uint64_t kMost = 512;
     constexpr int e = nmr::kBlockEdge;
-    const uint64_t nx = (b->nx + e - 1) / e, ny = (b->ny + e - 1) / e, nz = (b->nz + e - 1) / e, n = nx * ny * nz;
-    if (n > kMost) return NMR_OK;
-    int rc = NMR_OK;
-    if (n > L->ncap) {
-        if ((rc = grow(&L->bcount, n * 8, 0, s, bytes, L->ncap * 8))) return rc;
-        L->ncap = n;
-    }
-    b->bcount = L->bcount;
+    const uint64_t nx = (b->nx + e - 1) / e, ny = (b->ny + e - 1) / e, nz = (b->nz + e - 1) / e;
+    if (nx * ny * nz > kMost) return;
     b->nbx = (int)nx;
     b->nby = (int)ny;
     b->nbz = (int)nz;
-    HIP_TRY(nmr::launch_block_count(*b, s));
-    int total = 0;
-    HIP_TRY(hipMemcpyAsync(&total, b->overflow + 2, sizeof(total), hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
-    const size_t all = (size_t)total + nmr::kBlockThreads; // (a block's first load is a whole workgroup's)
-    if (all > L->bcap) {
-        if ((rc = grow(&L->blocks, all, 0, s, bytes, L->bcap))) return rc;
-        L->bcap = all;
-    }
-    b->blocks = L->blocks;
-    L->nbx = b->nbx;
-    L->nby = b->nby;
-    L->nbz = b->nbz;
-    return NMR_OK;
 }
 
 int pores_per_tile(int64_t groups)

@@ -592,8 +592,8 @@ __global__ void __launch_bounds__(kThreads) pore_link_kernel(PoreBuild b)
         if (s >= 2 && off[s] > 0xffu) wide = true;
         if ((s >= 2 || b.xoff) && off[s] > 0xffffu) over = true;
     }
-    if (over) b.overflow[0] = 1;
-    if (wide) b.overflow[1] = 1;
+    if (over) b.found[0] = 1;
+    if (wide) b.found[1] = 1;
     b.off8[slot] = (off[2] & 0xffu) | (off[3] & 0xffu) << 8 | (off[4] & 0xffu) << 16 | (off[5] & 0xffu) << 24;
     b.off16[slot] = make_uint2((off[2] & 0xffffu) | off[3] << 16, (off[4] & 0xffffu) | off[5] << 16);
     if (b.xoff) b.xoff[slot] = (off[0] & 0xffffu) | off[1] << 16;
