@@ -891,6 +891,8 @@ int use_pores(nmr_ctx* c, bool* yes)
     if (!c->brick_on || c->variant != -1 || !c->has_mask || !c->has_mag) return NMR_OK;
     int rc = refresh_inert(c);
     if (rc) return rc;
+    // (another velocity leaves the list, unless it makes pores read solids or none)
+    if (c->pl_tried && c->pl_reads_solids != pores_read_solids(c) && (rc = drop_pores(c))) return rc;
     if (!c->pl_tried) {
         if (c->no_alloc) return NMR_OK;
         if ((rc = build_pores(c))) return rc;
@@ -903,8 +905,8 @@ int use_pores(nmr_ctx* c, bool* yes)
     return NMR_OK;
 }
 
-// The mask or the velocity changes: the state goes back to the rows and the
-// list is rebuilt before its next use.
+// The mask changes, or which solids pores read: the state goes back to the rows
+// and the list is rebuilt before its next use.
 int drop_pores(nmr_ctx* c)
 {
     if (c->home & nmri::kHomePores) {
@@ -1364,7 +1366,6 @@ int nmr_hip_upload_velocity(nmr_ctx* ctx, const double* vx, const double* vy, co
     int rc = check_layout(layout);
     if (rc) return rc;
     if (!ctx->vel) return fail(NMR_ERR_STATE, "velocity upload without NMR_F_VELOCITY");
-    if ((rc = drop_pores(ctx))) return rc;
     const nmr_problem& p = ctx->prob;
     const int P = ctx->pitch, P1 = ctx->pitch1;
     {
@@ -1412,6 +1413,7 @@ int nmr_hip_upload_velocity(nmr_ctx* ctx, const double* vx, const double* vy, co
     ctx->inert_dirty = true;
     ctx->adv_valid = ctx->advb_valid = false;
     ctx->csum_valid = ctx->csumb_valid = false;
+    ctx->pl_vel_ok = false;
     return prepare(ctx);
 }
 
