@@ -226,7 +226,9 @@ int nmr_hip_last_run_ms(nmr_ctx* ctx, double* ms, int64_t* sweeps);
  * learned solve that the list does not take.  Small grids take several plain
  * upwind steps a launch.  0 always sweeps the row layout.  The fields are the
  * same bits either way.  Once mask and magnetization are uploaded, this and
- * nmr_hip_set_tile prepare (and allocate) what the next run takes. */
+ * nmr_hip_set_tile prepare (and allocate) what the next run takes; a call that
+ * fails leaves the choice as it was.  Where there is no memory for the list the
+ * tiles run. */
 int nmr_hip_set_layout(nmr_ctx* ctx, int32_t brick);
 /* Tile shape of the sweep kernel: variant index (-1 = automatic, -2 = a
  * one-thread-per-voxel kernel with the arithmetic of the sweeps, a

@@ -369,6 +369,7 @@ int ensure_pv_bricks(nmr_ctx* c);
 int state_bricks(nmr_ctx* c);
 int use_pores(nmr_ctx* c, bool* yes);
 int drop_pores(nmr_ctx* c);
+int release_pores(nmr_ctx* c);
 int state_pores(nmr_ctx* c);
 
 // Launch geometry of the general sweep: 256 threads, tiles of 4*lanes x
@@ -895,7 +896,12 @@ int use_pores(nmr_ctx* c, bool* yes)
     if (c->pl_tried && c->pl_reads_solids != pores_read_solids(c) && (rc = drop_pores(c))) return rc;
     if (!c->pl_tried) {
         if (c->no_alloc) return NMR_OK;
-        if ((rc = build_pores(c))) return rc;
+        rc = build_pores(c);
+        if (rc == NMR_ERR_NOMEM) {
+            rc = release_pores(c);
+            c->pl_tried = true; // the tiles, until the next mask
+        }
+        if (rc) return rc;
     }
     if (!c->pl_ok || !nmri::pores_pay((double)c->pl_slots, pore_problem(c))) return NMR_OK;
     if (!c->solids_tried) {
@@ -915,6 +921,17 @@ int drop_pores(nmr_ctx* c)
         c->home &= ~nmri::kHomePores;
     }
     c->pl_tried = c->pl_ok = false;
+    return NMR_OK;
+}
+
+// The same, and the list's memory is given back.
+int release_pores(nmr_ctx* c)
+{
+    (void)hipGetLastError(); // (an allocation that failed)
+    int rc = drop_pores(c);
+    if (rc) return rc;
+    HIP_TRY(hipStreamSynchronize(c->stream));
+    nmri::pores_free(&c->pl, &c->device_bytes);
     return NMR_OK;
 }
 
@@ -1125,12 +1142,26 @@ int presize_buffers(nmr_ctx* c)
     return rc;
 }
 
+// What a run over the tiles needs: the brick buffers with the velocity and
+// per-voxel arrays converted.
+int prepare_tiles(nmr_ctx* c)
+{
+    const bool brick = c->brick_on && bricks_fit(c);
+    int rc;
+    if (brick && ((rc = ensure_bricks(c)) || (rc = ensure_pv_bricks(c)))) return rc;
+    // the per-voxel velocity sums the sweeps read: upwind (the plain sweep,
+    // the general sweep's upwind stage) or centred (MacCormack)
+    if ((rc = velocity_sums(c, brick, c->prob.scheme == NMR_SCHEME_MACCORMACK))) return rc;
+    return presize_buffers(c);
+}
+
 // The one-time work of a solve, done by the uploads so that runs start at
 // once: the inert check, then the list of the pores with its data, or where
-// the next run takes the tiles the brick buffers with the velocity and
-// per-voxel arrays converted, and the partial-sum and signal buffers.  Which
-// of them is known once there is magnetization; a tile or layout that is set
-// later prepares for itself.
+// the next run takes the tiles their buffers, and the partial-sum and signal
+// buffers.  Which of them is known once there is magnetization; a tile or
+// layout that is set later prepares for itself.  Where there is no memory for
+// the list the tiles run, and where there is none for the tiles beside a list
+// that the run does not take, the list's is given back.
 int prepare(nmr_ctx* c)
 {
     if (!c->has_mask) return NMR_OK;
@@ -1139,15 +1170,29 @@ int prepare(nmr_ctx* c)
     bool pores = false;
     if ((rc = use_pores(c, &pores))) return rc;
     if (pores) {
-        if ((rc = state_pores(c)) || (rc = pore_data(c))) return rc;
-    } else {
-        const bool brick = c->brick_on && bricks_fit(c);
-        if (brick && ((rc = ensure_bricks(c)) || (rc = ensure_pv_bricks(c)))) return rc;
-        // the per-voxel velocity sums the sweeps read: upwind (the plain sweep,
-        // the general sweep's upwind stage) or centred (MacCormack)
-        if ((rc = velocity_sums(c, brick, c->prob.scheme == NMR_SCHEME_MACCORMACK))) return rc;
+        if (!(rc = state_pores(c)) && !(rc = pore_data(c))) rc = presize_buffers(c);
+        if (rc == NMR_ERR_NOMEM) {
+            if ((rc = release_pores(c))) return rc;
+            c->pl_tried = true;
+            pores = false;
+        }
+        if (rc) return rc;
     }
-    if ((rc = presize_buffers(c))) return rc;
+    if (!pores) {
+        // a list that the mask, or data that came since, made useless
+        const bool tried = c->pl_tried, unpaid = c->brick_on && c->variant == -1 && c->pl_ok && c->solids_ok;
+        if (c->pl.mem && (unpaid || !c->pl_ok)) {
+            if ((rc = release_pores(c))) return rc;
+            c->pl_tried = tried;
+            c->pl_unpaid = c->pl_unpaid || unpaid;
+        }
+        rc = prepare_tiles(c);
+        if (rc == NMR_ERR_NOMEM && c->pl.mem) { // (the list is built again when a run takes it)
+            if ((rc = release_pores(c))) return rc;
+            rc = prepare_tiles(c);
+        }
+        if (rc) return rc;
+    }
     HIP_TRY(hipStreamSynchronize(c->stream));
     return NMR_OK;
 }
@@ -1615,7 +1660,9 @@ int nmr_hip_set_layout(nmr_ctx* ctx, int32_t brick)
     if (brick != 0 && brick != 1) return fail(NMR_ERR_INVALID, "layout %d", (int)brick);
     if (ctx->brick_on == (brick != 0)) return NMR_OK;
     ctx->brick_on = brick != 0;
-    return prepare(ctx);
+    const int rc = prepare(ctx);
+    if (rc) ctx->brick_on = !ctx->brick_on;
+    return rc;
 }
 
 int nmr_hip_set_tile(nmr_ctx* ctx, int32_t variant, int32_t lz)
@@ -1625,9 +1672,15 @@ int nmr_hip_set_tile(nmr_ctx* ctx, int32_t variant, int32_t lz)
     if (variant == -2 && ctx->exact) return fail(NMR_ERR_UNSUPPORTED, "the per-voxel kernel has no exact phase");
     if (lz < 0) return fail(NMR_ERR_INVALID, "lz %d", (int)lz);
     if (ctx->variant == variant && ctx->lz == lz) return NMR_OK;
+    const int variant0 = ctx->variant, lz0 = ctx->lz;
     ctx->variant = variant;
     ctx->lz = lz;
-    return prepare(ctx);
+    const int rc = prepare(ctx);
+    if (rc) {
+        ctx->variant = variant0;
+        ctx->lz = lz0;
+    }
+    return rc;
 }
 
 int nmr_hip_signal(nmr_ctx* ctx, double* out)
@@ -2288,8 +2341,16 @@ int batch_use_pores(nmr_batch* b, bool* yes)
     const bool chosen = b->tuned && b->variant == b->tuned_variant && b->lz == b->tuned_lz &&
                         b->persistent == b->tuned_persistent;
     if (chosen ? !b->tuned_list : b->variant != -1) return NMR_OK;
-    if (!b->pl_tried)
-        if (int rc = build_batch_pores(b)) return rc;
+    if (!b->pl_tried) {
+        const int rc = build_batch_pores(b);
+        if (rc == NMR_ERR_NOMEM) (void)hipGetLastError(); // no memory for the list: the tiles run
+        else if (rc) return rc;
+    }
+    if (!b->pl_ok && b->pl.mem) { // (neither are the states in it)
+        HIP_TRY(hipStreamSynchronize(b->stream));
+        int64_t bytes = 0;
+        nmri::pores_free(&b->pl, &bytes);
+    }
     *yes = b->pl_ok;
     return NMR_OK;
 }

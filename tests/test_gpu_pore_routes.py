@@ -153,3 +153,66 @@ def test_a_velocity_uploaded_again_costs_what_it_does_for_the_tiles():
                 s.run(1)
     print(f"[uploads] velocity again: list {least[-1]:.3f}, tiles {least[4]:.3f} ms", flush=True)
     assert least[-1] <= 1.3 * least[4]
+
+
+class _Filled:
+    """Takes the device's free memory but for `leave` bytes."""
+
+    def __init__(self, leave):
+        self.hip, self.blocks = ctypes.CDLL("libamdhip64.so"), []
+        for size in (16 << 30, 1 << 30, 64 << 20, 8 << 20):
+            while self.free() - leave >= size:
+                p = ctypes.c_void_p()
+                if self.hip.hipMalloc(ctypes.byref(p), ctypes.c_size_t(size)) != 0:
+                    self.hip.hipGetLastError()
+                    break
+                self.blocks.append(p)
+
+    def free(self):
+        free, total = ctypes.c_size_t(), ctypes.c_size_t()
+        assert self.hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+        return free.value
+
+    def __enter__(self):
+        return self
+
+    def __exit__(self, *exc):
+        for p in self.blocks:
+            self.hip.hipFree(p)
+
+
+def test_no_memory_for_the_list_or_beside_it():
+    """384^3, one component, a list of 0.45 GB with 0.23 GB to build it, tiles of
+    0.45 GB.  With 0.6 GB left the upload takes the tiles, as it did before there
+    was a list; with 0.25 GB beside a list, setting a tile gives the list back."""
+    shape = (384, 384, 384)
+    rng = np.random.default_rng(12)
+    mask = (rng.random(shape, dtype=np.float32) < 0.3).astype(np.uint8)
+    m0 = rng.random(shape)
+    with _solver(shape, mask, [m0], 1, True) as s:
+        want = s.run(2), s.download_magnetization()[0]
+    with _solver(shape, mask, [m0], 1) as s:  # (every kernel of either way is loaded)
+        s.run(2)
+        s.set_tile(4)
+        s.run(2)
+    with HipSolver(shape, 1, DX, DT, D, 0.5, r1_bulk=0.4, rho1=4e-6, rho2=9e-6) as s:
+        s.upload_mask(mask)
+        with _Filled(600 << 20) as full:
+            print(f"[memory] {full.free() >> 20} MiB left before the upload", flush=True)
+            s.upload_magnetization(m0)
+            got = s.run(2), s.download_magnetization()[0]
+            print(f"[memory] {full.free() >> 20} MiB left", flush=True)
+    np.testing.assert_allclose(got[0], want[0], rtol=1e-12)
+    assert np.array_equal(got[1], want[1])
+    with _solver(shape, mask, [m0], 1) as s:
+        held = s.device_bytes()
+        first = s.run(1)
+        with _Filled(250 << 20) as full:
+            print(f"[memory] {full.free() >> 20} MiB left beside the list", flush=True)
+            s.set_tile(4)
+            got = np.concatenate([first, s.run(1)[1:]]), s.download_magnetization()[0]
+            s.set_tile(-1)  # and back: no memory to build the list again, or what the tiles leave
+            s.run(1)
+        assert s.device_bytes() < 1.5 * held
+    np.testing.assert_allclose(got[0], want[0], rtol=1e-12)
+    assert np.array_equal(got[1], want[1])
