@@ -293,8 +293,9 @@ int nmr_hip_batch_set_tile(nmr_batch* b, int32_t variant, int32_t lz, int32_t gr
  * times the four fastest again over three times the steps on the warm
  * device, and keeps the fastest of those; then times the list of the pores
  * against it.  Where the list is faster, runs take it as long as the tile
- * that this call returned is set.  The choice is cached per set of instance
- * shapes.  Any output pointer may be NULL. */
+ * that this call returned is set.  The tile is cached per set of instance
+ * shapes, the list against it per share of pores as well.  Any output pointer
+ * may be NULL. */
 int nmr_hip_batch_autotune(nmr_batch* b, int32_t trial_steps, int32_t* variant, int32_t* lz,
                            int32_t* persistent);
 /* GPU ms of the last run's steps and the voxel-steps they advanced. */

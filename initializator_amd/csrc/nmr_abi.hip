@@ -2072,8 +2072,9 @@ int nmr_hip_run_static(nmr_ctx* ctx, int64_t nsteps, const double* grad_sched, d
 namespace {
 
 std::mutex g_tune_mu;
-struct Tuned { int variant, lz, persistent; bool list; std::array<double, 7> cost; };
-std::map<std::vector<int>, Tuned> g_tune_cache; // shapes -> fastest launch
+struct Tuned { int variant, lz, persistent; std::array<double, 7> cost; };
+std::map<std::vector<int>, Tuned> g_tune_cache; // shapes -> fastest tile
+std::map<std::vector<int>, bool> g_list_cache;  // shapes and what fills them -> the list beats that tile
 
 void batch_free(nmr_batch* b)
 {
@@ -2841,36 +2842,15 @@ int nmr_hip_batch_autotune(nmr_batch* b, int32_t trial_steps, int32_t* variant, 
     for (const auto& I : b->inst)
         if (!I.uploaded) return fail(NMR_ERR_STATE, "autotune before every instance is uploaded");
     const std::vector<int> key = batch_key(b);
-    {
-        std::lock_guard<std::mutex> g(g_tune_mu);
-        auto it = g_tune_cache.find(key);
-        if (it != g_tune_cache.end()) {
-            b->variant = it->second.variant;
-            b->lz = it->second.lz;
-            b->persistent = it->second.persistent;
-            b->tuned_list = it->second.list;
-            set_tuned(b);
-            b->tile_cost = it->second.cost;
-            b->cur_variant = -2; // the per-instance shapes may have changed
-            if (variant) *variant = b->variant;
-            if (lz) *lz = b->lz;
-            if (persistent) *persistent = b->persistent;
-            return NMR_OK;
-        }
-    }
+    const int trials = std::max(1, (int)trial_steps);
     // trials on the layout the runs take
     const bool brick = b->brick_on && batch_bricks_fit(b);
-    {
-        int rc = brick ? batch_bricks(b) : nmri::batch_rows(b);
-        if (rc) return rc;
-    }
-    const int trials = std::max(1, (int)trial_steps);
     // GPU time per launch of (variant, lz, grid kind) over n launches after
     // one untimed: every trial reads the current buffer and writes the
     // other one, so the state is unchanged
     auto time_cfg = [&](int v, int l, int per, int n, double* ms_out) -> int {
-        int rc = batch_prepare(b, v, l, per, brick);
-        if (rc) return rc;
+        int rc = brick ? batch_bricks(b) : nmri::batch_rows(b);
+        if (rc || (rc = batch_prepare(b, v, l, per, brick))) return rc;
         if ((rc = batch_partials(b, 1, b->ntiles))) return rc;
         if ((rc = batch_launch_step(b, 0, b->parity, b->d_part))) return rc;
         HIP_TRY(hipEventRecord(b->ev0, b->stream));
@@ -2883,6 +2863,78 @@ int nmr_hip_batch_autotune(nmr_batch* b, int32_t trial_steps, int32_t* variant, 
         *ms_out = (double)ms / n;
         return NMR_OK;
     };
+    // the list of the pores against the tile that is set, whose time is best
+    // (0: not known): by what decides it beside the shapes, the share of pores
+    // (in sixteenths) and whether solids are read
+    auto tune_list = [&](double best) -> int {
+        b->tuned = b->tuned_list = false;
+        if (b->brick_on) {
+            int64_t pores = 0, voxels = 0;
+            bool solids = false;
+            for (int i = 0; i < b->ninst; i++) {
+                pores += b->inst[i].npore;
+                voxels += (int64_t)b->spec[i].nx * b->spec[i].ny * b->spec[i].nz;
+                solids = solids || (b->vel && !b->inst[i].inert);
+            }
+            std::vector<int> filled = key;
+            filled.push_back((int)(16 * pores / voxels));
+            filled.push_back((int)solids);
+            {
+                std::lock_guard<std::mutex> g(g_tune_mu);
+                auto it = g_list_cache.find(filled);
+                if (it != g_list_cache.end()) {
+                    b->tuned_list = it->second;
+                    set_tuned(b);
+                    return NMR_OK;
+                }
+            }
+            const int v = b->variant;
+            b->variant = -1;
+            bool list = false;
+            int rc = batch_use_pores(b, &list);
+            b->variant = v;
+            if (rc) return rc;
+            if (list) {
+                if (best <= 0.0 && (rc = time_cfg(v, b->lz, b->persistent, 3 * trials, &best))) return rc;
+                if ((rc = batch_state_pores(b)) || (rc = batch_partials(b, 1, b->pl_ntiles))) return rc;
+                if ((rc = batch_pore_step(b, 0, b->ppar, b->d_part))) return rc;
+                HIP_TRY(hipEventRecord(b->ev0, b->stream));
+                for (int r = 0; r < 3 * trials; r++)
+                    if ((rc = batch_pore_step(b, 0, b->ppar, b->d_part))) return rc;
+                HIP_TRY(hipEventRecord(b->ev1, b->stream));
+                HIP_TRY(hipEventSynchronize(b->ev1));
+                float ms = 0.f;
+                HIP_TRY(hipEventElapsedTime(&ms, b->ev0, b->ev1));
+                b->tuned_list = ms / (3 * trials) < best;
+                std::lock_guard<std::mutex> g(g_tune_mu);
+                g_list_cache[filled] = b->tuned_list;
+            }
+        }
+        set_tuned(b);
+        return NMR_OK;
+    };
+    auto answer = [&]() {
+        if (variant) *variant = b->variant;
+        if (lz) *lz = b->lz;
+        if (persistent) *persistent = b->persistent;
+        return NMR_OK;
+    };
+    bool known = false;
+    {
+        std::lock_guard<std::mutex> g(g_tune_mu);
+        auto it = g_tune_cache.find(key);
+        if ((known = it != g_tune_cache.end())) {
+            b->variant = it->second.variant;
+            b->lz = it->second.lz;
+            b->persistent = it->second.persistent;
+            b->tile_cost = it->second.cost;
+            b->cur_variant = -2; // the per-instance shapes may have changed
+        }
+    }
+    if (known) {
+        const int rc = tune_list(0.0);
+        return rc ? rc : answer();
+    }
     struct Trial { int v, l, per; double ms; };
     std::vector<Trial> done;
     // every one-step tile shape on the whole batch, then per-instance shapes
@@ -2941,36 +2993,12 @@ int nmr_hip_batch_autotune(nmr_batch* b, int32_t trial_steps, int32_t* variant, 
     b->variant = bv;
     b->lz = bl;
     b->persistent = bp;
-    // the list of the pores against the fastest tile
-    b->tuned = b->tuned_list = false;
-    if (b->brick_on) {
-        b->variant = -1;
-        bool list = false;
-        int rc = batch_use_pores(b, &list);
-        b->variant = bv;
-        if (rc) return rc;
-        if (list) {
-            if ((rc = batch_state_pores(b)) || (rc = batch_partials(b, 1, b->pl_ntiles))) return rc;
-            if ((rc = batch_pore_step(b, 0, b->ppar, b->d_part))) return rc;
-            HIP_TRY(hipEventRecord(b->ev0, b->stream));
-            for (int r = 0; r < 3 * trials; r++)
-                if ((rc = batch_pore_step(b, 0, b->ppar, b->d_part))) return rc;
-            HIP_TRY(hipEventRecord(b->ev1, b->stream));
-            HIP_TRY(hipEventSynchronize(b->ev1));
-            float ms = 0.f;
-            HIP_TRY(hipEventElapsedTime(&ms, b->ev0, b->ev1));
-            b->tuned_list = ms / (3 * trials) < best;
-        }
-    }
-    set_tuned(b);
     {
         std::lock_guard<std::mutex> g(g_tune_mu);
-        g_tune_cache[key] = {bv, bl, bp, b->tuned_list, b->tile_cost};
+        g_tune_cache[key] = {bv, bl, bp, b->tile_cost};
     }
-    if (variant) *variant = bv;
-    if (lz) *lz = bl;
-    if (persistent) *persistent = bp;
-    return NMR_OK;
+    const int rc = tune_list(best);
+    return rc ? rc : answer();
 }
 
 int nmr_hip_batch_last_run_ms(nmr_batch* b, double* ms, int64_t* voxel_steps)

@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 
 from initializator_amd import generators
-from initializator_amd.solver import HipSolver, check
+from initializator_amd.solver import BatchSolver, HipSolver, check
 
 pytestmark = pytest.mark.gpu
 
@@ -216,3 +216,42 @@ def test_no_memory_for_the_list_or_beside_it():
         assert s.device_bytes() < 1.5 * held
     np.testing.assert_allclose(got[0], want[0], rtol=1e-12)
     assert np.array_equal(got[1], want[1])
+
+
+def test_the_autotuner_does_not_take_another_batchs_choice_of_the_list():
+    """Three 96^3 instances whose list cannot be had (a solid that is not
+    finite) are tuned first; then others of the same shapes, a fifth of them
+    pores, for which the list takes less than half the tile's time.  Which of
+    them a run takes shows in the order of the signal's FP64 sums (of values over
+    16 decades: those of FP32 values of one size are exact in any order)."""
+    shape = (96, 96, 96)
+    size = 10.0 ** -(np.arange(96) / 6.0)[:, None, None]
+    masks = [generators.porosity(shape, 0.2, seed, sigma=2.0) for seed in range(3)]
+
+    def batch(bad=False):
+        b = BatchSolver([dict(shape=shape)] * 3, 2, DX, DT, D, 0.5, r1_bulk=0.4)
+        for i, m in enumerate(masks):
+            rng = np.random.default_rng(i)
+            m0 = [rng.random(shape) * size, (rng.random(shape) - 0.5) * size]
+            if bad and i == 1:
+                m0[0][tuple(np.argwhere(m == 0)[5])] = np.nan
+            b.upload(i, m, m0)
+        return b
+
+    def run(b):
+        out = b.run(20)
+        b.close()
+        return out
+
+    first = batch(True)
+    first.autotune(3)
+    first.close()
+    tuned = batch()
+    variant, lz, persistent = tuned.autotune(3)
+    tuned = run(tuned)
+    on_list = run(batch())
+    on_tile = batch()
+    on_tile.set_tile(variant, lz, persistent=persistent)
+    on_tile = run(on_tile)
+    assert not np.array_equal(on_list, on_tile)  # (else the next line shows nothing)
+    np.testing.assert_array_equal(tuned, on_list)
