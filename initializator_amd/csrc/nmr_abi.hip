@@ -2224,12 +2224,48 @@ nmr::PoreInst batch_coef(const nmr_problem& p, const nmr_batch_instance& s)
 // no tile is padded and the launch is even.  256 instances of edge 32-128:
 // 428.6 us a step against 1018 on the fastest tile (64x16 bricks).
 
+// Instance i as a domain of the list (its mask, window and velocity sums).
+void batch_domain(const nmr_batch* b, int i, nmr::PoreBuild* t)
+{
+    const nmr_problem& p = b->prob;
+    const nmr_batch_instance& s = b->spec[i];
+    const auto& I = b->inst[i];
+    t->mask = I.mask;
+    t->nx = s.nx;
+    t->ny = s.ny;
+    t->nz = s.nz;
+    t->pitch = I.pitch;
+    t->read_solids = b->vel && !I.inert;
+    t->w[0] = p.buffer[0]; t->w[1] = s.nx - p.buffer[0];
+    t->w[2] = p.buffer[1]; t->w[3] = s.ny - p.buffer[1];
+    t->w[4] = p.buffer[2]; t->w[5] = s.nz - p.buffer[2];
+    for (int q = 0; q < 3; q++) t->vel[q] = b->vel ? I.adv[q] : nullptr;
+}
+
+// Tiles of whole groups, instance by instance (the device arrays have room
+// for what the instances may grow to).
+int batch_tiles(nmr_batch* b)
+{
+    const uint32_t per = (uint32_t)b->pl_per;
+    std::vector<nmr::PoreTile> tiles;
+    std::vector<int> off(b->ninst + 1, 0);
+    for (int i = 0; i < b->ninst; i++) {
+        const auto& I = b->inst[i];
+        for (uint32_t g = I.slot0 / 64; g < I.slot1 / 64; g += per)
+            tiles.push_back({g, std::min(per, I.slot1 / 64 - g), (uint32_t)i});
+        off[i + 1] = (int)tiles.size();
+    }
+    HIP_TRY(hipMemcpy(b->d_ptiles, tiles.data(), tiles.size() * sizeof(tiles[0]), hipMemcpyHostToDevice));
+    HIP_TRY(hipMemcpy(b->d_poff, off.data(), off.size() * sizeof(int), hipMemcpyHostToDevice));
+    b->pl_ntiles = (int)tiles.size();
+    return NMR_OK;
+}
+
 // Builds the list for the uploaded instances.
 int build_batch_pores(nmr_batch* b)
 {
     b->pl_tried = true;
     b->pl_ok = b->pl_reads_solids = false;
-    const nmr_problem& p = b->prob;
     size_t rows = 0, planes = 0, voxels = 0;
     nmri::PoreProblem q{};
     q.nc = b->nc;
@@ -2238,8 +2274,8 @@ int build_batch_pores(nmr_batch* b)
         const nmr_batch_instance& s = b->spec[i];
         const auto& I = b->inst[i];
         if (!I.solids_ok || (b->nc == 3 && (s.nx > 65536 || s.ny > 65536))) return NMR_OK;
-        rows = std::max(rows, (size_t)s.ny * s.nz);
-        planes = std::max(planes, (size_t)s.nz);
+        rows += (size_t)s.ny * s.nz;
+        planes += (size_t)s.nz + 1;
         voxels = std::max(voxels, I.n_m);
         q.voxels += (double)s.nx * s.ny * s.nz;
         q.padded += nmri::pores_padded(s.nx, s.ny, s.nz);
@@ -2248,88 +2284,122 @@ int build_batch_pores(nmr_batch* b)
     nmr::PoreBuild t{};
     int rc = nmri::pores_temp(&t, rows, planes, voxels, b->stream);
     if (rc) return rc;
-    uint64_t* ends = nullptr;
     struct Temp {
         nmr::PoreBuild* t;
-        uint64_t** e;
-        ~Temp()
-        {
-            nmri::pores_drop_temp(t);
-            if (*e) (void)hipFree(*e);
-        }
-    } temp{&t, &ends};
-    HIP_TRY(hipMalloc((void**)&ends, (size_t)b->ninst * sizeof(uint64_t)));
-    auto domain = [&](int i) {
-        const nmr_batch_instance& s = b->spec[i];
-        const auto& I = b->inst[i];
-        t.mask = I.mask;
-        t.nx = s.nx;
-        t.ny = s.ny;
-        t.nz = s.nz;
-        t.pitch = I.pitch;
-        t.read_solids = b->vel && !I.inert;
-        t.w[0] = p.buffer[0]; t.w[1] = s.nx - p.buffer[0];
-        t.w[2] = p.buffer[1]; t.w[3] = s.ny - p.buffer[1];
-        t.w[4] = p.buffer[2]; t.w[5] = s.nz - p.buffer[2];
-    };
-    // slots of every instance
+        ~Temp() { nmri::pores_drop_temp(t); }
+    } temp{&t};
+    // slots of every instance, each counted from 0
+    uint32_t* const rows0 = t.rows;
+    uint64_t* const planes0 = t.planes;
     for (int i = 0; i < b->ninst; i++) {
-        domain(i);
-        t.first = 0;
+        batch_domain(b, i, &t);
         HIP_TRY(nmr::launch_pore_count(t, b->stream));
-        HIP_TRY(hipMemcpyAsync(ends + i, t.planes + t.nz, sizeof(uint64_t), hipMemcpyDeviceToDevice, b->stream));
+        t.rows += (size_t)t.ny * t.nz;
+        t.planes += (size_t)t.nz + 1;
     }
-    std::vector<uint64_t> n(b->ninst);
-    HIP_TRY(hipMemcpyAsync(n.data(), ends, n.size() * sizeof(uint64_t), hipMemcpyDeviceToHost, b->stream));
+    std::vector<uint64_t> h(planes), n(b->ninst);
+    HIP_TRY(hipMemcpyAsync(h.data(), planes0, planes * sizeof(uint64_t), hipMemcpyDeviceToHost, b->stream));
     HIP_TRY(hipStreamSynchronize(b->stream));
-    uint64_t end = 64;
-    for (uint64_t v : n) end += v;
+    uint64_t end = 64, room = 64;
+    size_t at = 0;
+    // room for an eighth more, so that another mask of an instance fits its place
+    auto with_room = [](uint64_t v) { return v + (v / 8 + 63) / 64 * 64; };
+    for (int i = 0; i < b->ninst; i++) {
+        at += (size_t)b->spec[i].nz + 1;
+        n[i] = h[at - 1];
+        end += n[i];
+        room += with_room(n[i]);
+    }
     q.solids = b->pl_reads_solids;
     if (!nmri::pores_fit(end, b->vel) || !nmri::pores_pay((double)end, q)) return NMR_OK;
+    const bool roomy = nmri::pores_fit(room, b->vel);
+    if (!roomy) room = end;
     int64_t bytes = 0;
     const nmri::PoreNeeds needs{b->nc, b->vel, b->pl_reads_solids, false, false};
-    if ((rc = nmri::pores_alloc(&b->pl, (uint32_t)end, needs, b->stream, &bytes))) return rc;
-    // link them; tiles of whole groups, instance by instance
+    if ((rc = nmri::pores_alloc(&b->pl, (uint32_t)room, needs, b->stream, &bytes))) return rc;
+    // link them
     int per = nmri::pores_per_tile((int64_t)(end / 64));
     const size_t S = (size_t)std::max(b->graph_steps, 2);
     while ((end / 64 / per) * S * b->nc * sizeof(double) > ((size_t)128 << 20)) per *= 2; // partial sums of a chunk
-    std::vector<nmr::PoreTile> tiles;
-    std::vector<int> off(b->ninst + 1, 0);
+    b->pl_per = per;
+    size_t most = 0; // tiles
     std::vector<nmr::PoreInst> pi(b->ninst);
     t.first = 64;
+    t.rows = rows0;
+    t.planes = planes0;
     for (int i = 0; i < b->ninst; i++) {
-        domain(i);
-        HIP_TRY(nmr::launch_pore_count(t, b->stream));
+        batch_domain(b, i, &t);
+        t.shift = t.first;
         nmri::pores_into(b->pl, &t, t.first + n[i]);
         HIP_TRY(nmr::launch_pore_link(t, b->stream));
+        t.rows += (size_t)t.ny * t.nz;
+        t.planes += (size_t)t.nz + 1;
         auto& I = b->inst[i];
         I.slot0 = (uint32_t)t.first;
         I.slot1 = (uint32_t)(t.first + n[i]);
-        if (b->vel)
-            for (int q = 0; q < 3; q++)
-                HIP_TRY(nmr::launch_pore_gather(I.adv[q], b->pl.vox, I.slot0, I.slot1, 4, 1 + q,
-                                                reinterpret_cast<float*>(b->pl.rec), b->stream));
-        for (uint32_t g = I.slot0 / 64; g < I.slot1 / 64; g += (uint32_t)per)
-            tiles.push_back({g, std::min((uint32_t)per, I.slot1 / 64 - g), (uint32_t)i});
-        off[i + 1] = (int)tiles.size();
-        pi[i] = batch_coef(p, b->spec[i]);
-        t.first += n[i];
+        t.first += roomy ? with_room(n[i]) : n[i];
+        I.slot2 = (uint32_t)t.first;
+        most += (I.slot2 - I.slot0) / 64 / per + 1;
+        pi[i] = batch_coef(b->prob, b->spec[i]);
     }
-    if (b->vel) HIP_TRY(nmr::launch_pore_record(b->pl.off8, b->pl.nslots, b->pl.rec, b->stream));
     nmri::PoreFound found{};
     if ((rc = nmri::pores_finish(&b->pl, t, b->stream, &found)) || found.overflow) return rc;
     for (void** q : {(void**)&b->d_pinst, (void**)&b->d_ptiles, (void**)&b->d_poff}) {
         if (*q) HIP_TRY(hipFree(*q));
         *q = nullptr;
     }
-    if ((rc = balloc(b->stream, &b->d_pinst, pi.size())) || (rc = balloc(b->stream, &b->d_ptiles, tiles.size())) ||
-        (rc = balloc(b->stream, &b->d_poff, off.size())))
+    if ((rc = balloc(b->stream, &b->d_pinst, pi.size())) || (rc = balloc(b->stream, &b->d_ptiles, most)) ||
+        (rc = balloc(b->stream, &b->d_poff, (size_t)b->ninst + 1)))
         return rc;
     HIP_TRY(hipMemcpy(b->d_pinst, pi.data(), pi.size() * sizeof(pi[0]), hipMemcpyHostToDevice));
-    HIP_TRY(hipMemcpy(b->d_ptiles, tiles.data(), tiles.size() * sizeof(tiles[0]), hipMemcpyHostToDevice));
-    HIP_TRY(hipMemcpy(b->d_poff, off.data(), off.size() * sizeof(int), hipMemcpyHostToDevice));
-    b->pl_ntiles = (int)tiles.size();
+    if ((rc = batch_tiles(b))) return rc;
     b->pl_ok = true;
+    return NMR_OK;
+}
+
+// Links instance i, which was uploaded again, in its place of the list, and
+// brings its state there if the others' are; *kept: it fits there, and the list
+// holds what it needs.
+int batch_relink(nmr_batch* b, int i, bool* kept)
+{
+    *kept = false;
+    auto& I = b->inst[i];
+    if (!I.solids_ok || (b->vel && !I.inert && !b->pl.aux)) return NMR_OK;
+    nmr::PoreBuild t{};
+    batch_domain(b, i, &t);
+    int rc = nmri::pores_temp(&t, (size_t)t.ny * t.nz, (size_t)t.nz, I.n_m, b->stream);
+    if (rc == NMR_ERR_NOMEM) {
+        (void)hipGetLastError();
+        return NMR_OK;
+    }
+    if (rc) return rc;
+    struct Temp {
+        nmr::PoreBuild* t;
+        ~Temp() { nmri::pores_drop_temp(t); }
+    } temp{&t};
+    t.first = I.slot0;
+    uint64_t end = 0;
+    HIP_TRY(nmr::launch_pore_count(t, b->stream));
+    HIP_TRY(hipMemcpyAsync(&end, t.planes + t.nz, sizeof(end), hipMemcpyDeviceToHost, b->stream));
+    HIP_TRY(hipStreamSynchronize(b->stream));
+    if (end > I.slot2) return NMR_OK;
+    bool any = end > I.slot0;
+    for (int k = 0; k < b->ninst; k++) any = any || (k != i && b->inst[k].slot1 > b->inst[k].slot0);
+    if (!any) return NMR_OK; // (no pore left in the whole batch)
+    HIP_TRY(hipMemsetAsync(b->pl.vox + I.slot0, 0xff, (size_t)(I.slot2 - I.slot0) * sizeof(*b->pl.vox), b->stream));
+    nmri::pores_into(b->pl, &t, end);
+    HIP_TRY(nmr::launch_pore_link(t, b->stream));
+    if (b->home & nmri::kHomePores)
+        for (int q = 0; q < b->nc; q++)
+            HIP_TRY(nmr::launch_pore_gather(I.m[b->parity][q], b->pl.vox, I.slot0, (uint32_t)end, b->nc, q,
+                                            b->pl.state[b->ppar], b->stream));
+    const bool wide = b->pl.wide;
+    nmri::PoreFound found{};
+    if ((rc = nmri::pores_finish(&b->pl, t, b->stream, &found)) || found.overflow) return rc;
+    b->pl.wide = b->pl.wide || wide;
+    I.slot1 = (uint32_t)end;
+    if ((rc = batch_tiles(b))) return rc;
+    *kept = true;
     return NMR_OK;
 }
 
@@ -2682,12 +2752,6 @@ int nmr_hip_batch_upload(nmr_batch* b, int32_t i, const uint8_t* mask, const dou
     auto& I = b->inst[i];
     const int P = I.pitch, P1 = I.pitch1;
     int rc = NMR_OK;
-    if (b->home & nmri::kHomePores) { // the other instances' states leave the list, which the new mask ends
-        if ((rc = nmri::batch_rows(b))) return rc;
-        HIP_TRY(hipStreamSynchronize(b->stream));
-        b->home &= ~nmri::kHomePores;
-    }
-    b->pl_tried = b->pl_ok = false;
     {
         std::vector<uint8_t> h(I.n_m, 0);
         int64_t np = 0;
@@ -2774,6 +2838,17 @@ int nmr_hip_batch_upload(nmr_batch* b, int32_t i, const uint8_t* mask, const dou
     I.solids_ok = f[1] == 0;
     I.uploaded = true;
     I.adv_bricks = false;
+    // the list goes on with the instance in its place; or the other instances'
+    // states leave it, and it is built again
+    bool kept = false;
+    if (b->pl_ok && (rc = batch_relink(b, i, &kept))) return rc;
+    if (!kept) {
+        if (b->home & nmri::kHomePores) {
+            if ((rc = nmri::batch_rows(b, i))) return rc;
+            b->home &= ~nmri::kHomePores;
+        }
+        b->pl_tried = b->pl_ok = false;
+    }
     // the rows hold the new state (both buffers); so do the bricks if they
     // are the home of the other instances
     if ((b->home & nmri::kHomeBricks) && (rc = batch_inst_to_bricks(b, i))) return rc;
@@ -3186,13 +3261,14 @@ int nmr_hip_batch_run(nmr_batch* b, int64_t nsteps, double* signal)
 
 namespace nmri {
 
-int batch_rows(nmr_batch* b)
+int batch_rows(nmr_batch* b, int but)
 {
     if (b->home & kHomeRows) return NMR_OK;
     for (int i = 0; i < b->ninst; i++) {
         const auto& s = b->spec[i];
         auto& I = b->inst[i];
         if (b->home & kHomePores) { // both row buffers still hold the solids' values
+            if (i == but) continue;
             for (int q = 0; q < b->nc; q++)
                 HIP_TRY(nmr::launch_pore_scatter(b->pl.state[b->ppar], b->pl.vox, I.slot0, I.slot1, b->nc, q, I.m[0][q],
                                                  I.m[1][q], b->stream));

@@ -254,7 +254,8 @@ struct nmr_batch {
         int inert = 0;
         bool solids_ok = false; // every solid's magnetization is finite
         int64_t npore = 0;
-        uint32_t slot0 = 0, slot1 = 0; // its slots in the list of pores
+        // its slots in the list of pores, and up to where it has room
+        uint32_t slot0 = 0, slot1 = 0, slot2 = 0;
         // upwind velocity sums of the plain sweep (rows), computed at upload
         float* adv[3] = {nullptr, nullptr, nullptr};
         // brick copies (8 x-voxels by 4 rows) of the state and the velocity sums
@@ -281,7 +282,7 @@ struct nmr_batch {
     nmr::PoreInst* d_pinst = nullptr;
     nmr::PoreTile* d_ptiles = nullptr;
     int* d_poff = nullptr; // first tile of every instance
-    int pl_ntiles = 0;
+    int pl_ntiles = 0, pl_per = 4; // tiles, and groups of a tile
     // the autotuner's choice: its tile, and whether the list was faster
     int tuned_variant = -1, tuned_lz = 0, tuned_persistent = 0;
     bool tuned = false, tuned_list = false;
@@ -335,6 +336,7 @@ int list_step(nmr_ctx* c, const nmr::Coef& cf);
 // Make the row buffers hold the current state (both of them, converted from
 // the bricks when only those hold it).
 int state_rows(nmr_ctx* c);
-// The same for every instance of a batch.
-int batch_rows(nmr_batch* b);
+// The same for every instance of a batch (but one, when only the list holds
+// the others).
+int batch_rows(nmr_batch* b, int but = -1);
 } // namespace nmri

@@ -250,6 +250,7 @@ struct PoreBuild {
     int read_solids;        // upwind velocity on pore-solid faces: solids next to pores get slots
     int w[6];               // signal window
     uint64_t first;         // first slot (a multiple of 64)
+    uint64_t shift;         // to add to planes, where they were counted from another slot
     int64_t count;          // groups of this domain (linking)
     uint32_t* rows;         // [nz*ny] slots before the row in its plane
     uint64_t* planes;       // [nz + 1] first slot of each plane
@@ -261,6 +262,8 @@ struct PoreBuild {
     uint2* off16;
     uint32_t* xoff;         // or null
     uint32_t* xy;           // or null
+    uint4* rec;             // records, to be written here from
+    const float* vel[3];    //   the velocity sums (row layout) unless they are null
     int* found;             // what is found on the way: [0] an offset that does not fit, [1] a group that needs
                             // 16-bit offsets, [2] slots of all blocks, [3] a solid that is not finite
     void* temp;             // what rows, planes, slotmap, bcount and found lie in

@@ -175,6 +175,7 @@ void pores_into(const PoreList& L, nmr::PoreBuild* b, uint64_t end)
     b->off16 = L.off16;
     b->xoff = L.xoff;
     b->xy = L.xy;
+    b->rec = L.rec;
     b->blocks = L.blocks;
     b->bcount_to = L.bcount;
     b->count = (int64_t)((end - b->first) / 64);

@@ -517,7 +517,7 @@ __global__ void __launch_bounds__(kThreads) pore_assign_kernel(PoreBuild b)
     const int lane = threadIdx.x & 63;
     for (int64_t row = (int64_t)blockIdx.x * kWaves + (threadIdx.x >> 6); row < nrows; row += (int64_t)gridDim.x * kWaves) {
         const int y = (int)(row % b.ny), z = (int)(row / b.ny);
-        uint32_t s0 = (uint32_t)b.planes[z] + b.rows[row];
+        uint32_t s0 = (uint32_t)(b.planes[z] + b.shift) + b.rows[row];
         for (int x0 = 0; x0 < b.nx; x0 += 64) {
             const int x = x0 + lane;
             const bool in = x < b.nx && has_slot(b, x, y, z);
@@ -594,7 +594,17 @@ __global__ void __launch_bounds__(kThreads) pore_link_kernel(PoreBuild b)
     }
     if (over) b.found[0] = 1;
     if (wide) b.found[1] = 1;
-    b.off8[slot] = (off[2] & 0xffu) | (off[3] & 0xffu) << 8 | (off[4] & 0xffu) << 16 | (off[5] & 0xffu) << 24;
+    const uint32_t off8 = (off[2] & 0xffu) | (off[3] & 0xffu) << 8 | (off[4] & 0xffu) << 16 | (off[5] & 0xffu) << 24;
+    b.off8[slot] = off8;
+    if (b.vel[0]) {
+        uint4 r = make_uint4(off8, 0u, 0u, 0u);
+        if (used) {
+            r.y = __float_as_uint(b.vel[0][o]);
+            r.z = __float_as_uint(b.vel[1][o]);
+            r.w = __float_as_uint(b.vel[2][o]);
+        }
+        b.rec[slot] = r;
+    }
     b.off16[slot] = make_uint2((off[2] & 0xffffu) | off[3] << 16, (off[4] & 0xffffu) | off[5] << 16);
     if (b.xoff) b.xoff[slot] = (off[0] & 0xffffu) | off[1] << 16;
     if (b.xy) b.xy[slot] = (uint32_t)x | ((uint32_t)y << 16);
