@@ -1633,23 +1633,28 @@ int nmr_hip_download_magnetization(nmr_ctx* ctx, double* mx, double* my, double*
                                ctx->stream));
         HIP_TRY(hipStreamSynchronize(ctx->stream));
         // interior plus the ghost layer each axis's boundary condition
-        // leaves (copy of the adjacent cell, opposite cell, or 0)
-        auto ghost = [](int i, int n, int bc, bool* zero) {
+        // leaves (copy of the adjacent cell, opposite cell, or 0: -1), row by
+        // row (128^3, one component: 1.0 ms; one cell at a time 2.2-2.7)
+        auto from = [](int i, int n, int bc) {
             if (i >= 1 && i <= n) return i - 1;
-            if (bc == NMR_BC_DIRICHLET) *zero = true;
+            if (bc == NMR_BC_DIRICHLET) return -1;
             if (bc == NMR_BC_PERIODIC) return i == 0 ? n - 1 : 0;
             return i == 0 ? 0 : n - 1;
         };
+        const int lo = from(0, p.nx, p.bc[0]), hi = from(p.nx + 1, p.nx, p.bc[0]);
         for (int k = 0; k < p.nz + 2; k++)
-            for (int j = 0; j < p.ny + 2; j++)
-                for (int i = 0; i < p.nx + 2; i++) {
-                    bool zero = false;
-                    const int ii = ghost(i, p.nx, p.bc[0], &zero);
-                    const int jj = ghost(j, p.ny, p.bc[1], &zero);
-                    const int kk = ghost(k, p.nz, p.bc[2], &zero);
-                    dst[q][pidx(p, i, j, k)] =
-                        zero ? 0.0 : h[(size_t)kk * p.ny * ctx->pitch + (size_t)jj * ctx->pitch + ii];
+            for (int j = 0; j < p.ny + 2; j++) {
+                const int jj = from(j, p.ny, p.bc[1]), kk = from(k, p.nz, p.bc[2]);
+                double* row = dst[q] + pidx(p, 0, j, k);
+                if (jj < 0 || kk < 0) {
+                    std::fill(row, row + p.nx + 2, 0.0);
+                    continue;
                 }
+                const float* src = h.data() + (size_t)kk * p.ny * ctx->pitch + (size_t)jj * ctx->pitch;
+                row[0] = lo < 0 ? 0.0 : (double)src[lo];
+                for (int i = 0; i < p.nx; i++) row[i + 1] = (double)src[i];
+                row[p.nx + 1] = hi < 0 ? 0.0 : (double)src[hi];
+            }
     }
     return NMR_OK;
 }

@@ -330,3 +330,24 @@ def test_an_instance_uploaded_again_costs_little_more_than_for_the_tiles():
         b.close()
     print(f"[uploads] an instance again and two steps: list {least[-1]:.2f}, tiles {least[4]:.2f} ms", flush=True)
     assert least[-1] <= 1.3 * least[4]
+
+
+@pytest.mark.parametrize("bc", [(0, 0, 0), (1, 1, 1), (2, 2, 2), (0, 1, 2), (2, 0, 1), (1, 2, 0)])
+@pytest.mark.parametrize("shape", [(1, 1, 1), (3, 5, 2), (4, 1, 9), (7, 6, 64)])
+def test_padded_download_is_the_interior_with_its_ghosts(shape, bc):
+    """After a step the padded layout holds the compact one and, a cell further,
+    what each axis's rule puts there: the cell beside, the opposite one, 0."""
+    rng = np.random.default_rng(14)
+    mask = (rng.random(shape) < 0.6).astype(np.uint8)
+    mask.flat[0] = 1
+    m0 = [rng.random(shape) for _ in range(3)]
+    with _solver(shape, mask, m0, 3, bc=bc) as s:
+        s.run(1)
+        inside, padded = s.download_magnetization(), s.download_magnetization(layout=1)
+    for a, b in zip(inside, padded):
+        want = a
+        for axis in (2, 1, 0):
+            width = [(0, 0)] * 3
+            width[axis] = (1, 1)
+            want = np.pad(want, width, mode={0: "edge", 1: "wrap", 2: "constant"}[bc[2 - axis]])
+        np.testing.assert_array_equal(b, want)
