@@ -824,7 +824,11 @@ int build_pores(nmr_ctx* c)
     b.first = 64;
     if (pore_plain(c) && !b.read_solids && p.scheme == NMR_SCHEME_UPWIND) nmri::pores_boxes(&b);
     const size_t rows = (size_t)p.ny * p.nz;
-    int rc = nmri::pores_temp(&b, rows, (size_t)p.nz, rows * c->pitch, c->stream);
+    // (a small grid's temporary arrays fit the partial sums that its runs take:
+    // allocating and freeing them took 0.25 ms of an upload at 64^3)
+    int rc = NMR_OK;
+    if (b.nbx && (rc = ensure_partials(c, (size_t)kChunkSteps * b.nbx * b.nby * b.nbz * c->nsig()))) return rc;
+    rc = nmri::pores_temp(&b, rows, (size_t)p.nz, rows * c->pitch, c->stream, c->partials, c->partials_cap * sizeof(double));
     if (rc) return rc;
     struct Temp {
         nmr::PoreBuild* b;

@@ -113,8 +113,10 @@ void pores_free(PoreList* L, int64_t* bytes);
 // Building: temporary arrays for domains of up to `rows` rows, `planes` planes
 // and `voxels` voxels (row layout); per domain, with first set,
 // launch_pore_count (planes[nz] is then the slot past its last one) and, with
-// the list's arrays taken by pores_into, launch_pore_link.
-int pores_temp(nmr::PoreBuild* b, size_t rows, size_t planes, size_t voxels, hipStream_t s);
+// the list's arrays taken by pores_into, launch_pore_link.  They lie in mem where
+// its bytes are enough.
+int pores_temp(nmr::PoreBuild* b, size_t rows, size_t planes, size_t voxels, hipStream_t s, void* mem = nullptr,
+               size_t bytes = 0);
 void pores_drop_temp(nmr::PoreBuild* b);
 void pores_into(const PoreList& L, nmr::PoreBuild* b, uint64_t end);
 // Gives the domain b its boxes, where the grid is small enough for them:

@@ -266,7 +266,7 @@ struct PoreBuild {
     const float* vel[3];    //   the velocity sums (row layout) unless they are null
     int* found;             // what is found on the way: [0] an offset that does not fit, [1] a group that needs
                             // 16-bit offsets, [2] slots of all blocks, [3] a solid that is not finite
-    void* temp;             // what rows, planes, slotmap, bcount and found lie in
+    void* temp;             // what rows, planes, slotmap, bcount and found lie in, where that is their own
     u32x4* blocks;          // the blocks' slots, or null
     uint32_t* bcount;       // [nblocks][8]: slots within 0 .. kBlockSteps faces of the box, the first one's place
     uint32_t* bcount_to;    // the same in the list

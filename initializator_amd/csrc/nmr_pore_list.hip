@@ -143,7 +143,7 @@ void pores_drop_temp(nmr::PoreBuild* b)
     b->temp = nullptr;
 }
 
-int pores_temp(nmr::PoreBuild* b, size_t rows, size_t planes, size_t voxels, hipStream_t s)
+int pores_temp(nmr::PoreBuild* b, size_t rows, size_t planes, size_t voxels, hipStream_t s, void* mem, size_t bytes)
 {
     const int boxes = b->nbx * b->nby * b->nbz;
     auto carve = [&](char* base) {
@@ -157,8 +157,11 @@ int pores_temp(nmr::PoreBuild* b, size_t rows, size_t planes, size_t voxels, hip
     };
     const size_t need = carve(nullptr);
     b->temp = nullptr;
-    HIP_TRY(hipMalloc(&b->temp, need));
-    carve(static_cast<char*>(b->temp));
+    if (need > bytes) {
+        HIP_TRY(hipMalloc(&b->temp, need));
+        mem = b->temp;
+    }
+    carve(static_cast<char*>(mem));
     b->found = reinterpret_cast<int*>(b->planes + planes + 1);
     const hipError_t e = hipMemsetAsync(b->found, 0, sizeof(PoreFound), s);
     if (e != hipSuccess) pores_drop_temp(b);
