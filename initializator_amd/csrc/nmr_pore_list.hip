@@ -203,7 +203,11 @@ void pores_boxes(nmr::PoreBuild* b)
     // velocity: 20^3 (27 boxes) 1.4 1.7 1.9 2.0 against 3.7 3.7 3.7 3.9; 48^3
     // (216) 1.4 1.8 2.2 2.4 against 3.7 3.9 3.8 4.0; 64^3 (512) 2.2 2.9 3.6 3.9
     // against 4.0 4.0 4.0 4.2; 80^3 (1000) 3.7 5.3 6.5 7.2 against 3.8 4.3 4.4
-    // 4.5; the porosity (0.15, 0.3, 0.5 at 64^3) hardly matters.
+    // 4.5.  With the porosity a thread's slots grow from one to three: 64^3, 0.3 /
+    // 0.6 / 1: one component 2.2 / 2.4 / 2.6 against 3.6 / 3.6 / 3.7, two with
+    // velocity 2.9 / 3.4 / 4.0 against 3.7 / 4.0 / 4.4, three 3.7 / 4.4 / 5.3
+    // against 4.1 / 4.4 / 4.9: the same or behind only for three with velocity
+    // at 0.6 and more.
     constexpr uint64_t kMost = 512;
     constexpr int e = nmr::kBlockEdge;
     const uint64_t nx = (b->nx + e - 1) / e, ny = (b->ny + e - 1) / e, nz = (b->nz + e - 1) / e;
